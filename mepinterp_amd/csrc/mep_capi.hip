@@ -586,9 +586,10 @@ static SepFT sep_args(mep_ctx* c) {
 }
 
 // mp (optional): the k-block is k0 .. k0+nb-1 of that Monkhorst-Pack mesh,
-// prepared by sep_prepare -> separable Fourier sums instead of the GEMM
+// prepared by sep_prepare -> separable Fourier sums instead of the GEMM.
+// ql: see launch_eigh
 static int interp_block(mep_ctx* c, int64_t nb, bool velo, int prec = MEP_PREC_FP64,
-                        const int32_t* mp = nullptr, int64_t k0 = 0) {
+                        const int32_t* mp = nullptr, int64_t k0 = 0, bool ql = false) {
   const bool sep = mp && c->sep && mp[0] == c->sep_mesh[0] && mp[1] == c->sep_mesh[1] &&
                    mp[2] == c->sep_mesh[2];
   const int64_t n = c->n;
@@ -650,10 +651,10 @@ static int interp_block(mep_ctx* c, int64_t nb, bool velo, int prec = MEP_PREC_F
   timed(c, K_EIGH, [&] {
     if (n > 32)
       launch_eigh_wide(c->st, (int)n, nb, c->dHk, c->ncols, c->packed, g, c->dE, c->dU, c->dinfo,
-                       c->dscr, c->var_eigh);
+                       c->dscr, c->var_eigh, ql);
     else
       launch_eigh(c->st, (int)n, nb, c->dHk, c->ncols, c->packed, g, c->dE, c->dU, c->dinfo,
-                  c->dscr, c->var_eigh);
+                  c->dscr, c->var_eigh, ql);
   });
   if (velo)
     timed(c, K_VELO, [&] {
@@ -994,7 +995,7 @@ static int run_block(mep_ctx* c, BandSetup& bs, int64_t k0, int64_t nb, const in
   const bool fuse = p->precision == MEP_PREC_FP64 && !bs.ext && c->packed && !c->tb &&
                     (c->flags & MEP_F_GAUGE_TRAFO) && !(c->flags & MEP_F_SEPARATE_VELO) &&
                     bandsum_can_fuse(bs.b);
-  CHK(interp_block(c, nb, !fuse, p->precision, mp, k0));
+  CHK(interp_block(c, nb, !fuse, p->precision, mp, k0, bs.ext && c->pos));
   CHK(band_block(c, bs, nb, weights ? c->dw : nullptr, fuse));
   return MEP_OK;
 }

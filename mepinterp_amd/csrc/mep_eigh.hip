@@ -14,12 +14,13 @@
 //      reflectors are stored in U's slot of the k-point, the diagonal phases
 //      P that make the subdiagonal real (T = P T_r P^H), d, e and tau in a
 //      side record.
-//   eigh_ql (one LANE per k-point, 64 k-points per wavefront): the implicit
-//      QL recurrence on T_r (EISPACK tql2 method).  A first pass with d, e in
-//      registers (eigh_ql_reg) gives the ascending eigenvalues and a
-//      separation verdict; only k-points with close eigenvalues run the
-//      second pass, which appends every sweep's Givens rotations (c_i, s_i)
-//      to a per-k record in HBM.
+//   eigh_sturm (one LANE per eigenvalue): the ascending eigenvalues of T_r as
+//      zeros of det(T_r - x) isolated by Sturm counts, and a separation
+//      verdict; only k-points with close eigenvalues run eigh_ql (one lane per
+//      k-point: the implicit QL recurrence, EISPACK tql2 method), which
+//      appends every sweep's Givens rotations (c_i, s_i) to a per-k record in
+//      HBM.  (The FP32 path, and FP64 where the caller asks for it, take
+//      the eigenvalues from QL as well.)
 //   eigh_vec (a team per k): the vectors of the real tridiagonal, directly
 //      from twisted factorizations for separated k-points or by replaying
 //      the rotations on Z (LDS, lane r <-> row r), then U = Q P Z: lane j
@@ -29,8 +30,8 @@
 //   largest-modulus component is made real and positive.
 // 32 < n <= 128: Householder with the matrix in one wavefront's LDS, a
 // workgroup's LDS or a workgroup's registers (eigh_house_lds / _wide /
-// _rows, MEP_VAR_EIGH), the QL passes (registers up to 48 bands, else LDS
-// columns), the tridiagonal vectors (eigh_replay_wide) and the blocked
+// _rows, MEP_VAR_EIGH), the eigenvalues (eigh_sturm_wide) and the rotations of
+// the listed k-points, the tridiagonal vectors (eigh_replay_wide) and the blocked
 // compact-WY back-transformation on FP64 MFMA (eigh_back_mfma).
 #include "mep_common.hpp"
 #include "mep_kernels.hpp"
@@ -712,55 +713,31 @@ __device__ __attribute__((always_inline)) inline void ql_one(int n, int64_t k, R
   sdw[5 * n] = (R)pos;
 }
 
-// One lane per k-point: implicit QL on the real tridiagonal (d, e) held in
-// LDS columns.  Every Givens rotation G(i, i+1; c, s) of every sweep is
-// appended, in application order, to the k-point's flat stream
-// rot[k][q] = (c, s), col[k][q] = i; the count goes to the side record.
-// Ascending eigenvalues go to E, each band's rank to the side record.
-// mode 0: every k-point records its rotations; mode 1: eigenvalues and the
-// separation verdict only; mode 2: the k-points with verdict -2 record.
+// The listed k-points (verdict -2), one lane each: implicit QL on the real
+// tridiagonal (d, e) held in LDS columns.  Every Givens rotation
+// G(i, i+1; c, s) of every sweep is appended, in application order, to the
+// k-point's flat stream rot[k][q] = (c, s), col[k][q] = i; the count goes to
+// the side record.  Ascending eigenvalues go to E, each band's rank to the
+// side record.
 template <int NMAX, class R>
-// mode 1: every k-point, eigenvalues and the separation verdict; the
-// k-points that need rotation records (count slot -2) are appended to
-// list[] (order immaterial: each is solved on its own).  mode 2: the listed
-// k-points again, recording the rotations.
-__global__ __launch_bounds__(64) void eigh_ql_kernel(int n, int64_t nk,
-                                                     R* __restrict__ side,
+__global__ __launch_bounds__(64) void eigh_ql_kernel(int n, R* __restrict__ side,
                                                      R* __restrict__ rot,
                                                      uint8_t* __restrict__ rcol,
                                                      double* __restrict__ E,
-                                                     int* __restrict__ info, int mode,
-                                                     int* __restrict__ list,
-                                                     int* __restrict__ count) {
+                                                     int* __restrict__ info,
+                                                     const int* __restrict__ list,
+                                                     const int* __restrict__ count) {
   __shared__ R ds[NMAX * 64], es[NMAX * 64];
   const int lane = threadIdx.x;
-  if (mode == 2) {
-    const int64_t cnt = *count;
-    for (int64_t i = (int64_t)blockIdx.x * 64 + lane; i < cnt; i += (int64_t)gridDim.x * 64)
-      ql_one<64, R, NMAX>(n, list[i], ds + lane, es + lane, side, rot, rcol, E, info, true);
-    return;
-  }
-  for (int64_t kb = (int64_t)blockIdx.x * 64; kb < nk; kb += (int64_t)gridDim.x * 64) {
-    const int64_t k = kb + lane;
-    bool again = false;
-    if (k < nk) {
-      ql_one<64, R, NMAX>(n, k, ds + lane, es + lane, side, rot, rcol, E, info, false);
-      again = side[k * side_len(n) + 5 * n] == R(-2);
-    }
-    const unsigned long long m = __ballot(again);
-    if (m) {
-      const int leader = __ffsll((long long)m) - 1;
-      int base = 0;
-      if (lane == leader) base = atomicAdd(count, __popcll(m));
-      base = __shfl(base, leader, 64);
-      if (again) list[base + __popcll(m & ((1ull << lane) - 1))] = (int)k;
-    }
-  }
+  const int64_t cnt = *count;
+  for (int64_t i = (int64_t)blockIdx.x * 64 + lane; i < cnt; i += (int64_t)gridDim.x * 64)
+    ql_one<64, R, NMAX>(n, list[i], ds + lane, es + lane, side, rot, rcol, E, info);
 }
 
-// Pass 1 of the QL stage (eigenvalues and the separation verdict) with d and
-// e in registers: one lane per k-point, NMAX <= 32, every array index a
-// compile-time constant, no LDS.  The active block always starts at index
+// Eigenvalues and the separation verdict by QL with d and e in registers (the
+// FP32 path, and FP64 for the sums with unbroadened poles, see launch_eigh):
+// one lane per k-point, NMAX <= 32, every array index a compile-time constant,
+// no LDS.  The k-points with verdict -2 are listed for eigh_ql.  The active block always starts at index
 // 0: when e[0] is negligible, d[0] is an eigenvalue and both arrays rotate
 // down by one (d[0] moves to the end), so after NMAX deflations d[j] holds
 // the j-th eigenvalue found, where ql_one's LDS column holds it.  Entries
@@ -903,46 +880,437 @@ __global__ __launch_bounds__(64) void eigh_ql_reg_kernel(int n, int64_t nk,
   }
 }
 
+// ---------------------------------------------------------------------------
+// Eigenvalues of the real tridiagonal, one LANE per eigenvalue (FP64).
+//
+// Lane j finds the j-th eigenvalue (ascending) as the zero of
+// p(x) = det(T - x) that the Sturm count isolates: the leading minors
+//   p_i = (d_i - x) p_{i-1} - e_{i-1}^2 p_{i-2}
+// cost one dependent fma a step (e^2 p_{i-2} is ready a step earlier), their
+// sign changes count the eigenvalues below x, and the last one is the
+// function whose zero is sought, so one recurrence serves both.  T is scaled
+// by a power of two to a Gershgorin bound in [1/2, 1).  e^2 is raised to at
+// least 1e-36 (a change of e far below the rounding of T), so sixteen steps
+// shrink a pair (p_{i-1}, p_i) to 1e-288 at the least; after every sixteenth
+// step a power of two is divided out and kept apart.  The computed minors are
+// those of a T whose entries differ by about one rounding each.
+//
+//   1. every lane evaluates one point of an even grid over the bound, and
+//      takes its bracket from the counts by binary search;
+//   2. a bracket that holds more eigenvalues than its own is halved;
+//   3. one that holds its own alone shrinks by inverse quadratic
+//      interpolation inside the bracket (Chandrupatla's rule; halving where
+//      that rule rejects it, or after 24 evaluations), and ends at a width of
+//      one rounding of the bound: no eigenvalue is accepted without its
+//      bracket.
+// 13 to 16 evaluations for the models tried (n = 8 ... 96), against the
+// implicit QL sweeps (one lane per k-point, about 1.7 n sweeps of n dependent
+// rotations of about 20 operations): the chain of a k-point is 13 n fma
+// instead of 1.7 n^2 rotations, and n lanes share it.
+//
+// Separation verdict as in ql_one.  A k-point with two eigenvalues that share
+// a bracket below half the separation limit is given up at once with verdict
+// -2 (the listed k-points are solved again by ql_one, which writes their E).
+// A record that is not finite is left to ql_one as well, which refuses it
+// unless the infinities stand alone.
+// ---------------------------------------------------------------------------
+struct SturmPoint {
+  double f;  // p(x) = f 2^e
+  int e, cnt;
+};
+
+// Bracket search of one lane.  a: the last point, b: the other end, c: the
+// point dropped last; values relative to 2^eref of the lane.
+struct SturmLane {
+  double a, b, c, fa, fb, fc;
+  int eref;
+  int ca, cb;      // counts at a and b
+  int other;       // eigenvalues of the bracket beside the lane's own
+  bool a_lo;       // a is the lower end
+  bool has_c, done;
+  static constexpr double TOL = 2.220446049250313e-16;  // final width (scaled)
+
+  __device__ inline void start(int j, double lo, double hi, const SturmPoint& pl,
+                               const SturmPoint& ph) {
+    a = lo;
+    b = hi;
+    eref = pl.e;
+    fa = pl.f;
+    fb = value(ph);
+    c = fc = 0.0;
+    ca = pl.cnt;
+    cb = ph.cnt;
+    other = cb - ca - 1;
+    a_lo = true;
+    has_c = false;
+  }
+  __device__ inline double value(const SturmPoint& s) const {
+    const int e = s.e - eref;  // far apart: zero or a huge value, and halving
+    return ldexp(s.f, e > 300 ? 300 : e);
+  }
+  __device__ inline double next(int it) const {
+    const double ba = b - a, half = fma(0.5, ba, a);
+    const double d1 = fb - fa;
+    double num = -fa, den = d1;  // the secant of the bracket, for its first step
+    bool ok = other == 0 && it < 24;
+    if (has_c) {
+      // 0 < xi < 1 and phi = d1 / d2 with phi^2 < xi, (1 - phi)^2 < 1 - xi
+      const double d2 = fb - fc, d3 = fc - fa;
+      const double A = fabs(ba), C = fabs(c - b), q = d2 * d2, d12 = d2 - d1;
+      ok = ok && C > A && d1 * d1 * C < A * q && d12 * d12 * C < (C - A) * q;
+      num = fa * (fc * ba * d3 - (c - a) * fb * d1);
+      den = (d1 * d2) * (d3 * ba);
+    }
+    double r = __builtin_amdgcn_rcp(den);
+    r = fma(r, fma(-den, r, 1.0), r);
+    const double t = num * r, g = 0.375 * TOL;
+    ok = ok && t > 0.0 && t < 1.0;
+    const double x = fma(t, ba, a), mn = fmin(a, b) + g, mx = fmax(a, b) - g;
+    return ok ? fmin(fmax(x, mn), mx) : half;
+  }
+  __device__ inline void update(int j, double x, const SturmPoint& s) {
+    const bool left = s.cnt <= j, same = left == a_lo;
+    c = same ? a : b;
+    fc = same ? fa : fb;
+    has_c = other == 0;
+    b = same ? b : a;
+    fb = same ? fb : fa;
+    cb = same ? cb : ca;
+    a = x;
+    fa = value(s);
+    ca = s.cnt;
+    a_lo = left;
+    other = abs(cb - ca) - 1;
+  }
+  __device__ inline double width() const { return fabs(b - a); }
+  // both ends were evaluated (the ends of the bound carry the counts -1, n + 1)
+  __device__ inline bool inside(int n) const {
+    return min(ca, cb) >= 0 && max(ca, cb) <= n;
+  }
+};
+
+// One step of the recurrence; the sign of the new minor is shifted into sg.
+__device__ inline void sturm_step(double dx, double e2, double& p0, double& p1, unsigned& sg) {
+  const double t = fma(dx, p1, -(e2 * p0));
+  sg = __builtin_amdgcn_alignbit(sg, (unsigned)__double2hiint(t), 31);
+  p0 = p1;
+  p1 = t;
+}
+__device__ inline void sturm_rescale(double& p0, double& p1, int& ex) {
+  const int e = __builtin_amdgcn_frexp_exp(fmax(fabs(p0), fabs(p1)));
+  p0 = ldexp(p0, -e);
+  p1 = ldexp(p1, -e);
+  ex += e;
+}
+
+// scale exponent of a record from its Gershgorin bound t (t > 0, finite)
+__device__ inline int sturm_exp(double t) { return __builtin_amdgcn_frexp_exp(t); }
+
+// separation limit of the verdict (FP64), and the width below which two
+// eigenvalues of one bracket are surely closer: half of it times a lower
+// bound of the largest modulus
+constexpr double STURM_SEP = 1e-5;
+
+// n <= 32: teams of NMAX lanes, T in LDS as pairs (d_i, e_{i-1}^2) that a
+// team reads together (one 16-byte broadcast a step); steps n .. of the last
+// block of eight are padding (d = 2, e = 0), which changes no sign.
+// Bound by FP64 issue where there are many k-points (n = 32, 262,144 k-points:
+// 0.86 ms; QL with one lane per k-point and T in registers 0.93 ms) and by the
+// chain where there are few (n = 24, 401 k-points: 16 us, QL 240 us).  With T
+// in every lane's registers: 1.11 ms and 14 us, so the LDS form serves both.
+template <int NMAX>
+__global__ __launch_bounds__(64) void eigh_sturm_kernel(
+    int n, int64_t nk, const double* __restrict__ side, double* __restrict__ side_out,
+    double* __restrict__ E, int* __restrict__ info, int* __restrict__ list,
+    int* __restrict__ count) {
+  constexpr int TEAMS = 64 / NMAX;
+  __shared__ mep_d2 Ts[TEAMS][NMAX + 1];
+  const int lane = threadIdx.x, j = lane % NMAX, base = lane - j;
+  const mep_d2* T = Ts[lane / NMAX];
+  for (int64_t kb = (int64_t)blockIdx.x * TEAMS; kb < nk; kb += (int64_t)gridDim.x * TEAMS) {
+    const int64_t k = kb + lane / NMAX;
+    const bool valid = k < nk;
+    const double* sd = side + (valid ? k : (int64_t)0) * side_len(n);
+    const double dj = j < n ? sd[j] : 0.0, ej = j + 1 < n ? sd[n + j] : 0.0;
+    const double em = (j > 0 && j < n) ? sd[n + j - 1] : 0.0;
+    const double rj = fabs(ej) + fabs(em);
+    double lo0 = j < n ? dj - rj : 1e308, hi0 = j < n ? dj + rj : -1e308;
+    double tot = fabs(dj) + fabs(ej), mx = fmax(fabs(dj), fabs(ej));  // |T| is at least mx
+#pragma unroll
+    for (int o = NMAX / 2; o > 0; o >>= 1) {
+      lo0 = fmin(lo0, __shfl_xor(lo0, o, 64));
+      hi0 = fmax(hi0, __shfl_xor(hi0, o, 64));
+      tot += __shfl_xor(tot, o, 64);
+      mx = fmax(mx, __shfl_xor(mx, o, 64));
+    }
+    const double tb = fmax(fabs(lo0), fabs(hi0));
+    const bool bad = !(tot < 1e308);  // also NaN
+    const int sx = bad || tb == 0.0 ? 0 : sturm_exp(tb);
+    {
+      const double es = ldexp(em, -sx);
+      mep_d2 v;
+      v.x = j < n ? ldexp(dj, -sx) : 2.0;
+      v.y = (j > 0 && j < n) ? fmax(es * es, 1e-36) : 0.0;
+      Ts[lane / NMAX][j] = v;
+    }
+    lo0 = ldexp(lo0, -sx) - 4e-16;
+    hi0 = ldexp(hi0, -sx) + 4e-16;
+    const double wclose = 0.5 * STURM_SEP * ldexp(mx, -sx);
+    __syncthreads();
+    auto eval = [&](double x) {
+      double p0 = 0.0, p1 = 1.0;
+      unsigned sg = 0;  // the signs of all n <= 32 minors, the first one's on top
+      int ex = 0;
+#pragma unroll
+      for (int b = 0; b < NMAX; b += 8) {
+        if (b < n) {  // uniform
+#pragma unroll
+          for (int i = b; i < b + 8; ++i) sturm_step(T[i].x - x, T[i].y, p0, p1, sg);
+          if (b == 8 && n > 16) sturm_rescale(p0, p1, ex);
+        }
+      }
+      return SturmPoint{p1, ex, (int)__popc(sg ^ (sg >> 1))};
+    };
+    SturmLane L;
+    {
+      const double step = (hi0 - lo0) / (double)(n + 1);
+      const SturmPoint g = eval(lo0 + (double)(j + 1) * step);
+      // the first grid point of the team with more than j eigenvalues below
+      int a = 0, b = n;
+#pragma unroll
+      for (int s = NMAX; s > 0; s >>= 1) {
+        const int mid = (a + b) >> 1;
+        const int c = __shfl(g.cnt, base + (mid < n ? mid : 0), 64);
+        if (a < b) {
+          if (c <= j) a = mid + 1;
+          else b = mid;
+        }
+      }
+      const int il = a > 0 ? a - 1 : 0, ih = a < n ? a : n - 1;
+      SturmPoint pl{__shfl(g.f, base + il, 64), __shfl(g.e, base + il, 64),
+                    __shfl(g.cnt, base + il, 64)};
+      SturmPoint ph{__shfl(g.f, base + ih, 64), __shfl(g.e, base + ih, 64),
+                    __shfl(g.cnt, base + ih, 64)};
+      double lo = lo0 + (double)(il + 1) * step, hi = lo0 + (double)(ih + 1) * step;
+      if (a == 0) { lo = lo0; pl = SturmPoint{0.0, ph.e, -1}; }  // no value there: halving
+      if (a == n) { hi = hi0; ph = SturmPoint{0.0, pl.e, n + 1}; }
+      L.start(j, lo, hi, pl, ph);
+      L.done = !valid || bad || j >= n || tb == 0.0;
+    }
+    bool close = false;
+    for (int it = 0; it < 90; ++it) {
+      // two eigenvalues in a bracket that is too narrow: the team is listed
+      const bool c = !L.done && L.other > 0 && L.inside(n) && L.width() < wclose;
+      const unsigned long long cm = __ballot(c);
+      if (cm) {
+        const unsigned long long tm = (NMAX == 64 ? ~0ull : ((1ull << (NMAX & 63)) - 1)) << base;
+        if (cm & tm) {
+          close = true;
+          L.done = true;
+        }
+      }
+      if (!__any(!L.done)) break;
+      const double x = L.done ? L.a : L.next(it);
+      const SturmPoint s = eval(x);
+      if (!L.done) {
+        L.update(j, x, s);
+        L.done = L.width() <= SturmLane::TOL;
+      }
+    }
+    double ev = tb == 0.0 ? 0.0 : ldexp(0.5 * (L.a + L.b), sx);
+    if (n == 1) ev = sd[0];
+    // the bracket of every lane closed, or the team is listed
+    if (valid && j < n && !L.done) atomicOr(info, 1);
+    // gap to the next eigenvalue and the largest modulus of the team
+    const double nx = __shfl(ev, base + (j + 1 < n ? j + 1 : j), 64);
+    double gap = j + 1 < n ? nx - ev : 1e30, big = j < n ? fabs(ev) : 0.0;
+#pragma unroll
+    for (int o = NMAX / 2; o > 0; o >>= 1) {
+      gap = fmin(gap, __shfl_xor(gap, o, 64));
+      big = fmax(big, __shfl_xor(big, o, 64));
+    }
+    const bool again = valid && (close || bad || !(gap >= STURM_SEP * big));
+    __syncthreads();  // T is rewritten by the next k-points
+    if (valid && j < n) E[k * n + j] = ev;
+    if (valid && j == 0) side_out[k * side_len(n) + 5 * n] = again ? -2.0 : -1.0;
+    const unsigned long long m = __ballot(again && j == 0);
+    if (m) {
+      const int leader = __ffsll((long long)m) - 1;
+      int at = 0;
+      if (lane == leader) at = atomicAdd(count, __popcll(m));
+      at = __shfl(at, leader, 64);
+      if (again && j == 0) list[at + __popcll(m & ((1ull << lane) - 1))] = (int)k;
+    }
+  }
+}
+
+// The same for 32 < n <= 128: one workgroup of ceil(n / 64) wavefronts per
+// k-point.  n = 96, 2,744 k-points: 107 us (QL in LDS columns 5.8 ms); n = 44,
+// 9,261 k-points: 93 us (QL in registers 820 us).
+template <int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void eigh_sturm_wide_kernel(
+    int n, int64_t nk, const double* __restrict__ side, double* __restrict__ side_out,
+    double* __restrict__ E, int* __restrict__ info, int* __restrict__ list,
+    int* __restrict__ count) {
+  constexpr int NM = 64 * WAVES;
+  __shared__ mep_d2 T[NM];
+  __shared__ double gf[NM], red[4][WAVES];
+  __shared__ int gc[NM], ge[NM], flag;
+  const int j = threadIdx.x, w = j >> 6;
+  for (int64_t k = blockIdx.x; k < nk; k += gridDim.x) {
+    const double* sd = side + k * side_len(n);
+    const double di = j < n ? sd[j] : 0.0, ei = j + 1 < n ? sd[n + j] : 0.0;
+    const double em = (j > 0 && j < n) ? sd[n + j - 1] : 0.0;
+    {
+      const double r = fabs(ei) + fabs(em);
+      double lo = j < n ? di - r : 1e308, hi = j < n ? di + r : -1e308;
+      double tot = fabs(di) + fabs(ei), mx = fmax(fabs(di), fabs(ei));
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) {
+        lo = fmin(lo, __shfl_xor(lo, o, 64));
+        hi = fmax(hi, __shfl_xor(hi, o, 64));
+        tot += __shfl_xor(tot, o, 64);
+        mx = fmax(mx, __shfl_xor(mx, o, 64));
+      }
+      if ((j & 63) == 0) {
+        red[0][w] = lo;
+        red[1][w] = hi;
+        red[2][w] = tot;
+        red[3][w] = mx;
+      }
+      if (j == 0) flag = 0;
+    }
+    __syncthreads();
+    double lo0 = red[0][0], hi0 = red[1][0], tot = red[2][0], mx = red[3][0];
+#pragma unroll
+    for (int v = 1; v < WAVES; ++v) {
+      lo0 = fmin(lo0, red[0][v]);
+      hi0 = fmax(hi0, red[1][v]);
+      tot += red[2][v];
+      mx = fmax(mx, red[3][v]);
+    }
+    const double tb = fmax(fabs(lo0), fabs(hi0));
+    const bool bad = !(tot < 1e308);
+    const int sx = bad || tb == 0.0 ? 0 : sturm_exp(tb);
+    {
+      const double es = ldexp(em, -sx);
+      mep_d2 v;
+      v.x = j < n ? ldexp(di, -sx) : 2.0;
+      v.y = (j > 0 && j < n) ? fmax(es * es, 1e-36) : 0.0;
+      T[j] = v;
+    }
+    lo0 = ldexp(lo0, -sx) - 4e-16;
+    hi0 = ldexp(hi0, -sx) + 4e-16;
+    const double wclose = 0.5 * STURM_SEP * ldexp(mx, -sx);
+    __syncthreads();
+    auto eval = [&](double x) {
+      double p0 = 0.0, p1 = 1.0;
+      unsigned sg = 0;
+      int ex = 0, neg = 0;
+      for (int b = 0; b < n; b += 16) {
+#pragma unroll
+        for (int h = 0; h < 16; h += 8)
+          if (b + h < n) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) sturm_step(T[b + h + i].x - x, T[b + h + i].y, p0, p1, sg);
+            neg += (int)__popc((sg ^ (sg >> 1)) & 0xffu);
+          }
+        sturm_rescale(p0, p1, ex);
+      }
+      return SturmPoint{p1, ex, neg};
+    };
+    SturmLane L;
+    {
+      const double step = (hi0 - lo0) / (double)(n + 1);
+      const SturmPoint g = eval(lo0 + (double)(j + 1) * step);
+      gc[j] = g.cnt;
+      gf[j] = g.f;
+      ge[j] = g.e;
+      __syncthreads();
+      int a = 0, b = n;
+      while (a < b) {
+        const int mid = (a + b) >> 1;
+        if (gc[mid] <= j) a = mid + 1;
+        else b = mid;
+      }
+      const int il = a > 0 ? a - 1 : 0, ih = a < n ? a : n - 1;
+      SturmPoint pl{gf[il], ge[il], gc[il]}, ph{gf[ih], ge[ih], gc[ih]};
+      double lo = lo0 + (double)(il + 1) * step, hi = lo0 + (double)(ih + 1) * step;
+      if (a == 0) { lo = lo0; pl = SturmPoint{0.0, ph.e, -1}; }  // no value there: halving
+      if (a == n) { hi = hi0; ph = SturmPoint{0.0, pl.e, n + 1}; }
+      L.start(j, lo, hi, pl, ph);
+      L.done = bad || j >= n || tb == 0.0;
+    }
+    __syncthreads();  // gf is reused for the eigenvalues
+    bool close = false;
+    for (int it = 0; it < 90; ++it) {
+      const bool c = !L.done && L.other > 0 && L.inside(n) && L.width() < wclose;
+      if (__any(c)) {
+        close = true;
+        break;
+      }
+      if (!__any(!L.done)) break;
+      const double x = L.done ? L.a : L.next(it);
+      const SturmPoint s = eval(x);
+      if (!L.done) {
+        L.update(j, x, s);
+        L.done = L.width() <= SturmLane::TOL;
+      }
+    }
+    if (close) L.done = true;
+    const double ev = tb == 0.0 ? 0.0 : ldexp(0.5 * (L.a + L.b), sx);
+    if (j < n && !L.done) atomicOr(info, 1);
+    gf[j] = ev;
+    if (close && (j & 63) == 0) flag = 1;
+    __syncthreads();
+    double gap = j + 1 < n ? gf[j + 1] - ev : 1e30, big = j < n ? fabs(ev) : 0.0;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      gap = fmin(gap, __shfl_xor(gap, o, 64));
+      big = fmax(big, __shfl_xor(big, o, 64));
+    }
+    if ((j & 63) == 0) {
+      red[0][w] = gap;
+      red[1][w] = big;
+    }
+    if (j < n) E[k * n + j] = ev;
+    __syncthreads();
+    if (j == 0) {
+#pragma unroll
+      for (int v = 1; v < WAVES; ++v) {
+        gap = fmin(gap, red[0][v]);
+        big = fmax(big, red[1][v]);
+      }
+      const bool again = flag || bad || !(gap >= STURM_SEP * big);
+      side_out[k * side_len(n) + 5 * n] = again ? -2.0 : -1.0;
+      if (again) list[atomicAdd(count, 1)] = (int)k;
+    }
+    __syncthreads();  // red, flag and T are rewritten by the next k-point
+  }
+}
+
 __global__ void zero_count_kernel(int* count) { *count = 0; }
 
-// the same for 32 < n <= 128: 32 lanes per workgroup, d and e in dynamic LDS
-// (n x 32 each); modes as eigh_ql_kernel (1: eigenvalues and the separation
-// verdict, listing the k-points that need rotation records; 2: the listed
-// k-points, recording)
-template <class R>
+// QL for 32 < n <= 128: 32 lanes per workgroup, d and e in dynamic LDS (n x 32
+// each).  rec: the listed k-points, recording; otherwise every k-point's
+// eigenvalues and verdict, listing those with -2.
 __global__ __launch_bounds__(32) void eigh_ql_wide_kernel(int n, int64_t nk,
-                                                          R* __restrict__ side,
-                                                          R* __restrict__ rot,
+                                                          double* __restrict__ side,
+                                                          double* __restrict__ rot,
                                                           uint8_t* __restrict__ rcol,
                                                           double* __restrict__ E,
-                                                          int* __restrict__ info, int mode,
+                                                          int* __restrict__ info, bool rec,
                                                           int* __restrict__ list,
                                                           int* __restrict__ count) {
   extern __shared__ double ql_smem[];
-  R* ds = reinterpret_cast<R*>(ql_smem);
-  R* es = ds + (int64_t)n * 32;
+  double* ds = ql_smem;
+  double* es = ds + (int64_t)n * 32;
   const int lane = threadIdx.x;
-  if (mode == 2) {
-    const int64_t cnt = *count;
-    for (int64_t i = (int64_t)blockIdx.x * 32 + lane; i < cnt; i += (int64_t)gridDim.x * 32)
-      ql_one<32, R>(n, list[i], ds + lane, es + lane, side, rot, rcol, E, info, true);
-    return;
-  }
-  for (int64_t kb = (int64_t)blockIdx.x * 32; kb < nk; kb += (int64_t)gridDim.x * 32) {
-    const int64_t k = kb + lane;
-    bool again = false;
-    if (k < nk) {
-      ql_one<32, R>(n, k, ds + lane, es + lane, side, rot, rcol, E, info, false);
-      again = side[k * side_len(n) + 5 * n] == R(-2);
-    }
-    const unsigned long long m = __ballot(again);
-    if (m) {
-      const int leader = __ffsll((long long)m) - 1;
-      int base = 0;
-      if (lane == leader) base = atomicAdd(count, __popcll(m));
-      base = __shfl(base, leader, 64);
-      if (again) list[base + __popcll(m & ((1ull << lane) - 1))] = (int)k;
-    }
+  const int64_t num = rec ? (int64_t)*count : nk;
+  for (int64_t i = (int64_t)blockIdx.x * 32 + lane; i < num; i += (int64_t)gridDim.x * 32) {
+    const int64_t k = rec ? list[i] : i;
+    ql_one<32, double>(n, k, ds + lane, es + lane, side, rot, rcol, E, info, rec);
+    if (!rec && side[k * side_len(n) + 5 * n] == -2.0) list[atomicAdd(count, 1)] = (int)k;
   }
 }
 
@@ -2189,7 +2557,7 @@ size_t eigh_back_mfma_lds(int n) {
 static size_t eigh_list_offset(int n, int64_t nk);
 
 void launch_eigh_wide(hipStream_t s, int n, int64_t nk, const zd* Hk, int64_t strideHk, int packed,
-                      const KGeom& g, double* E, zd* U, int* info, double* scratch, int house) {
+                      const KGeom& g, double* E, zd* U, int* info, double* scratch, int house, bool ql) {
   double* side = scratch;
   double* rot = side + nk * side_len(n);
   uint8_t* rcol = reinterpret_cast<uint8_t*>(rot + nk * 2 * rot_cap(n));
@@ -2199,7 +2567,7 @@ void launch_eigh_wide(hipStream_t s, int n, int64_t nk, const zd* Hk, int64_t st
                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lh);
   (void)hipFuncSetAttribute((const void*)eigh_replay_wide_kernel,
                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lr);
-  (void)hipFuncSetAttribute((const void*)eigh_ql_wide_kernel<double>,
+  (void)hipFuncSetAttribute((const void*)eigh_ql_wide_kernel,
                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lq);
   unsigned grid = (unsigned)(nk < 4096 ? nk : 4096);
   // measured crossovers (C3 models n = 36 ... 68, C5, seeded models n = 72 ... 128):
@@ -2238,21 +2606,19 @@ void launch_eigh_wide(hipStream_t s, int n, int64_t nk, const zd* Hk, int64_t st
   int64_t qb = (nk + 31) / 32;
   unsigned qgrid = (unsigned)(qb < 65536 ? qb : 65536);
   hipLaunchKernelGGL(zero_count_kernel, dim3(1), dim3(1), 0, s, count);
-  // eigenvalues and the separation verdict: d and e in registers up to 48
-  // bands (more k-points in flight than LDS columns allow), else in LDS
-  const int64_t qb64 = (nk + 63) / 64;
-  const unsigned qgrid64 = (unsigned)(qb64 < 65536 ? qb64 : 65536);
-  if (n <= 40)
-    hipLaunchKernelGGL((eigh_ql_reg_kernel<40, double>), dim3(qgrid64), dim3(64), 0, s, n, nk, side,
-                       E, info, list, count);
-  else if (n <= 48)
-    hipLaunchKernelGGL((eigh_ql_reg_kernel<48, double>), dim3(qgrid64), dim3(64), 0, s, n, nk, side,
-                       E, info, list, count);
+  // eigenvalues and the separation verdict, then the listed k-points
+  const unsigned sgrid = (unsigned)(nk < 65536 ? nk : 65536);
+  if (ql)
+    hipLaunchKernelGGL(eigh_ql_wide_kernel, dim3(qgrid), dim3(32), lq, s, n, nk, side, rot, rcol,
+                       E, info, false, list, count);
+  else if (n <= 64)
+    hipLaunchKernelGGL(eigh_sturm_wide_kernel<1>, dim3(sgrid), dim3(64), 0, s, n, nk, side, side, E,
+                       info, list, count);
   else
-    hipLaunchKernelGGL(eigh_ql_wide_kernel<double>, dim3(qgrid), dim3(32), lq, s, n, nk, side, rot,
-                       rcol, E, info, 1, list, count);
-  hipLaunchKernelGGL(eigh_ql_wide_kernel<double>, dim3(qgrid), dim3(32), lq, s, n, nk, side, rot,
-                     rcol, E, info, 2, list, count);
+    hipLaunchKernelGGL(eigh_sturm_wide_kernel<2>, dim3(sgrid), dim3(128), 0, s, n, nk, side, side,
+                       E, info, list, count);
+  hipLaunchKernelGGL(eigh_ql_wide_kernel, dim3(qgrid), dim3(32), lq, s, n, nk, side, rot, rcol,
+                     E, info, true, list, count);
   const int rthreads = n <= 64 ? 64 : 128;
   hipLaunchKernelGGL(eigh_replay_wide_kernel, dim3(grid), dim3(rthreads), lr, s, n, nk, side, rot,
                      rcol, E);
@@ -2291,7 +2657,7 @@ size_t eigh_scratch_bytes(int n, int64_t nk) {
 template <class R>
 static void launch_eigh_t(hipStream_t s, int n, int64_t nk, const typename cplx_of<R>::type* Hk,
                           int64_t strideHk, int packed, const KGeom& g, double* E,
-                          typename cplx_of<R>::type* U, int* info, void* scratch, int house) {
+                          typename cplx_of<R>::type* U, int* info, void* scratch, int house, bool ql) {
   R* side = reinterpret_cast<R*>(scratch);
   R* rot = side + nk * side_len(n);
   uint8_t* rcol = reinterpret_cast<uint8_t*>(rot + nk * 2 * rot_cap(n));
@@ -2324,10 +2690,15 @@ static void launch_eigh_t(hipStream_t s, int n, int64_t nk, const typename cplx_
     hipLaunchKernelGGL((eigh_house_kernel<NM, R>), dim3(grid), dim3(64), 0, s, n, nk, Hk, strideHk, \
                        packed, g.kpts, g.tau, U, side);                                          \
   hipLaunchKernelGGL(zero_count_kernel, dim3(1), dim3(1), 0, s, count);                        \
-  hipLaunchKernelGGL((eigh_ql_reg_kernel<NM, R>), dim3(qgrid), dim3(64), 0, s, n, nk, side, E,  \
+  if (ql || sizeof(R) != 8) {                                                                    \
+    hipLaunchKernelGGL((eigh_ql_reg_kernel<NM, R>), dim3(qgrid), dim3(64), 0, s, n, nk, side, E, \
+                       info, list, count);                                                       \
+  } else if constexpr (sizeof(R) == 8) {                                                         \
+    hipLaunchKernelGGL(eigh_sturm_kernel<NM>, dim3(grid), dim3(64), 0, s, n, nk, side, side, E,  \
+                       info, list, count);                                                       \
+  }                                                                                              \
+  hipLaunchKernelGGL((eigh_ql_kernel<NM, R>), dim3(qgrid), dim3(64), 0, s, n, side, rot, rcol, E, \
                      info, list, count);                                                         \
-  hipLaunchKernelGGL((eigh_ql_kernel<NM, R>), dim3(qgrid), dim3(64), 0, s, n, nk, side, rot,     \
-                     rcol, E, info, 2, list, count);                                             \
   hipLaunchKernelGGL((eigh_vec_kernel<NM, R>), dim3(grid), dim3(64), 0, s, n, nk, side, rot,     \
                      rcol, E, U);
   if (n <= 8) {
@@ -2341,11 +2712,11 @@ static void launch_eigh_t(hipStream_t s, int n, int64_t nk, const typename cplx_
 }
 
 void launch_eigh(hipStream_t s, int n, int64_t nk, const zd* Hk, int64_t strideHk, int packed,
-                 const KGeom& g, double* E, zd* U, int* info, double* scratch, int house) {
-  launch_eigh_t<double>(s, n, nk, Hk, strideHk, packed, g, E, U, info, scratch, house);
+                 const KGeom& g, double* E, zd* U, int* info, double* scratch, int house, bool ql) {
+  launch_eigh_t<double>(s, n, nk, Hk, strideHk, packed, g, E, U, info, scratch, house, ql);
 }
 
 void launch_eigh_f32(hipStream_t s, int n, int64_t nk, const zf* Hk, int64_t strideHk, int packed,
                      const KGeom& g, double* E, zf* U, int* info, double* scratch) {
-  launch_eigh_t<float>(s, n, nk, Hk, strideHk, packed, g, E, U, info, scratch, 0);
+  launch_eigh_t<float>(s, n, nk, Hk, strideHk, packed, g, E, U, info, scratch, 0, true);
 }

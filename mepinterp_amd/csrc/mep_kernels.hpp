@@ -51,12 +51,19 @@ void launch_ft_gemm_f32(hipStream_t s, int M, int N, int K, const float* Pt, con
 size_t eigh_scratch_bytes(int n, int64_t nk);
 // house: FP64 Householder variant for 16 < n <= 32 (1 = one k-point per
 // wavefront, 2 = two; 0 = the default, 1)
+// ql: eigenvalues by QL (one lane per k-point) instead of Sturm brackets (one
+// lane per eigenvalue).  The optical and gyrotropic sums with a position
+// operator divide by e_m - e_n - hw and (e_m - e_n)^2 - hw without a
+// broadening: next to such a pole a last-bit change of an eigenvalue moves the
+// sum by 1e-9 and more, so those runs keep the eigenvalues they always had.
 void launch_eigh(hipStream_t s, int n, int64_t nk, const zd* Hk, int64_t strideHk, int packed,
-                 const KGeom& g, double* E, zd* U, int* info, double* scratch, int house = 0);
+                 const KGeom& g, double* E, zd* U, int* info, double* scratch, int house = 0,
+                 bool ql = false);
 // house (32 < n): 1 = one 256-thread workgroup per k-point, 2 = one wavefront
 // per k-point with the matrix in LDS (n <= 64); 0 = the default (2 for n <= 52)
 void launch_eigh_wide(hipStream_t s, int n, int64_t nk, const zd* Hk, int64_t strideHk, int packed,
-                      const KGeom& g, double* E, zd* U, int* info, double* scratch, int house = 0);
+                      const KGeom& g, double* E, zd* U, int* info, double* scratch, int house = 0,
+                      bool ql = false);
 // the same in FP32 arithmetic (FP32 H(k) and U; eigenvalues written as FP64)
 void launch_eigh_f32(hipStream_t s, int n, int64_t nk, const zf* Hk, int64_t strideHk, int packed,
                      const KGeom& g, double* E, zf* U, int* info, double* scratch);
