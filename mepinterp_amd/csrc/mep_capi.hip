@@ -587,9 +587,10 @@ static SepFT sep_args(mep_ctx* c) {
 
 // mp (optional): the k-block is k0 .. k0+nb-1 of that Monkhorst-Pack mesh,
 // prepared by sep_prepare -> separable Fourier sums instead of the GEMM.
-// ql: see launch_eigh
+// ql: see launch_eigh; want: see VeloArgs
 static int interp_block(mep_ctx* c, int64_t nb, bool velo, int prec = MEP_PREC_FP64,
-                        const int32_t* mp = nullptr, int64_t k0 = 0, bool ql = false) {
+                        const int32_t* mp = nullptr, int64_t k0 = 0, bool ql = false,
+                        int want = VELO_A | VELO_DIAG | VELO_OM) {
   const bool sep = mp && c->sep && mp[0] == c->sep_mesh[0] && mp[1] == c->sep_mesh[1] &&
                    mp[2] == c->sep_mesh[2];
   const int64_t n = c->n;
@@ -602,6 +603,7 @@ static int interp_block(mep_ctx* c, int64_t nb, bool velo, int prec = MEP_PREC_F
   va.pos_op = c->pos ? 1 : 0;
   va.textbook = (c->flags & MEP_F_TEXTBOOK) ? 1 : 0;
   va.kubo_tol = c->kubo_tol;
+  va.want = want;
   va.scratch = reinterpret_cast<zd*>(c->dscr);  // free once the eigensolve is done
   va.scratch_bytes = eigh_scratch_bytes((int)n, c->kcap);
   if (velo && c->pos && !velo_pos_scratch_ok((int)n, va.scratch_bytes))
@@ -920,7 +922,7 @@ extern "C" int mep_curv_batch(mep_ctx* c, int64_t nk, const double* kpts, double
     int64_t nb = (nk - k0 < c->kcap) ? nk - k0 : c->kcap;
     HIPCHK(hipMemcpyAsync(c->dk, kpts + 3 * k0, sizeof(double) * 3 * nb, hipMemcpyHostToDevice,
                           c->st));
-    CHK(interp_block(c, nb, true));
+    CHK(interp_block(c, nb, true, MEP_PREC_FP64, nullptr, 0, false, 0));  // V alone is read
     timed(c, K_BANDSUM, [&] {
       launch_curv(c->st, (int)c->n, nb, c->dE, c->dV, ef, T_kelvin, c->dcurv);
     });
@@ -995,7 +997,11 @@ static int run_block(mep_ctx* c, BandSetup& bs, int64_t k0, int64_t nb, const in
   const bool fuse = p->precision == MEP_PREC_FP64 && !bs.ext && c->packed && !c->tb &&
                     (c->flags & MEP_F_GAUGE_TRAFO) && !(c->flags & MEP_F_SEPARATE_VELO) &&
                     bandsum_can_fuse(bs.b);
-  CHK(interp_block(c, nb, !fuse, p->precision, mp, k0, bs.ext && c->pos));
+  // the band sums read A and Omega on the diagonal (the Chern-Simons terms and
+  // get_gyro_D), the optical and gyrotropic ones A everywhere
+  const int want = (p->jobs & (MEP_JOB_KUBO | MEP_JOB_MEP | MEP_JOB_GYRO) ? VELO_DIAG : 0) |
+                   (bs.ext ? VELO_A : 0);
+  CHK(interp_block(c, nb, !fuse, p->precision, mp, k0, bs.ext && c->pos, want));
   CHK(band_block(c, bs, nb, weights ? c->dw : nullptr, fuse));
   return MEP_OK;
 }

@@ -70,15 +70,23 @@ void launch_eigh_f32(hipStream_t s, int n, int64_t nk, const zf* Hk, int64_t str
 
 // Velocity (and, with a position operator, connection and curvature) in
 // the Hamiltonian gauge.  V is written planar per k: V[k][a][i + n j].
+// With a position operator, `want` says what beside V is read afterwards: the
+// elements of A and Omega not asked for are left as they are.
+enum : int {
+  VELO_A = 1,     // A, every element
+  VELO_DIAG = 2,  // A and Omega on the band diagonal
+  VELO_OM = 4,    // A and Omega, every element
+};
 struct VeloArgs {
   int n, nmat;
+  int want = VELO_A | VELO_DIAG | VELO_OM;
   int packed;  // upper-triangle matrices (no position operator)
   int gauge_trafo;
   int pos_op;
   int textbook;
   double kubo_tol;
   zd* scratch;  // n > 32: 3 n x n per workgroup (up to 2048 workgroups); with a
-                // position operator and n > 16: 18 n x n per workgroup
+                // position operator 18 n x n per workgroup
   size_t scratch_bytes = 0;
 };
 // the scratch holds at least one position-operator slot (or none is needed)

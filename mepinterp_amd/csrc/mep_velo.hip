@@ -1,5 +1,5 @@
 // mep_velo.hip -- velocity (and connection / curvature) in the Hamiltonian
-// gauge, one k-point per wavefront.
+// gauge.
 //
 // Replaces W_to_H_gaugeTRAFO + get_velo (wann_interp.f90:100-101, 406-658).
 // Inputs per k: the Fourier GEMM output in the Wannier gauge, stacked as
@@ -14,6 +14,7 @@
 #include "mep_common.hpp"
 #include "mep_kernels.hpp"
 #include "mep_mfma.hpp"
+#include "mep_lane.hpp"
 
 struct TBPhase {
   double kx, ky, kz;
@@ -489,202 +490,410 @@ void launch_v_layout(hipStream_t s, int n, int64_t nk, const zd* src, zd* dst, b
 }
 
 // --------------------------------------------------------------------------
-// position operator present (n <= 16): PRB 74 195118 Eqs. 21-31 with the
-// reference's evaluation order (rotate_gauge :502-550, get_gauge_covar_deriv
-// :565-617, conn_gaugeTrafo :620-633, curv_gaugeTrafo :636-658, get_velo
-// :406-444).  textbook != 0 selects the printed equations instead.
+// Position operator: PRB 74 195118 Eqs. 21-31 with the reference's evaluation
+// order (rotate_gauge :502-550, get_gauge_covar_deriv :565-617,
+// conn_gaugeTrafo :620-633, curv_gaugeTrafo :636-658, get_velo :406-444);
+// textbook != 0 selects the printed equations instead.
+//   Hb_a = U^H dH_a U,  Ab_a = Hb_a U (reference) or U^H A_a U (textbook)
+//   D_a(i,j) = Hb_a(i,j) / (E_j - E_i) where |E_j - E_i| > kubo_tol, i != j
+//   A^(H)_a = Ab_a + i D_a,  V_a = Hb_a - i (E_j - E_i) X_a off the diagonal
+//   Om^(H)_c = U^H Om_c U - [D_a, X_b] + [D_b, X_a] - i [D_a, D_b]
+// with X = A^(H) (reference) or Ab (textbook) and c = (a, b) cyclic.  With
+// Y = X + i D the commutators are four products,
+//   X_b D_a - X_a D_b + D_b Y_a - D_a Y_b.
+// What is formed is what the caller reads (VeloArgs::want).  The band sums
+// read Omega on the diagonal only, which costs no product but Om_c U: the
+// rest of it are row and column sums of elementwise products,
+//   Om^(H)_c(i,i) = sum_m conj(U(m,i)) (Om_c U)(m,i)
+//     + sum_l [X_b(i,l) D_a(l,i) - X_a(i,l) D_b(l,i)]
+//     + sum_l [D_b(i,l) Y_a(l,i) - D_a(i,l) Y_b(l,i)].
 // --------------------------------------------------------------------------
-#define PM 16
-#define PLD (PM + 1)
 
-// C = op(A) * B over the n x n leading blocks of LDS matrices (ld PLD)
-__device__ inline void lds_mm(int n, const zd* A, bool adjA, const zd* B, zd* C) {
-  for (int idx = threadIdx.x; idx < n * n; idx += 64) {
-    int i = idx % n, j = idx / n;
-    zd s = zd{0.0, 0.0};
-    for (int l = 0; l < n; ++l) {
-      zd aa = adjA ? zconj(A[l + PLD * i]) : A[i + PLD * l];
-      s = zadd(s, zmul(aa, B[l + PLD * j]));
+// The Wannier-gauge matrices of one k-point, unpacked (n^2 each), with the
+// tight-binding epilogue from per-band phases f_m = e^{2 pi i k.tau_m} and
+// centres in LDS: n sincos a k-point instead of one an element and matrix.
+struct PosLoad {
+  const zd* X;
+  const zd* f;        // null: Wannier convention
+  const double* tau;  // (3, n)
+  int n;
+  const TBPhase* tb;
+  __device__ inline zd operator()(int mat, int i, int j) const {
+    const int64_t n2 = (int64_t)n * n, o = i + (int64_t)n * j;
+    zd x = X[mat * n2 + o];
+    if (!f) return x;
+    const double dt[3] = {tau[3 * j] - tau[3 * i], tau[3 * j + 1] - tau[3 * i + 1],
+                          tau[3 * j + 2] - tau[3 * i + 2]};
+    if (mat >= 1 && mat <= 3) {
+      x = zadd(x, zmuli(zscale(X[o], tb->c(mat - 1, dt))));
+    } else if (mat >= 7) {
+      // Omega_ab with (a,b) = (1,2), (2,0), (0,1)
+      const int a = (mat - 6) % 3, b = (mat - 5) % 3;
+      x = zadd(x, zmuli(zsub(zscale(X[(4 + b) * n2 + o], tb->c(a, dt)),
+                             zscale(X[(4 + a) * n2 + o], tb->c(b, dt)))));
     }
-    C[i + PLD * j] = s;
+    return zmul(zcmul(f[i], f[j]), x);
   }
+};
+// f_m and the centres of a workgroup's k-point into LDS (threads t < n)
+__device__ inline void pos_phases(const TBPhase& tb, int n, int t, zd* f, double* tau) {
+  if (!tb.tau || t >= n) return;
+  const double* tm = tb.tau + 3 * t;
+  double sn, cs;
+  sincos(2.0 * 3.14159265358979323846 * (tb.kx * tm[0] + tb.ky * tm[1] + tb.kz * tm[2]), &sn, &cs);
+  f[t] = zd{cs, sn};
+#pragma unroll
+  for (int a = 0; a < 3; ++a) tau[3 * t + a] = tm[a];
+}
+// Omega(3,3) of one element: antisymmetric, zero diagonal in (a, b)
+__device__ inline void pos_store_om(zd* O, zd oyz, zd ozx, zd oxy) {
+  O[0] = O[1 + 3 * 1] = O[2 + 3 * 2] = zd{0, 0};
+  O[1 + 3 * 2] = oyz;
+  O[2 + 3 * 1] = zsub(zd{0, 0}, oyz);
+  O[2 + 3 * 0] = ozx;
+  O[0 + 3 * 2] = zsub(zd{0, 0}, ozx);
+  O[0 + 3 * 1] = oxy;
+  O[1 + 3 * 0] = zsub(zd{0, 0}, oxy);
 }
 
-__global__ __launch_bounds__(64) void velo_pos_kernel(int n, int64_t nk, const zd* __restrict__ Hk,
-                                                      int64_t strideHk, TBPhase tb, int gauge_trafo,
-                                                      int textbook, double kubo_tol,
-                                                      const zd* __restrict__ U,
-                                                      const double* __restrict__ E,
-                                                      zd* __restrict__ V, zd* __restrict__ Aout,
-                                                      zd* __restrict__ Omout) {
-  __shared__ zd Us[PM * PLD], T1[PM * PLD], T2[PM * PLD];
-  __shared__ zd Hb[3][PM * PLD], Ab[3][PM * PLD], Dm[3][PM * PLD], Om[3][PM * PLD];
-  __shared__ zd Abar[3][PM * PLD];
-  __shared__ double Es[PM];
-  const int t = threadIdx.x;
-  const int N = n;
-  for (int64_t k = blockIdx.x; k < nk; k += gridDim.x) {
-    const TBPhase tk = tb.at(k);
-    const zd* X = Hk + k * strideHk;
-    const int64_t NN = (int64_t)n * n;
-    for (int idx = t; idx < n * n; idx += 64) {
-      int i = idx % n, j = idx / n;
-      Us[i + PLD * j] = U[k * NN + idx];
-      for (int a = 0; a < 3; ++a) {
-        Hb[a][i + PLD * j] = load_tb(X, 0, N, i, j, 1 + a, tk);
-        Ab[a][i + PLD * j] = load_tb(X, 0, N, i, j, 4 + a, tk);
-        Om[a][i + PLD * j] = load_tb(X, 0, N, i, j, 7 + a, tk);
-      }
-    }
-    if (t < n) Es[t] = E[k * n + t];
-    __syncthreads();
-    if (gauge_trafo) {
-      for (int a = 0; a < 3; ++a) {
-        // Hbar = U^H dH U ; tmp1 = dH U
-        lds_mm(n, Hb[a], false, Us, T1);
-        __syncthreads();
-        lds_mm(n, Us, true, T1, Hb[a]);
-        __syncthreads();
-        if (textbook) {
-          lds_mm(n, Ab[a], false, Us, T2);
-          __syncthreads();
-          lds_mm(n, Us, true, T2, Ab[a]);
-        } else {
-          // stale temporary: A = (U^H (dH U)) U
-          lds_mm(n, Us, true, T1, T2);
-          __syncthreads();
-          lds_mm(n, T2, false, Us, Ab[a]);
-        }
-        __syncthreads();
-        // Omega_bar = U^H Omega U
-        lds_mm(n, Us, true, Om[a], T2);
-        __syncthreads();
-        lds_mm(n, T2, false, Us, Om[a]);
-        __syncthreads();
-      }
-      // D_a,ij = Hbar_a,ij / (E_j - E_i) for i != j and |E_j - E_i| > kubo_tol
-      for (int idx = t; idx < n * n; idx += 64) {
-        int i = idx % n, j = idx / n;
-        double de = Es[j] - Es[i];
+// n <= 32: one k-point per workgroup of NM / 16 x NM / 16 wavefronts (one for
+// n <= 16), each owning one 16 x 16 tile of every product, as
+// velo_mfma_kernel: U and three planes in LDS, three components at a time on
+// FP64 MFMA, every result kept in the accumulators' layout so that D, A^(H),
+// V and the curvature's diagonal are formed in registers.  FULL: the whole
+// Omega (three more planes, for the commutators' operands).
+// 9 products for V alone, 12 with the diagonal of Omega, 27 in all.
+// n = 24, 4,096 k-points, V and the diagonals: 400 us (VALU products on
+// global-memory operands, every output: 3,277 us); n = 8, 32,768 k-points, V
+// alone: 222 us (LDS VALU products, every output: 1,490 us).
+template <int NM, bool FULL>
+__global__ __launch_bounds__(NM == 32 ? 256 : 64, 2) void velo_pos_kernel(
+    int n, int64_t nk, const zd* __restrict__ Hk, int64_t strideHk, TBPhase tb0, int gauge_trafo,
+    int textbook, double kubo_tol, int want, const zd* __restrict__ U, const double* __restrict__ E,
+    zd* __restrict__ V, zd* __restrict__ Aout, zd* __restrict__ Omout) {
+  constexpr int LD = NM + 1, PL = NM * LD, NT = NM == 32 ? 256 : 64, TD = NM / 16;
+  __shared__ zd Us[PL], Ds[3 * PL], Xs[FULL ? 3 * PL : 1];
+  __shared__ zd fph[NM], rsum[TD][3][NM], csum[TD][3][NM];
+  __shared__ double Es[NM], taus[3 * NM];
+  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+  const int n2 = n * n;
+  const int64_t NN = n2;
+  for (int c = t; c < PL; c += NT) {
+    Us[c] = Ds[c] = Ds[PL + c] = Ds[2 * PL + c] = zd{0.0, 0.0};
+    if (FULL) Xs[c] = Xs[PL + c] = Xs[2 * PL + c] = zd{0.0, 0.0};
+  }
+  const int rt = w % TD, ct = w / TD, r0 = 16 * rt, c0 = 16 * ct;
+  const int ar = r0 + (lane & 15), bc = c0 + (lane & 15), kq = lane >> 4;
+  const bool tile = r0 < n && c0 < n;  // wave-uniform
+  typedef zd Frag[3][4];  // three components, rows r0 + kq + 4 v of column bc
+  // R_a = P_a U (P in the planes) / R_a = U^H P_a
+  auto right = [&](const zd* P, Frag R) {
+    mep_v4d p1[3] = {}, p2[3] = {}, p3[3] = {};
+    if (tile)
+#pragma unroll
+      for (int k0 = 0; k0 < NM; k0 += 4) {
+        if (k0 >= n) break;
+        const int m = k0 + kq;
+        const zd b = ldz(Us + m + LD * bc);
+        const double bs = b.re + b.im;
+#pragma unroll
         for (int a = 0; a < 3; ++a) {
-          zd dv = zd{0.0, 0.0};
-          if (i != j && fabs(de) > kubo_tol)
-            dv = zd{Hb[a][i + PLD * j].re / de, Hb[a][i + PLD * j].im / de};
-          Dm[a][i + PLD * j] = dv;
-          Abar[a][i + PLD * j] = Ab[a][i + PLD * j];
+          const zd x = ldz(P + a * PL + ar + LD * m);
+          p1[a] = __builtin_amdgcn_mfma_f64_16x16x4f64(x.re, b.re, p1[a], 0, 0, 0);
+          p2[a] = __builtin_amdgcn_mfma_f64_16x16x4f64(x.im, b.im, p2[a], 0, 0, 0);
+          p3[a] = __builtin_amdgcn_mfma_f64_16x16x4f64(x.re + x.im, bs, p3[a], 0, 0, 0);
         }
       }
-      __syncthreads();
-      // A^(H) = A + i D
-      for (int idx = t; idx < n * n; idx += 64) {
-        int i = idx % n, j = idx / n;
-        for (int a = 0; a < 3; ++a)
-          Ab[a][i + PLD * j] = zadd(Ab[a][i + PLD * j], zmuli(Dm[a][i + PLD * j]));
-      }
-      __syncthreads();
-      // Omega^(H)_ab = Om_ab - [D_a, A_b] + [D_b, A_a] - i [D_a, D_b]
-      // for (a,b) in {(1,2), (2,0), (0,1)}; A is A^(H) (reference) or Abar
-      for (int c = 0; c < 3; ++c) {
-        int a = (c == 0) ? 1 : (c == 1) ? 2 : 0;
-        int b = (c == 0) ? 2 : (c == 1) ? 0 : 1;
-        zd(*Asrc)[PM * PLD] = textbook ? Abar : Ab;
-        for (int idx = t; idx < n * n; idx += 64) {
-          int i = idx % n, j = idx / n;
-          zd s = Om[c][i + PLD * j];
-          zd c1 = zd{0, 0}, c2 = zd{0, 0}, c3 = zd{0, 0};
-          for (int l = 0; l < n; ++l) {
-            // [D_a, A_b]_ij
-            c1 = zadd(c1, zsub(zmul(Dm[a][i + PLD * l], Asrc[b][l + PLD * j]),
-                               zmul(Asrc[b][i + PLD * l], Dm[a][l + PLD * j])));
-            // [D_b, A_a]_ij
-            c2 = zadd(c2, zsub(zmul(Dm[b][i + PLD * l], Asrc[a][l + PLD * j]),
-                               zmul(Asrc[a][i + PLD * l], Dm[b][l + PLD * j])));
-            // [D_a, D_b]_ij
-            c3 = zadd(c3, zsub(zmul(Dm[a][i + PLD * l], Dm[b][l + PLD * j]),
-                               zmul(Dm[b][i + PLD * l], Dm[a][l + PLD * j])));
-          }
-          s = zsub(s, c1);
-          s = zadd(s, c2);
-          s = zsub(s, zmuli(c3));
-          T1[i + PLD * j] = s;
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) R[a][v] = zd{p1[a][v] - p2[a][v], p3[a][v] - p1[a][v] - p2[a][v]};
+  };
+  auto left = [&](const zd* P, Frag R) {
+    mep_v4d p1[3] = {}, p2[3] = {}, p3[3] = {};
+    if (tile)
+#pragma unroll
+      for (int k0 = 0; k0 < NM; k0 += 4) {
+        if (k0 >= n) break;
+        const int m = k0 + kq;
+        const zd u = ldz(Us + m + LD * ar);
+        const double us = u.re - u.im;
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+          const zd y = ldz(P + a * PL + m + LD * bc);
+          p1[a] = __builtin_amdgcn_mfma_f64_16x16x4f64(u.re, y.re, p1[a], 0, 0, 0);
+          p2[a] = __builtin_amdgcn_mfma_f64_16x16x4f64(-u.im, y.im, p2[a], 0, 0, 0);
+          p3[a] = __builtin_amdgcn_mfma_f64_16x16x4f64(us, y.re + y.im, p3[a], 0, 0, 0);
         }
-        __syncthreads();
-        for (int idx = t; idx < n * n; idx += 64) {
-          int i = idx % n, j = idx / n;
-          Om[c][i + PLD * j] = T1[i + PLD * j];
-        }
-        __syncthreads();
       }
-    }
-    // velocity
-    for (int idx = t; idx < n * n; idx += 64) {
-      int i = idx % n, j = idx / n;
-      for (int a = 0; a < 3; ++a) {
-        zd v = Hb[a][i + PLD * j];
-        if (i != j) {
-          // V_nm = H_nm - i (E_m - E_n) A_nm
-          const zd* Asel = (gauge_trafo && textbook) ? Abar[a] : Ab[a];
-          zd ce = zd{0.0, Es[j] - Es[i]};
-          v = zsub(v, zmul(ce, Asel[i + PLD * j]));
-        }
-        V[k * 3 * NN + a * NN + idx] = v;
-        Aout[k * 3 * NN + a + 3 * (int64_t)idx] = Ab[a][i + PLD * j];
-      }
-      // Omega (3,3,n,n): antisymmetric, zero diagonal in (a,b)
-      zd* O = Omout + k * 9 * NN + 9 * (int64_t)idx;
-      zd oyz = Om[0][i + PLD * j], ozx = Om[1][i + PLD * j], oxy = Om[2][i + PLD * j];
-      O[0] = zd{0, 0};
-      O[1 + 3 * 1] = zd{0, 0};
-      O[2 + 3 * 2] = zd{0, 0};
-      O[1 + 3 * 2] = oyz;
-      O[2 + 3 * 1] = zsub(zd{0, 0}, oyz);
-      O[2 + 3 * 0] = ozx;
-      O[0 + 3 * 2] = zsub(zd{0, 0}, ozx);
-      O[0 + 3 * 1] = oxy;
-      O[1 + 3 * 0] = zsub(zd{0, 0}, oxy);
-    }
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) R[a][v] = zd{p1[a][v] - p2[a][v], p3[a][v] - p1[a][v] - p2[a][v]};
+  };
+  auto store = [&](const Frag R, zd* P) {  // every reader of P has passed a barrier
+    if (tile)
+#pragma unroll
+      for (int a = 0; a < 3; ++a)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) stz(P + a * PL + r0 + kq + 4 * v + LD * bc, R[a][v]);
+  };
+  for (int64_t k = blockIdx.x; k < nk; k += gridDim.x) {
+    const TBPhase tb = tb0.at(k);
+    const PosLoad ld{Hk + k * strideHk, tb.tau ? fph : nullptr, taus, n, &tb};
+    zd* Vk = V + k * 3 * NN;
+    zd* Ak = Aout + k * 3 * NN;
+    zd* Ok = Omout + k * 9 * NN;
+    __syncthreads();  // the previous k-point's readers are done
+    pos_phases(tb, n, t, fph, taus);
+    if (t < n) Es[t] = E[k * n + t];
+    for (int idx = t; idx < n2; idx += NT) stz(Us + idx % n + LD * (idx / n), U[k * NN + idx]);
     __syncthreads();
+    // three matrices mat0 .. mat0 + 2 into the planes
+    auto stage = [&](int mat0) {
+      for (int idx = t; idx < n2; idx += NT) {
+        const int i = idx % n, j = idx / n;
+#pragma unroll
+        for (int a = 0; a < 3; ++a) stz(Ds + a * PL + i + LD * j, ld(mat0 + a, i, j));
+      }
+    };
+    if (!gauge_trafo) {
+      for (int idx = t; idx < n2; idx += NT) {
+        const int i = idx % n, j = idx / n;
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+          const zd x = ld(4 + a, i, j);
+          zd v = ld(1 + a, i, j);
+          if (i != j) v = zsub(v, zmul(zd{0.0, Es[j] - Es[i]}, x));
+          Vk[a * NN + idx] = v;
+          Ak[a + 3 * (int64_t)idx] = x;
+        }
+        pos_store_om(Ok + 9 * (int64_t)idx, ld(7, i, j), ld(8, i, j), ld(9, i, j));
+      }
+      continue;
+    }
+    Frag hb, ab, tmp;
+    stage(1);
+    __syncthreads();
+    right(Ds, tmp);  // dH U
+    __syncthreads();
+    store(tmp, Ds);
+    __syncthreads();
+    left(Ds, hb);    // Hb
+    __syncthreads();
+    if (textbook) {
+      stage(4);
+      __syncthreads();
+      right(Ds, tmp);
+      __syncthreads();
+      store(tmp, Ds);
+      __syncthreads();
+      left(Ds, ab);
+      __syncthreads();
+      store(hb, Ds);
+      __syncthreads();
+    } else {
+      store(hb, Ds);
+      __syncthreads();
+      right(Ds, ab);
+    }
+    // D, A^(H) (over ab's place in X for the reference) and V, elementwise
+    Frag dm;
+    double de[4];
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int row = r0 + kq + 4 * v;
+      const bool in = row < n && bc < n;
+      de[v] = in ? Es[bc] - Es[row] : 0.0;
+      const bool far = in && row != bc && fabs(de[v]) > kubo_tol;
+      const double rd = far ? 1.0 / de[v] : 0.0;
+#pragma unroll
+      for (int a = 0; a < 3; ++a) {
+        dm[a][v] = zscale(hb[a][v], rd);
+        const zd ah = zadd(ab[a][v], zmuli(dm[a][v]));
+        if (!textbook) ab[a][v] = ah;  // ab = X from here on
+        if (in) {
+          zd vv = hb[a][v];
+          if (row != bc) vv = zsub(vv, zmul(zd{0.0, de[v]}, ab[a][v]));
+          Vk[a * NN + row + (int64_t)n * bc] = vv;
+          if ((want & VELO_A) || ((want & VELO_DIAG) && row == bc))
+            Ak[a + 3 * ((int64_t)row + (int64_t)n * bc)] = ah;
+        }
+      }
+    }
+    if (FULL) {
+      __syncthreads();  // Hb's readers are done
+      store(dm, Ds);
+      store(ab, Xs);
+      __syncthreads();
+      Frag cm;
+      {
+        mep_v4d p1[3] = {}, p2[3] = {}, p3[3] = {};
+        auto mac = [&](int c, zd x, zd y) {
+          p1[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(x.re, y.re, p1[c], 0, 0, 0);
+          p2[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(x.im, y.im, p2[c], 0, 0, 0);
+          p3[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(x.re + x.im, y.re + y.im, p3[c], 0, 0, 0);
+        };
+        if (tile)
+          for (int k0 = 0; k0 < n; k0 += 4) {
+            const int m = k0 + kq;
+            zd xr[3], dr[3], dc[3], yc[3];
+#pragma unroll
+            for (int a = 0; a < 3; ++a) {
+              xr[a] = ldz(Xs + a * PL + ar + LD * m);
+              dr[a] = ldz(Ds + a * PL + ar + LD * m);
+              dc[a] = ldz(Ds + a * PL + m + LD * bc);
+              yc[a] = zadd(ldz(Xs + a * PL + m + LD * bc), zmuli(dc[a]));
+            }
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+              const int a = (c + 1) % 3, b = (c + 2) % 3;
+              mac(c, xr[b], dc[a]);
+              mac(c, zscale(xr[a], -1.0), dc[b]);
+              mac(c, dr[b], yc[a]);
+              mac(c, zscale(dr[a], -1.0), yc[b]);
+            }
+          }
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+#pragma unroll
+          for (int v = 0; v < 4; ++v) cm[c][v] = zd{p1[c][v] - p2[c][v], p3[c][v] - p1[c][v] - p2[c][v]};
+      }
+      __syncthreads();
+      stage(7);
+      __syncthreads();
+      right(Ds, tmp);
+      __syncthreads();
+      store(tmp, Ds);
+      __syncthreads();
+      left(Ds, tmp);  // U^H Om U
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int row = r0 + kq + 4 * v;
+        if (row < n && bc < n)
+          pos_store_om(Ok + 9 * ((int64_t)row + (int64_t)n * bc), zadd(tmp[0][v], cm[0][v]),
+                       zadd(tmp[1][v], cm[1][v]), zadd(tmp[2][v], cm[2][v]));
+      }
+    } else if (want & VELO_DIAG) {
+      // D(l, i) of this thread's (i, l) from Hb's planes (no symmetry assumed)
+      zd cs[3] = {};
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int row = r0 + kq + 4 * v;
+        const bool far = row < n && bc < n && row != bc && fabs(de[v]) > kubo_tol;
+        const double rd = far ? -1.0 / de[v] : 0.0;
+        zd dt[3], y[3];
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+          dt[a] = zscale(ldz(Ds + a * PL + bc + LD * row), rd);
+          y[a] = zadd(ab[a][v], zmuli(dm[a][v]));
+        }
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+          const int a = (c + 1) % 3, b = (c + 2) % 3;
+          const zd f = zsub(zmul(ab[b][v], dt[a]), zmul(ab[a][v], dt[b]));
+          cs[c] = zadd(cs[c], zsub(zmul(dt[b], y[a]), zmul(dt[a], y[b])));
+          const zd rs = zd{row16_sum(f.re), row16_sum(f.im)};
+          if ((lane & 15) == 0) rsum[ct][c][row] = rs;  // zero beyond n
+        }
+      }
+      __syncthreads();  // Hb's readers are done
+      stage(7);
+      __syncthreads();
+      right(Ds, tmp);  // Om U
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+          cs[c] = zadd(cs[c], zcmul(ldz(Us + r0 + kq + 4 * v + LD * bc), tmp[c][v]));
+        const zd s = zd{rows4_sum(cs[c].re), rows4_sum(cs[c].im)};
+        if (kq == 0) csum[rt][c][bc] = s;
+      }
+      __syncthreads();
+      if (t < n) {
+        zd o[3];
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+          o[c] = zadd(rsum[0][c][t], csum[0][c][t]);
+          if (TD == 2 && n > 16) o[c] = zadd(o[c], zadd(rsum[TD - 1][c][t], csum[TD - 1][c][t]));
+        }
+        pos_store_om(Ok + 9 * ((int64_t)t + (int64_t)n * t), o[0], o[1], o[2]);
+      }
+    }
   }
 }
 
-// C = op(A) * B for n x n matrices of pitch n in global memory (the
-// workgroup's slot), 256 threads
+// C = sum over the terms of op(A) B for n x n matrices of pitch n in global
+// memory (the workgroup's slot): FP64 MFMA, the 16 x 16 tiles over four waves,
+// operands loaded in chunks of four steps ahead of their products.  aload(i, m)
+// and bload(m, j) return the elements; terms are run one after the other into
+// the same accumulators.
+template <class ALoad, class BLoad>
+__device__ inline void gmm_acc(int n, int ar, int bc, int kq, const ALoad& aload, const BLoad& bload,
+                               velo_v4d& p1, velo_v4d& p2, velo_v4d& p3) {
+  constexpr int CH = 4;
+  for (int m0 = 0; m0 < n; m0 += 4 * CH) {
+    zd av[CH], bv[CH];
+#pragma unroll
+    for (int i = 0; i < CH; ++i) {
+      const int m = m0 + 4 * i + kq;
+      av[i] = (m < n && ar < n) ? aload(ar, m) : zd{0.0, 0.0};
+      bv[i] = (m < n && bc < n) ? bload(m, bc) : zd{0.0, 0.0};
+    }
+#pragma unroll
+    for (int i = 0; i < CH; ++i) {
+      p1 = __builtin_amdgcn_mfma_f64_16x16x4f64(av[i].re, bv[i].re, p1, 0, 0, 0);
+      p2 = __builtin_amdgcn_mfma_f64_16x16x4f64(av[i].im, bv[i].im, p2, 0, 0, 0);
+      p3 = __builtin_amdgcn_mfma_f64_16x16x4f64(av[i].re + av[i].im, bv[i].re + bv[i].im, p3, 0, 0, 0);
+    }
+  }
+}
+// every tile of C: acc(ar, bc, kq, p1, p2, p3) forms it, out(row, col, value)
+// takes the elements
+template <class Acc, class Out>
+__device__ inline void gmm_tiles(int n, const Acc& acc, const Out& out) {
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lr = lane & 15, kq = lane >> 4, nt = (n + 15) / 16;
+  for (int it = wv; it < nt * nt; it += 4) {
+    const int r0 = 16 * (it % nt), bc = 16 * (it / nt) + lr;
+    velo_v4d p1 = {0, 0, 0, 0}, p2 = {0, 0, 0, 0}, p3 = {0, 0, 0, 0};
+    acc(r0 + lr, bc, kq, p1, p2, p3);
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int row = r0 + kq + 4 * v;
+      if (row < n && bc < n) out(row, bc, zd{p1[v] - p2[v], p3[v] - p1[v] - p2[v]});
+    }
+  }
+}
 __device__ inline void gmm(int n, const zd* A, bool adjA, const zd* B, zd* C) {
-  for (int idx = threadIdx.x; idx < n * n; idx += 256) {
-    const int i = idx % n, j = idx / n;
-    zd s0 = zd{0.0, 0.0}, s1 = zd{0.0, 0.0};
-    int l = 0;
-    for (; l + 1 < n; l += 2) {
-      const zd a0 = adjA ? zconj(A[l + (int64_t)n * i]) : A[i + (int64_t)n * l];
-      const zd a1 = adjA ? zconj(A[l + 1 + (int64_t)n * i]) : A[i + (int64_t)n * (l + 1)];
-      s0 = zadd(s0, zmul(a0, B[l + (int64_t)n * j]));
-      s1 = zadd(s1, zmul(a1, B[l + 1 + (int64_t)n * j]));
-    }
-    if (l < n) {
-      const zd a0 = adjA ? zconj(A[l + (int64_t)n * i]) : A[i + (int64_t)n * l];
-      s0 = zadd(s0, zmul(a0, B[l + (int64_t)n * j]));
-    }
-    C[i + (int64_t)n * j] = zadd(s0, s1);
-  }
+  gmm_tiles(
+      n,
+      [&](int ar, int bc, int kq, velo_v4d& p1, velo_v4d& p2, velo_v4d& p3) {
+        auto b = [&](int m, int j) { return B[m + (int64_t)n * j]; };
+        if (adjA)
+          gmm_acc(n, ar, bc, kq, [&](int i, int m) { return zconj(A[m + (int64_t)n * i]); }, b, p1,
+                  p2, p3);
+        else
+          gmm_acc(n, ar, bc, kq, [&](int i, int m) { return A[i + (int64_t)n * m]; }, b, p1, p2, p3);
+      },
+      [&](int i, int j, zd x) { C[i + (int64_t)n * j] = x; });
 }
 
-// The position-operator path for 16 < n <= 128: velo_pos_kernel's steps in
-// the same order (rotate_gauge :502-550, get_gauge_covar_deriv :565-617,
-// conn_gaugeTrafo :620-633, curv_gaugeTrafo :636-658, get_velo :406-444),
-// with its eighteen n x n matrices in the workgroup's slot of `slots`
-// (18 n^2 complex each; the slots lie in the consumed eigensolver records)
-// instead of LDS.
+// 32 < n <= 128: the same steps with the matrices in the workgroup's slot of
+// `slots` (18 n^2 complex each; the slots lie in the consumed eigensolver
+// records) instead of LDS, products on MFMA from L2.
 __global__ __launch_bounds__(256) void velo_pos_global_kernel(int n, int64_t nk,
                                                               const zd* __restrict__ Hk,
-                                                              int64_t strideHk, TBPhase tb,
+                                                              int64_t strideHk, TBPhase tb0,
                                                               int gauge_trafo, int textbook,
-                                                              double kubo_tol,
+                                                              double kubo_tol, int want,
                                                               const zd* __restrict__ U,
                                                               const double* __restrict__ E,
                                                               zd* __restrict__ V, zd* __restrict__ Aout,
                                                               zd* __restrict__ Omout,
                                                               zd* __restrict__ slots) {
-  __shared__ double Es[128];
+  __shared__ double Es[128], taus[3 * 128];
+  __shared__ zd fph[128];
   const int t = threadIdx.x;
   const int64_t NN = (int64_t)n * n;
   zd* base = slots + (int64_t)blockIdx.x * 18 * NN;
@@ -697,86 +906,103 @@ __global__ __launch_bounds__(256) void velo_pos_global_kernel(int n, int64_t nk,
     Om[a] = base + (12 + a) * NN;
     Abar[a] = base + (15 + a) * NN;
   }
+  const bool full = (want & VELO_OM) != 0, om = full || (want & VELO_DIAG);
   for (int64_t k = blockIdx.x; k < nk; k += gridDim.x) {
-    const TBPhase tk = tb.at(k);
-    const zd* X = Hk + k * strideHk;
+    const TBPhase tb = tb0.at(k);
+    const PosLoad ld{Hk + k * strideHk, tb.tau ? fph : nullptr, taus, n, &tb};
     __syncthreads();  // the previous k-point's reads of the slot are done
+    pos_phases(tb, n, t, fph, taus);
+    if (t < n) Es[t] = E[k * n + t];
+    __syncthreads();
     for (int idx = t; idx < n * n; idx += 256) {
       const int i = idx % n, j = idx / n;
       Us[idx] = U[k * NN + idx];
       for (int a = 0; a < 3; ++a) {
-        Hb[a][idx] = load_tb(X, 0, n, i, j, 1 + a, tk);
-        Ab[a][idx] = load_tb(X, 0, n, i, j, 4 + a, tk);
-        Om[a][idx] = load_tb(X, 0, n, i, j, 7 + a, tk);
+        Hb[a][idx] = ld(1 + a, i, j);
+        if (textbook || !gauge_trafo) Ab[a][idx] = ld(4 + a, i, j);
+        if (om || !gauge_trafo) Om[a][idx] = ld(7 + a, i, j);
       }
     }
-    if (t < n) Es[t] = E[k * n + t];
     __syncthreads();
     if (gauge_trafo) {
       for (int a = 0; a < 3; ++a) {
         gmm(n, Hb[a], false, Us, T1);  // dH U
+        if (textbook) gmm(n, Ab[a], false, Us, T2);
         __syncthreads();
-        gmm(n, Us, true, T1, Hb[a]);    // Hbar = U^H dH U
+        gmm(n, Us, true, T1, Hb[a]);   // Hb = U^H dH U
+        if (textbook) gmm(n, Us, true, T2, Ab[a]);
         __syncthreads();
-        if (textbook) {
-          gmm(n, Ab[a], false, Us, T2);
-          __syncthreads();
-          gmm(n, Us, true, T2, Ab[a]);
-        } else {
-          // stale temporary: A = (U^H (dH U)) U
-          gmm(n, Us, true, T1, T2);
-          __syncthreads();
-          gmm(n, T2, false, Us, Ab[a]);
+        if (!textbook) gmm(n, Hb[a], false, Us, Ab[a]);  // A = (U^H (dH U)) U
+        if (om) gmm(n, Om[a], false, Us, T2);
+        __syncthreads();
+        if (full) {
+          gmm(n, Us, true, T2, Om[a]);  // U^H Om U
+        } else if (om) {                // its diagonal
+          for (int i = t; i < n; i += 256) {
+            zd s = zd{0.0, 0.0};
+#pragma unroll 8
+            for (int m = 0; m < n; ++m)
+              s = zadd(s, zcmul(Us[m + (int64_t)n * i], T2[m + (int64_t)n * i]));
+            Om[a][i + (int64_t)n * i] = s;
+          }
         }
         __syncthreads();
-        gmm(n, Us, true, Om[a], T2);  // Omega_bar = U^H Omega U
-        __syncthreads();
-        gmm(n, T2, false, Us, Om[a]);
-        __syncthreads();
       }
-      // D_a,ij = Hbar_a,ij / (E_j - E_i) for i != j and |E_j - E_i| > kubo_tol
+      // D, Abar and A^(H) = Abar + i D
       for (int idx = t; idx < n * n; idx += 256) {
         const int i = idx % n, j = idx / n;
         const double de = Es[j] - Es[i];
+        const double rd = (i != j && fabs(de) > kubo_tol) ? 1.0 / de : 0.0;
         for (int a = 0; a < 3; ++a) {
-          zd dv = zd{0.0, 0.0};
-          if (i != j && fabs(de) > kubo_tol) dv = zd{Hb[a][idx].re / de, Hb[a][idx].im / de};
+          const zd dv = zscale(Hb[a][idx], rd), ab = Ab[a][idx];
           Dm[a][idx] = dv;
-          Abar[a][idx] = Ab[a][idx];
+          Abar[a][idx] = ab;
+          Ab[a][idx] = zadd(ab, zmuli(dv));
         }
       }
       __syncthreads();
-      // A^(H) = A + i D
-      for (int idx = t; idx < n * n; idx += 256)
-        for (int a = 0; a < 3; ++a) Ab[a][idx] = zadd(Ab[a][idx], zmuli(Dm[a][idx]));
-      __syncthreads();
-      // Omega^(H)_ab = Om_ab - [D_a, A_b] + [D_b, A_a] - i [D_a, D_b]
-      // for (a,b) in {(1,2), (2,0), (0,1)}; A is A^(H) (reference) or Abar
-      for (int c = 0; c < 3; ++c) {
-        const int a = (c == 0) ? 1 : (c == 1) ? 2 : 0;
-        const int b = (c == 0) ? 2 : (c == 1) ? 0 : 1;
-        zd* const* Asrc = textbook ? Abar : Ab;
-        for (int idx = t; idx < n * n; idx += 256) {
-          const int i = idx % n, j = idx / n;
-          zd s_ = Om[c][idx];
-          zd c1 = zd{0, 0}, c2 = zd{0, 0}, c3 = zd{0, 0};
-          for (int l = 0; l < n; ++l) {
-            const int64_t il = i + (int64_t)n * l, lj = l + (int64_t)n * j;
-            c1 = zadd(c1, zsub(zmul(Dm[a][il], Asrc[b][lj]), zmul(Asrc[b][il], Dm[a][lj])));
-            c2 = zadd(c2, zsub(zmul(Dm[b][il], Asrc[a][lj]), zmul(Asrc[a][il], Dm[b][lj])));
-            c3 = zadd(c3, zsub(zmul(Dm[a][il], Dm[b][lj]), zmul(Dm[b][il], Dm[a][lj])));
+      zd* const* X = textbook ? Abar : Ab;
+      auto Y = [&](int a, int64_t o) { return zadd(X[a][o], zmuli(Dm[a][o])); };
+      for (int c = 0; c < 3 && om; ++c) {
+        const int a = (c + 1) % 3, b = (c + 2) % 3;
+        if (full) {
+          gmm_tiles(
+              n,
+              [&](int ar, int bc, int kq, velo_v4d& p1, velo_v4d& p2, velo_v4d& p3) {
+                auto at = [&](const zd* M, double sg) {
+                  return [=](int i, int m) { return zscale(M[i + (int64_t)n * m], sg); };
+                };
+                auto bt = [&](const zd* M) {
+                  return [=](int m, int j) { return M[m + (int64_t)n * j]; };
+                };
+                gmm_acc(n, ar, bc, kq, at(X[b], 1.0), bt(Dm[a]), p1, p2, p3);
+                gmm_acc(n, ar, bc, kq, at(X[a], -1.0), bt(Dm[b]), p1, p2, p3);
+                gmm_acc(n, ar, bc, kq, at(Dm[b], 1.0),
+                        [&](int m, int j) { return Y(a, m + (int64_t)n * j); }, p1, p2, p3);
+                gmm_acc(n, ar, bc, kq, at(Dm[a], -1.0),
+                        [&](int m, int j) { return Y(b, m + (int64_t)n * j); }, p1, p2, p3);
+              },
+              // each element of Om_c is read and written by its own thread
+              [&](int i, int j, zd x) {
+                zd* o = Om[c] + i + (int64_t)n * j;
+                *o = zadd(*o, x);
+              });
+        } else {
+          for (int i = t; i < n; i += 256) {
+            zd s = Om[c][i + (int64_t)n * i];
+            for (int l = 0; l < n; ++l) {
+              const int64_t il = i + (int64_t)n * l, li = l + (int64_t)n * i;
+              s = zadd(s, zsub(zmul(X[b][il], Dm[a][li]), zmul(X[a][il], Dm[b][li])));
+              s = zadd(s, zsub(zmul(Dm[b][il], Y(a, li)), zmul(Dm[a][il], Y(b, li))));
+            }
+            Om[c][i + (int64_t)n * i] = s;
           }
-          s_ = zsub(s_, c1);
-          s_ = zadd(s_, c2);
-          s_ = zsub(s_, zmuli(c3));
-          T1[idx] = s_;
         }
-        __syncthreads();
-        for (int idx = t; idx < n * n; idx += 256) Om[c][idx] = T1[idx];
-        __syncthreads();
       }
+      __syncthreads();
     }
     // velocity, connection and curvature in the reference's layouts
+    const bool all = full || !gauge_trafo;
     for (int idx = t; idx < n * n; idx += 256) {
       const int i = idx % n, j = idx / n;
       for (int a = 0; a < 3; ++a) {
@@ -788,25 +1014,16 @@ __global__ __launch_bounds__(256) void velo_pos_global_kernel(int n, int64_t nk,
           v = zsub(v, zmul(ce, Asel[idx]));
         }
         V[k * 3 * NN + a * NN + idx] = v;
-        Aout[k * 3 * NN + a + 3 * (int64_t)idx] = Ab[a][idx];
+        if (all || (want & VELO_A) || i == j) Aout[k * 3 * NN + a + 3 * (int64_t)idx] = Ab[a][idx];
       }
-      zd* O = Omout + k * 9 * NN + 9 * (int64_t)idx;
-      const zd oyz = Om[0][idx], ozx = Om[1][idx], oxy = Om[2][idx];
-      O[0] = zd{0, 0};
-      O[1 + 3 * 1] = zd{0, 0};
-      O[2 + 3 * 2] = zd{0, 0};
-      O[1 + 3 * 2] = oyz;
-      O[2 + 3 * 1] = zsub(zd{0, 0}, oyz);
-      O[2 + 3 * 0] = ozx;
-      O[0 + 3 * 2] = zsub(zd{0, 0}, ozx);
-      O[0 + 3 * 1] = oxy;
-      O[1 + 3 * 0] = zsub(zd{0, 0}, oxy);
+      if (all || (om && i == j))
+        pos_store_om(Omout + k * 9 * NN + 9 * (int64_t)idx, Om[0][idx], Om[1][idx], Om[2][idx]);
     }
   }
 }
 
 bool velo_pos_scratch_ok(int n, size_t scratch_bytes) {
-  return n <= PM || scratch_bytes >= 18 * (size_t)n * n * sizeof(zd);
+  return n <= 32 || scratch_bytes >= 18 * (size_t)n * n * sizeof(zd);
 }
 
 void launch_velo(hipStream_t s, const VeloArgs& va, int64_t nk, const zd* Hk, int64_t strideHk,
@@ -817,9 +1034,20 @@ void launch_velo(hipStream_t s, const VeloArgs& va, int64_t nk, const zd* Hk, in
   tb.kpts = g.kpts;
   tb.tau = g.tau;
   for (int i = 0; i < 9; ++i) tb.cm[i] = g.cmat[i];
-  if (va.pos_op && va.n <= PM) {
-    hipLaunchKernelGGL(velo_pos_kernel, dim3(grid), dim3(64), 0, s, va.n, nk, Hk, strideHk, tb,
-                       va.gauge_trafo, va.textbook, va.kubo_tol, U, E, V, A, Om);
+  if (va.pos_op && va.n <= 32) {
+    const bool full = (va.want & VELO_OM) != 0;
+#define MEP_POS_LAUNCH(NM, FULL)                                                                   \
+  hipLaunchKernelGGL((velo_pos_kernel<NM, FULL>), dim3(grid), dim3(NM == 32 ? 256 : 64), 0, s,    \
+                     va.n, nk, Hk, strideHk, tb, va.gauge_trafo, va.textbook, va.kubo_tol,        \
+                     va.want, U, E, V, A, Om)
+    if (va.n <= 16) {
+      if (full) MEP_POS_LAUNCH(16, true);
+      else MEP_POS_LAUNCH(16, false);
+    } else {
+      if (full) MEP_POS_LAUNCH(32, true);
+      else MEP_POS_LAUNCH(32, false);
+    }
+#undef MEP_POS_LAUNCH
     return;
   }
   if (va.pos_op) {
@@ -830,8 +1058,8 @@ void launch_velo(hipStream_t s, const VeloArgs& va, int64_t nk, const zd* Hk, in
     if (pg > 2048) pg = 2048;
     if (pg < 1) pg = 1;  // the caller guarantees one slot (velo_pos_scratch_ok)
     hipLaunchKernelGGL(velo_pos_global_kernel, dim3((unsigned)pg), dim3(256), 0, s, va.n, nk, Hk,
-                       strideHk, tb, va.gauge_trafo, va.textbook, va.kubo_tol, U, E, V, A, Om,
-                       va.scratch);
+                       strideHk, tb, va.gauge_trafo, va.textbook, va.kubo_tol, va.want, U, E, V, A,
+                       Om, va.scratch);
     return;
   }
   if (va.n > 32 && va.n <= 16 * VL_MAXT && va.gauge_trafo) {
