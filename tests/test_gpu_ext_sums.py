@@ -14,7 +14,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("n,n_eF,n_hw,with_r,T", [
     (1, 1, 1, True, 300.0), (2, 3, 2, True, 300.0), (15, 1, 1, True, 0.0), (16, 2, 8, True, 300.0),
     (16, 1, 300, False, 300.0), (17, 2, 130, True, 300.0), (31, 7, 3, True, 300.0),
-    (32, 1, 5, True, 0.0), (32, 60, 1, True, 300.0), (72, 60, 1, False, 300.0), (33, 2, 3, True, 300.0)])
+    (32, 1, 5, True, 0.0), (32, 60, 1, True, 300.0), (72, 30, 1, False, 300.0), (33, 2, 3, True, 300.0)])
 def test_ext_sums_at_tile_and_item_edges(n, n_eF, n_hw, with_r, T):
     import oracle as O
     from mepinterp_amd import capi, models
