@@ -857,22 +857,44 @@ __global__ __launch_bounds__(BS_THREADS, 2) void bandsum_kernel(BandArgs b, doub
 }
 
 // ===========================================================================
-// 32 < n <= 128 (no position operator).  Same sums and the same record
-// layout; V and E are read from HBM / L2 instead of LDS, the workgroup's
-// accumulator record lives in `part` (one writer per entry, fixed order).
-//   per-band sums      thread (n0, part) over n = part, part + P, ...; parts
-//                      combined through LDS
-//   hw-resolved sums   a kernel of their own (hwsum_kernel below)
-//   itinerant terms    C_j column tiles on FP64 MFMA, wave item (tc, j)
-//                      accumulating over the row tiles in registers
-// LDS: E n | fd nef*n | S 2*9*256 | F2, F2m 2*9*n | red 4*36 | windows
+// 32 < n <= 128.  Same sums and the same record layout; V and E are read from
+// HBM / L2 instead of LDS, the workgroup's accumulator record lives in `part`
+// (one writer per entry, fixed order).
+//   pair phase       thread (n0, part) over n = part, part + P, ...; parts
+//                    combined through LDS.  HERM (V built here without a
+//                    position operator): V_a(n, n0) = conj V_a(n0, n), so one
+//                    coalesced read of V serves the Berry, local and, for a
+//                    single (hw, E_F), the velo / ohc sums; otherwise V(n, n0)
+//                    is read as stored
+//   hw-resolved sums a kernel of their own (hwsum_kernel below)
+//   itinerant terms  all three C_j on FP64 MFMA by wave item (16 x 16 tile);
+//                    the items' sums pass through the workgroup's slot
+// LDS: E n | fd nef*n | S 21*256 | F2, F2m 2*9*n | red 4*36 | windows
 // ===========================================================================
 static __device__ inline double rinv(const double* Es, int m, int c) {
   return (m == c) ? 0.0 : 1.0 / (Es[c] - Es[m]);  // 1 / (E_c - E_m)
 }
 
-constexpr int BW_CH = 4;  // four-deep MFMA steps per batch of operand loads
-__global__ __launch_bounds__(256) void bandsum_wide_kernel(BandArgs b, double Tsmear, AccLayout L,
+// complex elements of a workgroup's slot: three scaled planes and 18 sums of 16
+// columns for each 16 x 16 tile (at most the eigensolver record of a k-point)
+__host__ __device__ inline int64_t wide_slot(int n) {
+  const int64_t nt = (n + 15) / 16;
+  return 3 * (int64_t)n * n + nt * nt * (18 * 16 / 2);
+}
+size_t bandsum_wide_scratch(int n, int nblocks) { return sizeof(zd) * (size_t)wide_slot(n) * nblocks; }
+
+constexpr int BW_SLOTS = 21;  // per-band partial sums a thread leaves in LDS
+// lane group of 8 sums f over the bands and adds it to *dst (uniform call)
+static __device__ inline void band_item(int n, int nef, int ef, int g, bool valid, const double* fd,
+                                        const double* src, double w, double* dst) {
+  double s = 0.0;
+  if (valid)
+    for (int m0 = g; m0 < n; m0 += 8) s += fd[ef + nef * m0] * (src ? src[m0] : 1.0);
+  s = group8_sum(s);
+  if (valid && g == 0) *dst += w * s;
+}
+template <bool HERM>
+__global__ __launch_bounds__(256, 2) void bandsum_wide_kernel(BandArgs b, double Tsmear, AccLayout L,
                                                            int64_t nk, const double* __restrict__ E,
                                                            const zd* __restrict__ V,
                                                            const double* __restrict__ w,
@@ -884,9 +906,9 @@ __global__ __launch_bounds__(256) void bandsum_wide_kernel(BandArgs b, double Ts
   const int n = b.n, nef = b.n_ef, nhw = b.n_hw, nval = b.n_val;
   double* Es = smem;
   double* fd = Es + n;
-  double* S = fd + (int64_t)nef * n;  // [9][256]
-  double* S2 = S + 9 * 256;           // [9][256]
-  double* F2 = S2 + 9 * 256;          // [9][n]
+  double* S = fd + (int64_t)nef * n;  // [BW_SLOTS][256]
+  double* S2 = S + 9 * 256;
+  double* F2 = S + BW_SLOTS * 256;    // [9][n]
   double* F2m = F2 + 9 * n;           // [9][n]
   double* red = F2m + 9 * n;          // [4][36]
   uint8_t* win = reinterpret_cast<uint8_t*>(red + 4 * 36);  // [nval][n] lo, hi
@@ -896,6 +918,8 @@ __global__ __launch_bounds__(256) void bandsum_wide_kernel(BandArgs b, double Ts
   const bool doAHC = (b.jobs & MEP_JOB_AHC) != 0;
   const bool doK = (b.jobs & MEP_JOB_KUBO) != 0;
   const bool doNjob = (b.jobs & MEP_JOB_MEP) != 0;
+  const bool pmode = HERM && doAHC && (nhw * nef == 1);
+  const zd wq = zd{b.hw[0], b.eta}, w2 = zmul(wq, wq);
   const double tol = b.kubo_tol;
   double* acc = part + (int64_t)blockIdx.x * L.total;
   const int npad = n <= 64 ? 64 : 128, P = 256 / npad;
@@ -930,6 +954,151 @@ __global__ __launch_bounds__(256) void bandsum_wide_kernel(BandArgs b, double Ts
       }
     }
     __syncthreads();
+    if constexpr (HERM) {
+      // x_a = V_a(n0, n), P_ij = x_i conj(x_j) (i < j), r = 1 / (E0 - En), as
+      // the pair phase of bandsum_kernel
+      const bool doN = doNjob && pact && p0 < nval;
+      const double E0 = pact ? Es[p0] : 0.0, f0 = (pmode && pact) ? fd[p0] : 0.0;
+      double om[3] = {0.0, 0.0, 0.0}, gd[3] = {0.0, 0.0, 0.0}, gdm[3] = {0.0, 0.0, 0.0}, ps[24];
+      zd go[3], gom[3];
+#pragma unroll
+      for (int c = 0; c < 3; ++c) go[c] = gom[c] = zd{0.0, 0.0};
+#pragma unroll
+      for (int c = 0; c < 24; ++c) ps[c] = 0.0;
+      if (pact)
+#pragma unroll 2
+        for (int nn = pp; nn < n; nn += P) {
+          zd x[3], Pc[3];
+          double d[3];
+#pragma unroll
+          for (int a = 0; a < 3; ++a) {
+            x[a] = Vk[a * (int64_t)n2 + p0 + (int64_t)n * nn];
+            d[a] = zabs2(x[a]);
+          }
+#pragma unroll
+          for (int c = 0; c < 3; ++c) {
+            const zd xi = x[c == 2 ? 1 : 0], xj = x[c == 0 ? 1 : 2];
+            Pc[c] = zd{xi.re * xj.re + xi.im * xj.im, xi.im * xj.re - xi.re * xj.im};
+          }
+          const bool off = nn != p0;
+          const double dE = E0 - Es[nn];
+          const double r = off ? rcp_nr(dE) : 0.0, r2 = r * r, r3 = r2 * r;
+          const double r3m = (doN && fabs(dE * dE * dE) > tol) ? r3 : 0.0;
+#pragma unroll
+          for (int c = 0; c < 3; ++c) {
+            om[c] += r2 * Pc[c].im;
+            gd[c] += r3 * d[c];
+            gdm[c] += r3m * d[c];
+            go[c] = zd{go[c].re + r3 * Pc[c].re, go[c].im + r3 * Pc[c].im};
+            gom[c] = zd{gom[c].re + r3m * Pc[c].re, gom[c].im + r3m * Pc[c].im};
+          }
+          if (pmode) {
+            const double dfv = f0 - fd[nn];
+            const zd denv = zd{dE * dE - w2.re, -w2.im};
+            const zd deno = zmul(zd{dE, 0.0}, zd{dE - wq.re, -wq.im});
+            const double av = zabs2(denv), ao = zabs2(deno);
+            const double ia = rcp_nr(av * ao);
+            const double iv = ia * ao, io = ia * av;
+            const zd rv = off ? zd{denv.re * iv * dfv, -denv.im * iv * dfv} : zd{0.0, 0.0};
+            const zd ro = off ? zd{deno.re * io * dfv, -deno.im * io * dfv} : zd{0.0, 0.0};
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+              ps[2 * c] += rv.re * Pc[c].im;
+              ps[2 * c + 1] += rv.im * Pc[c].im;
+              ps[6 + 2 * c] += ro.re * Pc[c].re;
+              ps[7 + 2 * c] += ro.re * Pc[c].im;
+              ps[12 + 2 * c] += ro.im * Pc[c].re;
+              ps[13 + 2 * c] += ro.im * Pc[c].im;
+              ps[18 + c] += ro.re * d[c];
+              ps[21 + c] += ro.im * d[c];
+            }
+          }
+        }
+      // local terms: F3_ij = Re(z_l G_ik - z_k G_il), (j, k, l) cyclic, z =
+      // V(n0, n0), G_ik = sum_n r^3 x_i conj(x_k)
+      zd z[3];
+#pragma unroll
+      for (int a = 0; a < 3; ++a)
+        z[a] = pact ? Vk[a * (int64_t)n2 + p0 + (int64_t)n * p0] : zd{0.0, 0.0};
+      auto G = [&](const double* gd_, const zd* go_, int i, int k_) {
+        if (i == k_) return zd{gd_[i], 0.0};
+        const zd g = go_[i + k_ - 1];
+        return i < k_ ? g : zd{g.re, -g.im};
+      };
+#pragma unroll
+      for (int j = 0; j < 3; ++j) {
+        const int k_ = (j + 1) % 3, l = (j + 2) % 3;
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+          const zd a = G(gd, go, i, k_), bb = G(gd, go, i, l);
+          const zd am = G(gdm, gom, i, k_), bm = G(gdm, gom, i, l);
+          S[(i + 3 * j) * 256 + t] =
+              (z[l].re * a.re - z[l].im * a.im) - (z[k_].re * bb.re - z[k_].im * bb.im);
+          S[(9 + i + 3 * j) * 256 + t] =
+              (z[l].re * am.re - z[l].im * am.im) - (z[k_].re * bm.re - z[k_].im * bm.im);
+        }
+      }
+#pragma unroll
+      for (int c = 0; c < 3; ++c) S[(18 + c) * 256 + t] = om[c];
+      if (pmode) {
+        double v3[3];
+        scatter_sum24(ps, v3, lane);
+        const int base = 12 * ((lane >> 5) & 1) + 6 * ((lane >> 4) & 1) + 3 * ((lane >> 3) & 1);
+#pragma unroll
+        for (int q = 0; q < 3; ++q) v3[q] = group8_sum(v3[q]);
+        if ((lane & 7) == 0)
+#pragma unroll
+          for (int q = 0; q < 3; ++q) red[wv * 24 + base + q] = v3[q];
+      }
+      __syncthreads();
+      // the parts of a band into part 0's place
+      for (int e = t; e < BW_SLOTS * npad; e += 256) {
+        const int q = e / npad, m0 = e % npad;
+        double o = 0.0;
+        for (int u = 0; u < P; ++u) o += S[q * 256 + u * npad + m0];
+        S[q * 256 + m0] = o;
+      }
+      __syncthreads();
+      // Ne, kubo_ahc_tens (Omega_ij = -2 om, antisymmetric) and kubo_mep_LC
+      for (int base = 0; base < 8 * 13 * nef; base += 256) {
+        const int it = base + t, item = it >> 3, g = it & 7, c = item % 13, ef = item / 13;
+        const bool in = item < 13 * nef;
+        if (c >= 1 && c < 4) {
+          const int i = (c == 3) ? 1 : 0, j = (c == 1) ? 1 : 2;
+          double s = 0.0;
+          if (in && doAHC)
+            for (int m0 = g; m0 < n; m0 += 8) s += fd[ef + nef * m0] * S[(17 + c) * 256 + m0];
+          s = group8_sum(s);
+          if (in && doAHC && g == 0) {
+            acc[L.ahc + i + 3 * j + 9 * ef] += wk * (2.0 * s);
+            acc[L.ahc + j + 3 * i + 9 * ef] -= wk * (2.0 * s);
+          }
+        } else {
+          band_item(n, nef, ef, g, in && (c == 0 || doK), fd, c == 0 ? nullptr : S + (c - 4) * 256, wk,
+                    acc + (c == 0 ? L.Ne + ef : L.klc + (c - 4) + 9 * ef));
+        }
+      }
+      if (doNjob)
+        for (int it = t; it < 9 * nval; it += 256)
+          acc[L.nlc + it] += wk * S[(9 + it % 9) * 256 + it / 9];
+      // velo_ahc_tens / kubo_ohc_tens at the single (hw, E_F)
+      if (pmode && t < 18) {
+        const int q = t % 9, i = q % 3, j = q / 3, c = i + j - 1;
+        auto u = [&](int e) { return ((red[e] + red[24 + e]) + red[48 + e]) + red[72 + e]; };
+        zd val = zd{0.0, 0.0};
+        if (t < 9) {
+          if (i != j) val = (i < j) ? zd{u(2 * c), u(2 * c + 1)} : zd{-u(2 * c), -u(2 * c + 1)};
+        } else if (i == j) {
+          val = zd{-u(21 + i), u(18 + i)};
+        } else {
+          const double xr = u(6 + 2 * c), xi = u(7 + 2 * c), yr = u(12 + 2 * c), yi = u(13 + 2 * c);
+          val = (i < j) ? zd{xi - yr, xr + yi} : zd{-(xi + yr), xr - yi};
+        }
+        double* dst = acc + (t < 9 ? L.velo : L.ohc) + 2 * q;
+        dst[0] += wk * val.re;
+        dst[1] += wk * val.im;
+      }
+    } else {
     for (int ef = t; ef < nef; ef += 256) {
       double sN = 0.0;
       for (int m0 = 0; m0 < n; ++m0) sN += fd[ef + nef * m0];
@@ -1034,134 +1203,187 @@ __global__ __launch_bounds__(256) void bandsum_wide_kernel(BandArgs b, double Ts
         }
       __syncthreads();
     }
+    }
     // ---- itinerant (IC) terms on MFMA ----------------------------------------
     // B_a(m, n0) = V_a(m, n0) r(m, n0), r(m, n0) = 1 / (E_n0 - E_m) (0 on the
-    // diagonal): one division per pair, into the workgroup's slot of Bscr,
-    // so the MFMA loop below only loads (in chunks of BW_CH steps whose
-    // loads are all issued before the chunk's products).  Bscr holds B
-    // transposed (n0 + n m), so the 16 columns n0 of a tile load as one run
+    // diagonal): one reciprocal per pair, into the workgroup's slot of Bscr,
+    // transposed (n0 + n m), so the 16 columns n0 of a tile load as one run.
+    // A wave item is one 16 x 16 tile of all three C_j = V_k B_l - V_l B_k: six
+    // operands a step feed 18 products (four fed six with one C_j an item, which
+    // left the loop bound by L2 reads), and the next step's operands are in
+    // flight during a step's products.  With the one-read pair phase above: n =
+    // 96, 2,744 k-points 5.6 -> 2.9 ms; n = 44, 9,261 k-points 2.7 + 0.29 (its
+    // velo / ohc kernel) -> 1.7 ms.  Two row tiles an item (9 operands for 36
+    // products) spill: 3.1 and 1.75 ms; three wavefronts a SIMD spill too.
+    // The contraction with A_i(n0, n) = V_i(n0, n) r(n, n0)^2 comes straight
+    // from the accumulators; the items' sums go through the slot.
     if (doK || doNjob) {
       const int nt = (n + 15) / 16;
       const int lr = lane & 15, kq = lane >> 4;
-      zd* Bw = Bscr + (int64_t)blockIdx.x * 3 * n2;
+      zd* Bw = Bscr + (int64_t)blockIdx.x * wide_slot(n);
+      double* Pw = reinterpret_cast<double*>(Bw + 3 * (int64_t)n2);  // [item][18][16]
       for (int idx = t; idx < n2; idx += 256) {
         const int n0 = idx % n, m = idx / n;
-        const double rr = rinv(Es, m, n0);
+        const double rr = m == n0 ? 0.0 : rcp_nr(Es[n0] - Es[m]);
 #pragma unroll
-        for (int a = 0; a < 3; ++a)
-          Bw[a * (int64_t)n2 + idx] = zscale(Vk[a * (int64_t)n2 + m + (int64_t)n * n0], rr);
+        for (int a = 0; a < 3; ++a) {
+          const zd v = HERM ? zconj(Vk[a * (int64_t)n2 + idx]) : Vk[a * (int64_t)n2 + m + (int64_t)n * n0];
+          Bw[a * (int64_t)n2 + idx] = zscale(v, rr);
+        }
       }
       __syncthreads();
-      for (int item = wv; item < 3 * nt; item += 4) {
-        const int j = item / nt, tc = item % nt;
-        const int kk_ = (j + 1) % 3, ll_ = (j + 2) % 3;
-        const zd* Vk_ = Vk + kk_ * (int64_t)n2;
-        const zd* Vl_ = Vk + ll_ * (int64_t)n2;
-        const zd* Bk_ = Bw + kk_ * (int64_t)n2;
-        const zd* Bl_ = Bw + ll_ * (int64_t)n2;
-        const int c0 = 16 * tc, n0 = c0 + lr;
+      for (int item = wv; item < nt * nt; item += 4) {
+        const int r0 = 16 * (item / nt), n0 = 16 * (item % nt) + lr;
         const bool colok = n0 < n;
         const bool doN = doNjob && colok && n0 < nval;
-        double f2[3] = {0.0, 0.0, 0.0}, f2m[3] = {0.0, 0.0, 0.0};
-        for (int tr = 0; tr < nt; ++tr) {
-          const int r0 = 16 * tr, ar = r0 + lr;
-          mep_v4d p1 = {0, 0, 0, 0}, p2 = {0, 0, 0, 0}, p3 = {0, 0, 0, 0};
-          for (int m0 = 0; m0 < n; m0 += 4 * BW_CH) {
-            zd a0[BW_CH], a1[BW_CH], b0[BW_CH], b1[BW_CH];
+        const int nc = colok ? n0 : n - 1;  // padded rows and columns repeat the last: not used
+        const int ar = r0 + lr < n ? r0 + lr : n - 1;
+        mep_v4d p1[3] = {}, p2[3] = {}, p3[3] = {};
+        struct Step {
+          zd a[3], b[3];
+        };
+        auto load = [&](int m0, Step& s) {  // past the end: the last row, weight 0
+          const bool mok = m0 + kq < n;
+          const int64_t mo = (int64_t)n * (mok ? m0 + kq : n - 1);
 #pragma unroll
-            for (int i = 0; i < BW_CH; ++i) {
-              const int m = m0 + 4 * i + kq;
-              a0[i] = a1[i] = b0[i] = b1[i] = zd{0.0, 0.0};
-              if (m < n) {
-                if (ar < n) {
-                  a0[i] = Vk_[ar + (int64_t)n * m];
-                  a1[i] = Vl_[ar + (int64_t)n * m];
-                }
-                if (colok) {
-                  // uniform row base per step, one 32-bit lane offset
-                  const int64_t rb = (int64_t)n * (m0 + 4 * i);
-                  const int lo = n0 + n * kq;
-                  b0[i] = (Bl_ + rb)[lo];
-                  const zd bk = (Bk_ + rb)[lo];
-                  b1[i] = zd{-bk.re, -bk.im};
-                }
-              }
-            }
-#pragma unroll
-            for (int i = 0; i < BW_CH; ++i) {
-              if (m0 + 4 * i >= n) break;  // uniform
-              p1 = __builtin_amdgcn_mfma_f64_16x16x4f64(a0[i].re, b0[i].re, p1, 0, 0, 0);
-              p2 = __builtin_amdgcn_mfma_f64_16x16x4f64(a0[i].im, b0[i].im, p2, 0, 0, 0);
-              p3 = __builtin_amdgcn_mfma_f64_16x16x4f64(a0[i].re + a0[i].im, b0[i].re + b0[i].im, p3, 0, 0, 0);
-              p1 = __builtin_amdgcn_mfma_f64_16x16x4f64(a1[i].re, b1[i].re, p1, 0, 0, 0);
-              p2 = __builtin_amdgcn_mfma_f64_16x16x4f64(a1[i].im, b1[i].im, p2, 0, 0, 0);
-              p3 = __builtin_amdgcn_mfma_f64_16x16x4f64(a1[i].re + a1[i].im, b1[i].re + b1[i].im, p3, 0, 0, 0);
-            }
+          for (int c = 0; c < 3; ++c) {
+            s.b[c] = Bw[c * (int64_t)n2 + mo + nc];
+            s.a[c] = Vk[c * (int64_t)n2 + mo + ar];
           }
 #pragma unroll
-          for (int v = 0; v < 4; ++v) {
-            const int row = r0 + kq + 4 * v;
-            if (!colok || row >= n || row == n0) continue;
-            const zd cv = zd{p1[v] - p2[v], p3[v] - p1[v] - p2[v]};
-            const double rr = rinv(Es, row, n0);
-            const double rr2 = rr * rr;
-            zd ai[3];
+          for (int c = 0; c < 3; ++c) s.b[c] = zscale(s.b[c], mok ? 1.0 : 0.0);
+        };
+        auto mac = [&](const Step& s) {
+          double as[3], bs[3];
+#pragma unroll
+          for (int c = 0; c < 3; ++c) {
+            as[c] = s.a[c].re + s.a[c].im;
+            bs[c] = s.b[c].re + s.b[c].im;
+          }
+#pragma unroll
+          for (int j = 0; j < 3; ++j) {
+            const int kk = (j + 1) % 3, ll = (j + 2) % 3;
+            p1[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(s.a[kk].re, s.b[ll].re, p1[j], 0, 0, 0);
+            p2[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(s.a[kk].im, s.b[ll].im, p2[j], 0, 0, 0);
+            p3[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(as[kk], bs[ll], p3[j], 0, 0, 0);
+          }
+#pragma unroll
+          for (int j = 0; j < 3; ++j) {
+            const int kk = (j + 1) % 3, ll = (j + 2) % 3;
+            p1[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(s.a[ll].re, -s.b[kk].re, p1[j], 0, 0, 0);
+            p2[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(s.a[ll].im, -s.b[kk].im, p2[j], 0, 0, 0);
+            p3[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(as[ll], -bs[kk], p3[j], 0, 0, 0);
+          }
+        };
+        Step s0, s1;  // the next step's operands are in flight during this one's products
+        load(0, s0);
+        for (int m0 = 0; m0 < n; m0 += 8) {
+          load(m0 + 4, s1);
+          mac(s0);
+          load(m0 + 8, s0);
+          mac(s1);
+        }
+        double f2[9], f2m[9];
+#pragma unroll
+        for (int q = 0; q < 9; ++q) f2[q] = f2m[q] = 0.0;
+        // mep_niu keeps, for (n0, n), the m outside one window [lo, hi]: narrow
+        // windows take -Re[A C] here and add back the excluded terms below; wide
+        // windows sum the kept terms directly below; a window of n0 itself or of
+        // every m needs no second pass
+        auto wide = [&](int lo, int hi) { return 2 * (hi - lo + 1) > n; };
+        unsigned wterm = 0;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const int row = r0 + kq + 4 * v;
+          if (!colok || row >= n || row == n0) continue;
+          const double rr = rcp_nr(Es[n0] - Es[row]), rr2 = rr * rr;
+          bool narrow = false;
+          if (doN) {
+            const int lo = win[2 * (n0 * n + row)], hi = win[2 * (n0 * n + row) + 1];
+            const bool all = lo == 0 && hi == n - 1;
+            narrow = !all && !wide(lo, hi);
+            if (!all && !(lo == n0 && hi == n0)) wterm |= 1u << v;
+          }
+          zd ai[3];
+#pragma unroll
+          for (int i = 0; i < 3; ++i) ai[i] = zscale(Vk[i * (int64_t)n2 + n0 + (int64_t)n * row], rr2);
+#pragma unroll
+          for (int j = 0; j < 3; ++j) {
+            const zd cv = zd{p1[j][v] - p2[j][v], p3[j][v] - p1[j][v] - p2[j][v]};
 #pragma unroll
             for (int i = 0; i < 3; ++i) {
-              ai[i] = zscale(Vk[i * (int64_t)n2 + n0 + (int64_t)n * row], rr2);
-              f2[i] -= ai[i].re * cv.re - ai[i].im * cv.im;
-            }
-            if (doN) {
-              const int lo = win[2 * (n0 * n + row)], hi = win[2 * (n0 * n + row) + 1];
-              if (lo == 0 && hi == n - 1) continue;  // every m excluded
-              zd kept = zd{0.0, 0.0};
-              auto term = [&](int mm) {
-                const double rm = rinv(Es, mm, n0);
-                const zd bl = zscale(Vl_[mm + (int64_t)n * n0], rm);
-                const zd bk = zscale(Vk_[mm + (int64_t)n * n0], rm);
-                return zsub(zmul(Vk_[row + (int64_t)n * mm], bl), zmul(Vl_[row + (int64_t)n * mm], bk));
-              };
-              if (2 * (hi - lo + 1) > n) {
-                for (int mm = 0; mm < lo; ++mm) kept = zadd(kept, term(mm));
-                for (int mm = hi + 1; mm < n; ++mm) kept = zadd(kept, term(mm));
-              } else {
-                zd ex = zd{0.0, 0.0};
-                for (int mm = lo; mm <= hi; ++mm)
-                  if (mm != n0) ex = zadd(ex, term(mm));
-                kept = zsub(cv, ex);
-              }
-#pragma unroll
-              for (int i = 0; i < 3; ++i) f2m[i] -= ai[i].re * kept.re - ai[i].im * kept.im;
+              const double c = ai[i].re * cv.re - ai[i].im * cv.im;
+              f2[i + 3 * j] -= c;
+              f2m[i + 3 * j] -= narrow ? c : 0.0;
             }
           }
         }
-#pragma unroll
-        for (int i = 0; i < 3; ++i) {
-          f2[i] += __shfl_xor(f2[i], 16, 64);
-          f2[i] += __shfl_xor(f2[i], 32, 64);
-          f2m[i] += __shfl_xor(f2m[i], 16, 64);
-          f2m[i] += __shfl_xor(f2m[i], 32, 64);
-        }
-        if (kq == 0 && colok)
+        for (int v = 0; v < 4 && wterm >> v; ++v) {  // after the accumulators are dead
+          if (!((wterm >> v) & 1)) continue;
+          const int row = r0 + kq + 4 * v;
+          const int lo = win[2 * (n0 * n + row)], hi = win[2 * (n0 * n + row) + 1];
+          const bool wd = wide(lo, hi);
+          const double rr = rcp_nr(Es[n0] - Es[row]), rr2 = rr * rr;
+          zd ai[3], x[3];
 #pragma unroll
           for (int i = 0; i < 3; ++i) {
-            F2[(i + 3 * j) * n + n0] = f2[i];
-            F2m[(i + 3 * j) * n + n0] = f2m[i];
+            ai[i] = zscale(Vk[i * (int64_t)n2 + n0 + (int64_t)n * row], rr2);
+            x[i] = zd{0.0, 0.0};
           }
+          auto terms = [&](int from, int to) {
+            for (int mm = from; mm < to; ++mm) {
+              zd vm[3], bm[3];
+#pragma unroll
+              for (int c = 0; c < 3; ++c) {
+                vm[c] = Vk[c * (int64_t)n2 + row + (int64_t)n * mm];
+                bm[c] = Bw[c * (int64_t)n2 + n0 + (int64_t)n * mm];  // 0 for mm = n0
+              }
+#pragma unroll
+              for (int j = 0; j < 3; ++j) {
+                const int kk = (j + 1) % 3, ll = (j + 2) % 3;
+                x[j] = zadd(x[j], zsub(zmul(vm[kk], bm[ll]), zmul(vm[ll], bm[kk])));
+              }
+            }
+          };
+          if (wd) {  // kept terms: f2m -= Re(A x)
+            terms(0, lo);
+            terms(hi + 1, n);
+          } else {   // excluded terms: f2m += Re(A x)
+            terms(lo, hi + 1);
+          }
+#pragma unroll
+          for (int j = 0; j < 3; ++j)
+#pragma unroll
+            for (int i = 0; i < 3; ++i) {
+              const double c = ai[i].re * x[j].re - ai[i].im * x[j].im;
+              f2m[i + 3 * j] += wd ? -c : c;
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < 9; ++q) {
+          const double s0 = rows4_sum(f2[q]), s1 = rows4_sum(f2m[q]);
+          if (kq == 0) {
+            Pw[(item * 18 + q) * 16 + lr] = s0;
+            Pw[(item * 18 + 9 + q) * 16 + lr] = s1;
+          }
+        }
+      }
+      __syncthreads();
+      for (int e = t; e < 18 * n; e += 256) {  // F2 and F2m are neighbours
+        const int q = e / n, m0 = e % n;
+        double o = 0.0;
+        for (int tr = 0; tr < nt; ++tr) o += Pw[((tr * nt + m0 / 16) * 18 + q) * 16 + m0 % 16];
+        F2[e] = o;
       }
       __syncthreads();
       if (doK)
-        for (int it = t; it < 9 * nef; it += 256) {
-          const int q = it % 9, ef = it / 9;
-          double sI = 0.0;
-          for (int m0 = 0; m0 < n; ++m0) sI += fd[ef + nef * m0] * F2[q * n + m0];
-          acc[L.kic + q + 9 * ef] += wk * sI;
+        for (int base = 0; base < 8 * 9 * nef; base += 256) {
+          const int it = base + t, item = it >> 3, q = item % 9, ef = item / 9;
+          band_item(n, nef, ef, it & 7, item < 9 * nef, fd, F2 + q * n, wk, acc + L.kic + q + 9 * ef);
         }
       if (doNjob)
-        for (int it = t; it < 9 * nval; it += 256) {
-          const int q = it % 9, m0 = it / 9;
-          acc[L.nic + q + 9 * m0] += wk * F2m[q * n + m0];
-        }
+        for (int it = t; it < 9 * nval; it += 256)
+          acc[L.nic + it] += wk * F2m[(it % 9) * n + it / 9];
     }
     // ---- Chern-Simons terms (position operator: A and Omega) ---------------
     // kubo_mep_CS / mep_niu_CS (kubo_mep.f90:16-47, mep_niu.f90:20-45):
@@ -1197,7 +1419,7 @@ __global__ __launch_bounds__(256) void bandsum_wide_kernel(BandArgs b, double Ts
 
 size_t bandsum_wide_lds_bytes(const BandArgs& b) {
   const size_t n = b.n;
-  return sizeof(double) * (n + (size_t)b.n_ef * n + 2 * 9 * 256 + 2 * 9 * n + 4 * 36) +
+  return sizeof(double) * (n + (size_t)b.n_ef * n + BW_SLOTS * 256 + 2 * 9 * n + 4 * 36) +
          2 * (size_t)(b.n_val > 0 ? b.n_val : 1) * n;
 }
 
@@ -1688,11 +1910,17 @@ void launch_bandsum(hipStream_t s, const BandArgs& b, int64_t nk, const double* 
   double Tsmear = kB * b.T_kelvin;
   if (b.n > 32) {
     const size_t lds = bandsum_wide_lds_bytes(b);
-    (void)hipFuncSetAttribute((const void*)bandsum_wide_kernel,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    hipLaunchKernelGGL(bandsum_wide_kernel, dim3(nblocks), dim3(256), lds, s, b, Tsmear, L, nk, E,
-                       V, w, part, wide_scr, A, Om);
-    if (b.jobs & MEP_JOB_AHC) launch_hwsum(s, b, Tsmear, L, nk, E, V, w, nblocks, part);
+    auto go = [&](auto kernel) {
+      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+      hipLaunchKernelGGL(kernel, dim3(nblocks), dim3(256), lds, s, b, Tsmear, L, nk, E, V, w, part,
+                         wide_scr, A, Om);
+    };
+    if (b.v_herm) go(bandsum_wide_kernel<true>);
+    else go(bandsum_wide_kernel<false>);
+    // the single (hw, E_F) of a Hermitian V is summed in the pair phase
+    if (hw_many(b) || ((b.jobs & MEP_JOB_AHC) && !b.v_herm))
+      launch_hwsum(s, b, Tsmear, L, nk, E, V, w, nblocks, part);
   } else {
     if (b.n <= 16)
       launch_bs<16, false>(s, b, Tsmear, L, nk, E, V, A, Om, w, nblocks, part, nullptr);

@@ -792,14 +792,15 @@ static int band_setup(mep_ctx* c, const mep_run_params* p, int64_t kblock, BandS
 // velocity kernel is not launched and V never reaches HBM)
 static int band_block(mep_ctx* c, BandSetup& bs, int64_t nb, const double* w, bool fuse = false) {
   int nblk = (int)(nb < bs.nblocks ? nb : bs.nblocks);
+  if (c->n > 32 && bandsum_wide_scratch((int)c->n, nblk) > eigh_scratch_bytes((int)c->n, c->kcap))
+    return fail(MEP_ERR_ARG, "band sums: the k-block is too small for the workgroups' slots");
   VeloFuse vf;
   vf.Hk = c->dHk;
   vf.strideHk = c->ncols;
   vf.U = c->dU;
   timed(c, K_BANDSUM, [&] {
-    // n > 32: the eigensolver records (64 n^2 bytes or more per k-point of
-    // the block, consumed by now) hold the 48 n^2 bytes per workgroup of
-    // the wide kernel's scaled columns; nblk <= nb workgroups
+    // n > 32: the eigensolver records (consumed by now) hold the wide
+    // kernel's slots; nblk <= nb workgroups
     launch_bandsum(c->st, bs.b, nb, c->dE, c->dV, c->dA, c->dOm, w, nblk, c->dpart,
                    fuse ? &vf : nullptr, reinterpret_cast<zd*>(c->dscr));
     if (bs.ext)

@@ -134,8 +134,9 @@ struct VeloFuse {
   const zd* U;
 };
 bool bandsum_can_fuse(const BandArgs& b);
-// wide_scr (n > 32): 3 n^2 complex per workgroup (nblocks of them), the
-// columns of V scaled by 1 / (E_n0 - E_m) for the itinerant products
+// wide_scr (n > 32): bandsum_wide_scratch bytes, a slot per workgroup for the
+// columns of V scaled by 1 / (E_n0 - E_m) of the itinerant products and their sums
+size_t bandsum_wide_scratch(int n, int nblocks);
 void launch_bandsum(hipStream_t s, const BandArgs& b, int64_t nk, const double* E, const zd* V,
                     const zd* A, const zd* Om, const double* w, int nblocks, double* part,
                     const VeloFuse* fuse = nullptr, zd* wide_scr = nullptr);
