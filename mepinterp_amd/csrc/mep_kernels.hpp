@@ -91,7 +91,8 @@ struct VeloArgs {
 };
 // the scratch holds at least one position-operator slot (or none is needed)
 bool velo_pos_scratch_ok(int n, size_t scratch_bytes);
-void launch_velo(hipStream_t s, const VeloArgs& va, int64_t nk, const zd* Hk, int64_t strideHk,
+// Hk is consumed: above 32 bands the tight-binding phases go into it in place.
+void launch_velo(hipStream_t s, const VeloArgs& va, int64_t nk, zd* Hk, int64_t strideHk,
                  const KGeom& g, const zd* U, const double* E, zd* V, zd* A, zd* Om);
 
 // mixed precision: dH_a from the FP32 Fourier sum (no position operator),

@@ -47,6 +47,16 @@ struct TBPhase {
   }
 };
 
+// f_m and the centres of a workgroup's k-point into LDS (threads t < n)
+__device__ inline void pos_phases(const TBPhase& tb, int n, int t, zd* f, double* tau) {
+  if (!tb.tau || t >= n) return;
+  const double* tm = tb.tau + 3 * t;
+  double sn, cs;
+  sincos(2.0 * 3.14159265358979323846 * (tb.kx * tm[0] + tb.ky * tm[1] + tb.kz * tm[2]), &sn, &cs);
+  f[t] = zd{cs, sn};
+#pragma unroll
+  for (int a = 0; a < 3; ++a) tau[3 * t + a] = tm[a];
+}
 // Wannier-gauge element (row, col) of matrix `mat`: full column-major
 // matrices of N x N, or (packed) the upper triangles of Hermitian matrices
 // with (i <= j) at i + j(j+1)/2 and the lower half as conjugates.  HT is the
@@ -250,215 +260,194 @@ __global__ __launch_bounds__(256, 2) void velo_mfma_kernel(int n, int64_t nk,
 
 // --------------------------------------------------------------------------
 // 32 < n <= 128, no position operator: V_a = U^H dH_a U on FP64 MFMA, three
-// real products per complex one.  Pass 0 forms T_a = dH_a U for a = x, y, z
-// in the workgroup's slot Tscr[blockIdx] (3 n^2 complex), pass 1 V_a =
-// U^H T_a; the 3 nt^2 (component, 16 x 16 tile) items of a pass are spread
-// over the four waves, with one barrier per pass.  Operands come from L2 /
-// HBM in chunks of VW_CH four-deep steps: the chunk's loads are all issued
-// before its MFMAs, so their latencies overlap.
+// real products per complex one, operands from L2.
 // --------------------------------------------------------------------------
 typedef double velo_v4d __attribute__((ext_vector_type(4)));
-constexpr int VW_CH = 8;
 
-// lower-triangle tile p (row-major: (0,0), (1,0), (1,1), (2,0), ...) of an
-// edge of tiles: V_a = U^H T_a is Hermitian, so the second product forms
-// the tiles on and below the diagonal and writes each off-diagonal one
-// twice (V(c, r) = conj V(r, c))
-__device__ inline void lower_tile(int p, int* tr, int* tc) {
-  int r = (int)((sqrtf(8.0f * (float)p + 1.0f) - 1.0f) * 0.5f);
-  if ((r + 1) * (r + 2) / 2 <= p) ++r;
-  if (r * (r + 1) / 2 > p) --r;
-  *tr = r;
-  *tc = p - r * (r + 1) / 2;
-}
-
-template <int PASS>
-__device__ inline void velo_wide_pass(int n, int wv, int lane, const zd* __restrict__ X, int packed,
-                                      const TBPhase& tb, const zd* __restrict__ Uk,
-                                      zd* __restrict__ T, zd* __restrict__ Vk) {
-  const int lr = lane & 15, kq = lane >> 4;
-  const int n2 = n * n, nt = (n + 15) / 16;
-  const int nit = PASS == 0 ? nt * nt : nt * (nt + 1) / 2;  // tiles per component
-  for (int item = wv; item < 3 * nit; item += 4) {
-    const int a = item / nit, ti = item % nit;
-    int tr = ti / nt, tc = ti % nt;
-    if (PASS == 1) lower_tile(ti, &tr, &tc);
-    const int r0 = 16 * tr, c0 = 16 * tc;
-    const int ar = r0 + lr, bc = c0 + lr;
-    const zd* Ta = T + (int64_t)a * n2;
-    velo_v4d p1 = {0, 0, 0, 0}, p2 = {0, 0, 0, 0}, p3 = {0, 0, 0, 0};
-    for (int m0 = 0; m0 < n; m0 += 4 * VW_CH) {
-      zd av[VW_CH], bv[VW_CH];
+// The tight-binding epilogue of the packed dH_a, in place, with one sincos a
+// band: dH'_a(i, j) = conj(f_i) f_j (dH_a + i c_a(tau_j - tau_i) H), f_m =
+// e^{2 pi i k.tau_m}.  One k-point per workgroup.
+__global__ __launch_bounds__(256) void velo_tb_kernel(int n, int64_t nk, zd* __restrict__ Hk,
+                                                      int64_t strideHk, TBPhase tb0) {
+  __shared__ zd f[128];
+  __shared__ double tau[3 * 128];
+  const int t = threadIdx.x;
+  const int np = n * (n + 1) / 2;
+  for (int64_t k = blockIdx.x; k < nk; k += gridDim.x) {
+    const TBPhase tb = tb0.at(k);
+    zd* X = Hk + k * strideHk;
+    __syncthreads();
+    pos_phases(tb, n, t, f, tau);
+    __syncthreads();
+    for (int p = t; p < np; p += 256) {
+      // p = i + j (j + 1) / 2
+      int j = (int)((sqrtf(8.0f * (float)p + 1.0f) - 1.0f) * 0.5f);
+      if ((j + 1) * (j + 2) / 2 <= p) ++j;
+      if (j * (j + 1) / 2 > p) --j;
+      const int i = p - j * (j + 1) / 2;
+      const double dt[3] = {tau[3 * j] - tau[3 * i], tau[3 * j + 1] - tau[3 * i + 1],
+                            tau[3 * j + 2] - tau[3 * i + 2]};
+      const zd ph = zcmul(f[i], f[j]), h = X[p];
 #pragma unroll
-      for (int i = 0; i < VW_CH; ++i) {
-        const int m = m0 + 4 * i + kq;
-        av[i] = bv[i] = zd{0.0, 0.0};
-        if (m < n) {
-          if (ar < n)
-            av[i] = PASS == 0 ? load_tb(X, packed, n, ar, m, 1 + a, tb) : zconj(Uk[m + (int64_t)n * ar]);
-          if (bc < n) bv[i] = PASS == 0 ? Uk[m + (int64_t)n * bc] : Ta[m + (int64_t)n * bc];
-        }
-      }
-#pragma unroll
-      for (int i = 0; i < VW_CH; ++i) {
-        if (m0 + 4 * i >= n) break;  // uniform
-        p1 = __builtin_amdgcn_mfma_f64_16x16x4f64(av[i].re, bv[i].re, p1, 0, 0, 0);
-        p2 = __builtin_amdgcn_mfma_f64_16x16x4f64(av[i].im, bv[i].im, p2, 0, 0, 0);
-        p3 = __builtin_amdgcn_mfma_f64_16x16x4f64(av[i].re + av[i].im, bv[i].re + bv[i].im, p3, 0, 0, 0);
-      }
-    }
-    zd* out = PASS == 0 ? T + (int64_t)a * n2 : Vk + (int64_t)a * n2;
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const int row = r0 + kq + 4 * v;
-      if (row < n && bc < n) {
-        const zd z = zd{p1[v] - p2[v], p3[v] - p1[v] - p2[v]};
-        out[row + (int64_t)n * bc] = z;
-        if (PASS == 1 && tr != tc) out[bc + (int64_t)n * row] = zconj(z);
+      for (int a = 0; a < 3; ++a) {
+        zd* x = X + (int64_t)(1 + a) * np + p;
+        *x = zmul(ph, zadd(*x, zmuli(zscale(h, tb.c(a, dt)))));
       }
     }
   }
 }
 
-__global__ __launch_bounds__(256, 2) void velo_wide_kernel(int n, int64_t nk, const zd* __restrict__ Hk,
-                                                           int64_t strideHk, int packed, TBPhase tb0,
-                                                           int gauge_trafo, const zd* __restrict__ U,
-                                                           zd* __restrict__ V, zd* __restrict__ Tscr) {
-  const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
-  const int n2 = n * n;
-  zd* T = Tscr + (int64_t)blockIdx.x * 3 * n2;
-  for (int64_t k = blockIdx.x; k < nk; k += gridDim.x) {
-    const TBPhase tb = tb0.at(k);
-    const zd* X = Hk + k * strideHk;
+// A wavefront forms 16 columns of V (one of NT column tiles, 16 (NT - 1) < n <=
+// 16 NT).  T_a = dH_a U of its columns stays in its registers: the accumulator
+// of a tile (row lane / 16 + 4 v, column lane % 16) is the B operand of the
+// second product's steps as it stands, so T_a goes through neither LDS nor
+// memory and there is no barrier.  V_a = U^H T_a is Hermitian: the wavefront of
+// column tile c forms the row tiles c, c + 1, ... c + NT / 2 (mod NT), every
+// pair of tiles once and as many for each wavefront, and writes each
+// off-diagonal one twice.  dH_a is read from its packed upper triangle: below
+// the diagonal as conj dH_a(m, row), known per step outside the diagonal tile.
+// REG: the columns of U as well in registers, which takes half of the first
+// product's loads away (up to 64 bands; above, they would spill: n = 96 took
+// 2.4 ms so against 1.9).
+// The wavefronts of one k-point follow each other on one XCD (workgroup index
+// mod 8), so that dH_a and U come from its L2 after the first.  Bound by the
+// operand loads: 0.55 (n = 44) and 0.46 (n = 96) of the MFMA issue at two
+// wavefronts a SIMD; three with spills took 1.2 and 2.6 ms, two columns a
+// wavefront at one wavefront a SIMD 1.1 and 2.0.
+// n = 44, 9,261 k-points: 0.70 ms (U and one component at a time in LDS, T_a
+// through memory: 1.42); n = 96, 2,744: 1.92 ms (T_a through memory: 4.07).
+template <int NT, bool REG>
+__global__ __launch_bounds__(64, 2) void velo_wide_kernel(
+    int n, int64_t nk, const zd* __restrict__ Hk, int64_t strideHk, int gauge_trafo,
+    const zd* __restrict__ U, zd* __restrict__ V) {
+  const int lane = threadIdx.x, lr = lane & 15, kq = lane >> 4;
+  const int n2 = n * n, np = n * (n + 1) / 2;
+  const int64_t slots = (nk + 7) / 8 * NT;
+  constexpr int NS = 4 * NT;                      // steps of four
+  constexpr int GS = NT >= 7 ? 2 : 4, NQ = NS / GS;  // a group's loads are one group ahead
+  for (int64_t slot = blockIdx.x >> 3; slot < slots; slot += gridDim.x >> 3) {
+    const int64_t k = slot / NT * 8 + (blockIdx.x & 7);
+    const int c = (int)(slot % NT), bc = 16 * c + lr;
+    if (k >= nk) break;
+    const zd* X0 = Hk + k * strideHk + np;
     const zd* Uk = U + k * (int64_t)n2;
     zd* Vk = V + k * 3 * (int64_t)n2;
     if (!gauge_trafo) {
-      for (int idx = t; idx < 3 * n2; idx += 256)
-        Vk[idx] = load_tb(X, packed, n, (idx % n2) % n, (idx % n2) / n, 1 + idx / n2, tb);
+      for (int idx = 64 * c + lane; idx < n2; idx += 64 * NT) {
+        const int i = idx % n, j = idx / n, lo = i < j ? i : j, hi = i < j ? j : i;
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+          const zd x = X0[a * (int64_t)np + lo + hi * (hi + 1) / 2];
+          Vk[a * (int64_t)n2 + idx] = i > j ? zconj(x) : x;
+        }
+      }
       continue;
     }
-    velo_wide_pass<0>(n, wv, lane, X, packed, tb, Uk, T, Vk);
-    __syncthreads();  // T complete
-    velo_wide_pass<1>(n, wv, lane, X, packed, tb, Uk, T, Vk);
-    __syncthreads();  // T read before the next k-point overwrites it
-  }
-}
-
-// --------------------------------------------------------------------------
-// 32 < n <= 64, no position operator: the same products with the operands
-// in LDS.  Plane U holds U (pitch LV = n | 1, odd, so the 16-byte reads of
-// a 16-lane column tile fall in distinct banks); plane D holds dH_a (both
-// triangles, unpacked once per component), then T_a = dH_a U over it.  Per
-// component: stage dH_a | T = D U into registers | T over D | V_a = U^H T
-// to HBM.  The MFMA loop then issues two LDS reads and two adds per three
-// products (the L2 version above spends about fourteen VALU instructions per
-// product on addresses and guards, and VALU and FP64 MFMA issue serialise).
-// --------------------------------------------------------------------------
-constexpr int VL_MAXT = 4;  // 16 x 16 tiles per matrix edge (n <= 64)
-
-__host__ __device__ inline int velo_lds_pitch(int n) { return n | 1; }
-
-__global__ __launch_bounds__(256) void velo_lds_kernel(int n, int64_t nk, const zd* __restrict__ Hk,
-                                                       int64_t strideHk, int packed, TBPhase tb0,
-                                                       const zd* __restrict__ U,
-                                                       zd* __restrict__ V) {
-  extern __shared__ __attribute__((aligned(16))) double vl_smem[];
-  const int LV = velo_lds_pitch(n), PLV = LV * n;
-  zd* Us = reinterpret_cast<zd*>(vl_smem);
-  zd* Ds = Us + PLV;
-  const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
-  const int lr = lane & 15, kq = lane >> 4;
-  const int n2 = n * n, nt = (n + 15) / 16, ntile = nt * nt;
-  // tile rows / columns n .. 16 nt - 1 lie outside the planes: their
-  // operand loads read a clamped index and select zero
-  for (int64_t k = blockIdx.x; k < nk; k += gridDim.x) {
-    const TBPhase tb = tb0.at(k);
-    const zd* X = Hk + k * strideHk;
-    const zd* Uk = U + k * (int64_t)n2;
-    zd* Vk = V + k * 3 * (int64_t)n2;
-    __syncthreads();  // the previous k-point's last reads of U and T are done
-    for (int idx = t; idx < n2; idx += 256) stz(Us + idx % n + LV * (idx / n), Uk[idx]);
+    // row 4 s + kk; past the end (the last tile only): the last one, zero in U
+    auto row4 = [&](int s, int kk) {
+      const int m = 4 * s + kk;
+      return s < NS - 4 || m < n ? m : n - 1;
+    };
+    auto uload = [&](const zd* Uc, int s, int kk) {
+      zd u = Uc[row4(s, kk)];
+      if (s >= NS - 4) {
+        const bool ok = 4 * s + kk < n;
+        u.re = ok ? u.re : 0.0;
+        u.im = ok ? u.im : 0.0;
+      }
+      return u;
+    };
+    const zd* Ub = Uk + (int64_t)n * (bc < n ? bc : n - 1);
+    zd ur[REG ? NS : 1];
+    if constexpr (REG)
+#pragma unroll
+      for (int s = 0; s < NS; ++s) ur[s] = uload(Ub, s, kq);
+#pragma unroll 1
     for (int a = 0; a < 3; ++a) {
-      for (int idx = t; idx < n2; idx += 256) {
-        const int i = idx % n, j = idx / n;
-        stz(Ds + i + LV * j, load_tb(X, packed, n, i, j, 1 + a, tb));
-      }
-      __syncthreads();  // U and dH_a staged
-      // T = D U: up to VL_MAXT^2 / 4 tiles per wave, kept in registers
-      velo_v4d q1[4], q2[4], q3[4];
+      const zd* X = X0 + a * (int64_t)np;
+      zd T[NS];
+      {  // T(16 r ..) = sum over m of dH(row, m) U(m, col), GS steps a group
+        struct Group {
+          zd x[GS], u[REG ? 1 : GS];
+        } g[2];
+        auto load = [&](int q, Group& o) {
+          const int r = q / NQ, s0 = q % NQ * GS;
+          int kk = kq;
+          asm volatile("" : "+v"(kk));  // offsets are formed here, not kept across a
+          const int ar0 = 16 * r + lr, ar = r < NT - 1 || ar0 < n ? ar0 : n - 1;
+          const int low = ar * (ar + 1) / 2;
 #pragma unroll
-      for (int u = 0; u < 4; ++u) q1[u] = q2[u] = q3[u] = velo_v4d{0, 0, 0, 0};
+          for (int j = 0; j < GS; ++j) {
+            const int s = s0 + j, m = row4(s, kk);
+            const bool cj = s / 4 < r || (s / 4 == r && ar > m);
+            o.x[j] = X[cj ? m + low : ar + m * (m + 1) / 2];
+            o.x[j].im = cj ? -o.x[j].im : o.x[j].im;
+            if (!REG) o.u[REG ? 0 : j] = uload(Ub, s, kk);
+          }
+        };
+        load(0, g[0]);
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int tile = wv + 4 * u;
-        if (tile >= ntile) break;  // uniform
-        const int ar = 16 * (tile / nt) + lr, bc = 16 * (tile % nt) + lr;
-        const bool aok = ar < n, bok = bc < n;
-        const int arc = aok ? ar : 0, bcc = bok ? bc : 0;
-        for (int m0 = 0; m0 < n; m0 += 4) {
-          const int m = m0 + kq, mc = m < n ? m : 0;
-          zd x = ldz(Ds + arc + LV * mc), y = ldz(Us + mc + LV * bcc);
-          if (!(aok && m < n)) x = zd{0.0, 0.0};
-          if (!(bok && m < n)) y = zd{0.0, 0.0};
-          q1[u] = __builtin_amdgcn_mfma_f64_16x16x4f64(x.re, y.re, q1[u], 0, 0, 0);
-          q2[u] = __builtin_amdgcn_mfma_f64_16x16x4f64(x.im, y.im, q2[u], 0, 0, 0);
-          q3[u] = __builtin_amdgcn_mfma_f64_16x16x4f64(x.re + x.im, y.re + y.im, q3[u], 0, 0, 0);
+        for (int r = 0; r < NT; ++r) {
+          velo_v4d p1 = {}, p2 = {}, p3 = {};
+#pragma unroll
+          for (int sq = 0; sq < NQ; ++sq) {
+            const int q = r * NQ + sq;
+            if (q + 1 < NT * NQ) load(q + 1, g[(q + 1) & 1]);
+#pragma unroll
+            for (int j = 0; j < GS; ++j) {
+              const zd x = g[q & 1].x[j];
+              const zd u = REG ? ur[REG ? GS * sq + j : 0] : g[q & 1].u[REG ? 0 : j];
+              p1 = __builtin_amdgcn_mfma_f64_16x16x4f64(x.re, u.re, p1, 0, 0, 0);
+              p2 = __builtin_amdgcn_mfma_f64_16x16x4f64(x.im, u.im, p2, 0, 0, 0);
+              p3 = __builtin_amdgcn_mfma_f64_16x16x4f64(x.re + x.im, u.re + u.im, p3, 0, 0, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+          }
+#pragma unroll
+          for (int v = 0; v < 4; ++v) T[4 * r + v] = zd{p1[v] - p2[v], p3[v] - p1[v] - p2[v]};
         }
       }
-      __syncthreads();  // every wave has read dH_a
+      zd* Va = Vk + a * (int64_t)n2;
+      const int cnt = NT / 2 + ((NT & 1) || c < NT / 2 ? 1 : 0);
+#pragma unroll 1
+      for (int q = 0; q < cnt; ++q) {  // V(16 r ..) = sum over m of conj U(m, row) T(m, col)
+        const int r = c + q < NT ? c + q : c + q - NT;
+        const int ar = 16 * r + lr;
+        const zd* Ua = Uk + (int64_t)n * (ar < n ? ar : n - 1);
+        zd g[2][GS];
+        auto load = [&](int q4, zd* o) {
+          int kk = kq;
+          asm volatile("" : "+v"(kk));
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int tile = wv + 4 * u;
-        if (tile >= ntile) break;
-        const int r0 = 16 * (tile / nt), bc = 16 * (tile % nt) + lr;
+          for (int j = 0; j < GS; ++j) o[j] = uload(Ua, GS * q4 + j, kk);
+        };
+        load(0, g[0]);
+        velo_v4d p1 = {}, p2 = {}, p3 = {};
+#pragma unroll
+        for (int q4 = 0; q4 < NQ; ++q4) {
+          if (q4 + 1 < NQ) load(q4 + 1, g[(q4 + 1) & 1]);
+#pragma unroll
+          for (int j = 0; j < GS; ++j) {
+            const zd u = g[q4 & 1][j], x = T[GS * q4 + j];
+            p1 = __builtin_amdgcn_mfma_f64_16x16x4f64(u.re, x.re, p1, 0, 0, 0);
+            p2 = __builtin_amdgcn_mfma_f64_16x16x4f64(-u.im, x.im, p2, 0, 0, 0);
+            p3 = __builtin_amdgcn_mfma_f64_16x16x4f64(u.re - u.im, x.re + x.im, p3, 0, 0, 0);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-          const int row = r0 + kq + 4 * v;
-          if (row < n && bc < n)
-            stz(Ds + row + LV * bc, zd{q1[u][v] - q2[u][v], q3[u][v] - q1[u][v] - q2[u][v]});
-        }
-      }
-      __syncthreads();  // T complete
-      // V_a = U^H T, straight to HBM: the tiles on and below the diagonal
-      // (V_a is Hermitian), each off-diagonal one written twice
-      const int nlt = nt * (nt + 1) / 2;
-#pragma unroll
-      for (int u = 0; u < 3; ++u) {
-        const int tile = wv + 4 * u;
-        if (tile >= nlt) break;
-        int tr, tc;
-        lower_tile(tile, &tr, &tc);
-        const int r0 = 16 * tr;
-        const int ar = r0 + lr, bc = 16 * tc + lr;
-        const bool aok = ar < n, bok = bc < n;
-        const int arc = aok ? ar : 0, bcc = bok ? bc : 0;
-        velo_v4d p1 = {0, 0, 0, 0}, p2 = {0, 0, 0, 0}, p3 = {0, 0, 0, 0};
-        for (int m0 = 0; m0 < n; m0 += 4) {
-          const int m = m0 + kq, mc = m < n ? m : 0;
-          zd x = ldz(Us + mc + LV * arc), y = ldz(Ds + mc + LV * bcc);
-          x.im = -x.im;  // A(row, m) = conj(U(m, row))
-          if (!(aok && m < n)) x = zd{0.0, 0.0};
-          if (!(bok && m < n)) y = zd{0.0, 0.0};
-          p1 = __builtin_amdgcn_mfma_f64_16x16x4f64(x.re, y.re, p1, 0, 0, 0);
-          p2 = __builtin_amdgcn_mfma_f64_16x16x4f64(x.im, y.im, p2, 0, 0, 0);
-          p3 = __builtin_amdgcn_mfma_f64_16x16x4f64(x.re + x.im, y.re + y.im, p3, 0, 0, 0);
-        }
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const int row = r0 + kq + 4 * v;
+          const int row = 16 * r + kq + 4 * v;
           if (row < n && bc < n) {
             const zd z = zd{p1[v] - p2[v], p3[v] - p1[v] - p2[v]};
-            Vk[a * (int64_t)n2 + row + (int64_t)n * bc] = z;
-            if (tr != tc) Vk[a * (int64_t)n2 + bc + (int64_t)n * row] = zconj(z);
+            Va[row + (int64_t)n * bc] = z;
+            if (r != c) Va[bc + (int64_t)n * row] = zconj(z);
           }
         }
       }
-      __syncthreads();  // T read before the next component's dH overwrites it
     }
   }
 }
-
-size_t velo_lds_bytes(int n) { return sizeof(zd) * 2 * (size_t)velo_lds_pitch(n) * n; }
 
 // V (3,n,n) per k: planar [a][i + n j]  <->  reference (a fastest)
 __global__ void v_planar_to_ref(int n, int64_t nk, const zd* __restrict__ Vp, zd* __restrict__ Vr) {
@@ -535,16 +524,6 @@ struct PosLoad {
     return zmul(zcmul(f[i], f[j]), x);
   }
 };
-// f_m and the centres of a workgroup's k-point into LDS (threads t < n)
-__device__ inline void pos_phases(const TBPhase& tb, int n, int t, zd* f, double* tau) {
-  if (!tb.tau || t >= n) return;
-  const double* tm = tb.tau + 3 * t;
-  double sn, cs;
-  sincos(2.0 * 3.14159265358979323846 * (tb.kx * tm[0] + tb.ky * tm[1] + tb.kz * tm[2]), &sn, &cs);
-  f[t] = zd{cs, sn};
-#pragma unroll
-  for (int a = 0; a < 3; ++a) tau[3 * t + a] = tm[a];
-}
 // Omega(3,3) of one element: antisymmetric, zero diagonal in (a, b)
 __device__ inline void pos_store_om(zd* O, zd oyz, zd ozx, zd oxy) {
   O[0] = O[1 + 3 * 1] = O[2 + 3 * 2] = zd{0, 0};
@@ -1026,7 +1005,7 @@ bool velo_pos_scratch_ok(int n, size_t scratch_bytes) {
   return n <= 32 || scratch_bytes >= 18 * (size_t)n * n * sizeof(zd);
 }
 
-void launch_velo(hipStream_t s, const VeloArgs& va, int64_t nk, const zd* Hk, int64_t strideHk,
+void launch_velo(hipStream_t s, const VeloArgs& va, int64_t nk, zd* Hk, int64_t strideHk,
                  const KGeom& g, const zd* U, const double* E, zd* V, zd* A, zd* Om) {
   unsigned grid = (unsigned)(nk < 65536 ? nk : 65536);
   TBPhase tb;
@@ -1062,22 +1041,27 @@ void launch_velo(hipStream_t s, const VeloArgs& va, int64_t nk, const zd* Hk, in
                        Om, va.scratch);
     return;
   }
-  if (va.n > 32 && va.n <= 16 * VL_MAXT && va.gauge_trafo) {
-    const size_t lds = velo_lds_bytes(va.n);
-    (void)hipFuncSetAttribute((const void*)velo_lds_kernel,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    unsigned lgrid = (unsigned)(nk < 8192 ? nk : 8192);
-    hipLaunchKernelGGL(velo_lds_kernel, dim3(lgrid), dim3(256), lds, s, va.n, nk, Hk, strideHk,
-                       va.packed, tb, U, V);
-    return;
-  }
   if (va.n > 32) {
-    // T slots: 3 n^2 complex per workgroup (48 n^2 bytes), within the
-    // eigensolver's rotation records that va.scratch reuses (64 n^2 bytes or
-    // more per k-point of the block, and there are at least wgrid of them)
-    unsigned wgrid = (unsigned)(nk < 2048 ? nk : 2048);
-    hipLaunchKernelGGL(velo_wide_kernel, dim3(wgrid), dim3(256), 0, s, va.n, nk, Hk, strideHk,
-                       va.packed, tb, va.gauge_trafo, U, V, va.scratch);
+    if (tb.tau)
+      hipLaunchKernelGGL(velo_tb_kernel, dim3(grid), dim3(256), 0, s, va.n, nk, Hk, strideHk, tb);
+    const int nt = (va.n + 15) / 16;
+    // 8 slots of a column each, at most 65536 times 8 workgroups
+    const int64_t slots = (nk + 7) / 8 * nt;
+    const unsigned wgrid = 8 * (unsigned)(slots < 65536 ? slots : 65536);
+#define MEP_VELO_WIDE(NT)                                                                    \
+  case NT:                                                                                   \
+    hipLaunchKernelGGL((velo_wide_kernel<NT, (NT <= 4)>), dim3(wgrid), dim3(64), 0, s, va.n,      \
+                       nk, Hk, strideHk, va.gauge_trafo, U, V);                              \
+    break;
+    switch (nt) {
+      MEP_VELO_WIDE(3)
+      MEP_VELO_WIDE(4)
+      MEP_VELO_WIDE(5)
+      MEP_VELO_WIDE(6)
+      MEP_VELO_WIDE(7)
+      MEP_VELO_WIDE(8)
+    }
+#undef MEP_VELO_WIDE
     return;
   }
   hipLaunchKernelGGL(velo_mfma_kernel<zd>, dim3(grid), dim3(256), 0, s, va.n, nk, Hk, strideHk,
