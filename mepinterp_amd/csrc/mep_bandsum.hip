@@ -1424,47 +1424,54 @@ size_t bandsum_wide_lds_bytes(const BandArgs& b) {
 }
 
 // ===========================================================================
-// velo_ahc_tens / kubo_ohc_tens for 32 < n <= 128: per k, the pairs (x, y),
-// x != y, whose occupations differ at some E_F are compacted, in pair order,
-// into LDS chunks of up to 256 records (dE, f_x - f_y per E_F, the 9
-// Im(V_i(x,y) V_j(y,x)) and the 9 complex V_i(y,x) V_j(x,y)); thread
-// (slot, split) walks every split-th record for its IPT items = (hw, E_F),
-// accumulating in registers over all k; the splits are combined once at the
-// end.  Items beyond 256 IPT are taken in further passes over the k-points.
+// velo_ahc_tens / kubo_ohc_tens over a list of items (hw, E_F): per k, the
+// pairs x < y whose occupations differ at some E_F are compacted, in pair
+// order, into LDS chunks of up to 256 records; thread (slot, split) walks
+// every split-th record for its IPT items, accumulating in registers over all
+// k; the splits are combined once at the end.  Items beyond 256 IPT are taken
+// in further passes over the k-points.
+//
+// A record stands for (x, y) and (y, x).  With dE = E_x - E_y, f = f_x - f_y,
+// w = hw + i eta and P_ij = V_i(y, x) V_j(x, y), the two orders' weights are
+//   velo  g Im(P_ji - P_ij),  g = f / (dE^2 - w^2)
+//   ohc   f / (dE (dE - w)) P_ij - f / (dE (dE + w)) P_ji
+//         = g (P_ij - P_ji) + w g (P_ij + P_ji) / dE
+// so one complex g serves all of them: the sums of g A, A_c = P_ij - P_ji, and
+// of g S, S_ij = (P_ij + P_ji) / dE, are what the items keep, and w enters once
+// at the end.  With D = (dE - hw)(dE + hw) + eta^2 (no cancellation at
+// resonance) and B = 2 hw eta, g = (D + i B) r, r = f / (D^2 + B^2): the items
+// sum D r v and r v over the real values v of A and S, and B waits as well.
+// Hermitian V: Im A (3), Re S (3) and S_ii (3), the others being zero; general
+// V: those of all 18.
+//
+// Bound by FP64 VALU issue: 2 x 9 fma and about 13 more a record and item
+// (Hermitian V); four items a thread take the reads of a record from LDS off
+// the LDS return path.
+// n = 96, 256 frequencies, 2,744 k-points: 2.8 ms (three denominators for the
+// two orders, 24 sums an item: 4.2); n = 20, 80 items, 24,273: 0.50 ms (0.88);
+// general V, n = 14, 16 items, 2,730: 40 us (59).
 // ===========================================================================
 constexpr int HW_CH = 256;  // pair candidates per chunk (one per thread)
-constexpr int HW_IPT = 2;   // items per thread, Hermitian V
 
-
-// Records per pair (x, y) of differing occupation: dE, w_k (f_x - f_y) for
-// every E_F, then the V products.  General V: 9 Im(V_i(x,y) V_j(y,x)) and 9
-// complex V_i(y,x) V_j(x,y) (27 values).  V built here (Hermitian): with
-// P_ij = x_i conj(x_j), x_a = V_a(x, y), only Im P_ij and P_ij (i < j) and
-// |x_i|^2 (12 values), and the items accumulate sum rv Im P_ij,
-// X = sum Re(ro) P_ij, Y = sum Im(ro) P_ij and the same of |x_i|^2.
 template <bool HERM>
-__host__ __device__ constexpr int hw_vals() { return HERM ? 12 : 27; }
-template <bool HERM>
-__host__ __device__ constexpr int hw_accs() { return HERM ? 24 : 36; }
+__host__ __device__ constexpr int hw_vals() { return HERM ? 9 : 18; }
 
-// IPT items per thread: every record read from LDS feeds IPT items (the
-// LDS return path, not the VALU, limits one item per thread).
 template <bool HERM, int IPT>
-__global__ __launch_bounds__(256, IPT > 1 ? 2 : 3) void hwsum_kernel(BandArgs b, double Tsmear, AccLayout L,
+__global__ __launch_bounds__(256, 2) void hwsum_kernel(BandArgs b, double Tsmear, AccLayout L,
                                                        int64_t nk, const double* __restrict__ E,
                                                        const zd* __restrict__ V,
                                                        const double* __restrict__ w,
                                                        double* __restrict__ part) {
-  constexpr int NV = hw_vals<HERM>(), NA = hw_accs<HERM>(), HA = NA / 2;
+  constexpr int NV = hw_vals<HERM>(), NP = NV / 3;  // values; values of A, S and S_ii each
   extern __shared__ double smem[];
   const int n = b.n, nef = b.n_ef, nhw = b.n_hw;
-  const int PS = 1 + nef + NV;  // doubles per record: dE, dfv[nef], the products
+  const int PS = 1 + nef + NV;  // doubles per record: dE, f[nef], v[NV]
   double* Es = smem;
   double* fd = Es + n;
   int* cnt_w = reinterpret_cast<int*>(fd + (int64_t)nef * n);  // [4] per-wave counts
   double* st = fd + (int64_t)nef * n + 4;  // [HW_CH][PS]; reused for the split reduction
   const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
-  const int n2 = n * n;
+  const int n2 = n * n, npair = n * (n - 1) / 2;
   const bool finiteT = b.T_kelvin > 1e-2;
   const int items = nhw * nef;
   double* accp = part + (int64_t)blockIdx.x * L.total;
@@ -1478,20 +1485,21 @@ __global__ __launch_bounds__(256, IPT > 1 ? 2 : 3) void hwsum_kernel(BandArgs b,
     const bool act = split < S;
     bool iok[IPT];
     int ef[IPT];
-    zd wh[IPT], wh2[IPT];
+    double wr[IPT], B2[IPT];
+    const double eta2 = b.eta * b.eta;
 #pragma unroll
     for (int u = 0; u < IPT; ++u) {
       iok[u] = act && slot + IWT * u < IW;
       const int it = g0 + (iok[u] ? slot + IWT * u : 0);
       ef[u] = it / nhw;
-      wh[u] = zd{b.hw[it % nhw], b.eta};
-      wh2[u] = zmul(wh[u], wh[u]);
+      wr[u] = b.hw[it % nhw];
+      B2[u] = 4.0 * wr[u] * wr[u] * eta2;
     }
-    double acc[IPT][NA];
+    double aD[IPT][NV], aR[IPT][NV];  // sums of D r v and of r v
 #pragma unroll
     for (int u = 0; u < IPT; ++u)
 #pragma unroll
-      for (int q = 0; q < NA; ++q) acc[u][q] = 0.0;
+      for (int q = 0; q < NV; ++q) aD[u][q] = aR[u][q] = 0.0;
     for (int64_t k = blockIdx.x; k < nk; k += gridDim.x) {
       const double wk = w ? w[k] : 1.0;
       const zd* Vk = V + k * 3 * (int64_t)n2;
@@ -1507,13 +1515,15 @@ __global__ __launch_bounds__(256, IPT > 1 ? 2 : 3) void hwsum_kernel(BandArgs b,
           fd[idx] = finiteT ? 1.0 / (1.0 + exp((e - f) / Tsmear)) : ((e < f) ? 1.0 : 0.0);
         }
       }
-      for (int c0 = 0; c0 < n2; c0 += HW_CH) {
+      for (int c0 = 0; c0 < npair; c0 += HW_CH) {
         __syncthreads();  // fd ready; the previous chunk consumed
-        const int pidx = c0 + t;
-        const int x = pidx % n, y = pidx / n;
-        // Hermitian V: one record per unordered pair x < y, summed for both
-        // orders below; general V: every ordered pair
-        bool keep = pidx < n2 && (HERM ? x < y : x != y);
+        // pair x < y, p = x + y (y - 1) / 2
+        const int p = c0 + t;
+        int y = (int)((sqrtf(8.0f * (float)p + 1.0f) + 1.0f) * 0.5f);
+        if (y * (y + 1) / 2 <= p) ++y;
+        if (y * (y - 1) / 2 > p) --y;
+        const int x = p - y * (y - 1) / 2;
+        bool keep = p < npair;
         if (keep) {
           bool any = false;
           for (int e_ = 0; e_ < nef; ++e_) any |= fd[e_ + nef * x] != fd[e_ + nef * y];
@@ -1528,199 +1538,124 @@ __global__ __launch_bounds__(256, IPT > 1 ? 2 : 3) void hwsum_kernel(BandArgs b,
         const int cnt = cnt_w[0] + cnt_w[1] + cnt_w[2] + cnt_w[3];
         if (keep) {
           double* sp = st + (int64_t)(base + below) * PS;
-          sp[0] = Es[x] - Es[y];
+          const double dE = Es[x] - Es[y], iE = 1.0 / dE;
+          sp[0] = dE;
           for (int e_ = 0; e_ < nef; ++e_) sp[1 + e_] = wk * (fd[e_ + nef * x] - fd[e_ + nef * y]);
-          double* pq = sp + 1 + nef;
+          double* v = sp + 1 + nef;
           zd vxy[3];
 #pragma unroll
           for (int a = 0; a < 3; ++a) vxy[a] = Vk[a * (int64_t)n2 + x + (int64_t)n * y];
-          if constexpr (HERM) {
-            // pq: Im P_c (3), P_c (3 complex), |x_a|^2 (3); c = (0,1), (0,2), (1,2)
+          // v: A_c, S_c (c = (0,1), (0,2), (1,2)), S_ii
+          if constexpr (HERM) {  // V(y, x) = conj V(x, y): Im A, Re S, S_ii
 #pragma unroll
             for (int c = 0; c < 3; ++c) {
               const zd xi = vxy[c == 2 ? 1 : 0], xj = vxy[c == 0 ? 1 : 2];
-              const zd P = zd{xi.re * xj.re + xi.im * xj.im, xi.im * xj.re - xi.re * xj.im};
-              pq[c] = P.im;
-              pq[3 + 2 * c] = P.re;
-              pq[4 + 2 * c] = P.im;
-              pq[9 + c] = zabs2(vxy[c]);
+              v[c] = 2.0 * (xi.re * xj.im - xi.im * xj.re);
+              v[3 + c] = 2.0 * (xi.re * xj.re + xi.im * xj.im) * iE;
+              v[6 + c] = 2.0 * zabs2(vxy[c]) * iE;
             }
           } else {
             zd vyx[3];
 #pragma unroll
             for (int a = 0; a < 3; ++a) vyx[a] = Vk[a * (int64_t)n2 + y + (int64_t)n * x];
 #pragma unroll
-            for (int j = 0; j < 3; ++j)
-#pragma unroll
-              for (int i = 0; i < 3; ++i) {
-                const int q = i + 3 * j;
-                pq[q] = zmul(vxy[i], vyx[j]).im;
-                const zd q2 = zmul(vyx[i], vxy[j]);
-                pq[9 + 2 * q] = q2.re;
-                pq[9 + 2 * q + 1] = q2.im;
-              }
+            for (int c = 0; c < 3; ++c) {
+              const int i = c == 2 ? 1 : 0, j = c == 0 ? 1 : 2;
+              const zd pij = zmul(vyx[i], vxy[j]), pji = zmul(vyx[j], vxy[i]);
+              const zd A = zsub(pij, pji), Sc = zscale(zadd(pij, pji), iE);
+              const zd Sd = zscale(zmul(vyx[c], vxy[c]), 2.0 * iE);
+              v[2 * c] = A.re;
+              v[2 * c + 1] = A.im;
+              v[6 + 2 * c] = Sc.re;
+              v[7 + 2 * c] = Sc.im;
+              v[12 + 2 * c] = Sd.re;
+              v[13 + 2 * c] = Sd.im;
+            }
           }
         }
         __syncthreads();
-        // one record (dE, the weight f of each item, the products pq) into
-        // the items' sums
-        auto consume = [&](const double dE, const double* fv, const double* pq) {
+        if (act)
+          for (int j = split; j < cnt; j += S) {
+            const double* sp = st + (int64_t)j * PS;
+            const double dE = sp[0];
+            double v[NV];
+#pragma unroll
+            for (int q = 0; q < NV; ++q) v[q] = sp[1 + nef + q];
 #pragma unroll
             for (int u = 0; u < IPT; ++u) {
-              const double f = fv[u];
-              if constexpr (HERM) {
-                // the record of x < y stands for (x, y) and (y, x): (y, x) has
-                // -dE, -f and conj P, so its velo term equals (x, y)'s and its
-                // ohc weight is ro2 = -f / (dE (dE + w)).  One reciprocal for
-                // the three denominators; f = 0 records (another E_F differs)
-                // contribute exactly zero.
-                // with p = dE - w, q = dE + w: denv = p q, deno = dE p and
-                // the (y, x) denominator dE q, so R = f / (dE |p|^2 |q|^2)
-                // gives rv = 2 f / denv = 2 dE R conj(p q),
-                // ro = f / deno = |q|^2 R conj(p), ro2 = -|p|^2 R conj(q)
-                const double wr = wh[u].re, wi = wh[u].im;
-                const double pr = dE - wr, qr = dE + wr;
-                const double ap = pr * pr + wi * wi, aq = qr * qr + wi * wi;
-                const double R = f * rcp_nr(dE * ap * aq);
-                const double Rq = R * aq, Rp = R * ap, Rd = 2.0 * R * dE;
-                const zd rv = zd{(dE * dE - wh2[u].re) * Rd, wh2[u].im * Rd};
-                const double t1 = pr * Rq, t2 = qr * Rp;
-                const zd sp = zd{t1 - t2, wi * (Rq + Rp)};  // ro + ro2
-                const zd sm = zd{t1 + t2, wi * (Rq - Rp)};  // ro - ro2
-                // acc: [0..5] rv Im P_c, [6..11] Re(ro) |x_a|^2 then Im(ro) |x_a|^2,
-                // [12..17] Re(ro) P_c, [18..23] Im(ro) P_c, over both orders
+              // f = 0 records (another E_F differs) contribute exactly zero
+              const double D = (dE - wr[u]) * (dE + wr[u]) + eta2;
+              const double r = sp[1 + ef[u]] * rcp_nr(D * D + B2[u]), Dr = D * r;
 #pragma unroll
-                for (int c = 0; c < 3; ++c) {
-                  acc[u][2 * c] += pq[c] * rv.re;
-                  acc[u][2 * c + 1] += pq[c] * rv.im;
-                  acc[u][6 + c] += sp.re * pq[9 + c];
-                  acc[u][9 + c] += sp.im * pq[9 + c];
-                  acc[u][12 + 2 * c] += sp.re * pq[3 + 2 * c];
-                  acc[u][13 + 2 * c] += sm.re * pq[4 + 2 * c];
-                  acc[u][18 + 2 * c] += sp.im * pq[3 + 2 * c];
-                  acc[u][19 + 2 * c] += sm.im * pq[4 + 2 * c];
-                }
-              } else {
-                const zd denv = zd{dE * dE - wh2[u].re, -wh2[u].im};
-                const zd deno = zmul(zd{dE, 0.0}, zd{dE - wh[u].re, -wh[u].im});
-                const double av = zabs2(denv), ao = zabs2(deno);
-                // one reciprocal for both denominators
-                const double fi = f * rcp_nr(av * ao);
-                const double iv = fi * ao, io = fi * av;
-                const zd rv = zd{denv.re * iv, -denv.im * iv};
-                const zd ro = zd{deno.re * io, -deno.im * io};
-                // acc: [0..17] velo_q (re, im), [18..35] ohc_q (re, im)
-#pragma unroll
-                for (int q = 0; q < 9; ++q) {
-                  const double vim = pq[q];
-                  acc[u][2 * q] += vim * rv.re;
-                  acc[u][2 * q + 1] += vim * rv.im;
-                  // i * (q2o * ro)
-                  const double qr = pq[9 + 2 * q], qi = pq[9 + 2 * q + 1];
-                  acc[u][18 + 2 * q] -= qr * ro.im + qi * ro.re;
-                  acc[u][18 + 2 * q + 1] += qr * ro.re - qi * ro.im;
-                }
+              for (int q = 0; q < NV; ++q) {
+                aD[u][q] += Dr * v[q];
+                aR[u][q] += r * v[q];
               }
             }
-        };
-        if constexpr (HERM && IPT > 1) {
-          // the m records j = split, split + S, ... taken in pairs in two
-          // register sets, so one record's LDS loads are in flight while the
-          // other is summed.  No exit between a load and its use (the
-          // compiler would sink the loads to the use): past the last record
-          // the loads repeat it, and an odd m's extra record adds with
-          // weight 0 (exactly nothing: dE != 0 in every record)
-          if (act && split < cnt) {
-            constexpr int RW = 1 + IPT + NV;
-            const int m = (cnt - 1 - split) / S + 1;
-            auto rec = [&](int i) { return st + (int64_t)(split + (i < m ? i : m - 1) * S) * PS; };
-            auto ld = [&](const double* p, double* r) {
-              r[0] = p[0];
-#pragma unroll
-              for (int u = 0; u < IPT; ++u) r[1 + u] = p[1 + ef[u]];
-#pragma unroll
-              for (int q = 0; q < NV; ++q) r[1 + IPT + q] = p[1 + nef + q];
-            };
-            double ra[RW], rb[RW];
-            ld(rec(0), ra);
-            for (int i = 0; i < m; i += 2) {
-              ld(rec(i + 1), rb);
-              consume(ra[0], ra + 1, ra + 1 + IPT);
-              ld(rec(i + 2), ra);
-              double fb[IPT];
-#pragma unroll
-              for (int u = 0; u < IPT; ++u) fb[u] = (i + 1 < m) ? rb[1 + u] : 0.0;
-              consume(rb[0], fb, rb + 1 + IPT);
-            }
           }
-        } else if (act) {
-#pragma unroll 2
-          for (int j = split; j < cnt; j += S) {  // several records' LDS loads in flight
-            const double* sp = st + (int64_t)j * PS;
-            double fv[IPT];
-#pragma unroll
-            for (int u = 0; u < IPT; ++u) fv[u] = sp[1 + ef[u]];
-            consume(sp[0], fv, sp + 1 + nef);
-          }
-        }
       }
     }
-    // combine the splits of each item in two halves of the accumulators
-    // (red[split][item][HA] over the staging area); each half holds
-    // everything its outputs need
-    for (int half = 0; half < 2; ++half) {
+    // combine the splits of each item, A, S and S_ii in turn, in
+    // red[split][item][2 NP] over the staging area, and add what each gives:
+    // with G = sum g v (g = (D + i B) r), velo_ij = -Im part of A's sums (as a
+    // complex g), ohc_ij = i (G_A + w G_S), ohc_ji = i (w G_S - G_A), ohc_ii =
+    // i w G_Sii
+#pragma unroll
+    for (int third = 0; third < 3; ++third) {
       __syncthreads();
       if (act)
 #pragma unroll
         for (int u = 0; u < IPT; ++u)
           if (iok[u])
 #pragma unroll
-            for (int q = 0; q < HA; ++q)
-              st[(split * IW + slot + IWT * u) * HA + q] = acc[u][half * HA + q];
-      __syncthreads();
-      auto red = [&](int i2, int q) {
-        double sR = 0.0;
-        for (int u = 0; u < S; ++u) sR += st[(u * IW + i2) * HA + q];
-        return sR;
-      };
-      if constexpr (!HERM) {
-        for (int o = t; o < IW * 18; o += 256) {
-          const int i2 = o / 18, q = o % 18;
-          const int item = g0 + i2, hh = item % nhw, e2 = item / nhw;
-          accp[(half ? L.ohc : L.velo) + 2 * 9 * (hh + (int64_t)nhw * e2) + q] += red(i2, q);
-        }
-      } else {
-        // half 0: velo (antisymmetric, zero diagonal) and the ohc diagonal;
-        // half 1: the ohc off-diagonal entries
-        const int per = half ? 12 : 24;
-        for (int o = t; o < IW * per; o += 256) {
-          const int i2 = o / per, r = o % per;
-          const int item = g0 + i2, hh = item % nhw, e2 = item / nhw;
-          const int64_t rec = 2 * 9 * (hh + (int64_t)nhw * e2);
-          if (half == 0) {
-            if (r < 18) {  // velo_q, q = i + 3j, component r % 2
-              const int q = r / 2, cpx = r % 2, i = q % 3, j = q / 3;
-              if (i != j) {
-                const double v = red(i2, 2 * (i + j - 1) + cpx);
-                accp[L.velo + rec + r] += (i < j) ? v : -v;
-              }
-            } else {       // ohc_ii = i sum ro |x_i|^2 = (-Y, X)
-              const int i = (r - 18) / 2, cpx = (r - 18) % 2;
-              const double v = cpx ? red(i2, 6 + i) : -red(i2, 9 + i);
-              accp[L.ohc + rec + 2 * (4 * i) + cpx] += v;
+            for (int q = 0; q < NP; ++q) {
+              double* o = st + (split * IW + slot + IWT * u) * 2 * NP;
+              o[q] = aD[u][third * NP + q];
+              o[NP + q] = aR[u][third * NP + q];
             }
-          } else {         // ohc_ij (i < j) = (Xi - Yr, Xr + Yi); ohc_ji = (-(Xi + Yr), Xr - Yi)
-            const int c = r / 4, sel = r % 4;  // sel: (ij re, ij im, ji re, ji im)
-            const int i = (c == 2) ? 1 : 0, j = (c == 0) ? 1 : 2;
-            const double xr = red(i2, 2 * c), xi = red(i2, 2 * c + 1);
-            const double yr = red(i2, 6 + 2 * c), yi = red(i2, 6 + 2 * c + 1);
-            double v;
-            int q;
-            if (sel == 0) { v = xi - yr; q = i + 3 * j; }
-            else if (sel == 1) { v = xr + yi; q = i + 3 * j; }
-            else if (sel == 2) { v = -(xi + yr); q = j + 3 * i; }
-            else { v = xr - yi; q = j + 3 * i; }
-            accp[L.ohc + rec + 2 * q + (sel & 1)] += v;
+      __syncthreads();
+      for (int o = t; o < IW * 3; o += 256) {
+        const int i2 = o / 3, c = o % 3;
+        const int item = g0 + i2, hh = item % nhw, e2 = item / nhw;
+        const zd wq = zd{b.hw[hh], b.eta};
+        const double B = 2.0 * wq.re * wq.im;
+        auto G = [&](int q) {  // sum of g v_q over the splits
+          double sD = 0.0, sR = 0.0;
+          for (int u = 0; u < S; ++u) {
+            sD += st[(u * IW + i2) * 2 * NP + q];
+            sR += st[(u * IW + i2) * 2 * NP + NP + q];
+          }
+          return zd{sD, B * sR};
+        };
+        zd Gi = zd{0.0, 0.0}, Z;  // sum of g Im v; sum of g v
+        if constexpr (HERM) {
+          const zd x = G(c);
+          Gi = x;
+          Z = third == 0 ? zmuli(x) : x;
+        } else {
+          const zd x = G(2 * c);
+          Gi = G(2 * c + 1);
+          Z = zadd(x, zmuli(Gi));
+        }
+        double* av = accp + L.velo + 2 * 9 * (hh + (int64_t)nhw * e2);
+        double* ao = accp + L.ohc + 2 * 9 * (hh + (int64_t)nhw * e2);
+        const int i = c == 2 ? 1 : 0, j = c == 0 ? 1 : 2;
+        auto add = [](double* p, const zd& z, double sgn) {
+          p[0] += sgn * z.re;
+          p[1] += sgn * z.im;
+        };
+        if (third == 0) {
+          add(av + 2 * (i + 3 * j), Gi, -1.0);
+          add(av + 2 * (j + 3 * i), Gi, 1.0);
+          add(ao + 2 * (i + 3 * j), zmuli(Z), 1.0);
+          add(ao + 2 * (j + 3 * i), zmuli(Z), -1.0);
+        } else {
+          const zd iwZ = zmuli(zmul(wq, Z));
+          if (third == 1) {
+            add(ao + 2 * (i + 3 * j), iwZ, 1.0);
+            add(ao + 2 * (j + 3 * i), iwZ, 1.0);
+          } else {
+            add(ao + 2 * 4 * c, iwZ, 1.0);
           }
         }
       }
@@ -1728,19 +1663,19 @@ __global__ __launch_bounds__(256, IPT > 1 ? 2 : 3) void hwsum_kernel(BandArgs b,
   }
 }
 
-// items per thread: two for Hermitian V with many items (C5's 256
-// frequencies: 94.5 -> 83.4 ms per 32^3); few items (the single (hw, E_F)
-// pair sums) keep one, at the higher occupancy
+// items per thread: four from eight items on (n = 96, 256 items: 2.8 ms, one
+// 3.1; n = 20, 80 items: 0.50, 0.51); general V's 36 sums an item leave
+// registers for two, which was slower (n = 14, 16 items: 52 us, one 40)
 static int hwsum_ipt(const BandArgs& b) {
-  return (b.v_herm && (int64_t)b.n_hw * b.n_ef >= 128) ? HW_IPT : 1;
+  return b.v_herm && (int64_t)b.n_hw * b.n_ef >= 8 ? 4 : 1;
 }
 
+// (the records' room is what the number of Fermi levels is limited by: 13 and
+// 28 doubles beside a record's levels)
 size_t hwsum_lds_bytes(const BandArgs& b) {
-  const size_t nv = b.v_herm ? hw_vals<true>() : hw_vals<false>();
-  const size_t ha = (b.v_herm ? hw_accs<true>() : hw_accs<false>()) / 2;
-  const size_t ps = 1 + (size_t)b.n_ef + nv;
-  const size_t ipt = (size_t)hwsum_ipt(b);
-  const size_t stage = (size_t)HW_CH * ps > 256 * ipt * ha ? (size_t)HW_CH * ps : 256 * ipt * ha;
+  const size_t ps = (size_t)b.n_ef + (b.v_herm ? 13 : 28);
+  const size_t red = 256 * 24;  // the split reduction: 24 doubles a thread at most
+  const size_t stage = (size_t)HW_CH * ps > red ? (size_t)HW_CH * ps : red;
   return sizeof(double) * ((size_t)b.n + (size_t)b.n_ef * b.n + 4 + stage);
 }
 
@@ -1883,22 +1818,14 @@ static void launch_hwsum(hipStream_t s, const BandArgs& b, double Tsmear, const 
                          int64_t nk, const double* E, const zd* V, const double* w, int nblocks,
                          double* part) {
   const size_t lh = hwsum_lds_bytes(b);
-  if (b.v_herm && hwsum_ipt(b) == HW_IPT) {
-    (void)hipFuncSetAttribute((const void*)hwsum_kernel<true, HW_IPT>,
+  auto go = [&](auto kernel) {
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lh);
-    hipLaunchKernelGGL((hwsum_kernel<true, HW_IPT>), dim3(nblocks), dim3(256), lh, s, b, Tsmear, L,
-                       nk, E, V, w, part);
-  } else if (b.v_herm) {
-    (void)hipFuncSetAttribute((const void*)hwsum_kernel<true, 1>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lh);
-    hipLaunchKernelGGL((hwsum_kernel<true, 1>), dim3(nblocks), dim3(256), lh, s, b, Tsmear, L, nk,
-                       E, V, w, part);
-  } else {
-    (void)hipFuncSetAttribute((const void*)hwsum_kernel<false, 1>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lh);
-    hipLaunchKernelGGL((hwsum_kernel<false, 1>), dim3(nblocks), dim3(256), lh, s, b, Tsmear, L, nk,
-                       E, V, w, part);
-  }
+    hipLaunchKernelGGL(kernel, dim3(nblocks), dim3(256), lh, s, b, Tsmear, L, nk, E, V, w, part);
+  };
+  if (!b.v_herm) go(hwsum_kernel<false, 1>);
+  else if (hwsum_ipt(b) == 4) go(hwsum_kernel<true, 4>);
+  else go(hwsum_kernel<true, 1>);
 }
 
 void launch_bandsum(hipStream_t s, const BandArgs& b, int64_t nk, const double* E, const zd* V,
