@@ -14,12 +14,12 @@
 // Per k the workgroup stages in LDS the three velocity planes V_a (padded
 // column-major) and the antisymmetric reciprocal table
 // r(m, n) = 1 / (E_n - E_m) (0 on the diagonal), so no band sum divides.
-//   pair phase    lane (n0, part) of every wave walks n = part, part + P,
-//                 ...; wave 0 sums the Berry curvature of n0 (and finds the
-//                 Niu exclusion windows), wave 1 the local (LC) MEP terms,
-//                 waves 2-3 (single (hw, E_F)) the velo/ohc pair sums; the
-//                 band sums are wavefront shuffle reductions (several
-//                 (hw, E_F) items: hwsum_kernel, launched after this one);
+//   pair phase    Hermitian V: each wave takes 8 bands n0, lane (n0, part)
+//                 walks n = part, part + 8, ..., and the sums over the parts
+//                 are scattered over the lanes; general V: wave 0 the Berry
+//                 curvature, wave 1 the local (LC) MEP terms, wave 2 the
+//                 velo/ohc pair sums (single (hw, E_F); several items:
+//                 hwsum_kernel, launched after this one);
 //   itinerant     C_j = V_k B_l - V_l B_k, (j,k,l) cyclic, with
 //                 B_l(m, n0) = V_l(m, n0) r(m, n0): three complex n x n
 //                 products on FP64 MFMA (three real products per complex
@@ -57,22 +57,28 @@ AccLayout acc_layout(const BandArgs& b) {
 
 constexpr int BS_THREADS = 256;
 
-// LDS plan: V planes (zd) 3*PL | r table PL | E NMAX | fd nef*NMAX |
-// F2 guarded NT*9*NMAX | IC tile sums 9*NT*NT*nef | red NMAX |
-// per-band Berry and LC tensors 18*NMAX | pair sums 96 | acc total |
-// Niu windows 2*NMAX*NMAX bytes              (doubles after the V planes)
+// LDS plan: V planes (zd) 3*PL | E NMAX | r table PL | fd nef*NMAX | IC per
+// band NT*9*NMAX, twice (all terms, Niu-kept terms) | red NMAX | per-band
+// Berry and LC tensors 18*NMAX | pair sums 40 | acc total | Niu windows
+// 2*NMAX*NMAX bytes                         (doubles after the V planes)
 template <int NMAX>
 struct BsLds {
   static constexpr int LD = NMAX + 1;
   static constexpr int PL = NMAX * LD;
   static constexpr int NT = NMAX / 16;  // 16-row tiles per matrix
   static size_t doubles(int nef, int64_t total) {
-    return (size_t)PL + NMAX + (size_t)nef * NMAX + (size_t)NT * 9 * NMAX +
-           (size_t)9 * NT * NT * nef + NMAX + 18 * NMAX + 96 + (size_t)total;
+    return (size_t)PL + NMAX + (size_t)nef * NMAX + 2 * (size_t)NT * 9 * NMAX + NMAX + 18 * NMAX +
+           40 + (size_t)total;
   }
   static size_t bytes(int nef, int64_t total) {
     return sizeof(zd) * 3 * (size_t)PL + sizeof(double) * doubles(nef, total) +
            2 * (size_t)NMAX * NMAX;
+  }
+  // what the number of Fermi levels is limited by (above a few levels more
+  // than the kernel takes)
+  static size_t limit_bytes(int nef, int64_t total) {
+    return bytes(nef, total) + 56 * sizeof(double) + sizeof(double) * 9 * NT * (NT * (size_t)nef) -
+           sizeof(double) * 9 * NT * NMAX;
   }
 };
 
@@ -83,7 +89,15 @@ struct BsLds {
 // the same order as velo_mfma_kernel (so V, and every sum, is bit-identical
 // to the two-kernel path).  n in 17..32, no position operator, Wannier
 // convention.
-template <int NMAX, bool FUSED>
+//
+// Bound by issue: the FP64 MFMA products take 0.45 of the time at n = 32 and do
+// not overlap with the VALU work of the other phases, so what counts is the
+// instructions: one sum instead of two where the Niu guards exclude nothing
+// (decided per k-point), per-k reductions scattered over the lanes or kept in
+// registers over all k-points, one weight per pair.
+// n = 32, 262,144 k-points, all tensors: 15.8 ms (17.6 before these); n = 20,
+// 24,273, five Fermi levels, V read: 0.85 ms (1.11).
+template <int NMAX, bool FUSED, bool HERM>
 __global__ __launch_bounds__(BS_THREADS, 2) void bandsum_kernel(BandArgs b, double Tsmear,
                                                                 AccLayout L, int64_t gap,
                                                                 int64_t nk,
@@ -100,22 +114,21 @@ __global__ __launch_bounds__(BS_THREADS, 2) void bandsum_kernel(BandArgs b, doub
   constexpr int LD = S_::LD, PL = S_::PL, NT = S_::NT;
   // U's plane (PL complex) lives over the per-k tables between the r table
   // and the accumulators while V is formed
-  static_assert(!FUSED || (NMAX == 32 && PL + NMAX + NT * 9 * NMAX + NMAX + 18 * NMAX + 96 >= 2 * PL),
+  static_assert(!FUSED || (NMAX == 32 && HERM && PL + 2 * NT * 9 * NMAX + NMAX >= 2 * PL),
                 "fused velocities: U's plane must fit below the accumulators");
   extern __shared__ __attribute__((aligned(16))) double smem[];
   const int n = b.n, nef = b.n_ef, nhw = b.n_hw, nval = b.n_val;
   zd* Vs = reinterpret_cast<zd*>(smem);
-  double* Rs = reinterpret_cast<double*>(Vs + 3 * PL);
-  double* Es = Rs + PL;
-  double* fd = Es + NMAX;
-  double* QF = fd + (int64_t)nef * NMAX;        // [NT][9][NMAX] guarded IC per band
-  double* TS = QF + NT * 9 * NMAX;              // [3*NT*NT tiles][3][nef] Kubo IC tile sums
-  double* red = TS + 9 * NT * NT * nef;
+  double* Es = reinterpret_cast<double*>(Vs + 3 * PL);
+  double* Rs = Es + NMAX;
+  double* fd = Rs + PL;
+  double* QK = fd + (int64_t)nef * NMAX;        // [NT][9][NMAX] IC per band, row tile by row tile
+  double* QF = QK + NT * 9 * NMAX;              // the same over the Niu-kept terms
+  double* red = QF + NT * 9 * NMAX;
   double* OMA = red + NMAX;                     // [9][NMAX] Berry curvature per band
   double* F3A = OMA + 9 * NMAX;                 // [9][NMAX] Kubo LC tensor per band
-  double* PW = F3A + 9 * NMAX;                  // velo / ohc pair sums: [4 waves][24]
-                                                // (Hermitian V) or [36] (general V)
-  double* acc = PW + 96;
+  double* PW = F3A + 9 * NMAX;                  // velo / ohc pair sums [36] (general V)
+  double* acc = PW + 40;
   uint8_t* win = reinterpret_cast<uint8_t*>(acc + L.total);  // [n0][n] lo, hi
   const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
   const int n2 = n * n;
@@ -124,10 +137,9 @@ __global__ __launch_bounds__(BS_THREADS, 2) void bandsum_kernel(BandArgs b, doub
   const bool doK = (b.jobs & MEP_JOB_KUBO) != 0;
   const bool doNjob = (b.jobs & MEP_JOB_MEP) != 0;
   const bool pmode = doAHC && (nhw * nef == 1);
-  // V(n, m) = conj(V(m, n)) holds for V built here without a position
-  // operator (with one, the reference's connection is not Hermitian; V from
-  // a caller is taken as it is)
-  const bool herm = b.v_herm != 0;
+  // HERM: V(n, m) = conj(V(m, n)), which holds for V built here without a
+  // position operator (with one, the reference's connection is not Hermitian;
+  // V from a caller is taken as it is)
   const double tol = b.kubo_tol;
   for (int64_t c = t; c < L.total; c += BS_THREADS) acc[c] = 0.0;
   // V planes, r, E and fd are staged for indices < n only: their padding
@@ -136,6 +148,8 @@ __global__ __launch_bounds__(BS_THREADS, 2) void bandsum_kernel(BandArgs b, doub
 
   const zd wq = zd{b.hw[0], b.eta};
   const zd w2 = zmul(wq, wq);
+  const double eta2 = b.eta * b.eta, B2 = 4.0 * wq.re * wq.re * eta2;
+  double pacc[3] = {0.0, 0.0, 0.0};  // Hermitian V: this lane's velo / ohc pair sums, over all k
 
   // FUSED: U and the packed dH_a of a k-point, loaded into registers during
   // the last (light) phase of the previous k-point
@@ -143,6 +157,7 @@ __global__ __launch_bounds__(BS_THREADS, 2) void bandsum_kernel(BandArgs b, doub
   constexpr int ND = (NMAX * (NMAX + 1) / 2 + BS_THREADS - 1) / BS_THREADS;
   const int np = n * (n + 1) / 2;
   zd ut[FUSED ? NU : 1], dt[3][FUSED ? ND : 1];
+  double et = 0.0;
   auto fetch = [&](int64_t kk) {
     const int tt = threadIdx.x;
     const bool ok = kk < nk;
@@ -160,6 +175,7 @@ __global__ __launch_bounds__(BS_THREADS, 2) void bandsum_kernel(BandArgs b, doub
       for (int a = 0; a < 3; ++a)
         dt[a][u] = (ok && p < np) ? X[(int64_t)(1 + a) * np + p] : zd{0.0, 0.0};
     }
+    et = (ok && tt < n) ? E[kk * n + tt] : 0.0;
   };
   if constexpr (FUSED) fetch(blockIdx.x);
 
@@ -179,8 +195,11 @@ __global__ __launch_bounds__(BS_THREADS, 2) void bandsum_kernel(BandArgs b, doub
       // dH_a, then V_a from the accumulators into the V planes.  Rows and
       // columns >= n stay zero in every plane, so no operand load is guarded.
       zd* Us = reinterpret_cast<zd*>(Rs);
-      for (int c = t; c < PL; c += BS_THREADS) stz(Us + c, zd{0.0, 0.0});
-      __syncthreads();  // U's plane is zero
+      if (n < NMAX) {
+        for (int c = t; c < PL; c += BS_THREADS) stz(Us + c, zd{0.0, 0.0});
+        __syncthreads();  // U's plane is zero
+      }
+      if (t < n) Es[t] = et;
 #pragma unroll
       for (int u = 0; u < NU; ++u) {
         const int idx = t + BS_THREADS * u;
@@ -256,11 +275,14 @@ __global__ __launch_bounds__(BS_THREADS, 2) void bandsum_kernel(BandArgs b, doub
           const int row = r0 + kq + 4 * v;
           stz(Vs + a * PL + row + LD * bc, zd{q1[a][v] - q2[a][v], q3[a][v] - q1[a][v] - q2[a][v]});
         }
-      // the r table, E and the occupations are zero again, E in its slot
-      const int zn = PL + NMAX + nef * NMAX;
-      for (int c = t; c < zn; c += BS_THREADS) {
-        const int e = c - PL;
-        Rs[c] = (e >= 0 && e < n) ? E[k * n + e] : 0.0;
+      // the r table's diagonal and padding are zero again
+      if (n < NMAX) {
+        for (int c = t; c < PL; c += BS_THREADS) {
+          const int i = c % LD, j = c / LD;
+          if (i >= n || j >= n || i == j) Rs[c] = 0.0;
+        }
+      } else if (t < NMAX) {
+        Rs[t + LD * t] = 0.0;
       }
     } else {
     const zd* Vk = V + k * 3 * (int64_t)n2;
@@ -276,7 +298,7 @@ __global__ __launch_bounds__(BS_THREADS, 2) void bandsum_kernel(BandArgs b, doub
           const int j = jb + JS * jj;
           vt[a][jj] = (i < n && j < n) ? Vk[a * n2 + i + n * j] : zd{0.0, 0.0};
         }
-      const double et = (t < n) ? E[k * n + t] : 0.0;
+      et = (t < n) ? E[k * n + t] : 0.0;
 #pragma unroll
       for (int a = 0; a < 3; ++a)
 #pragma unroll
@@ -286,8 +308,21 @@ __global__ __launch_bounds__(BS_THREADS, 2) void bandsum_kernel(BandArgs b, doub
         }
       if (t < n) Es[t] = et;
     }
-    }
     __syncthreads();
+    }
+    // mep_niu's guards exclude nothing where, with g the gap to the nearest
+    // band, g^3 > kubo_tol for every valence band (the energies are sorted and
+    // rounding is monotone, so every |(E0-En)^2 (E0-Em)| and |E0-En|^3 is at
+    // least that): such a k-point needs no windows and no second sums.  The
+    // same in every wavefront.  (n = 32, 16 valence bands over 4 Ha: 95 of 100
+    // k-points at the default kubo_tol.)
+    bool clean = true;
+    if (doNjob && lane < n && lane < nval) {
+      const double g0 = lane > 0 ? Es[lane] - Es[lane - 1] : HUGE_VAL;
+      const double g1 = lane < n - 1 ? Es[lane + 1] - Es[lane] : HUGE_VAL;
+      clean = g0 * g0 * g0 > tol && g1 * g1 * g1 > tol;
+    }
+    clean = __ballot(!clean) == 0;
     // ---- r(m, c) = 1 / (E_c - E_m); occupations ---------------------------
     {
       // one division per pair m < c: r(c, m) = -r(m, c) exactly in IEEE
@@ -303,7 +338,7 @@ __global__ __launch_bounds__(BS_THREADS, 2) void bandsum_kernel(BandArgs b, doub
         Rs[c + LD * m] = -v;
       }
     }
-    if (doNjob)
+    if (doNjob && !clean)
       for (int idx = t; idx < nval * NMAX; idx += BS_THREADS) {
         // mep_niu's guard |(E0-En)^2 (E0-Em)| > kubo_tol: energies are
         // sorted, so the excluded m of (n0, n) form one range around n0
@@ -328,7 +363,7 @@ __global__ __launch_bounds__(BS_THREADS, 2) void bandsum_kernel(BandArgs b, doub
     }
     __syncthreads();
 
-    if (!herm) {
+    if constexpr (!HERM) {
       // ==== pair phase, general V (position operator: the reference's
       // connection makes V non-Hermitian, so V(n, n0) is read as stored).
       // Lane (p0, pp) of each wave walks n = pp, pp + P, ...: wave 0 the
@@ -461,22 +496,17 @@ __global__ __launch_bounds__(BS_THREADS, 2) void bandsum_kernel(BandArgs b, doub
       const double E0 = Es[n0];
       double om[3] = {0.0, 0.0, 0.0};        // sum r^2 Im P_ij
       double gd[3] = {0.0, 0.0, 0.0};        // sum r^3 |x_i|^2
-      double gdm[3] = {0.0, 0.0, 0.0};       // the same over Niu-kept n
-      zd go[3], gom[3];                      // sum r^3 P_ij (i < j), kept
+      zd go[3];                              // sum r^3 P_ij (i < j)
       double ps[24];                         // velo / ohc pair sums
 #pragma unroll
-      for (int c = 0; c < 3; ++c) go[c] = gom[c] = zd{0.0, 0.0};
+      for (int c = 0; c < 3; ++c) go[c] = zd{0.0, 0.0};
 #pragma unroll
       for (int c = 0; c < 24; ++c) ps[c] = 0.0;
       const double f0 = pmode ? fd[n0] : 0.0;
-      for (int nn = part; nn < n; nn += 8) {
+      auto pair = [&](int nn, zd* P, double* d) {
         zd x[3];
 #pragma unroll
         for (int a = 0; a < 3; ++a) x[a] = ldz(Vs + a * PL + n0 + LD * nn);
-        const double r = Rs[nn + LD * n0];
-        const double r2 = r * r, r3 = r2 * r;
-        zd P[3];
-        double d[3];
 #pragma unroll
         for (int a = 0; a < 3; ++a) d[a] = x[a].re * x[a].re + x[a].im * x[a].im;
 #pragma unroll
@@ -484,57 +514,50 @@ __global__ __launch_bounds__(BS_THREADS, 2) void bandsum_kernel(BandArgs b, doub
           const zd xi = x[c == 2 ? 1 : 0], xj = x[c == 0 ? 1 : 2];
           P[c] = zd{xi.re * xj.re + xi.im * xj.im, xi.im * xj.re - xi.re * xj.im};
         }
+      };
+      for (int nn = part; nn < n; nn += 8) {
+        zd P[3];
+        double d[3];
+        pair(nn, P, d);
+        const double r = Rs[nn + LD * n0];
+        const double r2 = r * r, r3 = r2 * r;
         if (doAHC)
 #pragma unroll
           for (int c = 0; c < 3; ++c) om[c] += r2 * P[c].im;
         if (doK || doNjob) {
-          const double dn = E0 - Es[nn];
-          const double r3m = (doN && fabs(dn * dn * dn) > tol) ? r3 : 0.0;
 #pragma unroll
-          for (int a = 0; a < 3; ++a) {
-            gd[a] += r3 * d[a];
-            gdm[a] += r3m * d[a];
-          }
+          for (int a = 0; a < 3; ++a) gd[a] += r3 * d[a];
 #pragma unroll
-          for (int c = 0; c < 3; ++c) {
-            go[c] = zd{go[c].re + r3 * P[c].re, go[c].im + r3 * P[c].im};
-            gom[c] = zd{gom[c].re + r3m * P[c].re, gom[c].im + r3m * P[c].im};
-          }
+          for (int c = 0; c < 3; ++c) go[c] = zd{go[c].re + r3 * P[c].re, go[c].im + r3 * P[c].im};
         }
         if (pmode) {
-          const double dE = E0 - Es[nn];
-          const double dfv = f0 - fd[nn];
-          const zd denv = zd{dE * dE - w2.re, -w2.im};
-          const zd deno = zmul(zd{dE, 0.0}, zd{dE - wq.re, -wq.im});
-          // one reciprocal for both denominators
-          const double av = zabs2(denv), ao = zabs2(deno);
-          const double ia = rcp_nr(av * ao);
-          const double iv = ia * ao, io = ia * av;
-          // selects, not a branch, drop n == n0 (where 1/deno is not finite)
-          const bool off = nn != n0;
-          const zd rv = off ? zd{denv.re * iv * dfv, -denv.im * iv * dfv} : zd{0.0, 0.0};
-          const zd ro = off ? zd{deno.re * io * dfv, -deno.im * io * dfv} : zd{0.0, 0.0};
+          // both orders of a pair weigh g = f / (dE^2 - w^2) = (D + i B) q and
+          // w g / dE (see hwsum_kernel): the sums of D q v and q v, v = Im P,
+          // Re P / dE, |x|^2 / dE.  Selects, not a branch, drop pairs of equal
+          // occupation, n = n0 among them
+          const double dE = E0 - Es[nn], f = f0 - fd[nn];
+          const bool on = f != 0.0 && nn != n0 && n0 < n;
+          const double D = (dE - wq.re) * (dE + wq.re) + eta2;
+          const double q = on ? f * rcp_nr(D * D + B2) : 0.0, Dq = D * q;
+          const double rs = on ? r : 0.0, qr = q * rs, Dqr = Dq * rs;
 #pragma unroll
           for (int c = 0; c < 3; ++c) {
-            ps[2 * c] += rv.re * P[c].im;
-            ps[2 * c + 1] += rv.im * P[c].im;
-            ps[6 + 2 * c] += ro.re * P[c].re;
-            ps[7 + 2 * c] += ro.re * P[c].im;
-            ps[12 + 2 * c] += ro.im * P[c].re;
-            ps[13 + 2 * c] += ro.im * P[c].im;
-            ps[18 + c] += ro.re * d[c];
-            ps[21 + c] += ro.im * d[c];
+            ps[c] += Dq * P[c].im;
+            ps[3 + c] += q * P[c].im;
+            ps[6 + c] += Dqr * P[c].re;
+            ps[9 + c] += qr * P[c].re;
+            ps[12 + c] += Dqr * d[c];
+            ps[15 + c] += qr * d[c];
           }
         }
       }
       // local terms of n0: F3_ij = Re(z_l G_ik - z_k G_il), (j, k, l) cyclic,
       // z = V(n0, n0), G_ik = sum_n r^3 x_i conj(x_k) (Hermitian in i, k)
-      double v24[24];
-      {
-        zd z[3];
+      zd z[3];
 #pragma unroll
-        for (int a = 0; a < 3; ++a) z[a] = ldz(Vs + a * PL + n0 + LD * n0);
-        auto G = [&](const double* gd_, const zd* go_, int i, int k) {
+      for (int a = 0; a < 3; ++a) z[a] = ldz(Vs + a * PL + n0 + LD * n0);
+      auto local = [&](const double* gd_, const zd* go_, double* o) {
+        auto G = [&](int i, int k) {
           if (i == k) return zd{gd_[i], 0.0};
           const zd g = go_[i + k - 1];
           return i < k ? g : zd{g.re, -g.im};
@@ -544,52 +567,66 @@ __global__ __launch_bounds__(BS_THREADS, 2) void bandsum_kernel(BandArgs b, doub
           const int k = (j + 1) % 3, l = (j + 2) % 3;
 #pragma unroll
           for (int i = 0; i < 3; ++i) {
-            const zd a = G(gd, go, i, k), bb = G(gd, go, i, l);
-            const zd am = G(gdm, gom, i, k), bm = G(gdm, gom, i, l);
-            v24[i + 3 * j] = (z[l].re * a.re - z[l].im * a.im) - (z[k].re * bb.re - z[k].im * bb.im);
-            v24[9 + i + 3 * j] =
-                (z[l].re * am.re - z[l].im * am.im) - (z[k].re * bm.re - z[k].im * bm.im);
+            const zd a = G(i, k), bb = G(i, l);
+            o[i + 3 * j] = (z[l].re * a.re - z[l].im * a.im) - (z[k].re * bb.re - z[k].im * bb.im);
           }
         }
+      };
+      // sums over the 8 parts (lane bits 3-5), scattered: lane (n0, g) ends
+      // with the slots 8 g5 + 4 g4 + 2 g3 + s, s < 2, of its n0
+      double v16[16], v2[2];
+      local(gd, go, v16);
+#pragma unroll
+      for (int c = 0; c < 3; ++c) v16[9 + c] = om[c];
+#pragma unroll
+      for (int c = 12; c < 16; ++c) v16[c] = 0.0;
+      scatter_sum<16>(v16, v2, lane);
+      const int base2 = 8 * ((lane >> 5) & 1) + 4 * ((lane >> 4) & 1) + 2 * ((lane >> 3) & 1);
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        const int slot = base2 + s;
+        if (slot < 9) {
+          F3A[slot * NMAX + n0] = v2[s];
+          if (clean && doN) acc[L.nlc + slot + 9 * n0] += wk * v2[s];
+        } else if (slot < 12) {  // Omega_ij = -2 v, Omega_ji = 2 v for pair (i, j)
+          const int c = slot - 9, i = (c == 2) ? 1 : 0, j = (c == 0) ? 1 : 2;
+          OMA[(i + 3 * j) * NMAX + n0] = -2.0 * v2[s];
+          OMA[(j + 3 * i) * NMAX + n0] = 2.0 * v2[s];
+          OMA[4 * c * NMAX + n0] = 0.0;
+        }
+      }
+      if (!clean) {  // the local terms over the Niu-kept n
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
-          v24[18 + c] = om[c];
-          v24[21 + c] = 0.0;
+          gd[c] = 0.0;
+          go[c] = zd{0.0, 0.0};
         }
-      }
-      // sums over the 8 parts (lane bits 3-5), scattered: lane (n0, g) ends
-      // with the slots 12 g5 + 6 g4 + 3 g3 + s, s < 3, of its n0
-      double v3[3];
-      scatter_sum24(v24, v3, lane);
-      {
-        const int base = 12 * ((lane >> 5) & 1) + 6 * ((lane >> 4) & 1) + 3 * ((lane >> 3) & 1);
+#pragma unroll 1
+        for (int nn = part; nn < n; nn += 8) {
+          zd P[3];
+          double d[3];
+          pair(nn, P, d);
+          const double r = Rs[nn + LD * n0], dn = E0 - Es[nn];
+          const double r3 = (doN && fabs(dn * dn * dn) > tol) ? r * r * r : 0.0;
 #pragma unroll
-        for (int s = 0; s < 3; ++s) {
-          const int slot = base + s;
-          if (slot < 9) {
-            F3A[slot * NMAX + n0] = v3[s];
-          } else if (slot < 18) {
-            if (doN) acc[L.nlc + (slot - 9) + 9 * n0] += wk * v3[s];
-          } else if (slot < 21) {  // Omega_ij = -2 v, Omega_ji = 2 v for pair (i, j)
-            const int c = slot - 18, i = (c == 2) ? 1 : 0, j = (c == 0) ? 1 : 2;
-            OMA[(i + 3 * j) * NMAX + n0] = -2.0 * v3[s];
-            OMA[(j + 3 * i) * NMAX + n0] = 2.0 * v3[s];
-          } else {                 // Omega_ii = 0
-            OMA[4 * (slot - 21) * NMAX + n0] = 0.0;
-          }
+          for (int a = 0; a < 3; ++a) gd[a] += r3 * d[a];
+#pragma unroll
+          for (int c = 0; c < 3; ++c) go[c] = zd{go[c].re + r3 * P[c].re, go[c].im + r3 * P[c].im};
         }
+        local(gd, go, v16);
+#pragma unroll
+        for (int c = 9; c < 16; ++c) v16[c] = 0.0;
+        scatter_sum<16>(v16, v2, lane);
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+          if (doN && base2 + s < 9) acc[L.nlc + base2 + s + 9 * n0] += wk * v2[s];
       }
       if (pmode) {
-        scatter_sum24(ps, v3, lane);
-        const int base = 12 * ((lane >> 5) & 1) + 6 * ((lane >> 4) & 1) + 3 * ((lane >> 3) & 1);
+        double v3[3];
+        scatter_sum<24>(ps, v3, lane);
 #pragma unroll
-        for (int s = 0; s < 3; ++s) v3[s] = group8_sum(v3[s]);
-        if ((lane & 7) == 0)
-#pragma unroll
-          for (int s = 0; s < 3; ++s) PW[wv * 24 + base + s] = v3[s];
+        for (int s = 0; s < 3; ++s) pacc[s] += wk * v3[s];
       }
-    } else if (pmode && lane < 24) {
-      PW[wv * 24 + lane] = 0.0;
     }
     }
     // (the Hall and optical conductivities of several (hw, E_F) items run in
@@ -625,8 +662,7 @@ __global__ __launch_bounds__(BS_THREADS, 2) void bandsum_kernel(BandArgs b, doub
         mep_v4d p1[JN], p2[JN], p3[JN];
 #pragma unroll
         for (int jj = 0; jj < JN; ++jj) p1[jj] = p2[jj] = p3[jj] = mep_v4d{0, 0, 0, 0};
-#pragma unroll
-        for (int k0 = 0; k0 < NMAX; k0 += 4) {
+        auto step = [&](int k0) {
           const int m = k0 + kq;
           const double rr = Rs[m + LD * bc];
           zd a[NP], s[NP];
@@ -653,7 +689,13 @@ __global__ __launch_bounds__(BS_THREADS, 2) void bandsum_kernel(BandArgs b, doub
             p2[jj] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[ll].im, -s[kk].im, p2[jj], 0, 0, 0);
             p3[jj] = __builtin_amdgcn_mfma_f64_16x16x4f64(as[ll], -ss[kk], p3[jj], 0, 0, 0);
           }
-        }
+        };
+        constexpr int K1 = NMAX == 32 ? 24 : NMAX;  // one branch for the last quarter
+#pragma unroll
+        for (int k0 = 0; k0 < K1; k0 += 4) step(k0);
+        if (n > K1)
+#pragma unroll
+          for (int k0 = K1; k0 < NMAX; k0 += 4) step(k0);
         // contraction with A_i(n0, n) = V_i(n0, n) r(n, n0)^2, n0 = column;
         // r(n, n0) = 0 for n = n0 and outside n, so those rows add nothing.
         // f2[i + 3 jj]: component (i, j) with j = jj (JN == 3) or jsel
@@ -677,7 +719,7 @@ __global__ __launch_bounds__(BS_THREADS, 2) void bandsum_kernel(BandArgs b, doub
           const double rr2 = rr * rr;
           bool narrow = false;
           wterm[v] = false;
-          if (doN && row < n && row != n0) {
+          if (!clean && doN && row < n && row != n0) {
             const int lo = win[2 * (n0 * NMAX + row)], hi = win[2 * (n0 * NMAX + row) + 1];
             const bool all = lo == 0 && hi == n - 1;
             narrow = !all && !wide(lo, hi);
@@ -693,12 +735,12 @@ __global__ __launch_bounds__(BS_THREADS, 2) void bandsum_kernel(BandArgs b, doub
             for (int i = 0; i < 3; ++i) {
               const double c = ai[i].re * cv.re - ai[i].im * cv.im;
               f2[i + 3 * jj] -= c;
-              f2m[i + 3 * jj] -= narrow ? c : 0.0;
+              if (!clean) f2m[i + 3 * jj] -= narrow ? c : 0.0;
             }
           }
         }
         // window terms, after the accumulators are dead
-        if (doN)
+        if (!clean && doN)
 #pragma unroll 1
           for (int v = 0; v < 4; ++v) {
             if (!wterm[v]) continue;
@@ -735,44 +777,45 @@ __global__ __launch_bounds__(BS_THREADS, 2) void bandsum_kernel(BandArgs b, doub
               for (int i = 0; i < 3; ++i) f2m[i + 3 * jj] += ai[i].re * x.re - ai[i].im * x.im;
             }
           }
-        // sum the 4 row groups of the block (lanes l, l^16, l^32, l^48)
+        // sums over the 4 row groups of the block (lane bits 4, 5), scattered:
+        // group g holds the slots NS g .. NS g + NS - 1
+        constexpr int NS = (JN == 3) ? 3 : 1;
+        const int jb = (JN == 3) ? 0 : 3 * jsel;  // component of f2[0]
+        auto put = [&](const double* f, double* Q) {
+          double h[2 * NS], o[NS];
+          auto at = [&](int q) { return q < 3 * JN ? f[q < 3 * JN ? q : 0] : 0.0; };
 #pragma unroll
-        for (int q = 0; q < 3 * JN; ++q) {
-          f2[q] = rows4_sum(f2[q]);
-          f2m[q] = rows4_sum(f2m[q]);
-        }
-        const int jb = (JN == 3) ? 0 : jsel;  // component of f2[3 * 0 ..]
-        if (kq == 0 && colok)
+          for (int q = 0; q < 2 * NS; ++q) h[q] = swap32_sum(at(q), at(q + 2 * NS));
 #pragma unroll
-          for (int q = 0; q < 3 * JN; ++q) QF[(tr * 9 + q + 3 * jb) * NMAX + n0] = f2m[q];
-        // kubo_mep_IC: f-weighted sum over the block's 16 bands
-        if (doK)
-          for (int ef = 0; ef < nef; ++ef) {
-            const double f = (colok && kq == 0) ? fd[ef + nef * n0] : 0.0;
+          for (int q = 0; q < NS; ++q) o[q] = swap16_sum(h[q], h[q + NS]);
 #pragma unroll
-            for (int q = 0; q < 3 * JN; ++q) {
-              const int i = q % 3, j = q / 3 + jb;
-              const double s = row16_sum(f * f2[q]);
-              if (lane == 0) TS[((j * NB + blk) * 3 + i) * nef + ef] = s;
-            }
-          }
+          for (int q = 0; q < NS; ++q)
+            if (colok && NS * kq + q < 3 * JN) Q[(tr * 9 + jb + NS * kq + q) * NMAX + n0] = o[q];
+        };
+        put(f2, QK);
+        if (!clean) put(f2m, QF);
       }
     }
     __syncthreads();
     if constexpr (FUSED) fetch(k + gridDim.x);  // in flight during the sums below
     // ---- sums over the bands n0 and over the waves' partial records --------
-    // Ne, kubo_ahc_tens (-sum f Omega) and kubo_mep_LC for every E_F
+    // Ne, kubo_ahc_tens (-sum f Omega), kubo_mep_LC and kubo_mep_IC for every E_F
     // for every E_F; item (c, ef) is summed by 8 lanes, lane g taking the
     // bands m0 = g, g + 8, ...
-    for (int base = 0; base < 8 * 19 * nef; base += BS_THREADS) {
+    for (int base = 0; base < 8 * 28 * nef; base += BS_THREADS) {
       const int it = base + t, item = it >> 3, g = it & 7;
-      const int c = item % 19, ef = item / 19;
-      const bool valid = item < 19 * nef &&
+      const int c = item % 28, ef = item / 28;
+      const bool valid = item < 28 * nef &&
                          (c == 0 || (c < 10 && doAHC) || (c >= 10 && doK));
       double s = 0.0;
       if (valid) {
-        const double* src = (c == 0) ? nullptr : (c < 10) ? OMA + (c - 1) * NMAX : F3A + (c - 10) * NMAX;
-        for (int m0 = g; m0 < n; m0 += 8) s += fd[ef + nef * m0] * (src ? src[m0] : 1.0);
+        const double* src = (c == 0)   ? nullptr
+                            : (c < 10) ? OMA + (c - 1) * NMAX
+                            : (c < 19) ? F3A + (c - 10) * NMAX
+                                       : QK + (c - 19) * NMAX;
+        const double* src2 = (NT == 2 && c >= 19) ? src + 9 * NMAX : nullptr;
+        for (int m0 = g; m0 < n; m0 += 8)
+          s += fd[ef + nef * m0] * (src2 ? src[m0] + src2[m0] : src ? src[m0] : 1.0);
       }
       s = group8_sum(s);  // the loop bounds are uniform over the wave
       if (valid && g == 0) {
@@ -780,45 +823,26 @@ __global__ __launch_bounds__(BS_THREADS, 2) void bandsum_kernel(BandArgs b, doub
           acc[L.Ne + ef] += wk * s;
         else if (c < 10)
           acc[L.ahc + (c - 1) + 9 * ef] -= wk * s;
-        else
+        else if (c < 19)
           acc[L.klc + (c - 10) + 9 * ef] += wk * s;
+        else
+          acc[L.kic + (c - 19) + 9 * ef] += wk * s;
       }
     }
-    // velo_ahc_tens / kubo_ohc_tens at the single (hw, E_F): the last 18
-    // threads, o = q (velo) and 9 + q (ohc)
-    if (pmode && t >= BS_THREADS - 18) {
-      const int o = t - (BS_THREADS - 18);  // 0..8 velo, 9..17 ohc
-      const int q = o % 9, i = q % 3, j = q / 3, c = i + j - 1;
-      auto u = [&](int e) { return ((PW[e] + PW[24 + e]) + PW[48 + e]) + PW[72 + e]; };
-      zd val = zd{0.0, 0.0};
-      if (!herm) {
-        val = zd{PW[2 * o], PW[2 * o + 1]};
-      } else if (o < 9) {  // velo: sum rv Im P_ij, antisymmetric in (i, j)
-        if (i != j) val = (i < j) ? zd{u(2 * c), u(2 * c + 1)} : zd{-u(2 * c), -u(2 * c + 1)};
-      } else {      // ohc: i sum ro conj(P_ij) = i conj(X - iY) for X = sum Re(ro) P, Y = sum Im(ro) P
-        if (i == j) {
-          val = zd{-u(21 + i), u(18 + i)};
-        } else {
-          const double xr = u(6 + 2 * c), xi = u(7 + 2 * c), yr = u(12 + 2 * c), yi = u(13 + 2 * c);
-          val = (i < j) ? zd{xi - yr, xr + yi} : zd{-(xi + yr), xr - yi};
-        }
-      }
-      double* dst = acc + (o < 9 ? L.velo : L.ohc) + 2 * q;
-      dst[0] += wk * val.re;
-      dst[1] += wk * val.im;
+    // general V: velo_ahc_tens / kubo_ohc_tens at the single (hw, E_F), the
+    // last 18 threads, o = q (velo) and 9 + q (ohc)
+    if (!HERM && pmode && t >= BS_THREADS - 18) {
+      const int o = t - (BS_THREADS - 18);
+      double* dst = acc + (o < 9 ? L.velo : L.ohc) + 2 * (o % 9);
+      dst[0] += wk * PW[2 * o];
+      dst[1] += wk * PW[2 * o + 1];
     }
-    if (doK)
-      for (int it = t; it < 9 * nef; it += BS_THREADS) {
-        const int q = it % 9, ef = it / 9, i = q % 3, j = q / 3;
-        double s = 0.0;
-        for (int tt = 0; tt < NT * NT; ++tt) s += TS[((j * NT * NT + tt) * 3 + i) * nef + ef];
-        acc[L.kic + q + 9 * ef] += wk * s;
-      }
     if (doNjob)
       for (int it = t; it < 9 * nval; it += BS_THREADS) {
         const int q = it % 9, n0 = it / 9;
         double s = 0.0;
-        for (int tr = 0; tr < NT; ++tr) s += QF[(tr * 9 + q) * NMAX + n0];
+        const double* Q = clean ? QK : QF;
+        for (int tr = 0; tr < NT; ++tr) s += Q[(tr * 9 + q) * NMAX + n0];
         acc[L.nic + q + 9 * n0] += wk * s;
       }
     // ---- Chern-Simons term (needs A and Omega) ------------------------------
@@ -850,6 +874,36 @@ __global__ __launch_bounds__(BS_THREADS, 2) void bandsum_kernel(BandArgs b, doub
     }
   }
   __syncthreads();
+  if (HERM && pmode) {
+    // the pair sums of the 8 bands of a group, then of the wavefronts that had
+    // bands (8 to a wavefront); every pair was summed in both orders
+    const int base = 12 * ((lane >> 5) & 1) + 6 * ((lane >> 4) & 1) + 3 * ((lane >> 3) & 1);
+#pragma unroll
+    for (int s = 0; s < 3; ++s) {
+      const double v = group8_sum(pacc[s]);
+      if ((lane & 7) == 0) QK[wv * 24 + base + s] = v;
+    }
+    __syncthreads();
+    if (t < 9) {
+      const int i = t % 3, j = t / 3, c = i + j - 1;
+      const double B = 2.0 * wq.re * wq.im;
+      auto u = [&](int e) { return ((QK[e] + QK[24 + e]) + QK[48 + e]) + QK[72 + e]; };
+      auto g = [&](int e) { return zd{u(e), B * u(e + 3)}; };  // sum of g v
+      zd av = zd{0.0, 0.0}, ao;
+      if (i == j) {      // ohc_ii = i w sum g |x_i|^2 / dE
+        ao = zmuli(zmul(wq, g(12 + i)));
+      } else {           // velo_ij = M, ohc_ij = M + i w N (i < j); -M for j > i
+        const zd M = g(c), iwN = zmuli(zmul(wq, g(6 + c)));
+        av = i < j ? M : zd{-M.re, -M.im};
+        ao = zadd(av, iwN);
+      }
+      acc[L.velo + 2 * t] += av.re;
+      acc[L.velo + 2 * t + 1] += av.im;
+      acc[L.ohc + 2 * t] += ao.re;
+      acc[L.ohc + 2 * t + 1] += ao.im;
+    }
+    __syncthreads();
+  }
   // the record in HBM holds the velo / ohc block (gap entries from L.velo)
   // that this layout leaves out
   double* out = part + (int64_t)blockIdx.x * (L.total + gap);
@@ -1042,7 +1096,7 @@ __global__ __launch_bounds__(256, 2) void bandsum_wide_kernel(BandArgs b, double
       for (int c = 0; c < 3; ++c) S[(18 + c) * 256 + t] = om[c];
       if (pmode) {
         double v3[3];
-        scatter_sum24(ps, v3, lane);
+        scatter_sum<24>(ps, v3, lane);
         const int base = 12 * ((lane >> 5) & 1) + 6 * ((lane >> 4) & 1) + 3 * ((lane >> 3) & 1);
 #pragma unroll
         for (int q = 0; q < 3; ++q) v3[q] = group8_sum(v3[q]);
@@ -1781,17 +1835,17 @@ static AccLayout lds_layout(const BandArgs& b, const AccLayout& L, int64_t* gap)
   return S;
 }
 
-template <int NMAX, bool FUSED>
+template <int NMAX, bool FUSED, bool HERM>
 static void launch_bs(hipStream_t s, const BandArgs& b, double Tsmear, const AccLayout& L,
                       int64_t nk, const double* E, const zd* V, const zd* A, const zd* Om,
                       const double* w, int nblocks, double* part, const VeloFuse* f) {
   int64_t gap;
   const AccLayout S = lds_layout(b, L, &gap);
   size_t lds = BsLds<NMAX>::bytes(b.n_ef, S.total);
-  (void)hipFuncSetAttribute((const void*)bandsum_kernel<NMAX, FUSED>,
+  (void)hipFuncSetAttribute((const void*)bandsum_kernel<NMAX, FUSED, HERM>,
                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-  hipLaunchKernelGGL((bandsum_kernel<NMAX, FUSED>), dim3(nblocks), dim3(BS_THREADS), lds, s, b,
-                     Tsmear, S, gap, nk, E, V, A, Om, w, part, f ? f->Hk : nullptr,
+  hipLaunchKernelGGL((bandsum_kernel<NMAX, FUSED, HERM>), dim3(nblocks), dim3(BS_THREADS), lds, s,
+                     b, Tsmear, S, gap, nk, E, V, A, Om, w, part, f ? f->Hk : nullptr,
                      f ? f->strideHk : (int64_t)0, f ? f->U : nullptr);
 }
 
@@ -1803,7 +1857,8 @@ size_t bandsum_lds_bytes(const BandArgs& b) {
   }
   int64_t gap;
   const AccLayout S = lds_layout(b, L, &gap);
-  const size_t a = b.n <= 16 ? BsLds<16>::bytes(b.n_ef, S.total) : BsLds<32>::bytes(b.n_ef, S.total);
+  const size_t a = b.n <= 16 ? BsLds<16>::limit_bytes(b.n_ef, S.total)
+                              : BsLds<32>::limit_bytes(b.n_ef, S.total);
   const size_t h = hw_many(b) ? hwsum_lds_bytes(b) : 0;
   return a > h ? a : h;
 }
@@ -1849,12 +1904,15 @@ void launch_bandsum(hipStream_t s, const BandArgs& b, int64_t nk, const double* 
     if (hw_many(b) || ((b.jobs & MEP_JOB_AHC) && !b.v_herm))
       launch_hwsum(s, b, Tsmear, L, nk, E, V, w, nblocks, part);
   } else {
-    if (b.n <= 16)
-      launch_bs<16, false>(s, b, Tsmear, L, nk, E, V, A, Om, w, nblocks, part, nullptr);
-    else if (fuse)
-      launch_bs<32, true>(s, b, Tsmear, L, nk, E, V, A, Om, w, nblocks, part, fuse);
-    else
-      launch_bs<32, false>(s, b, Tsmear, L, nk, E, V, A, Om, w, nblocks, part, nullptr);
+    if (b.n <= 16) {
+      if (b.v_herm) launch_bs<16, false, true>(s, b, Tsmear, L, nk, E, V, A, Om, w, nblocks, part, nullptr);
+      else launch_bs<16, false, false>(s, b, Tsmear, L, nk, E, V, A, Om, w, nblocks, part, nullptr);
+    } else if (fuse) {
+      launch_bs<32, true, true>(s, b, Tsmear, L, nk, E, V, A, Om, w, nblocks, part, fuse);
+    } else {
+      if (b.v_herm) launch_bs<32, false, true>(s, b, Tsmear, L, nk, E, V, A, Om, w, nblocks, part, nullptr);
+      else launch_bs<32, false, false>(s, b, Tsmear, L, nk, E, V, A, Om, w, nblocks, part, nullptr);
+    }
     if (hw_many(b)) launch_hwsum(s, b, Tsmear, L, nk, E, V, w, nblocks, part);
   }
 }

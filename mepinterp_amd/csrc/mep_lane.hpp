@@ -104,16 +104,17 @@ __device__ inline T team_bcast(T v, int src) {
   }
   return r;
 }
-// Sums of 24 values over lane bits 3-5, scattered: lane l ends with the
-// slots 12 b5 + 6 b4 + 3 b3 + s (s < 3) of l's bits b5 b4 b3, each summed
-// over the 8 lanes that share l's bits 0-2.
-__device__ inline void scatter_sum24(const double* v, double* o, int lane) {
-  double h[12], q[6];
+// Sums of N values (a multiple of 8) over lane bits 3-5, scattered: lane l ends
+// with the slots N/2 b5 + N/4 b4 + N/8 b3 + s (s < N/8) of l's bits b5 b4 b3,
+// each summed over the 8 lanes that share l's bits 0-2.
+template <int N>
+__device__ inline void scatter_sum(const double* v, double* o, int lane) {
+  double h[N / 2], q[N / 4];
 #pragma unroll
-  for (int j = 0; j < 12; ++j) h[j] = swap32_sum(v[j], v[j + 12]);
+  for (int j = 0; j < N / 2; ++j) h[j] = swap32_sum(v[j], v[j + N / 2]);
 #pragma unroll
-  for (int j = 0; j < 6; ++j) q[j] = swap16_sum(h[j], h[j + 6]);
+  for (int j = 0; j < N / 4; ++j) q[j] = swap16_sum(h[j], h[j + N / 4]);
   const bool b3 = (lane & 8) != 0;
 #pragma unroll
-  for (int j = 0; j < 3; ++j) o[j] = ror8_sum(q[j], q[j + 3], b3);
+  for (int j = 0; j < N / 8; ++j) o[j] = ror8_sum(q[j], q[j + N / 8], b3);
 }

@@ -1,0 +1,39 @@
+"""The band sums up to 32 bands against the oracle at the edges of their
+branches: k-points whose Niu windows are all trivial (a small tolerance), some
+wide (the default) and nearly everything excluded (a large one), one and four
+matrix tiles, the last quarter of the band range present or not, velocities
+formed in the kernel or read, general V, one and several Fermi levels, and the
+pair sums at zero temperature, frequency and broadening."""
+import numpy as np
+import pytest
+
+from conftest import oracle_model, rand_kpts
+
+pytestmark = pytest.mark.gpu
+
+KEYS = ("Ne", "ahc", "ahc_velo", "ohc", "kubo_ic", "kubo_lc", "kubo_cs", "niu_ic", "niu_lc", "niu_cs")
+
+
+@pytest.mark.parametrize("n,pos,tb,n_eF", [(2, False, False, 1), (9, False, True, 2), (16, False, False, 1),
+                                           (17, False, False, 1), (24, False, True, 1), (25, False, False, 1),
+                                           (32, False, False, 1), (32, False, False, 3), (7, True, False, 1),
+                                           (24, True, True, 1), (25, True, False, 2), (32, True, False, 1)])
+@pytest.mark.parametrize("tol", [1e-13, 1e-5, 3e-2])
+def test_band_sums_match_oracle(n, pos, tb, n_eF, tol):
+    import oracle as O
+    from mepinterp_amd import capi, models
+    m = models.make_random(seed=500 + n, n=n, L=1, with_r=pos, tb=tb)
+    om = oracle_model(m, kubo_tol=tol)
+    k = rand_kpts(5, seed=n)
+    still = not pos and n_eF == 1
+    kw = dict(n_eF=n_eF, eF_min=-0.01, eF_max=0.01, n_hw=1, hw_min=0.0 if still else 0.02,
+              hw_max=0.0 if still else 0.02, T_kelvin=0.0 if still else 300.0,
+              eta=0.0 if still else 0.002, valence_bands=max(1, n // 2))
+    with capi.Engine(m["R_frac"], m["H"], r=m["r"], wf_centers=m["wf_centers"], a_latt=m["a_latt"],
+                     kubo_tol=tol) as eng:
+        g = eng.run_kpts(k, capi.Engine.params(
+            jobs=capi.MEP_JOB_AHC | capi.MEP_JOB_KUBO | capi.MEP_JOB_MEP, **kw))
+    o = O.accumulate(om, O.RunParams(do_ahc=True, do_kubo=True, do_mep=True, **kw), k)
+    for q in KEYS:
+        # 1e-9, the sums' tolerance (these gaps are 1e-3 and more)
+        assert np.max(np.abs(g[q] - o[q])) <= 1e-9 * np.max(np.abs(o[q])), q
