@@ -1811,6 +1811,178 @@ __global__ __launch_bounds__(64 * RP_WAVES) void reduce_parts_kernel(int nblocks
   }
 }
 
+// ===========================================================================
+// n <= 32, no magnetoelectric sums, up to HALL_EF Fermi levels, V in memory:
+// N_el, kubo_ahc_tens and, for a single (hw, E_F), velo_ahc_tens and
+// kubo_ohc_tens, over the pairs x < y of as many k-points at a time as fill the
+// workgroup, one pair a thread.  Every sum is over pairs, so it stays in the
+// thread's registers over all k-points and is reduced once: no per-band tables,
+// and only the occupations go through LDS.  With P_ij = V_i(y, x) V_j(x, y),
+// A_c = P_ij - P_ji and S_ij = P_ij + P_ji, the curvatures of x and y give
+//   ahc_ij = sum ((f_x + f_y) Im S_ij - (f_x - f_y) Im A_c) / dE^2   (ji: + A)
+// and the velo / ohc sums are hwsum_kernel's.  General V: nothing is assumed of
+// V(y, x).
+// Bound by the reads of V (at 8 bands, 32,768 k-points: 34 us; the band-sum
+// kernel, with three of its wavefronts waiting on the fourth's shuffles, 411).
+// Several Fermi levels cost 9 sums each: from HALL_EF on, the band-sum kernel.
+// ===========================================================================
+constexpr int HALL_EF = 4, HALL_KB = 32;
+
+template <int NEF, bool PMODE>
+__global__ __launch_bounds__(256, 2) void hall_kernel(BandArgs b, double Tsmear, AccLayout L,
+                                                      int64_t nk, const double* __restrict__ E,
+                                                      const zd* __restrict__ V,
+                                                      const double* __restrict__ w,
+                                                      double* __restrict__ part) {
+  static_assert(!PMODE || NEF == 1, "");
+  constexpr int NA = 9 * NEF, NQ = PMODE ? 36 : 0;
+  __shared__ double Es[128], fd[NEF * 128], wks[HALL_KB], red[4 * (NA + NQ + NEF)];
+  const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+  const int n = b.n, n2 = n * n, npair = n * (n - 1) / 2;
+  const bool finiteT = b.T_kelvin > 1e-2, doAHC = (b.jobs & MEP_JOB_AHC) != 0;
+  // k-points at a time: KB n <= 128
+  int KB = npair ? 256 / npair : HALL_KB;
+  KB = KB < 1 ? 1 : KB > HALL_KB ? HALL_KB : KB;
+  const double wr = b.hw[0], eta2 = b.eta * b.eta, B2 = 4.0 * wr * wr * eta2;
+  double ah[NA], pv[NQ + 1], ne[NEF];  // per level: S (3), A (3), S_ii (3); D q v, q v
+#pragma unroll
+  for (int q = 0; q < NA; ++q) ah[q] = 0.0;
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) pv[q] = 0.0;
+#pragma unroll
+  for (int e = 0; e < NEF; ++e) ne[e] = 0.0;
+  for (int64_t k0 = (int64_t)blockIdx.x * KB; k0 < nk; k0 += (int64_t)gridDim.x * KB) {
+    const int kb = nk - k0 < KB ? (int)(nk - k0) : KB;
+    __syncthreads();
+    for (int c = t; c < kb * n; c += 256) {
+      const double e = E[k0 * n + c], wk = w ? w[k0 + c / n] : 1.0;
+      Es[c] = e;
+#pragma unroll
+      for (int ef = 0; ef < NEF; ++ef) {
+        double f;
+        if (b.fd_in) f = b.fd_in[(k0 * n + c) * NEF + ef];
+        else f = finiteT ? 1.0 / (1.0 + exp((e - b.ef[ef]) / Tsmear)) : ((e < b.ef[ef]) ? 1.0 : 0.0);
+        fd[c * NEF + ef] = f;
+        ne[ef] += wk * f;
+      }
+      if (c % n == 0) wks[c / n] = wk;
+    }
+    __syncthreads();
+    if (!doAHC) continue;
+    for (int c = t; c < kb * npair; c += 256) {
+      const int kk = c / npair, p = c - kk * npair;
+      // pair x < y, p = x + y (y - 1) / 2
+      int y = (int)((sqrtf(8.0f * (float)p + 1.0f) + 1.0f) * 0.5f);
+      if (y * (y + 1) / 2 <= p) ++y;
+      if (y * (y - 1) / 2 > p) --y;
+      const int x = p - y * (y - 1) / 2;
+      const zd* Vk = V + (k0 + kk) * 3 * (int64_t)n2;
+      zd vxy[3], vyx[3];
+#pragma unroll
+      for (int a = 0; a < 3; ++a) {
+        vxy[a] = Vk[a * n2 + x + n * y];
+        vyx[a] = Vk[a * n2 + y + n * x];
+      }
+      const double wk = wks[kk], dE = Es[kk * n + x] - Es[kk * n + y], r = 1.0 / dE;
+      const double* fx = fd + (kk * n + x) * NEF;
+      const double* fy = fd + (kk * n + y) * NEF;
+      zd A[3], S[3], Sd[3];
+#pragma unroll
+      for (int q = 0; q < 3; ++q) {
+        const int i = q == 2 ? 1 : 0, j = q == 0 ? 1 : 2;
+        const zd pij = zmul(vyx[i], vxy[j]), pji = zmul(vyx[j], vxy[i]);
+        A[q] = zsub(pij, pji);
+        S[q] = zadd(pij, pji);
+        Sd[q] = zscale(zmul(vyx[q], vxy[q]), 2.0);
+      }
+      const double wr2 = wk * (r * r);
+#pragma unroll
+      for (int ef = 0; ef < NEF; ++ef) {
+        const double s = wr2 * (fx[ef] + fy[ef]), d = wr2 * (fx[ef] - fy[ef]);
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+          ah[9 * ef + q] += s * S[q].im;
+          ah[9 * ef + 3 + q] += d * A[q].im;
+          ah[9 * ef + 6 + q] += s * Sd[q].im;
+        }
+      }
+      if constexpr (PMODE) {
+        // selects drop pairs of equal occupation
+        const double f = fx[0] - fy[0];
+        const bool on = f != 0.0;
+        const double D = (dE - wr) * (dE + wr) + eta2;
+        const double g = on ? wk * f * rcp_nr(D * D + B2) : 0.0, Dg = D * g;
+        const double rs = on ? r : 0.0, gr = g * rs, Dgr = Dg * rs;
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+          pv[2 * q] += Dg * A[q].re;
+          pv[2 * q + 1] += Dg * A[q].im;
+          pv[6 + 2 * q] += Dgr * S[q].re;
+          pv[7 + 2 * q] += Dgr * S[q].im;
+          pv[12 + 2 * q] += Dgr * Sd[q].re;
+          pv[13 + 2 * q] += Dgr * Sd[q].im;
+          pv[18 + 2 * q] += g * A[q].re;
+          pv[19 + 2 * q] += g * A[q].im;
+          pv[24 + 2 * q] += gr * S[q].re;
+          pv[25 + 2 * q] += gr * S[q].im;
+          pv[30 + 2 * q] += gr * Sd[q].re;
+          pv[31 + 2 * q] += gr * Sd[q].im;
+        }
+      }
+    }
+  }
+  // the workgroup's sums, wavefront by wavefront
+  constexpr int NR = NA + NQ + NEF;
+  auto put = [&](int q, double v) {
+    v = rows4_sum(row16_sum(v));
+    if (lane == 0) red[wv * NR + q] = v;
+  };
+#pragma unroll
+  for (int q = 0; q < NA; ++q) put(q, ah[q]);
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) put(NA + q, pv[q]);
+#pragma unroll
+  for (int q = 0; q < NEF; ++q) put(NA + NQ + q, ne[q]);
+  __syncthreads();
+  auto R = [&](int q) { return ((red[q] + red[NR + q]) + red[2 * NR + q]) + red[3 * NR + q]; };
+  double* out = part + (int64_t)blockIdx.x * L.total;
+  if (t < NEF) out[L.Ne + t] += R(NA + NQ + t);
+  if (doAHC && t < 9 * NEF) {
+    const int ef = t / 9, i = t % 3, j = t / 3 % 3, c = i + j - 1;
+    double v;
+    if (i == j) v = R(9 * ef + 6 + i);
+    else v = i < j ? R(9 * ef + c) - R(9 * ef + 3 + c) : R(9 * ef + c) + R(9 * ef + 3 + c);
+    out[L.ahc + t] += v;
+  }
+  if (PMODE && doAHC && t >= 64 && t < 73) {
+    const int o = t - 64, i = o % 3, j = o / 3, c = i + j - 1;
+    const zd wq = zd{wr, b.eta};
+    const double B = 2.0 * wr * b.eta;
+    auto G = [&](int q) {  // sum of g v over the complex value q of A, S or S_ii
+      const double dr = R(NA + 2 * q), di = R(NA + 2 * q + 1);
+      const double br = B * R(NA + 18 + 2 * q), bi = B * R(NA + 19 + 2 * q);
+      return zd{dr - bi, di + br};
+    };
+    auto Gi = [&](int q) { return zd{R(NA + 2 * q + 1), B * R(NA + 19 + 2 * q)}; };  // g Im v
+    zd av = zd{0.0, 0.0}, ao;
+    if (i == j) {
+      ao = zmuli(zmul(wq, G(6 + i)));
+    } else {
+      const zd gi = Gi(c), iA = zmuli(G(c)), iwS = zmuli(zmul(wq, G(3 + c)));
+      av = i < j ? zd{-gi.re, -gi.im} : gi;
+      ao = i < j ? zadd(iwS, iA) : zsub(iwS, iA);
+    }
+    out[L.velo + 2 * o] += av.re;
+    out[L.velo + 2 * o + 1] += av.im;
+    out[L.ohc + 2 * o] += ao.re;
+    out[L.ohc + 2 * o + 1] += ao.im;
+  }
+}
+
+static bool hall_only(const BandArgs& b) {
+  return b.n <= 32 && b.n_ef <= HALL_EF && !(b.jobs & (MEP_JOB_KUBO | MEP_JOB_MEP));
+}
+
 // n <= 32: the Hall and optical conductivities of several (hw, E_F) items
 // (velo_ahc_tens / kubo_ohc_tens over a frequency list or several Fermi
 // levels) run in hwsum_kernel, every item on its own threads, reading V
@@ -1904,7 +2076,16 @@ void launch_bandsum(hipStream_t s, const BandArgs& b, int64_t nk, const double* 
     if (hw_many(b) || ((b.jobs & MEP_JOB_AHC) && !b.v_herm))
       launch_hwsum(s, b, Tsmear, L, nk, E, V, w, nblocks, part);
   } else {
-    if (b.n <= 16) {
+    if (!fuse && hall_only(b)) {
+      auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(nblocks), dim3(256), 0, s, b, Tsmear, L, nk, E, V, w, part);
+      };
+      if (b.n_ef == 1 && !hw_many(b)) go(hall_kernel<1, true>);
+      else if (b.n_ef == 1) go(hall_kernel<1, false>);
+      else if (b.n_ef == 2) go(hall_kernel<2, false>);
+      else if (b.n_ef == 3) go(hall_kernel<3, false>);
+      else go(hall_kernel<4, false>);
+    } else if (b.n <= 16) {
       if (b.v_herm) launch_bs<16, false, true>(s, b, Tsmear, L, nk, E, V, A, Om, w, nblocks, part, nullptr);
       else launch_bs<16, false, false>(s, b, Tsmear, L, nk, E, V, A, Om, w, nblocks, part, nullptr);
     } else if (fuse) {

@@ -37,3 +37,33 @@ def test_band_sums_match_oracle(n, pos, tb, n_eF, tol):
     for q in KEYS:
         # 1e-9, the sums' tolerance (these gaps are 1e-3 and more)
         assert np.max(np.abs(g[q] - o[q])) <= 1e-9 * np.max(np.abs(o[q])), q
+
+
+@pytest.mark.parametrize("n,pos,n_eF,n_hw", [
+    (1, False, 1, 1), (2, True, 1, 1), (4, True, 1, 1), (8, True, 1, 1), (8, True, 2, 3), (16, True, 1, 1),
+    (17, True, 1, 1), (23, True, 3, 1), (24, True, 4, 1), (24, True, 5, 1), (32, True, 1, 1), (32, True, 1, 4),
+    (5, False, 1, 1), (16, False, 1, 1), (16, False, 4, 2), (20, False, 2, 1), (24, False, 1, 1)])
+@pytest.mark.parametrize("T", [0.0, 300.0])
+def test_hall_sums_alone_match_oracle(n, pos, n_eF, n_hw, T):
+    """No magnetoelectric sums: as many k-points at a time as fill a workgroup
+    (42 cannot be one k-point, 37 no multiple of any), one pair a thread or
+    two rounds, up to four Fermi levels and more, weights."""
+    import oracle as O
+    from mepinterp_amd import capi, models
+    m = models.make_random(seed=800 + n, n=n, L=1, with_r=pos)
+    om = oracle_model(m)
+    nk = 37
+    k = rand_kpts(nk, seed=n)
+    wt = np.random.default_rng(n).uniform(0.5, 2.0, size=nk)
+    kw = dict(n_eF=n_eF, eF_min=-0.02, eF_max=0.02, n_hw=n_hw, hw_min=0.01, hw_max=0.05, T_kelvin=T,
+              eta=0.003, valence_bands=1)
+    with capi.Engine(m["R_frac"], m["H"], r=m["r"], a_latt=m["a_latt"]) as eng:
+        g = eng.run_kpts(k, capi.Engine.params(jobs=capi.MEP_JOB_AHC, **kw), weights=wt)
+    o = {}
+    for i in range(nk):
+        one = O.accumulate(om, O.RunParams(do_ahc=True, **kw), np.asfortranarray(k[:, i:i + 1]))
+        for q in KEYS[:4]:
+            o[q] = o.get(q, 0.0) + wt[i] * np.asarray(one[q])
+    for q in KEYS[:4]:
+        # 1e-9, the sums' tolerance
+        assert np.max(np.abs(g[q] - o[q])) <= 1e-9 * np.max(np.abs(o[q])), q
