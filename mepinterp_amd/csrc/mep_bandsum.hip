@@ -1786,28 +1786,57 @@ void launch_curv(hipStream_t s, int n, int64_t nk, const double* E, const zd* V,
                      T_kelvin > 1e-2 ? 1 : 0, out);
 }
 
-// acc[c] += sum over the nblocks partial records of part[g][c].  A
-// workgroup takes 64 consecutive c (one per lane, coalesced rows); its 16
-// wavefronts take the records g = w, w + 16, ... in order, and the 16 wave
-// sums are added in wave order: a fixed summation order, so the result is
-// deterministic.
-constexpr int RP_WAVES = 16;
-__global__ __launch_bounds__(64 * RP_WAVES) void reduce_parts_kernel(int nblocks, int64_t len,
-                                                                    const double* __restrict__ part,
-                                                                    double* __restrict__ acc) {
-  __shared__ double ws[RP_WAVES][64];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int64_t c = blockIdx.x * (int64_t)64 + lane;
+// acc[c] = sum over the nblocks partial records of part[g][c], for one or two
+// sets of records (len2 = 0: one).  A workgroup takes 16 consecutive c (128
+// bytes of a record); thread (r, c) sums the records r, r + 64, ... with up to
+// 16 loads in flight, and the 64 row sums are added in two steps of fixed
+// order, so the result is deterministic.  Latency-bound at the usual record of
+// a few hundred sums, which is why the columns are spread over many
+// workgroups: 505 sums of 1,024 records 9 us (64 columns a workgroup, one
+// load in flight: 21 to 33).
+constexpr int RP_COLS = 16, RP_ROWS = 64;
+__global__ __launch_bounds__(RP_COLS * RP_ROWS) void reduce_parts_kernel(
+    int nblocks, int64_t len, const double* __restrict__ part, double* __restrict__ acc,
+    int64_t len2, const double* __restrict__ part2, double* __restrict__ acc2) {
+  __shared__ double ws[RP_ROWS][RP_COLS + 1];
+  const int col = threadIdx.x % RP_COLS, row = threadIdx.x / RP_COLS;
+  const int64_t nb1 = (len + RP_COLS - 1) / RP_COLS;
+  int64_t blk = blockIdx.x;
+  if (blk >= nb1) {
+    blk -= nb1;
+    len = len2;
+    part = part2;
+    acc = acc2;
+  }
+  const int64_t c = blk * RP_COLS + col;
   double s = 0.0;
-  if (c < len)
-    for (int g = w; g < nblocks; g += RP_WAVES) s += part[(int64_t)g * len + c];
-  ws[w][lane] = s;
-  __syncthreads();
-  if (w == 0 && c < len) {
-    double t = 0.0;
+  if (c < len) {
+    double v[16];
+    for (int g0 = row; g0 < nblocks; g0 += 16 * RP_ROWS) {
 #pragma unroll
-    for (int v = 0; v < RP_WAVES; ++v) t += ws[v][lane];
-    acc[c] += t;
+      for (int u = 0; u < 16; ++u) {
+        const int g = g0 + u * RP_ROWS;
+        v[u] = g < nblocks ? part[(int64_t)g * len + c] : 0.0;
+      }
+#pragma unroll
+      for (int u = 0; u < 16; ++u) s += v[u];
+    }
+  }
+  ws[row][col] = s;
+  __syncthreads();
+  double t = 0.0;
+  if (row < 8) {
+#pragma unroll
+    for (int v = 0; v < 8; ++v) t += ws[row * 8 + v][col];
+  }
+  __syncthreads();
+  if (row < 8) ws[row][col] = t;
+  __syncthreads();
+  if (row == 0 && c < len) {
+    double r = 0.0;
+#pragma unroll
+    for (int v = 0; v < 8; ++v) r += ws[v][col];
+    acc[c] = r;
   }
 }
 
@@ -2098,10 +2127,11 @@ void launch_bandsum(hipStream_t s, const BandArgs& b, int64_t nk, const double* 
   }
 }
 
-void launch_reduce_parts(hipStream_t s, int nblocks, int64_t len, const double* part, double* acc) {
-  int64_t nb = (len + 63) / 64;
-  hipLaunchKernelGGL(reduce_parts_kernel, dim3((unsigned)nb), dim3(64 * RP_WAVES), 0, s, nblocks,
-                     len, part, acc);
+void launch_reduce_parts(hipStream_t s, int nblocks, int64_t len, const double* part, double* acc,
+                         int64_t len2, const double* part2, double* acc2) {
+  const int64_t nb = (len + RP_COLS - 1) / RP_COLS + (len2 + RP_COLS - 1) / RP_COLS;
+  hipLaunchKernelGGL(reduce_parts_kernel, dim3((unsigned)nb), dim3(RP_COLS * RP_ROWS), 0, s, nblocks,
+                     len, part, acc, len2, part2, acc2);
 }
 
 __global__ void fill_zero_kernel(double* __restrict__ p, int64_t n) {

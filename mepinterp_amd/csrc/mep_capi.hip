@@ -782,7 +782,6 @@ static int band_setup(mep_ctx* c, const mep_run_params* p, int64_t kblock, BandS
     HIPCHK(hipMalloc(&c->dacc, sizeof(double) * rec));
     c->acc_cap = rec;
   }
-  launch_fill_zero(c->st, c->dacc, rec);
   launch_fill_zero(c->st, c->dpart, need);
   HIPCHK(hipGetLastError());
   return MEP_OK;
@@ -844,10 +843,8 @@ static void for_each_output(const BandSetup& bs, const mep_run_params* p, mep_su
 static void reduce_records(mep_ctx* c, const BandSetup& bs) {
   // the partial records accumulate over every k-block of the run
   timed(c, K_REDUCE, [&] {
-    launch_reduce_parts(c->st, bs.nblocks, bs.L.total, c->dpart, c->dacc);
-    if (bs.ext)
-      launch_reduce_parts(c->st, bs.nblocks, bs.X.total, c->dpart + (int64_t)bs.nblocks * bs.L.total,
-                          c->dacc + bs.L.total);
+    launch_reduce_parts(c->st, bs.nblocks, bs.L.total, c->dpart, c->dacc, bs.ext ? bs.X.total : 0,
+                        c->dpart + (int64_t)bs.nblocks * bs.L.total, c->dacc + bs.L.total);
   });
 }
 
@@ -1150,7 +1147,6 @@ static int bg_capture(BatchGraph* g, int32_t n_models, mep_ctx* const* ctxs,
     for (int32_t i = 0; i < n_models && rc == MEP_OK; ++i) {
       mep_ctx* c = ctxs[i];
       const int64_t rec = band_record_len(bs[i]);
-      launch_fill_zero(c->st, c->dacc, rec);
       launch_fill_zero(c->st, c->dpart, (int64_t)bs[i].nblocks * rec);
     }
     for (int64_t r = 0; r < rounds && rc == MEP_OK; ++r)
@@ -1484,7 +1480,6 @@ extern "C" int mep_run_kpts_static(mep_ctx* c, int64_t nk, const double* kpts,
   else
     launch_linspace(c->st, p->hw_min, p->hw_max, p->n_hw, c->dhw);
   const int64_t rec = band_record_len(bs);
-  launch_fill_zero(c->st, c->dacc, rec);
   launch_fill_zero(c->st, c->dpart, (int64_t)bs.nblocks * rec);
   HIPCHK(hipGetLastError());
   CHK(run_block(c, bs, 0, nk, nullptr, kpts, weights, p));

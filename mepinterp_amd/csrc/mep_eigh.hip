@@ -56,7 +56,9 @@ __global__ __launch_bounds__(64) void eigh_house_kernel(int n, int64_t nk,
                                                         const double* __restrict__ kpts,
                                                         const double* __restrict__ tau,
                                                         typename cplx_of<R>::type* __restrict__ U,
-                                                        R* __restrict__ side) {
+                                                        R* __restrict__ side,
+                                                        int* __restrict__ count) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) *count = 0;  // the list is empty
   using Z = typename cplx_of<R>::type;
   constexpr int TEAMS = 64 / NMAX;
   constexpr int LDA = NMAX;
@@ -198,7 +200,9 @@ __global__ __launch_bounds__(64, 4) void eigh_house_half_kernel(int n, int64_t n
                                                              const double* __restrict__ kpts,
                                                              const double* __restrict__ tau,
                                                              zd* __restrict__ U,
-                                                             double* __restrict__ side) {
+                                                             double* __restrict__ side,
+                                                             int* __restrict__ count) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) *count = 0;  // the list is empty
   constexpr int NMAX = 32, HC = 16;
   __shared__ zd vv[NMAX], ww[NMAX], sub[NMAX], fph[NMAX];
   __shared__ double tauv[NMAX];
@@ -401,7 +405,9 @@ __global__ __launch_bounds__(64, 2) void eigh_house_row2_kernel(int n, int64_t n
                                                               const double* __restrict__ kpts,
                                                               const double* __restrict__ tau,
                                                               zd* __restrict__ U,
-                                                              double* __restrict__ side) {
+                                                              double* __restrict__ side,
+                                                              int* __restrict__ count) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) *count = 0;  // the list is empty
   constexpr int NMAX = 32, LDV = NMAX + 1;  // LDV: the two k-points' vectors in other banks
   __shared__ __attribute__((aligned(16))) zd vv[2 * LDV], ww[2 * LDV];
   __shared__ zd sub[2 * NMAX], fph[2 * NMAX];
@@ -1289,7 +1295,6 @@ __global__ __launch_bounds__(64 * WAVES) void eigh_sturm_wide_kernel(
   }
 }
 
-__global__ void zero_count_kernel(int* count) { *count = 0; }
 
 // QL for 32 < n <= 128: 32 lanes per workgroup, d and e in dynamic LDS (n x 32
 // each).  rec: the listed k-points, recording; otherwise every k-point's
@@ -1664,7 +1669,9 @@ __global__ __launch_bounds__(256) void eigh_house_wide_kernel(int n, int64_t nk,
                                                               const double* __restrict__ kpts,
                                                               const double* __restrict__ tau,
                                                               zd* __restrict__ U,
-                                                              double* __restrict__ side) {
+                                                              double* __restrict__ side,
+                                                              int* __restrict__ count) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) *count = 0;  // the list is empty
   extern __shared__ double hw_smem[];
   const int np = n * (n + 1) / 2;
   zd* Lw = reinterpret_cast<zd*>(hw_smem);
@@ -1823,7 +1830,9 @@ __global__ __launch_bounds__(64) void eigh_house_lds_kernel(int n, int64_t nk,
                                                             const double* __restrict__ kpts,
                                                             const double* __restrict__ tau,
                                                             zd* __restrict__ U,
-                                                            double* __restrict__ side) {
+                                                            double* __restrict__ side,
+                                                            int* __restrict__ count) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) *count = 0;  // the list is empty
   extern __shared__ __attribute__((aligned(16))) double hl_smem[];
   zd* A = reinterpret_cast<zd*>(hl_smem);  // A(r, c) at A[r + n c]
   zd* vv = A + (int64_t)n * n;
@@ -1988,7 +1997,9 @@ __global__ __launch_bounds__(4 * NMAX, NMAX <= 96 ? 3 : 2) void eigh_house_rows_
                                                                   const double* __restrict__ kpts,
                                                                   const double* __restrict__ tau,
                                                                   zd* __restrict__ U,
-                                                                  double* __restrict__ side) {
+                                                                  double* __restrict__ side,
+                                                                  int* __restrict__ count) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) *count = 0;  // the list is empty
   constexpr int NW = NMAX / 16, NC = NMAX / 4;
   __shared__ __attribute__((aligned(16))) zd vv[2][NMAX];
   __shared__ __attribute__((aligned(16))) zd ww[2][NMAX];
@@ -2561,6 +2572,8 @@ void launch_eigh_wide(hipStream_t s, int n, int64_t nk, const zd* Hk, int64_t st
   double* side = scratch;
   double* rot = side + nk * side_len(n);
   uint8_t* rcol = reinterpret_cast<uint8_t*>(rot + nk * 2 * rot_cap(n));
+  int* list = reinterpret_cast<int*>(reinterpret_cast<uint8_t*>(scratch) + eigh_list_offset(n, nk));
+  int* count = list + nk;
   const size_t lh = eigh_house_wide_lds(n), lr = eigh_replay_wide_lds(n);
   const size_t lq = sizeof(double) * 2 * (size_t)n * 32;
   (void)hipFuncSetAttribute((const void*)eigh_house_wide_kernel,
@@ -2580,32 +2593,29 @@ void launch_eigh_wide(hipStream_t s, int n, int64_t nk, const zd* Hk, int64_t st
     const unsigned rgrid = (unsigned)(nk < 65536 ? nk : 65536);
     if (n <= 64)
       hipLaunchKernelGGL(eigh_house_rows_kernel<64>, dim3(rgrid), dim3(256), 0, s, n, nk, Hk,
-                         strideHk, packed, g.kpts, g.tau, U, side);
+                         strideHk, packed, g.kpts, g.tau, U, side, count);
     else if (n <= 80)
       hipLaunchKernelGGL(eigh_house_rows_kernel<80>, dim3(rgrid), dim3(320), 0, s, n, nk, Hk,
-                         strideHk, packed, g.kpts, g.tau, U, side);
+                         strideHk, packed, g.kpts, g.tau, U, side, count);
     else if (n <= 96)
       hipLaunchKernelGGL(eigh_house_rows_kernel<96>, dim3(rgrid), dim3(384), 0, s, n, nk, Hk,
-                         strideHk, packed, g.kpts, g.tau, U, side);
+                         strideHk, packed, g.kpts, g.tau, U, side, count);
     else
       hipLaunchKernelGGL(eigh_house_rows_kernel<128>, dim3(rgrid), dim3(512), 0, s, n, nk, Hk,
-                         strideHk, packed, g.kpts, g.tau, U, side);
+                         strideHk, packed, g.kpts, g.tau, U, side, count);
   } else if (house == 2 && n <= 64) {
     const size_t ll = eigh_house_lds_bytes(n);
     (void)hipFuncSetAttribute((const void*)eigh_house_lds_kernel,
                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)ll);
     const unsigned lgrid = (unsigned)(nk < 65536 ? nk : 65536);
     hipLaunchKernelGGL(eigh_house_lds_kernel, dim3(lgrid), dim3(64), ll, s, n, nk, Hk, strideHk,
-                       packed, g.kpts, g.tau, U, side);
+                       packed, g.kpts, g.tau, U, side, count);
   } else {
     hipLaunchKernelGGL(eigh_house_wide_kernel, dim3(grid), dim3(256), lh, s, n, nk, Hk, strideHk,
-                       packed, g.kpts, g.tau, U, side);
+                       packed, g.kpts, g.tau, U, side, count);
   }
-  int* list = reinterpret_cast<int*>(reinterpret_cast<uint8_t*>(scratch) + eigh_list_offset(n, nk));
-  int* count = list + nk;
   int64_t qb = (nk + 31) / 32;
   unsigned qgrid = (unsigned)(qb < 65536 ? qb : 65536);
-  hipLaunchKernelGGL(zero_count_kernel, dim3(1), dim3(1), 0, s, count);
   // eigenvalues and the separation verdict, then the listed k-points
   const unsigned sgrid = (unsigned)(nk < 65536 ? nk : 65536);
   if (ql)
@@ -2676,20 +2686,19 @@ static void launch_eigh_t(hipStream_t s, int n, int64_t nk, const typename cplx_
     if (house == 2) {                                                                            \
       if (g.tau)                                                                                 \
         hipLaunchKernelGGL(eigh_house_row2_kernel<true>, dim3(h2grid), dim3(64), 0, s, n, nk,    \
-                           Hk, strideHk, packed, g.kpts, g.tau, U, side);                        \
+                           Hk, strideHk, packed, g.kpts, g.tau, U, side, count);                        \
       else                                                                                       \
         hipLaunchKernelGGL(eigh_house_row2_kernel<false>, dim3(h2grid), dim3(64), 0, s, n, nk,   \
-                           Hk, strideHk, packed, g.kpts, g.tau, U, side);                        \
+                           Hk, strideHk, packed, g.kpts, g.tau, U, side, count);                        \
     } else if (g.tau)                                                                            \
       hipLaunchKernelGGL(eigh_house_half_kernel<true>, dim3(hgrid), dim3(64), 0, s, n, nk, Hk,    \
-                         strideHk, packed, g.kpts, g.tau, U, side);                              \
+                         strideHk, packed, g.kpts, g.tau, U, side, count);                              \
     else                                                                                         \
       hipLaunchKernelGGL(eigh_house_half_kernel<false>, dim3(hgrid), dim3(64), 0, s, n, nk, Hk,   \
-                         strideHk, packed, g.kpts, g.tau, U, side);                              \
+                         strideHk, packed, g.kpts, g.tau, U, side, count);                              \
   } else                                                                                         \
     hipLaunchKernelGGL((eigh_house_kernel<NM, R>), dim3(grid), dim3(64), 0, s, n, nk, Hk, strideHk, \
-                       packed, g.kpts, g.tau, U, side);                                          \
-  hipLaunchKernelGGL(zero_count_kernel, dim3(1), dim3(1), 0, s, count);                        \
+                       packed, g.kpts, g.tau, U, side, count);                                          \
   if (ql || sizeof(R) != 8) {                                                                    \
     hipLaunchKernelGGL((eigh_ql_reg_kernel<NM, R>), dim3(qgrid), dim3(64), 0, s, n, nk, side, E, \
                        info, list, count);                                                       \

@@ -141,7 +141,8 @@ size_t bandsum_wide_scratch(int n, int nblocks);
 void launch_bandsum(hipStream_t s, const BandArgs& b, int64_t nk, const double* E, const zd* V,
                     const zd* A, const zd* Om, const double* w, int nblocks, double* part,
                     const VeloFuse* fuse = nullptr, zd* wide_scr = nullptr);
-void launch_reduce_parts(hipStream_t s, int nblocks, int64_t len, const double* part, double* acc);
+void launch_reduce_parts(hipStream_t s, int nblocks, int64_t len, const double* part, double* acc,
+                         int64_t len2, const double* part2, double* acc2);
 
 // optical / photogalvanic / gyrotropic sums (MEP_JOB_OPT, MEP_JOB_GYRO):
 // record layout (complex interleaved doubles) and launcher; n_wf <= 128,
