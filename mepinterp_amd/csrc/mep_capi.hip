@@ -102,6 +102,8 @@ struct mep_ctx {
   double* dpart = nullptr;
   int64_t part_cap = 0;
   double* dacc = nullptr;
+  uint8_t* hpin = nullptr;  // pinned transfer buffer (pin below)
+  size_t hpin_cap = 0;
   int64_t acc_cap = 0;
   double* def = nullptr;
   double* dhw = nullptr;
@@ -436,6 +438,7 @@ extern "C" int mep_ctx_destroy(mep_ctx* c) {
   hipFree(c->dXb); hipFree(c->dPh); hipFree(c->dY1);
   hipFree(c->dpart); hipFree(c->dacc); hipFree(c->def); hipFree(c->dhw); hipFree(c->dfd);
   hipFree(c->dcurv);
+  if (c->hpin) hipHostFree(c->hpin);
   for (auto e : c->pool) hipEventDestroy(e);
   if (c->st) hipStreamDestroy(c->st);
   delete c;
@@ -666,16 +669,46 @@ static int interp_block(mep_ctx* c, int64_t nb, bool velo, int prec = MEP_PREC_F
   return MEP_OK;
 }
 
-static int check_info(mep_ctx* c) {
-  int info = 0;
-  HIPCHK(hipMemcpyAsync(&info, c->dinfo, sizeof(int), hipMemcpyDeviceToHost, c->st));
-  HIPCHK(hipStreamSynchronize(c->st));
+static int info_status(mep_ctx* c, int info) {
   if (info) {
     hipMemsetAsync(c->dinfo, 0, sizeof(int), c->st);
     hipStreamSynchronize(c->st);
     return fail(MEP_ERR_EIG, "eigensolver did not converge (zheevd info != 0 equivalent)");
   }
   return MEP_OK;
+}
+
+static int check_info(mep_ctx* c) {
+  int info = 0;
+  HIPCHK(hipMemcpyAsync(&info, c->dinfo, sizeof(int), hipMemcpyDeviceToHost, c->st));
+  HIPCHK(hipStreamSynchronize(c->st));
+  return info_status(c, info);
+}
+
+// The context's pinned buffer for the small transfers of a call: copies from or
+// to the caller's pageable memory hold the host until each is done (15 to 30 us
+// apiece at any size), copies through this buffer are queued, and the call
+// waits once.  Every call ends with its stream idle, so the buffer is free at
+// its start.  nullptr above 1 MiB (where the extra host copy costs more than
+// the waits) or if it cannot be allocated: the caller copies directly.
+static uint8_t* pin(mep_ctx* c, size_t bytes) {
+  if (bytes > (size_t)1 << 20) return nullptr;
+  if (bytes > c->hpin_cap) {
+    if (hipStreamSynchronize(c->st) != hipSuccess) return nullptr;
+    size_t cap = (size_t)1 << 16;
+    while (cap < bytes) cap *= 2;
+    if (c->hpin) hipHostFree(c->hpin);
+    c->hpin = nullptr;
+    c->hpin_cap = 0;
+    void* q = nullptr;
+    if (hipHostMalloc(&q, cap, hipHostMallocDefault) != hipSuccess) {
+      (void)hipGetLastError();
+      return nullptr;
+    }
+    c->hpin = static_cast<uint8_t*>(q);
+    c->hpin_cap = cap;
+  }
+  return c->hpin;
 }
 
 static void linspace(double lo, double hi, int n, std::vector<double>& out) {
@@ -740,6 +773,12 @@ static int band_plan(mep_ctx* c, const mep_run_params* p, int64_t kblock, BandSe
 
 static int64_t band_record_len(const BandSetup& bs) { return bs.L.total + (bs.ext ? bs.X.total : 0); }
 
+// a run's part of the pinned buffer: E_F and frequencies, the record, the
+// eigensolver's status
+static size_t run_pin_bytes(const mep_run_params* p, int64_t rec) {
+  return sizeof(double) * ((size_t)p->n_eF + (size_t)p->n_hw + (size_t)rec + 1);
+}
+
 static int band_setup(mep_ctx* c, const mep_run_params* p, int64_t kblock, BandSetup& bs) {
   CHK(band_plan(c, p, kblock, bs));
   BandArgs& b = bs.b;
@@ -764,11 +803,19 @@ static int band_setup(mep_ctx* c, const mep_run_params* p, int64_t kblock, BandS
     HIPCHK(hipMalloc(&c->dhw, sizeof(double) * hw.size()));
     c->hw_cap = hw.size();
   }
-  HIPCHK(hipMemcpy(c->def, ef.data(), sizeof(double) * ef.size(), hipMemcpyHostToDevice));
-  HIPCHK(hipMemcpy(c->dhw, hw.data(), sizeof(double) * hw.size(), hipMemcpyHostToDevice));
+  const int64_t rec = band_record_len(bs);
+  if (double* h = reinterpret_cast<double*>(pin(c, run_pin_bytes(p, rec)))) {
+    memcpy(h, ef.data(), sizeof(double) * ef.size());
+    memcpy(h + ef.size(), hw.data(), sizeof(double) * hw.size());
+    HIPCHK(hipMemcpyAsync(c->def, h, sizeof(double) * ef.size(), hipMemcpyHostToDevice, c->st));
+    HIPCHK(hipMemcpyAsync(c->dhw, h + ef.size(), sizeof(double) * hw.size(), hipMemcpyHostToDevice,
+                          c->st));
+  } else {
+    HIPCHK(hipMemcpy(c->def, ef.data(), sizeof(double) * ef.size(), hipMemcpyHostToDevice));
+    HIPCHK(hipMemcpy(c->dhw, hw.data(), sizeof(double) * hw.size(), hipMemcpyHostToDevice));
+  }
   b.ef = c->def;
   b.hw = c->dhw;
-  const int64_t rec = band_record_len(bs);
   int64_t need = (int64_t)bs.nblocks * rec;
   if (need > c->part_cap) {
     ++c->gen;
@@ -848,18 +895,42 @@ static void reduce_records(mep_ctx* c, const BandSetup& bs) {
   });
 }
 
-static int unpack(mep_ctx* c, const BandSetup& bs, const mep_run_params* p, int64_t nk,
-                  mep_sums* out) {
+// the reduction of a run's records and the transfer of the result, queued
+static int queue_results(mep_ctx* c, const BandSetup& bs, const mep_run_params* p) {
   reduce_records(c, bs);
   HIPCHK(hipGetLastError());
   const int64_t rec = band_record_len(bs);
-  std::vector<double> h(rec);
-  HIPCHK(hipMemcpyAsync(h.data(), c->dacc, sizeof(double) * rec, hipMemcpyDeviceToHost, c->st));
-  HIPCHK(hipStreamSynchronize(c->st));
+  if (double* h = reinterpret_cast<double*>(pin(c, run_pin_bytes(p, rec)))) {
+    h += p->n_eF + p->n_hw;
+    HIPCHK(hipMemcpyAsync(h, c->dacc, sizeof(double) * rec, hipMemcpyDeviceToHost, c->st));
+    HIPCHK(hipMemcpyAsync(h + rec, c->dinfo, sizeof(int), hipMemcpyDeviceToHost, c->st));
+  }
+  return MEP_OK;
+}
+
+// wait for them and fill the caller's arrays
+static int unpack(mep_ctx* c, const BandSetup& bs, const mep_run_params* p, int64_t nk,
+                  mep_sums* out) {
+  const int64_t rec = band_record_len(bs);
+  std::vector<double> hv;
+  const double* h = nullptr;
+  if (run_pin_bytes(p, rec) <= c->hpin_cap) {  // where queue_results used it
+    h = reinterpret_cast<const double*>(c->hpin) + p->n_eF + p->n_hw;
+    HIPCHK(hipStreamSynchronize(c->st));
+    int info;
+    memcpy(&info, h + rec, sizeof(int));
+    CHK(info_status(c, info));
+  } else {
+    CHK(check_info(c));
+    hv.resize((size_t)rec);
+    HIPCHK(hipMemcpyAsync(hv.data(), c->dacc, sizeof(double) * rec, hipMemcpyDeviceToHost, c->st));
+    HIPCHK(hipStreamSynchronize(c->st));
+    h = hv.data();
+  }
   resolve_times(c);
   if (!out) return MEP_OK;
   for_each_output(bs, p, out, [&](double* dst, int64_t off, int64_t len) {
-    if (dst) memcpy(dst, h.data() + off, sizeof(double) * len);
+    if (dst) memcpy(dst, h + off, sizeof(double) * len);
   });
   out->n_k = nk;
   return MEP_OK;
@@ -877,6 +948,42 @@ extern "C" int mep_interp_batch(mep_ctx* c, int64_t nk, const double* kpts, doub
     return fail(MEP_ERR_ARG, "mep_interp_batch: a position operator needs A_ka and Om_kab");
   CHK(ensure_ws(c, nk));
   const int64_t n = c->n, n2 = n * n;
+  // k-points, E, V, A, Omega and the status through the pinned buffer
+  const size_t bk = sizeof(double) * 3 * (size_t)nk, be = sizeof(double) * (size_t)(n * nk);
+  const size_t bv = V_ka ? sizeof(zd) * 3 * (size_t)(n2 * nk) : 0, bo = V_ka && c->pos ? 3 * bv : 0;
+  const size_t bytes = bk + be + bv + (V_ka && c->pos ? bv : 0) + bo + sizeof(double);
+  uint8_t* h = nk <= c->kcap ? pin(c, bytes) : nullptr;
+  if (h) {
+    memcpy(h, kpts, bk);
+    HIPCHK(hipMemcpyAsync(c->dk, h, bk, hipMemcpyHostToDevice, c->st));
+    CHK(interp_block(c, nk, V_ka != nullptr));
+    struct Part {
+      void* dst;
+      const void* src;
+      size_t len;
+    } part[5];
+    int np = 0, info = 0;
+    part[np++] = {e_k, c->dE, be};
+    if (V_ka) {
+      launch_v_layout(c->st, (int)n, nk, c->dV, c->dHk, true);
+      HIPCHK(hipGetLastError());
+      part[np++] = {V_ka, c->dHk, bv};
+      if (c->pos) {
+        part[np++] = {A_ka, c->dA, bv};
+        part[np++] = {Om_kab, c->dOm, bo};
+      }
+    }
+    part[np++] = {&info, c->dinfo, sizeof(int)};
+    uint8_t* q = h + bk;
+    for (int i = 0; i < np; q += part[i++].len)
+      HIPCHK(hipMemcpyAsync(q, part[i].src, part[i].len, hipMemcpyDeviceToHost, c->st));
+    HIPCHK(hipStreamSynchronize(c->st));
+    q = h + bk;
+    for (int i = 0; i < np; q += part[i++].len) memcpy(part[i].dst, q, part[i].len);
+    CHK(info_status(c, info));
+    resolve_times(c);
+    return MEP_OK;
+  }
   for (int64_t k0 = 0; k0 < nk; k0 += c->kcap) {
     int64_t nb = (nk - k0 < c->kcap) ? nk - k0 : c->kcap;
     HIPCHK(hipMemcpyAsync(c->dk, kpts + 3 * k0, sizeof(double) * 3 * nb, hipMemcpyHostToDevice,
@@ -972,6 +1079,7 @@ extern "C" int mep_bandsum_batch(mep_ctx* c, int64_t nk, const double* e_k, cons
     }
     CHK(band_block(c, bs, nb, nullptr));
   }
+  CHK(queue_results(c, bs, p));
   return unpack(c, bs, p, nk, out);
 }
 
@@ -1014,7 +1122,7 @@ static int run_common(mep_ctx* c, int64_t nk, const int32_t* mp, const double* k
     int64_t nb = (nk - k0 < c->kcap) ? nk - k0 : c->kcap;
     CHK(run_block(c, bs, k0, nb, mp, kpts, weights, p));
   }
-  CHK(check_info(c));
+  CHK(queue_results(c, bs, p));
   return unpack(c, bs, p, nk, out);
 }
 
@@ -1049,10 +1157,9 @@ extern "C" int mep_run_batch(int32_t n_models, mep_ctx* const* ctxs, const int32
       const int64_t nb = (nk[i] - k0 < c->kcap) ? nk[i] - k0 : c->kcap;
       CHK(run_block(c, bs[i], k0, nb, mp_grids + 3 * i, nullptr, nullptr, &params[i]));
     }
-  for (int32_t i = 0; i < n_models; ++i) {
-    CHK(check_info(ctxs[i]));
+  for (int32_t i = 0; i < n_models; ++i) CHK(queue_results(ctxs[i], bs[i], &params[i]));
+  for (int32_t i = 0; i < n_models; ++i)
     CHK(unpack(ctxs[i], bs[i], &params[i], nk[i], outs ? &outs[i] : nullptr));
-  }
   return MEP_OK;
 }
 
