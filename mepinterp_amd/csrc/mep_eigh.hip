@@ -1977,7 +1977,7 @@ __global__ __launch_bounds__(64) void eigh_house_lds_kernel(int n, int64_t nk,
 // keeps register arrays in scratch)
 __device__ inline zd zsel(bool c, zd a, zd b) { return zd{c ? a.re : b.re, c ? a.im : b.im}; }
 
-// Householder reduction for 32 < n <= NMAX (NMAX = 64, 80, 96, 128) with the
+// Householder reduction for 32 < n <= NMAX (NMAX = 48, 64, 80, 96, 128) with the
 // matrix in registers: a workgroup of NMAX / 16 wavefronts per k-point,
 // lane 4 r + q of wave w holding row i = 16 w + r, columns j = 4 (jj + s) + q
 // (jj < NMAX / 4), where s = kc / 4 for the column kc being reduced: every
@@ -1990,8 +1990,14 @@ __device__ inline zd zsel(bool c, zd a, zd b) { return zd{c ? a.re : b.re, c ? a
 // hold columns > kc - 4 (uniform skip); rows of finished waves skip it too.
 // v goes to U's column kc as it is made.  Three barriers per column (LDS
 // buffers alternate between columns).  Same outputs as the other kernels.
+// The loops take CH or CU entries at a time, their LDS reads first, with zeros
+// past the end instead of a test per entry, and v's one corrected element (at
+// kc + 1) is selected in the two entries that can hold it: bound by the LDS
+// return path and the chain of sums at three wavefronts a SIMD.  n = 96, 2,744
+// k-points: 2.51 ms (one entry at a time, selects on each: 3.73); n = 52,
+// 3,570: 0.62 ms (0.84).
 template <int NMAX>
-__global__ __launch_bounds__(4 * NMAX, NMAX <= 96 ? 3 : 2) void eigh_house_rows_kernel(int n, int64_t nk,
+__global__ __launch_bounds__(4 * NMAX, NMAX <= 48 ? 4 : NMAX <= 96 ? 3 : 2) void eigh_house_rows_kernel(int n, int64_t nk,
                                                                   const zd* __restrict__ Hk,
                                                                   int64_t strideHk, int packed,
                                                                   const double* __restrict__ kpts,
@@ -2001,13 +2007,18 @@ __global__ __launch_bounds__(4 * NMAX, NMAX <= 96 ? 3 : 2) void eigh_house_rows_
                                                                   int* __restrict__ count) {
   if (blockIdx.x == 0 && threadIdx.x == 0) *count = 0;  // the list is empty
   constexpr int NW = NMAX / 16, NC = NMAX / 4;
-  __shared__ __attribute__((aligned(16))) zd vv[2][NMAX];
-  __shared__ __attribute__((aligned(16))) zd ww[2][NMAX];
+  // entries past the end of a row's shifted array: zero
+  constexpr int CH = 4, CU = NMAX == 64 || NMAX == 128 ? 4 : 2;  // chunks of the two loops
+  __shared__ __attribute__((aligned(16))) zd vv[2][NMAX + 4 * CH];
+  __shared__ __attribute__((aligned(16))) zd ww[2][NMAX + 4 * CH];
   __shared__ __attribute__((aligned(16))) zd sub[NMAX];
   __shared__ __attribute__((aligned(16))) zd fph[NMAX];
   __shared__ double red[2][2][NW];
   const double two_pi = 6.283185307179586476925;
   const zd zero = zd{0.0, 0.0};
+  if (threadIdx.x < 4 * CH)
+#pragma unroll
+    for (int b = 0; b < 2; ++b) vv[b][NMAX + threadIdx.x] = ww[b][NMAX + threadIdx.x] = zero;
   for (int64_t k = blockIdx.x; k < nk; k += gridDim.x) {
     int t = threadIdx.x;
     asm volatile("" : "+v"(t));
@@ -2083,23 +2094,28 @@ __global__ __launch_bounds__(4 * NMAX, NMAX <= 96 ? 3 : 2) void eigh_house_rows_
       const zd v0 = zsub(x0, alpha);
       const double vn2 = 2.0 * xn * (xn + ax0);
       const double tk = refl ? 2.0 * rcp_nr(vn2) : 0.0;
-      auto vget = [&](int j) {  // v_j (zero at and above kc, and without a reflection)
-        const zd x = vv[b][j];
-        return zsel(!refl, zero, zsel(j == kc + 1, v0, x));
-      };
-      const zd vi = zsel(i < n, vget(i), zero);
+      // v_j: x_j, but v0 at kc + 1 (an entry 0 or 1), and zero at and above kc.
+      // Without a reflection tau = 0 and neither p nor an update is used.
+      auto vfix = [&](int jj, zd x) { return jj < 2 ? zsel(4 * (jj + s) + q == kc + 1, v0, x) : x; };
+      const zd vi = zsel(i < n && refl, zsel(i == kc + 1, v0, vv[b][i]), zero);
       const bool active = 16 * wv + 15 > kc;  // uniform: the wave has rows > kc
       zd p = zero;
       if (active) {
         zd p2[2] = {zero, zero};
 #pragma unroll
-        for (int jj = 0; jj < NC; ++jj) {
-          if (jj >= NC - s) continue;  // uniform: entries past the shifted end
-          const int j = 4 * (jj + s) + q;
-          const zd a_ = row[jj], b_ = vget(j);
-          zd& c = p2[jj & 1];
-          c.re = fma(a_.re, b_.re, fma(-a_.im, b_.im, c.re));
-          c.im = fma(a_.re, b_.im, fma(a_.im, b_.re, c.im));
+        for (int j0 = 0; j0 < NC; j0 += CH) {
+          if (j0 >= NC - s) continue;  // uniform: entries past the shifted end
+          const zd* vb = &vv[b][4 * s + q];
+          zd b_[CH];
+#pragma unroll
+          for (int u = 0; u < CH; ++u) b_[u] = ldz(vb + 4 * (j0 + u));
+#pragma unroll
+          for (int u = 0; u < CH; ++u) {
+            const zd a_ = row[j0 + u], bb = vfix(j0 + u, b_[u]);
+            zd& c = p2[u & 1];
+            c.re = fma(a_.re, bb.re, fma(-a_.im, bb.im, c.re));
+            c.im = fma(a_.re, bb.im, fma(a_.im, bb.re, c.im));
+          }
         }
         p = zadd(p2[0], p2[1]);
       }
@@ -2129,15 +2145,25 @@ __global__ __launch_bounds__(4 * NMAX, NMAX <= 96 ? 3 : 2) void eigh_house_rows_
       __syncthreads();  // (3)
       if (refl && active) {
 #pragma unroll
-        for (int jj = 0; jj < NC; ++jj) {
-          if (jj >= NC - s) continue;  // uniform
-          const int j = 4 * (jj + s) + q;
-          // A(i, j) -= v_i conj(w_j) + w_i conj(v_j)  (zero for j <= kc or i <= kc)
-          const zd vj = vget(j), wj = ww[b][j];
-          zd r_ = row[jj];
-          r_.re = fma(-vi.re, wj.re, fma(-vi.im, wj.im, fma(-wi_.re, vj.re, fma(-wi_.im, vj.im, r_.re))));
-          r_.im = fma(-vi.im, wj.re, fma(vi.re, wj.im, fma(-wi_.im, vj.re, fma(wi_.re, vj.im, r_.im))));
-          row[jj] = r_;
+        for (int j0 = 0; j0 < NC; j0 += CU) {
+          if (j0 >= NC - s) continue;  // uniform
+          const zd* vb = &vv[b][4 * s + q];
+          const zd* wb = &ww[b][4 * s + q];
+          zd v_[CU], w_[CU];
+#pragma unroll
+          for (int u = 0; u < CU; ++u) {
+            v_[u] = ldz(vb + 4 * (j0 + u));
+            w_[u] = ldz(wb + 4 * (j0 + u));
+          }
+#pragma unroll
+          for (int u = 0; u < CU; ++u) {
+            // A(i, j) -= v_i conj(w_j) + w_i conj(v_j)  (zero for j <= kc or i <= kc)
+            const zd vj = vfix(j0 + u, v_[u]), wj = w_[u];
+            zd r_ = row[j0 + u];
+            r_.re = fma(-vi.re, wj.re, fma(-vi.im, wj.im, fma(-wi_.re, vj.re, fma(-wi_.im, vj.im, r_.re))));
+            r_.im = fma(-vi.im, wj.re, fma(vi.re, wj.im, fma(-wi_.im, vj.re, fma(wi_.re, vj.im, r_.im))));
+            row[j0 + u] = r_;
+          }
         }
       }
     }
@@ -2583,15 +2609,23 @@ void launch_eigh_wide(hipStream_t s, int n, int64_t nk, const zd* Hk, int64_t st
   (void)hipFuncSetAttribute((const void*)eigh_ql_wide_kernel,
                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lq);
   unsigned grid = (unsigned)(nk < 4096 ? nk : 4096);
-  // measured crossovers (C3 models n = 36 ... 68, C5, seeded models n = 72 ... 128):
-  // one wavefront with the matrix in LDS up to 44, registers to 64, the LDS
-  // workgroup to 88 (five or six wavefronts of registers sit unevenly on the
-  // four SIMDs), registers above
-  if (house == 0) house = n <= 44 ? 2 : n <= 64 ? 3 : n <= 88 ? 1 : 3;
+  // measured crossovers (seeded models, runs of 1.6 to 2.5 ms): one wavefront
+  // with the matrix in LDS up to 34 bands (n = 33: 1.80 ms, registers 1.82; n =
+  // 36: 1.66, 1.61; n = 44: 1.61, 1.30), registers to 64, the LDS workgroup to
+  // 72 (five wavefronts of registers sit unevenly on the four SIMDs; n = 68:
+  // 2.41, 2.49; n = 76: 2.56, 2.30), registers above.  The kernels round
+  // differently; with ql (sums over unbroadened poles, where a last bit of E
+  // shows) the choice is the one those sums have always had.
+  if (house == 0)
+    house = ql ? (n <= 44 ? 2 : n <= 64 ? 3 : n <= 88 ? 1 : 3)
+               : (n <= 34 ? 2 : n <= 64 ? 3 : n <= 72 ? 1 : 3);
   if (house == 3) {
     // the matrix in registers, NMAX / 16 wavefronts per k-point
     const unsigned rgrid = (unsigned)(nk < 65536 ? nk : 65536);
-    if (n <= 64)
+    if (n <= 48)
+      hipLaunchKernelGGL(eigh_house_rows_kernel<48>, dim3(rgrid), dim3(192), 0, s, n, nk, Hk,
+                         strideHk, packed, g.kpts, g.tau, U, side, count);
+    else if (n <= 64)
       hipLaunchKernelGGL(eigh_house_rows_kernel<64>, dim3(rgrid), dim3(256), 0, s, n, nk, Hk,
                          strideHk, packed, g.kpts, g.tau, U, side, count);
     else if (n <= 80)
