@@ -929,8 +929,8 @@ static __device__ inline double rinv(const double* Es, int m, int c) {
   return (m == c) ? 0.0 : 1.0 / (Es[c] - Es[m]);  // 1 / (E_c - E_m)
 }
 
-// complex elements of a workgroup's slot: three scaled planes and 18 sums of 16
-// columns for each 16 x 16 tile (at most the eigensolver record of a k-point)
+// complex elements of a workgroup's slot: three scaled planes (general V) and 18
+// sums of 16 columns for each 16 x 16 tile (at most the eigensolver record of a k-point)
 __host__ __device__ inline int64_t wide_slot(int n) {
   const int64_t nt = (n + 15) / 16;
   return 3 * (int64_t)n * n + nt * nt * (18 * 16 / 2);
@@ -957,6 +957,7 @@ __global__ __launch_bounds__(256, 2) void bandsum_wide_kernel(BandArgs b, double
                                                            const zd* __restrict__ A,
                                                            const zd* __restrict__ Om) {
   extern __shared__ double smem[];
+  __shared__ uint8_t ord[2 * 64];  // the wave items' row and column tiles
   const int n = b.n, nef = b.n_ef, nhw = b.n_hw, nval = b.n_val;
   double* Es = smem;
   double* fd = Es + n;
@@ -973,12 +974,35 @@ __global__ __launch_bounds__(256, 2) void bandsum_wide_kernel(BandArgs b, double
   const bool doK = (b.jobs & MEP_JOB_KUBO) != 0;
   const bool doNjob = (b.jobs & MEP_JOB_MEP) != 0;
   const bool pmode = HERM && doAHC && (nhw * nef == 1);
-  const zd wq = zd{b.hw[0], b.eta}, w2 = zmul(wq, wq);
+  const zd wq = zd{b.hw[0], b.eta};
+  const double eta2 = b.eta * b.eta, B2 = 4.0 * wq.re * wq.re * eta2;
   const double tol = b.kubo_tol;
   double* acc = part + (int64_t)blockIdx.x * L.total;
   const int npad = n <= 64 ? 64 : 128, P = 256 / npad;
   const int p0 = t % npad, pp = t / npad;
   const bool pact = p0 < n;
+
+  if (t == 0) {
+    // 2 x 2 tiles at a time, (a, b) and then (b, a): the four wavefronts share
+    // their operands in L1
+    const int nt = (n + 15) / 16, nq = (nt + 1) / 2;
+    int c = 0;
+    auto quad = [&](int a, int b_) {
+      for (int u = 0; u < 4; ++u) {
+        const int tr = 2 * a + (u & 1), tc = 2 * b_ + (u >> 1);
+        if (tr < nt && tc < nt) {
+          ord[2 * c] = (uint8_t)tr;
+          ord[2 * c + 1] = (uint8_t)tc;
+          ++c;
+        }
+      }
+    };
+    for (int a = 0; a < nq; ++a)
+      for (int b_ = a; b_ < nq; ++b_) {
+        quad(a, b_);
+        if (a != b_) quad(b_, a);
+      }
+  }
 
   for (int64_t k = blockIdx.x; k < nk; k += gridDim.x) {
     const double wk = w ? w[k] : 1.0;
@@ -986,17 +1010,34 @@ __global__ __launch_bounds__(256, 2) void bandsum_wide_kernel(BandArgs b, double
     __syncthreads();
     if (t < n) Es[t] = E[k * n + t];
     __syncthreads();
+    // the valence bands whose Niu guards exclude something: not those with g^3 >
+    // kubo_tol, g the gap to the nearest band (see bandsum_kernel).  Bit n0 of
+    // dirty, the same in every wavefront; only these have windows
+    uint64_t dirty[2] = {0, 0};
     if (doNjob)
-      for (int idx = t; idx < nval * n; idx += 256) {
-        const int nn = idx % n, n0 = idx / n;
-        if (nn == n0) continue;
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const int n0 = 64 * q + lane;
+        bool d = false;
+        if (n0 < n && n0 < nval) {
+          const double g0 = n0 > 0 ? Es[n0] - Es[n0 - 1] : HUGE_VAL;
+          const double g1 = n0 < n - 1 ? Es[n0 + 1] - Es[n0] : HUGE_VAL;
+          d = !(g0 * g0 * g0 > tol && g1 * g1 * g1 > tol);
+        }
+        dirty[q] = __ballot(d);
+      }
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+      for (uint64_t m = dirty[q]; m; m &= m - 1) {
+        const int n0 = 64 * q + __builtin_ctzll(m), nn = t;
+        if (nn >= n || nn == n0) continue;
         const double E0 = Es[n0], dn = E0 - Es[nn];
         const double dn2 = dn * dn;
         int lo = n0, hi = n0;
         while (lo > 0 && !(fabs(dn2 * (E0 - Es[lo - 1])) > tol)) --lo;
         while (hi < n - 1 && !(fabs(dn2 * (E0 - Es[hi + 1])) > tol)) ++hi;
-        win[2 * idx] = (uint8_t)lo;
-        win[2 * idx + 1] = (uint8_t)hi;
+        win[2 * (n0 * n + nn)] = (uint8_t)lo;
+        win[2 * (n0 * n + nn) + 1] = (uint8_t)hi;
       }
     for (int idx = t; idx < nef * n; idx += 256) {
       if (b.fd_in) {
@@ -1011,12 +1052,14 @@ __global__ __launch_bounds__(256, 2) void bandsum_wide_kernel(BandArgs b, double
     if constexpr (HERM) {
       // x_a = V_a(n0, n), P_ij = x_i conj(x_j) (i < j), r = 1 / (E0 - En), as
       // the pair phase of bandsum_kernel
-      const bool doN = doNjob && pact && p0 < nval;
+      // gd, go: over the n that mep_niu keeps, gx, gy: over those it excludes
+      // (few), which the Kubo sums add
+      const bool guard = pact && ((dirty[p0 >> 6] >> (p0 & 63)) & 1);
       const double E0 = pact ? Es[p0] : 0.0, f0 = (pmode && pact) ? fd[p0] : 0.0;
-      double om[3] = {0.0, 0.0, 0.0}, gd[3] = {0.0, 0.0, 0.0}, gdm[3] = {0.0, 0.0, 0.0}, ps[24];
-      zd go[3], gom[3];
+      double om[3] = {0.0, 0.0, 0.0}, gd[3] = {0.0, 0.0, 0.0}, gx[3] = {0.0, 0.0, 0.0}, ps[24];
+      zd go[3], gy[3];
 #pragma unroll
-      for (int c = 0; c < 3; ++c) go[c] = gom[c] = zd{0.0, 0.0};
+      for (int c = 0; c < 3; ++c) go[c] = gy[c] = zd{0.0, 0.0};
 #pragma unroll
       for (int c = 0; c < 24; ++c) ps[c] = 0.0;
       if (pact)
@@ -1037,34 +1080,34 @@ __global__ __launch_bounds__(256, 2) void bandsum_wide_kernel(BandArgs b, double
           const bool off = nn != p0;
           const double dE = E0 - Es[nn];
           const double r = off ? rcp_nr(dE) : 0.0, r2 = r * r, r3 = r2 * r;
-          const double r3m = (doN && fabs(dE * dE * dE) > tol) ? r3 : 0.0;
+          const bool ex = guard && !(fabs(dE * dE * dE) > tol);
+          const double r3k = ex ? 0.0 : r3;
 #pragma unroll
           for (int c = 0; c < 3; ++c) {
             om[c] += r2 * Pc[c].im;
-            gd[c] += r3 * d[c];
-            gdm[c] += r3m * d[c];
-            go[c] = zd{go[c].re + r3 * Pc[c].re, go[c].im + r3 * Pc[c].im};
-            gom[c] = zd{gom[c].re + r3m * Pc[c].re, gom[c].im + r3m * Pc[c].im};
+            gd[c] += r3k * d[c];
+            go[c] = zd{go[c].re + r3k * Pc[c].re, go[c].im + r3k * Pc[c].im};
           }
-          if (pmode) {
-            const double dfv = f0 - fd[nn];
-            const zd denv = zd{dE * dE - w2.re, -w2.im};
-            const zd deno = zmul(zd{dE, 0.0}, zd{dE - wq.re, -wq.im});
-            const double av = zabs2(denv), ao = zabs2(deno);
-            const double ia = rcp_nr(av * ao);
-            const double iv = ia * ao, io = ia * av;
-            const zd rv = off ? zd{denv.re * iv * dfv, -denv.im * iv * dfv} : zd{0.0, 0.0};
-            const zd ro = off ? zd{deno.re * io * dfv, -deno.im * io * dfv} : zd{0.0, 0.0};
+          if (ex)
 #pragma unroll
             for (int c = 0; c < 3; ++c) {
-              ps[2 * c] += rv.re * Pc[c].im;
-              ps[2 * c + 1] += rv.im * Pc[c].im;
-              ps[6 + 2 * c] += ro.re * Pc[c].re;
-              ps[7 + 2 * c] += ro.re * Pc[c].im;
-              ps[12 + 2 * c] += ro.im * Pc[c].re;
-              ps[13 + 2 * c] += ro.im * Pc[c].im;
-              ps[18 + c] += ro.re * d[c];
-              ps[21 + c] += ro.im * d[c];
+              gx[c] += r3 * d[c];
+              gy[c] = zd{gy[c].re + r3 * Pc[c].re, gy[c].im + r3 * Pc[c].im};
+            }
+          if (pmode) {  // the weights of bandsum_kernel's pair phase
+            const double f = f0 - fd[nn];
+            const bool on = f != 0.0 && off;
+            const double D = (dE - wq.re) * (dE + wq.re) + eta2;
+            const double q = on ? f * rcp_nr(D * D + B2) : 0.0, Dq = D * q;
+            const double rs = on ? r : 0.0, qr = q * rs, Dqr = Dq * rs;
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+              ps[c] += Dq * Pc[c].im;
+              ps[3 + c] += q * Pc[c].im;
+              ps[6 + c] += Dqr * Pc[c].re;
+              ps[9 + c] += qr * Pc[c].re;
+              ps[12 + c] += Dqr * d[c];
+              ps[15 + c] += qr * d[c];
             }
           }
         }
@@ -1074,23 +1117,35 @@ __global__ __launch_bounds__(256, 2) void bandsum_wide_kernel(BandArgs b, double
 #pragma unroll
       for (int a = 0; a < 3; ++a)
         z[a] = pact ? Vk[a * (int64_t)n2 + p0 + (int64_t)n * p0] : zd{0.0, 0.0};
-      auto G = [&](const double* gd_, const zd* go_, int i, int k_) {
-        if (i == k_) return zd{gd_[i], 0.0};
-        const zd g = go_[i + k_ - 1];
-        return i < k_ ? g : zd{g.re, -g.im};
-      };
+      auto local = [&](const double* gd_, const zd* go_, double* o) {
+        auto G = [&](int i, int k_) {
+          if (i == k_) return zd{gd_[i], 0.0};
+          const zd g = go_[i + k_ - 1];
+          return i < k_ ? g : zd{g.re, -g.im};
+        };
 #pragma unroll
-      for (int j = 0; j < 3; ++j) {
-        const int k_ = (j + 1) % 3, l = (j + 2) % 3;
+        for (int j = 0; j < 3; ++j) {
+          const int k_ = (j + 1) % 3, l = (j + 2) % 3;
 #pragma unroll
-        for (int i = 0; i < 3; ++i) {
-          const zd a = G(gd, go, i, k_), bb = G(gd, go, i, l);
-          const zd am = G(gdm, gom, i, k_), bm = G(gdm, gom, i, l);
-          S[(i + 3 * j) * 256 + t] =
-              (z[l].re * a.re - z[l].im * a.im) - (z[k_].re * bb.re - z[k_].im * bb.im);
-          S[(9 + i + 3 * j) * 256 + t] =
-              (z[l].re * am.re - z[l].im * am.im) - (z[k_].re * bm.re - z[k_].im * bm.im);
+          for (int i = 0; i < 3; ++i) {
+            const zd a = G(i, k_), bb = G(i, l);
+            o[i + 3 * j] = (z[l].re * a.re - z[l].im * a.im) - (z[k_].re * bb.re - z[k_].im * bb.im);
+          }
         }
+      };
+      {
+        double f3[9];
+        local(gd, go, f3);
+#pragma unroll
+        for (int q = 0; q < 9; ++q) S[(9 + q) * 256 + t] = f3[q];
+        if (__ballot(guard)) {
+          double fx[9];
+          local(gx, gy, fx);
+#pragma unroll
+          for (int q = 0; q < 9; ++q) f3[q] += fx[q];
+        }
+#pragma unroll
+        for (int q = 0; q < 9; ++q) S[q * 256 + t] = f3[q];
       }
 #pragma unroll
       for (int c = 0; c < 3; ++c) S[(18 + c) * 256 + t] = om[c];
@@ -1136,21 +1191,23 @@ __global__ __launch_bounds__(256, 2) void bandsum_wide_kernel(BandArgs b, double
         for (int it = t; it < 9 * nval; it += 256)
           acc[L.nlc + it] += wk * S[(9 + it % 9) * 256 + it / 9];
       // velo_ahc_tens / kubo_ohc_tens at the single (hw, E_F)
-      if (pmode && t < 18) {
-        const int q = t % 9, i = q % 3, j = q / 3, c = i + j - 1;
+      if (pmode && t < 9) {
+        const int i = t % 3, j = t / 3, c = i + j - 1;
+        const double B = 2.0 * wq.re * wq.im;
         auto u = [&](int e) { return ((red[e] + red[24 + e]) + red[48 + e]) + red[72 + e]; };
-        zd val = zd{0.0, 0.0};
-        if (t < 9) {
-          if (i != j) val = (i < j) ? zd{u(2 * c), u(2 * c + 1)} : zd{-u(2 * c), -u(2 * c + 1)};
-        } else if (i == j) {
-          val = zd{-u(21 + i), u(18 + i)};
+        auto g = [&](int e) { return zd{u(e), B * u(e + 3)}; };  // sum of g v
+        zd av = zd{0.0, 0.0}, ao;
+        if (i == j) {
+          ao = zmuli(zmul(wq, g(12 + i)));
         } else {
-          const double xr = u(6 + 2 * c), xi = u(7 + 2 * c), yr = u(12 + 2 * c), yi = u(13 + 2 * c);
-          val = (i < j) ? zd{xi - yr, xr + yi} : zd{-(xi + yr), xr - yi};
+          const zd M = g(c), iwN = zmuli(zmul(wq, g(6 + c)));
+          av = i < j ? M : zd{-M.re, -M.im};
+          ao = zadd(av, iwN);
         }
-        double* dst = acc + (t < 9 ? L.velo : L.ohc) + 2 * q;
-        dst[0] += wk * val.re;
-        dst[1] += wk * val.im;
+        acc[L.velo + 2 * t] += wk * av.re;
+        acc[L.velo + 2 * t + 1] += wk * av.im;
+        acc[L.ohc + 2 * t] += wk * ao.re;
+        acc[L.ohc + 2 * t + 1] += wk * ao.im;
       }
     } else {
     for (int ef = t; ef < nef; ef += 256) {
@@ -1260,57 +1317,68 @@ __global__ __launch_bounds__(256, 2) void bandsum_wide_kernel(BandArgs b, double
     }
     // ---- itinerant (IC) terms on MFMA ----------------------------------------
     // B_a(m, n0) = V_a(m, n0) r(m, n0), r(m, n0) = 1 / (E_n0 - E_m) (0 on the
-    // diagonal): one reciprocal per pair, into the workgroup's slot of Bscr,
-    // transposed (n0 + n m), so the 16 columns n0 of a tile load as one run.
+    // diagonal).  Hermitian V: formed in the step from conj V_a(n0, m), which
+    // loads as one run of the 16 columns n0, so V is all that is read (a scaled
+    // copy per workgroup doubled a working set that the caches miss as it is);
+    // general V: scaled planes in the workgroup's slot of Bscr, transposed.
     // A wave item is one 16 x 16 tile of all three C_j = V_k B_l - V_l B_k: six
-    // operands a step feed 18 products (four fed six with one C_j an item, which
-    // left the loop bound by L2 reads), and the next step's operands are in
-    // flight during a step's products.  With the one-read pair phase above: n =
-    // 96, 2,744 k-points 5.6 -> 2.9 ms; n = 44, 9,261 k-points 2.7 + 0.29 (its
-    // velo / ohc kernel) -> 1.7 ms.  Two row tiles an item (9 operands for 36
-    // products) spill: 3.1 and 1.75 ms; three wavefronts a SIMD spill too.
-    // The contraction with A_i(n0, n) = V_i(n0, n) r(n, n0)^2 comes straight
-    // from the accumulators; the items' sums go through the slot.
+    // operands a step feed 18 products, and the next step's operands are in
+    // flight during a step's products; the four wavefronts take 2 x 2 tiles, whose
+    // operands they share in L1.  Two row tiles an item (9 operands for 36
+    // products) spill, three wavefronts a SIMD too.  The contraction with
+    // A_i(n0, n) = V_i(n0, n) r(n, n0)^2 comes straight from the accumulators;
+    // the items' sums go through the slot.  Bound by the operands' way from
+    // beyond L2 and by MFMA issue (0.5 of it).
+    // n = 96, 2,744 k-points: 2.5 ms (one C_j an item, V read three times: 5.6;
+    // with scaled planes and tiles in row order 3.0); n = 44, 9,261: 1.48 ms
+    // (3.0 with its velo / ohc kernel; 1.72).
     if (doK || doNjob) {
       const int nt = (n + 15) / 16;
       const int lr = lane & 15, kq = lane >> 4;
       zd* Bw = Bscr + (int64_t)blockIdx.x * wide_slot(n);
       double* Pw = reinterpret_cast<double*>(Bw + 3 * (int64_t)n2);  // [item][18][16]
-      for (int idx = t; idx < n2; idx += 256) {
-        const int n0 = idx % n, m = idx / n;
-        const double rr = m == n0 ? 0.0 : rcp_nr(Es[n0] - Es[m]);
+      if constexpr (!HERM) {
+        for (int idx = t; idx < n2; idx += 256) {
+          const int n0 = idx % n, m = idx / n;
+          const double rr = m == n0 ? 0.0 : rcp_nr(Es[n0] - Es[m]);
 #pragma unroll
-        for (int a = 0; a < 3; ++a) {
-          const zd v = HERM ? zconj(Vk[a * (int64_t)n2 + idx]) : Vk[a * (int64_t)n2 + m + (int64_t)n * n0];
-          Bw[a * (int64_t)n2 + idx] = zscale(v, rr);
+          for (int a = 0; a < 3; ++a)
+            Bw[a * (int64_t)n2 + idx] = zscale(Vk[a * (int64_t)n2 + m + (int64_t)n * n0], rr);
         }
+        __syncthreads();
       }
-      __syncthreads();
       for (int item = wv; item < nt * nt; item += 4) {
-        const int r0 = 16 * (item / nt), n0 = 16 * (item % nt) + lr;
+        const int tr = ord[2 * item], tc = ord[2 * item + 1];
+        const int r0 = 16 * tr, n0 = 16 * tc + lr;
         const bool colok = n0 < n;
-        const bool doN = doNjob && colok && n0 < nval;
+        // this column has windows; without any in the tile, the kept sums are all
+        const bool doN = colok && ((dirty[n0 >> 6] >> (n0 & 63)) & 1);
+        const bool anyN = __ballot(doN) != 0;
         const int nc = colok ? n0 : n - 1;  // padded rows and columns repeat the last: not used
         const int ar = r0 + lr < n ? r0 + lr : n - 1;
         mep_v4d p1[3] = {}, p2[3] = {}, p3[3] = {};
+        const double E0 = Es[nc];
         struct Step {
           zd a[3], b[3];
+          double r;
         };
         auto load = [&](int m0, Step& s) {  // past the end: the last row, weight 0
           const bool mok = m0 + kq < n;
           const int64_t mo = (int64_t)n * (mok ? m0 + kq : n - 1);
 #pragma unroll
           for (int c = 0; c < 3; ++c) {
-            s.b[c] = Bw[c * (int64_t)n2 + mo + nc];
+            s.b[c] = HERM ? Vk[c * (int64_t)n2 + mo + nc] : Bw[c * (int64_t)n2 + mo + nc];
             s.a[c] = Vk[c * (int64_t)n2 + mo + ar];
           }
-#pragma unroll
-          for (int c = 0; c < 3; ++c) s.b[c] = zscale(s.b[c], mok ? 1.0 : 0.0);
+          s.r = HERM ? E0 - Es[mok ? m0 + kq : n - 1] : 1.0;
+          if (!mok || (HERM && m0 + kq == nc)) s.r = 0.0;  // no such m; r(n0, n0) = 0
         };
-        auto mac = [&](const Step& s) {
+        auto mac = [&](Step& s) {
           double as[3], bs[3];
+          const double r = HERM ? (s.r != 0.0 ? rcp_nr(s.r) : 0.0) : s.r;
 #pragma unroll
           for (int c = 0; c < 3; ++c) {
+            s.b[c] = zd{s.b[c].re * r, s.b[c].im * (HERM ? -r : r)};
             as[c] = s.a[c].re + s.a[c].im;
             bs[c] = s.b[c].re + s.b[c].im;
           }
@@ -1351,7 +1419,7 @@ __global__ __launch_bounds__(256, 2) void bandsum_wide_kernel(BandArgs b, double
           const int row = r0 + kq + 4 * v;
           if (!colok || row >= n || row == n0) continue;
           const double rr = rcp_nr(Es[n0] - Es[row]), rr2 = rr * rr;
-          bool narrow = false;
+          bool narrow = !doN;
           if (doN) {
             const int lo = win[2 * (n0 * n + row)], hi = win[2 * (n0 * n + row) + 1];
             const bool all = lo == 0 && hi == n - 1;
@@ -1368,7 +1436,7 @@ __global__ __launch_bounds__(256, 2) void bandsum_wide_kernel(BandArgs b, double
             for (int i = 0; i < 3; ++i) {
               const double c = ai[i].re * cv.re - ai[i].im * cv.im;
               f2[i + 3 * j] -= c;
-              f2m[i + 3 * j] -= narrow ? c : 0.0;
+              if (anyN) f2m[i + 3 * j] -= narrow ? c : 0.0;
             }
           }
         }
@@ -1387,10 +1455,12 @@ __global__ __launch_bounds__(256, 2) void bandsum_wide_kernel(BandArgs b, double
           auto terms = [&](int from, int to) {
             for (int mm = from; mm < to; ++mm) {
               zd vm[3], bm[3];
+              const double rm = HERM ? (mm == n0 ? 0.0 : rcp_nr(Es[n0] - Es[mm])) : 1.0;
 #pragma unroll
               for (int c = 0; c < 3; ++c) {
                 vm[c] = Vk[c * (int64_t)n2 + row + (int64_t)n * mm];
-                bm[c] = Bw[c * (int64_t)n2 + n0 + (int64_t)n * mm];  // 0 for mm = n0
+                bm[c] = HERM ? zscale(zconj(Vk[c * (int64_t)n2 + n0 + (int64_t)n * mm]), rm)
+                             : Bw[c * (int64_t)n2 + n0 + (int64_t)n * mm];  // 0 for mm = n0
               }
 #pragma unroll
               for (int j = 0; j < 3; ++j) {
@@ -1415,10 +1485,10 @@ __global__ __launch_bounds__(256, 2) void bandsum_wide_kernel(BandArgs b, double
         }
 #pragma unroll
         for (int q = 0; q < 9; ++q) {
-          const double s0 = rows4_sum(f2[q]), s1 = rows4_sum(f2m[q]);
+          const double s0 = rows4_sum(f2[q]), s1 = anyN ? rows4_sum(f2m[q]) : s0;
           if (kq == 0) {
-            Pw[(item * 18 + q) * 16 + lr] = s0;
-            Pw[(item * 18 + 9 + q) * 16 + lr] = s1;
+            Pw[((tr * nt + tc) * 18 + q) * 16 + lr] = s0;
+            Pw[((tr * nt + tc) * 18 + 9 + q) * 16 + lr] = s1;
           }
         }
       }

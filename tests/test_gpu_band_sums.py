@@ -1,9 +1,10 @@
-"""The band sums up to 32 bands against the oracle at the edges of their
-branches: k-points whose Niu windows are all trivial (a small tolerance), some
-wide (the default) and nearly everything excluded (a large one), one and four
-matrix tiles, the last quarter of the band range present or not, velocities
-formed in the kernel or read, general V, one and several Fermi levels, and the
-pair sums at zero temperature, frequency and broadening."""
+"""The band sums against the oracle at the edges of their branches: k-points
+whose Niu windows are all trivial (a small tolerance), some wide (the default)
+and nearly everything excluded (a large one), one and four matrix tiles, the
+last quarter of the band range present or not, above 32 bands odd and even
+numbers of tiles, velocities formed in the kernel or read, general V, one and
+several Fermi levels, and the pair sums at zero temperature, frequency and
+broadening."""
 import numpy as np
 import pytest
 
@@ -17,7 +18,9 @@ KEYS = ("Ne", "ahc", "ahc_velo", "ohc", "kubo_ic", "kubo_lc", "kubo_cs", "niu_ic
 @pytest.mark.parametrize("n,pos,tb,n_eF", [(2, False, False, 1), (9, False, True, 2), (16, False, False, 1),
                                            (17, False, False, 1), (24, False, True, 1), (25, False, False, 1),
                                            (32, False, False, 1), (32, False, False, 3), (7, True, False, 1),
-                                           (24, True, True, 1), (25, True, False, 2), (32, True, False, 1)])
+                                           (24, True, True, 1), (25, True, False, 2), (32, True, False, 1),
+                                           (33, False, False, 1), (48, False, True, 2), (65, False, False, 1),
+                                           (100, False, False, 1), (36, True, False, 1)])
 @pytest.mark.parametrize("tol", [1e-13, 1e-5, 3e-2])
 def test_band_sums_match_oracle(n, pos, tb, n_eF, tol):
     import oracle as O
