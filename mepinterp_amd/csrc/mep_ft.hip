@@ -93,6 +93,9 @@ __global__ void phase_real_f32_kernel(int64_t nk, int Kh, int has_zero,
 // Tiles are mapped XCD-aware: workgroups go round-robin over the 8 XCDs,
 // so each XCD receives a contiguous range of tiles, i.e. all column tiles
 // of a few k-row tiles, and the phase rows they share stay in its L2.
+// 60,000 x 2,400 x 343: 1.86 ms, 0.7 of the MFMA issue; the rest is the first
+// chunk's latency, the 1.15 GB of results and the barriers (1.97 ms with an
+// address and a bounds test in VALU instructions for every load).
 // --------------------------------------------------------------------------
 typedef double v4d __attribute__((ext_vector_type(4)));
 
@@ -125,16 +128,26 @@ __global__ __launch_bounds__(256, 2) void ft_gemm_f64_kernel(int M, int N, int K
 #pragma unroll
     for (int j = 0; j < 4; ++j) acc[i][j] = v4d{0.0, 0.0, 0.0, 0.0};
 
-  // staging map: thread -> (kk = tid/128 + 2 it, col = tid%128), 8 per operand
-  const int sc = tid & 127, sk = tid >> 7;
+  // staging map: thread -> (kk = tid/128 + 2 it, col = tid%128), 8 per operand.
+  // A row of the chunk is uniform over a wavefront, so its address is scalar
+  // and a load costs no VALU instruction (they do not overlap with the FP64
+  // products); columns past the end repeat the last one (not stored), rows
+  // past K are zero in X
+  const int sc = tid & 127, sk = __builtin_amdgcn_readfirstlane(tid >> 7);
+  const int am = (int)(m0 + sc < M ? sc : M - 1 - m0), bn = (int)(n0 + sc < N ? sc : N - 1 - n0);
   double ra[8], rb[8];
   auto gload = [&](int k0) {
+    const bool full = k0 + DG_KC <= K;  // uniform
 #pragma unroll
     for (int it = 0; it < 8; ++it) {
-      const int kk = k0 + sk + 2 * it;
-      ra[it] = (kk < K && m0 + sc < M) ? Pt[(int64_t)kk * M + m0 + sc] : 0.0;
-      rb[it] = (kk < K && n0 + sc < N) ? X[(int64_t)kk * N + n0 + sc] : 0.0;
+      const int kk = k0 + sk + 2 * it, kr = full || kk < K ? kk : K - 1;
+      ra[it] = (Pt + ((int64_t)kr * M + m0))[(unsigned)am];
+      rb[it] = (X + ((int64_t)kr * N + n0))[(unsigned)bn];
     }
+    if (!full)
+#pragma unroll
+      for (int it = 0; it < 8; ++it)
+        if (k0 + sk + 2 * it >= K) rb[it] = 0.0;
   };
   auto lstore = [&](int buf) {
 #pragma unroll
