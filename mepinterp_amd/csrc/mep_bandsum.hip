@@ -178,6 +178,26 @@ __global__ __launch_bounds__(BS_THREADS, 2) void bandsum_kernel(BandArgs b, doub
     et = (ok && tt < n) ? E[kk * n + tt] : 0.0;
   };
   if constexpr (FUSED) fetch(blockIdx.x);
+  // where those elements go in LDS, the same for every k-point: U(i, j) at
+  // uo, dH's element p = i + j (j + 1) / 2 at (i, j) (low half) and (j, i)
+  // (high half), out of range: all ones
+  uint32_t uo[FUSED ? NU : 1], po[FUSED ? ND : 1];
+  if constexpr (FUSED) {
+#pragma unroll
+    for (int u = 0; u < NU; ++u) {
+      const int idx = t + BS_THREADS * u;
+      uo[u] = idx < n2 ? idx % n + LD * (idx / n) : ~0u;
+    }
+#pragma unroll
+    for (int u = 0; u < ND; ++u) {
+      const int p = t + BS_THREADS * u;
+      int j = (int)((sqrtf(8.0f * (float)p + 1.0f) - 1.0f) * 0.5f);
+      if ((j + 1) * (j + 2) / 2 <= p) ++j;
+      if (j * (j + 1) / 2 > p) --j;
+      const int i = p - j * (j + 1) / 2;
+      po[u] = p < np ? (uint32_t)(i + LD * j) | (uint32_t)(j + LD * i) << 16 : ~0u;
+    }
+  }
 
   for (int64_t k = blockIdx.x; k < nk; k += gridDim.x) {
     // the thread index is made opaque per k-point: otherwise the compiler
@@ -202,22 +222,15 @@ __global__ __launch_bounds__(BS_THREADS, 2) void bandsum_kernel(BandArgs b, doub
       if (t < n) Es[t] = et;
 #pragma unroll
       for (int u = 0; u < NU; ++u) {
-        const int idx = t + BS_THREADS * u;
-        if (idx < n2) stz(Us + idx % n + LD * (idx / n), ut[u]);
+        if (uo[u] != ~0u) stz(Us + uo[u], ut[u]);
       }
 #pragma unroll
       for (int u = 0; u < ND; ++u) {
-        const int p = t + BS_THREADS * u;
-        if (p >= np) continue;
-        // element p of the packed upper triangle: (i, j), i <= j, p = i + j(j+1)/2
-        int j = (int)((sqrtf(8.0f * (float)p + 1.0f) - 1.0f) * 0.5f);
-        if ((j + 1) * (j + 2) / 2 <= p) ++j;
-        if (j * (j + 1) / 2 > p) --j;
-        const int i = p - j * (j + 1) / 2;
+        if (po[u] == ~0u) continue;
 #pragma unroll
         for (int a = 0; a < 3; ++a) {
-          stz(Vs + a * PL + j + LD * i, zconj(dt[a][u]));
-          stz(Vs + a * PL + i + LD * j, dt[a][u]);  // last: the diagonal keeps the value as stored
+          stz(Vs + a * PL + (po[u] >> 16), zconj(dt[a][u]));
+          stz(Vs + a * PL + (po[u] & 0xffff), dt[a][u]);  // last: the diagonal keeps the value as stored
         }
       }
       __syncthreads();
