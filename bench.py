@@ -204,7 +204,7 @@ def main():
     for name, fl in (("velo", velo_flop_k), ("bandsum", bs_flop_k)):
         ms, cnt = split[name]
         if cnt == 0:
-            stages[name] = {"fused_into": "bandsum_kernel<32, true>"}
+            stages[name] = {"fused_into": "bandsum_kernel<32, true, true>"}
             continue
         ach = fl * nk / (ms * 1e-3) / 1e12
         stages[name] = {"bound": "mfma", "flop_per_k": fl, "achieved_tflops": ach,
