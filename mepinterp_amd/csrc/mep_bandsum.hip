@@ -58,29 +58,33 @@ AccLayout acc_layout(const BandArgs& b) {
 constexpr int BS_THREADS = 256;
 
 // LDS plan: V planes (zd) 3*PL | E NMAX | r table PL | fd nef*NMAX | IC per
-// band NT*9*NMAX, twice (all terms, Niu-kept terms) | red NMAX | per-band
-// Berry and LC tensors 18*NMAX | pair sums 40 | acc total | Niu windows
-// 2*NMAX*NMAX bytes                         (doubles after the V planes)
-template <int NMAX>
+// band NT*9*NMAX, twice (all terms, Niu-kept terms) | pair sums or Chern-Simons
+// terms 36 | per-band Berry and LC tensors (3 or 9 + 9)*NMAX | acc total
+//                                           (doubles after the V planes)
+// At 32 bands and one E_F this stays below half of the LDS, two workgroups a
+// CU, for every number of valence bands.
+template <int NMAX, bool HERM>
 struct BsLds {
   static constexpr int LD = NMAX + 1;
   static constexpr int PL = NMAX * LD;
   static constexpr int NT = NMAX / 16;  // 16-row tiles per matrix
-  static size_t doubles(int nef, int64_t total) {
-    return (size_t)PL + NMAX + (size_t)nef * NMAX + 2 * (size_t)NT * 9 * NMAX + NMAX + 18 * NMAX +
-           40 + (size_t)total;
-  }
+  static constexpr int OM = HERM ? 3 : 9;  // rows of the Berry curvature
   static size_t bytes(int nef, int64_t total) {
-    return sizeof(zd) * 3 * (size_t)PL + sizeof(double) * doubles(nef, total) +
-           2 * (size_t)NMAX * NMAX;
-  }
-  // what the number of Fermi levels is limited by (above a few levels more
-  // than the kernel takes)
-  static size_t limit_bytes(int nef, int64_t total) {
-    return bytes(nef, total) + 56 * sizeof(double) + sizeof(double) * 9 * NT * (NT * (size_t)nef) -
-           sizeof(double) * 9 * NT * NMAX;
+    return sizeof(zd) * 3 * (size_t)PL +
+           sizeof(double) * ((size_t)PL + NMAX + (size_t)nef * NMAX + 2 * (size_t)NT * 9 * NMAX + 36 +
+                             (OM + 9) * NMAX + (size_t)total);
   }
 };
+// what the number of Fermi levels is limited by (above a few levels more than
+// the kernel takes): V and r, E and the occupations, per-band tables of 27 (45
+// with two row tiles) rows and one more, sums of 9 per level and tile, 96, the
+// record and two bytes per pair of bands
+static size_t bs_limit_bytes(int nmax, int nef, int64_t total) {
+  const size_t pl = (size_t)nmax * (nmax + 1), nt = nmax / 16, m = nmax;
+  return sizeof(zd) * 3 * pl + 2 * m * m +
+         sizeof(double) * (pl + m + nef * m + nt * 9 * m + 9 * nt * nt * nef + m + 18 * m + 96 +
+                           (size_t)total);
+}
 
 
 // FUSED: V is not read from HBM but formed in the V planes from the packed
@@ -110,11 +114,11 @@ __global__ __launch_bounds__(BS_THREADS, 2) void bandsum_kernel(BandArgs b, doub
                                                                 const zd* __restrict__ Hk,
                                                                 int64_t strideHk,
                                                                 const zd* __restrict__ U) {
-  using S_ = BsLds<NMAX>;
+  using S_ = BsLds<NMAX, HERM>;
   constexpr int LD = S_::LD, PL = S_::PL, NT = S_::NT;
   // U's plane (PL complex) lives over the per-k tables between the r table
   // and the accumulators while V is formed
-  static_assert(!FUSED || (NMAX == 32 && HERM && PL + 2 * NT * 9 * NMAX + NMAX >= 2 * PL),
+  static_assert(!FUSED || (NMAX == 32 && HERM && PL + 2 * NT * 9 * NMAX >= 2 * PL),
                 "fused velocities: U's plane must fit below the accumulators");
   extern __shared__ __attribute__((aligned(16))) double smem[];
   const int n = b.n, nef = b.n_ef, nhw = b.n_hw, nval = b.n_val;
@@ -124,12 +128,11 @@ __global__ __launch_bounds__(BS_THREADS, 2) void bandsum_kernel(BandArgs b, doub
   double* fd = Rs + PL;
   double* QK = fd + (int64_t)nef * NMAX;        // [NT][9][NMAX] IC per band, row tile by row tile
   double* QF = QK + NT * 9 * NMAX;              // the same over the Niu-kept terms
-  double* red = QF + NT * 9 * NMAX;
-  double* OMA = red + NMAX;                     // [9][NMAX] Berry curvature per band
-  double* F3A = OMA + 9 * NMAX;                 // [9][NMAX] Kubo LC tensor per band
-  double* PW = F3A + 9 * NMAX;                  // velo / ohc pair sums [36] (general V)
-  double* acc = PW + 40;
-  uint8_t* win = reinterpret_cast<uint8_t*>(acc + L.total);  // [n0][n] lo, hi
+  double* PW = QF + NT * 9 * NMAX;              // velo / ohc pair sums [36] (general V)
+  double* red = PW;                             // Chern-Simons terms, once those are read
+  double* OMA = PW + 36;                        // [OM][NMAX] Berry curvature per band
+  double* F3A = OMA + S_::OM * NMAX;            // [9][NMAX] Kubo LC tensor per band
+  double* acc = F3A + 9 * NMAX;
   const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
   const int n2 = n * n;
   const bool finiteT = b.T_kelvin > 1e-2;
@@ -351,20 +354,6 @@ __global__ __launch_bounds__(BS_THREADS, 2) void bandsum_kernel(BandArgs b, doub
         Rs[c + LD * m] = -v;
       }
     }
-    if (doNjob && !clean)
-      for (int idx = t; idx < nval * NMAX; idx += BS_THREADS) {
-        // mep_niu's guard |(E0-En)^2 (E0-Em)| > kubo_tol: energies are
-        // sorted, so the excluded m of (n0, n) form one range around n0
-        const int nn = idx % NMAX, n0 = idx / NMAX;
-        if (nn >= n || nn == n0) continue;
-        const double E0 = Es[n0], dn = E0 - Es[nn];
-        const double dn2 = dn * dn;
-        int lo = n0, hi = n0;
-        while (lo > 0 && !(fabs(dn2 * (E0 - Es[lo - 1])) > tol)) --lo;
-        while (hi < n - 1 && !(fabs(dn2 * (E0 - Es[hi + 1])) > tol)) ++hi;
-        win[2 * (n0 * NMAX + nn)] = (uint8_t)lo;
-        win[2 * (n0 * NMAX + nn) + 1] = (uint8_t)hi;
-      }
     for (int idx = t; idx < nef * n; idx += BS_THREADS) {
       if (b.fd_in) {
         fd[idx] = b.fd_in[k * (int64_t)nef * n + idx];
@@ -601,11 +590,8 @@ __global__ __launch_bounds__(BS_THREADS, 2) void bandsum_kernel(BandArgs b, doub
         if (slot < 9) {
           F3A[slot * NMAX + n0] = v2[s];
           if (clean && doN) acc[L.nlc + slot + 9 * n0] += wk * v2[s];
-        } else if (slot < 12) {  // Omega_ij = -2 v, Omega_ji = 2 v for pair (i, j)
-          const int c = slot - 9, i = (c == 2) ? 1 : 0, j = (c == 0) ? 1 : 2;
-          OMA[(i + 3 * j) * NMAX + n0] = -2.0 * v2[s];
-          OMA[(j + 3 * i) * NMAX + n0] = 2.0 * v2[s];
-          OMA[4 * c * NMAX + n0] = 0.0;
+        } else if (slot < 12) {  // Omega_ij = -2 v, Omega_ji = 2 v, Omega_ii = 0
+          OMA[(slot - 9) * NMAX + n0] = v2[s];
         }
       }
       if (!clean) {  // the local terms over the Niu-kept n
@@ -725,6 +711,7 @@ __global__ __launch_bounds__(BS_THREADS, 2) void bandsum_kernel(BandArgs b, doub
         // rows whose window holds more than n0 itself (the others need no
         // second pass) and is not the whole band range
         bool wterm[4];
+        unsigned win[4];  // lo, hi << 8
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
           const int row = r0 + kq + 4 * v;
@@ -732,8 +719,15 @@ __global__ __launch_bounds__(BS_THREADS, 2) void bandsum_kernel(BandArgs b, doub
           const double rr2 = rr * rr;
           bool narrow = false;
           wterm[v] = false;
+          win[v] = 0;
           if (!clean && doN && row < n && row != n0) {
-            const int lo = win[2 * (n0 * NMAX + row)], hi = win[2 * (n0 * NMAX + row) + 1];
+            // mep_niu's guard |(E0-En)^2 (E0-Em)| > kubo_tol: energies are
+            // sorted, so the excluded m of (n0, n) form one range around n0
+            const double E0 = Es[n0], dn = E0 - Es[row], dn2 = dn * dn;
+            int lo = n0, hi = n0;
+            while (lo > 0 && !(fabs(dn2 * (E0 - Es[lo - 1])) > tol)) --lo;
+            while (hi < n - 1 && !(fabs(dn2 * (E0 - Es[hi + 1])) > tol)) ++hi;
+            win[v] = (unsigned)lo | (unsigned)hi << 8;
             const bool all = lo == 0 && hi == n - 1;
             narrow = !all && !wide(lo, hi);
             wterm[v] = !all && !(lo == n0 && hi == n0);
@@ -756,9 +750,10 @@ __global__ __launch_bounds__(BS_THREADS, 2) void bandsum_kernel(BandArgs b, doub
         if (!clean && doN)
 #pragma unroll 1
           for (int v = 0; v < 4; ++v) {
-            if (!wterm[v]) continue;
+            const unsigned wv_ = v == 0 ? win[0] : v == 1 ? win[1] : v == 2 ? win[2] : win[3];
+            if (!(v == 0 ? wterm[0] : v == 1 ? wterm[1] : v == 2 ? wterm[2] : wterm[3])) continue;
             const int row = r0 + kq + 4 * v;
-            const int lo = win[2 * (n0 * NMAX + row)], hi = win[2 * (n0 * NMAX + row) + 1];
+            const int lo = (int)(wv_ & 255), hi = (int)(wv_ >> 8);
             const bool wd = wide(lo, hi);
             const double rr = Rs[row + LD * n0];
             const double rr2 = rr * rr;
@@ -815,31 +810,40 @@ __global__ __launch_bounds__(BS_THREADS, 2) void bandsum_kernel(BandArgs b, doub
     // Ne, kubo_ahc_tens (-sum f Omega), kubo_mep_LC and kubo_mep_IC for every E_F
     // for every E_F; item (c, ef) is summed by 8 lanes, lane g taking the
     // bands m0 = g, g + 8, ...
-    for (int base = 0; base < 8 * 28 * nef; base += BS_THREADS) {
+    // (Hermitian V: the three Berry sums are each two entries)
+    constexpr int NO = S_::OM, NI = 1 + NO + 18;
+    for (int base = 0; base < 8 * NI * nef; base += BS_THREADS) {
       const int it = base + t, item = it >> 3, g = it & 7;
-      const int c = item % 28, ef = item / 28;
-      const bool valid = item < 28 * nef &&
-                         (c == 0 || (c < 10 && doAHC) || (c >= 10 && doK));
+      const int c = item % NI, ef = item / NI;
+      const bool valid = item < NI * nef &&
+                         (c == 0 || (c <= NO && doAHC) || (c > NO && doK));
       double s = 0.0;
       if (valid) {
-        const double* src = (c == 0)   ? nullptr
-                            : (c < 10) ? OMA + (c - 1) * NMAX
-                            : (c < 19) ? F3A + (c - 10) * NMAX
-                                       : QK + (c - 19) * NMAX;
-        const double* src2 = (NT == 2 && c >= 19) ? src + 9 * NMAX : nullptr;
+        const double* src = (c == 0)        ? nullptr
+                            : (c <= NO)     ? OMA + (c - 1) * NMAX
+                            : (c <= NO + 9) ? F3A + (c - 1 - NO) * NMAX
+                                            : QK + (c - 10 - NO) * NMAX;
+        const double* src2 = (NT == 2 && c > NO + 9) ? src + 9 * NMAX : nullptr;
         for (int m0 = g; m0 < n; m0 += 8)
           s += fd[ef + nef * m0] * (src2 ? src[m0] + src2[m0] : src ? src[m0] : 1.0);
       }
       s = group8_sum(s);  // the loop bounds are uniform over the wave
       if (valid && g == 0) {
-        if (c == 0)
+        if (c == 0) {
           acc[L.Ne + ef] += wk * s;
-        else if (c < 10)
-          acc[L.ahc + (c - 1) + 9 * ef] -= wk * s;
-        else if (c < 19)
-          acc[L.klc + (c - 10) + 9 * ef] += wk * s;
-        else
-          acc[L.kic + (c - 19) + 9 * ef] += wk * s;
+        } else if (c <= NO) {
+          if constexpr (HERM) {
+            const int i = (c == 3) ? 1 : 0, j = (c == 1) ? 1 : 2;
+            acc[L.ahc + i + 3 * j + 9 * ef] += wk * (2.0 * s);
+            acc[L.ahc + j + 3 * i + 9 * ef] -= wk * (2.0 * s);
+          } else {
+            acc[L.ahc + (c - 1) + 9 * ef] -= wk * s;
+          }
+        } else if (c <= NO + 9) {
+          acc[L.klc + (c - 1 - NO) + 9 * ef] += wk * s;
+        } else {
+          acc[L.kic + (c - 10 - NO) + 9 * ef] += wk * s;
+        }
       }
     }
     // general V: velo_ahc_tens / kubo_ohc_tens at the single (hw, E_F), the
@@ -2103,13 +2107,13 @@ static bool hw_many(const BandArgs& b) {
   return (b.jobs & MEP_JOB_AHC) && (int64_t)b.n_hw * b.n_ef > 1;
 }
 
-// The n <= 32 kernel's accumulators in LDS: the record's layout without the
-// velo / ohc block when hwsum_kernel fills it (then N_hw does not bound the
-// LDS); *gap is the length of the block left out
-static AccLayout lds_layout(const BandArgs& b, const AccLayout& L, int64_t* gap) {
+// The n <= 32 kernel's accumulators in LDS: the record's layout, with drop
+// without the velo / ohc block (which hwsum_kernel fills, or nobody); *gap is
+// the length of the block left out
+static AccLayout lds_layout(const AccLayout& L, bool drop, int64_t* gap) {
   AccLayout S = L;
   *gap = 0;
-  if (hw_many(b)) {
+  if (drop) {
     *gap = L.kic - L.velo;
     S.ohc = L.velo;
     S.kic -= *gap; S.klc -= *gap; S.kcs -= *gap;
@@ -2124,8 +2128,8 @@ static void launch_bs(hipStream_t s, const BandArgs& b, double Tsmear, const Acc
                       int64_t nk, const double* E, const zd* V, const zd* A, const zd* Om,
                       const double* w, int nblocks, double* part, const VeloFuse* f) {
   int64_t gap;
-  const AccLayout S = lds_layout(b, L, &gap);
-  size_t lds = BsLds<NMAX>::bytes(b.n_ef, S.total);
+  const AccLayout S = lds_layout(L, hw_many(b) || !(b.jobs & MEP_JOB_AHC), &gap);
+  size_t lds = BsLds<NMAX, HERM>::bytes(b.n_ef, S.total);
   (void)hipFuncSetAttribute((const void*)bandsum_kernel<NMAX, FUSED, HERM>,
                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   hipLaunchKernelGGL((bandsum_kernel<NMAX, FUSED, HERM>), dim3(nblocks), dim3(BS_THREADS), lds, s,
@@ -2140,9 +2144,8 @@ size_t bandsum_lds_bytes(const BandArgs& b) {
     return a > h ? a : h;
   }
   int64_t gap;
-  const AccLayout S = lds_layout(b, L, &gap);
-  const size_t a = b.n <= 16 ? BsLds<16>::limit_bytes(b.n_ef, S.total)
-                              : BsLds<32>::limit_bytes(b.n_ef, S.total);
+  const AccLayout S = lds_layout(L, hw_many(b), &gap);
+  const size_t a = bs_limit_bytes(b.n <= 16 ? 16 : 32, b.n_ef, S.total);
   const size_t h = hw_many(b) ? hwsum_lds_bytes(b) : 0;
   return a > h ? a : h;
 }

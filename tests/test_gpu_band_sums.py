@@ -22,7 +22,7 @@ KEYS = ("Ne", "ahc", "ahc_velo", "ohc", "kubo_ic", "kubo_lc", "kubo_cs", "niu_ic
                                            (33, False, False, 1), (48, False, True, 2), (65, False, False, 1),
                                            (100, False, False, 1), (36, True, False, 1)])
 @pytest.mark.parametrize("tol", [1e-13, 1e-5, 3e-2])
-def test_band_sums_match_oracle(n, pos, tb, n_eF, tol):
+def test_band_sums_match_oracle(n, pos, tb, n_eF, tol, n_val=None):
     import oracle as O
     from mepinterp_amd import capi, models
     m = models.make_random(seed=500 + n, n=n, L=1, with_r=pos, tb=tb)
@@ -31,7 +31,7 @@ def test_band_sums_match_oracle(n, pos, tb, n_eF, tol):
     still = not pos and n_eF == 1
     kw = dict(n_eF=n_eF, eF_min=-0.01, eF_max=0.01, n_hw=1, hw_min=0.0 if still else 0.02,
               hw_max=0.0 if still else 0.02, T_kelvin=0.0 if still else 300.0,
-              eta=0.0 if still else 0.002, valence_bands=max(1, n // 2))
+              eta=0.0 if still else 0.002, valence_bands=n_val or max(1, n // 2))
     with capi.Engine(m["R_frac"], m["H"], r=m["r"], wf_centers=m["wf_centers"], a_latt=m["a_latt"],
                      kubo_tol=tol) as eng:
         g = eng.run_kpts(k, capi.Engine.params(
@@ -70,3 +70,24 @@ def test_hall_sums_alone_match_oracle(n, pos, n_eF, n_hw, T):
     for q in KEYS[:4]:
         # 1e-9, the sums' tolerance
         assert np.max(np.abs(g[q] - o[q])) <= 1e-9 * np.max(np.abs(o[q])), q
+
+
+@pytest.mark.parametrize("n,pos,n_eF", [(16, False, 1), (32, False, 1), (32, True, 3), (31, False, 2)])
+def test_every_band_a_valence_band(n, pos, n_eF):
+    """The largest tables of the n <= 32 kernel."""
+    test_band_sums_match_oracle(n, pos, False, n_eF, 1e-5, n_val=n)
+
+
+def test_no_hall_sums_with_a_long_frequency_list():
+    """Without Hall sums the frequencies take no room beside the tables: the
+    magnetoelectric sums are those of a single frequency, bit for bit."""
+    from mepinterp_amd import capi, models
+    m = models.make_random(seed=532, n=32, L=1, with_r=True)
+    k = rand_kpts(3, seed=2)
+    kw = dict(jobs=capi.MEP_JOB_KUBO | capi.MEP_JOB_MEP, n_eF=1, eF_min=0.0, eF_max=0.0, hw_min=0.01,
+              hw_max=0.02, T_kelvin=300.0, eta=0.004, valence_bands=2)
+    with capi.Engine(m["R_frac"], m["H"], r=m["r"], a_latt=m["a_latt"]) as eng:
+        one = eng.run_kpts(k, capi.Engine.params(n_hw=1, **kw))
+        many = eng.run_kpts(k, capi.Engine.params(n_hw=300, **kw))
+    for q in KEYS[4:]:
+        assert np.array_equal(one[q], many[q]), q
