@@ -99,7 +99,7 @@ static size_t bs_limit_bytes(int nmax, int nef, int64_t total) {
 // instructions: one sum instead of two where the Niu guards exclude nothing
 // (decided per k-point), per-k reductions scattered over the lanes or kept in
 // registers over all k-points, one weight per pair.
-// n = 32, 262,144 k-points, all tensors: 15.8 ms (17.6 before these); n = 20,
+// n = 32, 262,144 k-points, all tensors: 15.2 ms (17.6 before these); n = 20,
 // 24,273, five Fermi levels, V read: 0.85 ms (1.11).
 template <int NMAX, bool FUSED, bool HERM>
 __global__ __launch_bounds__(BS_THREADS, 2) void bandsum_kernel(BandArgs b, double Tsmear,
