@@ -908,9 +908,11 @@ static int queue_results(mep_ctx* c, const BandSetup& bs, const mep_run_params* 
   return MEP_OK;
 }
 
-// wait for them and fill the caller's arrays
+// wait for them and fill the caller's arrays.  solved: the call ran the
+// eigensolver, whose status decides; otherwise a status that an earlier failed
+// call left is not this call's
 static int unpack(mep_ctx* c, const BandSetup& bs, const mep_run_params* p, int64_t nk,
-                  mep_sums* out) {
+                  mep_sums* out, bool solved = true) {
   const int64_t rec = band_record_len(bs);
   std::vector<double> hv;
   const double* h = nullptr;
@@ -919,9 +921,9 @@ static int unpack(mep_ctx* c, const BandSetup& bs, const mep_run_params* p, int6
     HIPCHK(hipStreamSynchronize(c->st));
     int info;
     memcpy(&info, h + rec, sizeof(int));
-    CHK(info_status(c, info));
+    if (solved) CHK(info_status(c, info));
   } else {
-    CHK(check_info(c));
+    if (solved) CHK(check_info(c));
     hv.resize((size_t)rec);
     HIPCHK(hipMemcpyAsync(hv.data(), c->dacc, sizeof(double) * rec, hipMemcpyDeviceToHost, c->st));
     HIPCHK(hipStreamSynchronize(c->st));
@@ -1080,7 +1082,7 @@ extern "C" int mep_bandsum_batch(mep_ctx* c, int64_t nk, const double* e_k, cons
     CHK(band_block(c, bs, nb, nullptr));
   }
   CHK(queue_results(c, bs, p));
-  return unpack(c, bs, p, nk, out);
+  return unpack(c, bs, p, nk, out, false);
 }
 
 // one k-block of a run: k-points (generated or uploaded), interpolation and
