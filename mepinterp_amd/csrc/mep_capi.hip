@@ -104,6 +104,7 @@ struct mep_ctx {
   double* dacc = nullptr;
   uint8_t* hpin = nullptr;  // pinned transfer buffer (pin below)
   size_t hpin_cap = 0;
+  bool hpin_busy = false;   // copies from or into it may be under way
   int64_t acc_cap = 0;
   double* def = nullptr;
   double* dhw = nullptr;
@@ -688,13 +689,17 @@ static int check_info(mep_ctx* c) {
 // The context's pinned buffer for the small transfers of a call: copies from or
 // to the caller's pageable memory hold the host until each is done (15 to 30 us
 // apiece at any size), copies through this buffer are queued, and the call
-// waits once.  Every call ends with its stream idle, so the buffer is free at
-// its start.  nullptr above 1 MiB (where the extra host copy costs more than
+// waits once (and clears hpin_busy).  A call that ends in an error may leave
+// copies on the stream: the next one waits for them here.  One call of pin per
+// entry point.  nullptr above 1 MiB (where the extra host copy costs more than
 // the waits) or if it cannot be allocated: the caller copies directly.
 static uint8_t* pin(mep_ctx* c, size_t bytes) {
   if (bytes > (size_t)1 << 20) return nullptr;
-  if (bytes > c->hpin_cap) {
+  if (c->hpin_busy) {
     if (hipStreamSynchronize(c->st) != hipSuccess) return nullptr;
+    c->hpin_busy = false;
+  }
+  if (bytes > c->hpin_cap) {
     size_t cap = (size_t)1 << 16;
     while (cap < bytes) cap *= 2;
     if (c->hpin) hipHostFree(c->hpin);
@@ -708,6 +713,7 @@ static uint8_t* pin(mep_ctx* c, size_t bytes) {
     c->hpin = static_cast<uint8_t*>(q);
     c->hpin_cap = cap;
   }
+  c->hpin_busy = true;
   return c->hpin;
 }
 
@@ -895,13 +901,20 @@ static void reduce_records(mep_ctx* c, const BandSetup& bs) {
   });
 }
 
+// the record's place in the pinned buffer that band_setup made room in (nullptr:
+// it did not, the record is copied directly)
+static double* pinned_record(const mep_ctx* c, const mep_run_params* p, int64_t rec) {
+  if (run_pin_bytes(p, rec) > c->hpin_cap) return nullptr;
+  return reinterpret_cast<double*>(c->hpin) + p->n_eF + p->n_hw;
+}
+
 // the reduction of a run's records and the transfer of the result, queued
 static int queue_results(mep_ctx* c, const BandSetup& bs, const mep_run_params* p) {
   reduce_records(c, bs);
   HIPCHK(hipGetLastError());
   const int64_t rec = band_record_len(bs);
-  if (double* h = reinterpret_cast<double*>(pin(c, run_pin_bytes(p, rec)))) {
-    h += p->n_eF + p->n_hw;
+  if (double* h = pinned_record(c, p, rec)) {
+    c->hpin_busy = true;
     HIPCHK(hipMemcpyAsync(h, c->dacc, sizeof(double) * rec, hipMemcpyDeviceToHost, c->st));
     HIPCHK(hipMemcpyAsync(h + rec, c->dinfo, sizeof(int), hipMemcpyDeviceToHost, c->st));
   }
@@ -915,10 +928,10 @@ static int unpack(mep_ctx* c, const BandSetup& bs, const mep_run_params* p, int6
                   mep_sums* out, bool solved = true) {
   const int64_t rec = band_record_len(bs);
   std::vector<double> hv;
-  const double* h = nullptr;
-  if (run_pin_bytes(p, rec) <= c->hpin_cap) {  // where queue_results used it
-    h = reinterpret_cast<const double*>(c->hpin) + p->n_eF + p->n_hw;
+  const double* h = pinned_record(c, p, rec);
+  if (h) {
     HIPCHK(hipStreamSynchronize(c->st));
+    c->hpin_busy = false;
     int info;
     memcpy(&info, h + rec, sizeof(int));
     if (solved) CHK(info_status(c, info));
@@ -980,6 +993,7 @@ extern "C" int mep_interp_batch(mep_ctx* c, int64_t nk, const double* kpts, doub
     for (int i = 0; i < np; q += part[i++].len)
       HIPCHK(hipMemcpyAsync(q, part[i].src, part[i].len, hipMemcpyDeviceToHost, c->st));
     HIPCHK(hipStreamSynchronize(c->st));
+    c->hpin_busy = false;
     q = h + bk;
     for (int i = 0; i < np; q += part[i++].len) memcpy(part[i].dst, q, part[i].len);
     CHK(info_status(c, info));
@@ -1128,12 +1142,29 @@ static int run_common(mep_ctx* c, int64_t nk, const int32_t* mp, const double* k
   return unpack(c, bs, p, nk, out);
 }
 
+// Ends a batch: unless it is done, every context that the set-up reached is
+// waited for and its eigensolver status cleared, so that an error of one model
+// leaves nothing on the other models' streams and no status for their next call.
+struct BatchEnd {
+  mep_ctx* const* ctxs;
+  int32_t n = 0;  // contexts reached
+  bool done = false;
+  ~BatchEnd() {
+    for (int32_t i = 0; i < n && !done; ++i) {
+      mep_ctx* c = ctxs[i];
+      hipMemsetAsync(c->dinfo, 0, sizeof(int), c->st);
+      if (hipStreamSynchronize(c->st) == hipSuccess) c->hpin_busy = false;
+    }
+  }
+};
+
 extern "C" int mep_run_batch(int32_t n_models, mep_ctx* const* ctxs, const int32_t* mp_grids,
                              const mep_run_params* params, mep_sums* outs) {
   if (n_models < 1 || !ctxs || !mp_grids || !params)
     return fail(MEP_ERR_ARG, "mep_run_batch: bad argument");
   std::vector<BandSetup> bs((size_t)n_models);
   std::vector<int64_t> nk((size_t)n_models);
+  BatchEnd end{ctxs};
   int64_t rounds = 0;
   for (int32_t i = 0; i < n_models; ++i) {
     mep_ctx* c = ctxs[i];
@@ -1144,6 +1175,7 @@ extern "C" int mep_run_batch(int32_t n_models, mep_ctx* const* ctxs, const int32
     if (mp[0] < 1 || mp[1] < 1 || mp[2] < 1)
       return fail(MEP_ERR_ARG, "mep_run_batch: mp_grid entries must be >= 1");
     nk[i] = (int64_t)mp[0] * mp[1] * mp[2];
+    end.n = i + 1;
     CHK(ensure_ws(c, nk[i]));
     CHK(sep_prepare(c, mp));
     CHK(band_setup(c, &params[i], c->kcap, bs[i]));
@@ -1162,6 +1194,7 @@ extern "C" int mep_run_batch(int32_t n_models, mep_ctx* const* ctxs, const int32
   for (int32_t i = 0; i < n_models; ++i) CHK(queue_results(ctxs[i], bs[i], &params[i]));
   for (int32_t i = 0; i < n_models; ++i)
     CHK(unpack(ctxs[i], bs[i], &params[i], nk[i], outs ? &outs[i] : nullptr));
+  end.done = true;
   return MEP_OK;
 }
 
@@ -1296,6 +1329,7 @@ extern "C" int mep_run_batch_graph(int32_t n_models, mep_ctx* const* ctxs,
     return fail(MEP_ERR_ARG, "mep_run_batch_graph: bad argument");
   std::vector<BandSetup> bs((size_t)n_models);
   std::vector<int64_t> nk((size_t)n_models);
+  BatchEnd end{ctxs};
   int64_t rounds = 0;
   for (int32_t i = 0; i < n_models; ++i) {
     mep_ctx* c = ctxs[i];
@@ -1310,6 +1344,7 @@ extern "C" int mep_run_batch_graph(int32_t n_models, mep_ctx* const* ctxs,
     if (params[i].hw_lst && params[i].n_hw < 1)
       return fail(MEP_ERR_ARG, "mep_run_batch_graph: n_hw must be >= 1");
     nk[i] = (int64_t)mp[0] * mp[1] * mp[2];
+    end.n = i + 1;
     CHK(ensure_ws(c, nk[i]));
     CHK(sep_prepare(c, mp));
     CHK(band_setup(c, &params[i], c->kcap, bs[i]));
@@ -1317,7 +1352,10 @@ extern "C" int mep_run_batch_graph(int32_t n_models, mep_ctx* const* ctxs,
     if (nblk > rounds) rounds = nblk;
   }
   // the uploads of the set-up precede the graph on every context's stream
-  for (int32_t i = 0; i < n_models; ++i) HIPCHK(hipStreamSynchronize(ctxs[i]->st));
+  for (int32_t i = 0; i < n_models; ++i) {
+    HIPCHK(hipStreamSynchronize(ctxs[i]->st));
+    ctxs[i]->hpin_busy = false;
+  }
   BatchGraph* g = nullptr;
   {
     std::lock_guard<std::mutex> lk(g_bg_mu);
@@ -1367,6 +1405,7 @@ extern "C" int mep_run_batch_graph(int32_t n_models, mep_ctx* const* ctxs,
       outs[i].n_k = nk[i];
     }
   }
+  end.done = true;
   return MEP_OK;
 }
 

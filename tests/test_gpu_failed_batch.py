@@ -42,3 +42,34 @@ def test_band_sums_of_given_bands_after_a_failed_graph_batch(n):
             got = eng.bandsum(e, V, p)
             for q in JOBS_KEYS:
                 assert np.array_equal(got[q], ref[q]), q
+
+
+@pytest.mark.parametrize("graph", [False, True])
+def test_next_calls_after_a_failed_batch(graph):
+    """The first model is refused while the others, which take longer, are still
+    at work: an interpolation and a run on each of them right after the error
+    equal those of engines that saw no failed batch, bit for bit."""
+    from mepinterp_amd import capi
+    n, mesh = 40, (16, 16, 8)
+    p = _params(n)
+    k = rand_kpts(3, seed=1)
+
+    def calls(eng):
+        return eng.interp(k, velo=False)[0], eng.run_mesh((4, 3, 2), p), eng.interp(k)
+    ref = []
+    for seed in (6, 7):
+        with _engine(n, seed) as eng:
+            eng.run_mesh(mesh, p)  # the same workspace as below
+            ref.append(calls(eng))
+    with _engine(n, 6) as b, _engine(n, 7) as c, _engine(8, 4, nan=True) as a:
+        for _ in range(2):
+            with pytest.raises(capi.MepError):
+                capi.run_batch([a, b, c], [(2, 2, 1), mesh, mesh], [_params(8), p, p],
+                               graph=graph)
+            for eng, (e0, s0, v0) in zip((c, b), (ref[1], ref[0])):
+                e1, s1, v1 = calls(eng)
+                assert np.array_equal(e1, e0)
+                for q in JOBS_KEYS:
+                    assert np.array_equal(s1[q], s0[q]), q
+                for g, r in zip(v1[:2], v0[:2]):
+                    assert np.array_equal(g, r)
