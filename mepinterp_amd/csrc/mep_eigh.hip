@@ -742,9 +742,9 @@ __global__ __launch_bounds__(64) void eigh_ql_kernel(int n, R* __restrict__ side
 
 // Eigenvalues and the separation verdict by QL with d and e in registers (the
 // FP32 path, and FP64 for the sums with unbroadened poles, see launch_eigh):
-// one lane per k-point, NMAX <= 32, every array index a compile-time constant,
-// no LDS.  The k-points with verdict -2 are listed for eigh_ql.  The active block always starts at index
-// 0: when e[0] is negligible, d[0] is an eigenvalue and both arrays rotate
+// one lane per k-point, NMAX <= 48, every array index a compile-time constant,
+// no LDS.  The k-points with verdict -2 are listed for eigh_ql.  The active block
+// always starts at index 0: when e[0] is negligible, d[0] is an eigenvalue and both arrays rotate
 // down by one (d[0] moves to the end), so after NMAX deflations d[j] holds
 // the j-th eigenvalue found, where ql_one's LDS column holds it.  Entries
 // n .. NMAX-1 are decoupled padding (e = 0) that deflates as soon as it
@@ -2650,9 +2650,20 @@ void launch_eigh_wide(hipStream_t s, int n, int64_t nk, const zd* Hk, int64_t st
   }
   int64_t qb = (nk + 31) / 32;
   unsigned qgrid = (unsigned)(qb < 65536 ? qb : 65536);
-  // eigenvalues and the separation verdict, then the listed k-points
+  // eigenvalues and the separation verdict, then the listed k-points.  QL: with
+  // d and e in registers up to 48 bands, which holds more k-points in flight than
+  // LDS columns do (with the reduction and the vectors, 4,096 k-points: n = 36 1.19
+  // ms, LDS columns 1.63; n = 48 1.59, 2.42)
   const unsigned sgrid = (unsigned)(nk < 65536 ? nk : 65536);
-  if (ql)
+  const int64_t qb64 = (nk + 63) / 64;
+  const unsigned qgrid64 = (unsigned)(qb64 < 65536 ? qb64 : 65536);
+  if (ql && n <= 40)
+    hipLaunchKernelGGL((eigh_ql_reg_kernel<40, double>), dim3(qgrid64), dim3(64), 0, s, n, nk, side,
+                       E, info, list, count);
+  else if (ql && n <= 48)
+    hipLaunchKernelGGL((eigh_ql_reg_kernel<48, double>), dim3(qgrid64), dim3(64), 0, s, n, nk, side,
+                       E, info, list, count);
+  else if (ql)
     hipLaunchKernelGGL(eigh_ql_wide_kernel, dim3(qgrid), dim3(32), lq, s, n, nk, side, rot, rcol,
                        E, info, false, list, count);
   else if (n <= 64)

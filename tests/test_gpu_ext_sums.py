@@ -38,3 +38,22 @@ def test_ext_sums_at_tile_and_item_edges(n, n_eF, n_hw, with_r, T):
         err = np.max(np.abs(g[key] - ref))
         # 1e-9, the sums' tolerance (n = 1 has no pairs: zero on both sides)
         assert err <= 1e-9 * scale, (key, err, scale)
+
+
+@pytest.mark.parametrize("n", [40, 41, 48, 49])
+def test_ext_sums_at_the_edges_of_the_register_ql(n):
+    """Eigenvalues by QL in registers (two widths) and in LDS columns.  The
+    frequencies lie above every gap, so no unbroadened pole is near."""
+    import oracle as O
+    from mepinterp_amd import capi, models
+    m = models.make_random(seed=60 + n, n=n, L=1, with_r=True)
+    k = rand_kpts(70, seed=n)  # more than the 64 k-points of a workgroup
+    width = 2.0 * np.max(np.sum(np.abs(m["H"]), axis=(1, 2)))  # of the spectrum, at most
+    kw = dict(n_eF=2, eF_min=-0.02, eF_max=0.02, n_hw=2, hw_min=width, hw_max=2.0 * width,
+              T_kelvin=300.0, eta=0.004, valence_bands=1)
+    with capi.Engine(m["R_frac"], m["H"], r=m["r"], a_latt=m["a_latt"]) as eng:
+        g = eng.run_kpts(k, capi.Engine.params(jobs=capi.MEP_JOB_OPT, **kw))
+    o = O.accumulate(oracle_model(m), O.RunParams(do_opt=True, **kw), k)
+    for key in ("opt_s", "opt_a", "photo"):
+        # 1e-9, the sums' tolerance
+        assert np.max(np.abs(g[key] - o[key])) <= 1e-9 * np.max(np.abs(o[key])), key
