@@ -137,7 +137,10 @@ int mep_interp_batch(mep_ctx *ctx, int64_t nk, const double *kpts, double *e_k, 
    mep_niu_IC/LC/CS (mep_niu.f90:20-159).  With nk = 1 the outputs are the
    reference functions' results.  fd_distrib(n_eF,n,nk) supplies the
    occupations as the reference's kubo_* arguments do; NULL = fd_stat of
-   e_k at the p->n_eF Fermi levels and p->T_kelvin.                          */
+   e_k at the p->n_eF Fermi levels and p->T_kelvin.  e_k is ascending at each
+   k-point, as get_wann_interp returns it: which m the guard of mep_niu_IC
+   excludes for a pair (n0, n) is searched outward from n0 by index, and ends
+   at the first m that is kept.  The other sums do not depend on the order.   */
 int mep_bandsum_batch(mep_ctx *ctx, int64_t nk, const double *e_k, const double *V_ka,
                       const double *A_ka, const double *Om_kab, const double *fd_distrib,
                       const mep_run_params *p, mep_sums *out);

@@ -331,12 +331,14 @@ __global__ __launch_bounds__(BS_THREADS, 2) void bandsum_kernel(BandArgs b, doub
     // rounding is monotone, so every |(E0-En)^2 (E0-Em)| and |E0-En|^3 is at
     // least that): such a k-point needs no windows and no second sums.  The
     // same in every wavefront.  (n = 32, 16 valence bands over 4 Ha: 95 of 100
-    // k-points at the default kubo_tol.)
+    // k-points at the default kubo_tol.)  General V: the energies may be a
+    // caller's, in any order, so that the neighbouring index need not be the
+    // nearest band; a k-point out of order is not clean.
     bool clean = true;
-    if (doNjob && lane < n && lane < nval) {
+    if (doNjob && lane < n && (!HERM || lane < nval)) {
       const double g0 = lane > 0 ? Es[lane] - Es[lane - 1] : HUGE_VAL;
       const double g1 = lane < n - 1 ? Es[lane + 1] - Es[lane] : HUGE_VAL;
-      clean = g0 * g0 * g0 > tol && g1 * g1 * g1 > tol;
+      clean = lane < nval ? g0 * g0 * g0 > tol && g1 * g1 * g1 > tol : g0 >= 0.0;
     }
     clean = __ballot(!clean) == 0;
     // ---- r(m, c) = 1 / (E_c - E_m); occupations ---------------------------
@@ -1028,21 +1030,31 @@ __global__ __launch_bounds__(256, 2) void bandsum_wide_kernel(BandArgs b, double
     if (t < n) Es[t] = E[k * n + t];
     __syncthreads();
     // the valence bands whose Niu guards exclude something: not those with g^3 >
-    // kubo_tol, g the gap to the nearest band (see bandsum_kernel).  Bit n0 of
-    // dirty, the same in every wavefront; only these have windows
+    // kubo_tol, g the gap to the nearest band (see bandsum_kernel), nor, at a
+    // k-point out of order, any.  Bit n0 of dirty, the same in every wavefront;
+    // only these have windows
     uint64_t dirty[2] = {0, 0};
-    if (doNjob)
+    if (doNjob) {
+      bool up = true;  // ascending
 #pragma unroll
       for (int q = 0; q < 2; ++q) {
         const int n0 = 64 * q + lane;
         bool d = false;
-        if (n0 < n && n0 < nval) {
+        if (n0 < n && (!HERM || n0 < nval)) {
           const double g0 = n0 > 0 ? Es[n0] - Es[n0 - 1] : HUGE_VAL;
           const double g1 = n0 < n - 1 ? Es[n0 + 1] - Es[n0] : HUGE_VAL;
-          d = !(g0 * g0 * g0 > tol && g1 * g1 * g1 > tol);
+          d = n0 < nval && !(g0 * g0 * g0 > tol && g1 * g1 * g1 > tol);
+          up = up && (HERM || g0 >= 0.0);
         }
         dirty[q] = __ballot(d);
       }
+      if (!HERM && __ballot(!up)) {
+        auto low = [](int c) { return c >= 64 ? ~0ull : c > 0 ? (1ull << c) - 1 : 0ull; };
+        const int nv = nval < n ? nval : n;
+        dirty[0] = low(nv);
+        dirty[1] = low(nv - 64);
+      }
+    }
 #pragma unroll
     for (int q = 0; q < 2; ++q)
       for (uint64_t m = dirty[q]; m; m &= m - 1) {

@@ -91,3 +91,26 @@ def test_no_hall_sums_with_a_long_frequency_list():
         many = eng.run_kpts(k, capi.Engine.params(n_hw=300, **kw))
     for q in KEYS[4:]:
         assert np.array_equal(one[q], many[q]), q
+
+
+@pytest.mark.parametrize("n", [5, 16, 20, 32, 36, 70])
+def test_given_bands_out_of_order(n):
+    """A close band that is no neighbour by index: its whole row is excluded by
+    the guards of the Niu terms, every other row keeps all but n0."""
+    import oracle as O
+    from mepinterp_amd import capi, models
+    # rows of the close band: at most delta^2 0.6 n <= 1.1e-3, the others: at
+    # least 0.59^2 delta = 1.7e-3
+    tol, delta, nk, nv = 1.2e-3, 5e-3, 3, max(2, n // 2)
+    rng = np.random.default_rng(n)
+    e = np.repeat(0.6 * np.arange(n)[:, None], nk, axis=1)
+    e[n - 1] = e[1] + delta
+    V = rng.standard_normal((3, n, n, nk)) + 1j * rng.standard_normal((3, n, n, nk))
+    m = models.make_random(seed=n, n=n, L=1)
+    with capi.Engine(m["R_frac"], m["H"], a_latt=m["a_latt"], kubo_tol=tol) as eng:
+        g = eng.bandsum(e, V, capi.Engine.params(jobs=capi.MEP_JOB_MEP, valence_bands=nv))
+    for q, f in (("niu_ic", O.mep_niu_ic), ("niu_lc", O.mep_niu_lc)):
+        ref = sum(f(np.asfortranarray(V[..., i]), np.ascontiguousarray(e[:, i]), nv, tol)
+                  for i in range(nk))
+        # 1e-9, the sums' tolerance
+        assert np.max(np.abs(g[q] - ref)) <= 1e-9 * np.max(np.abs(ref)), q
