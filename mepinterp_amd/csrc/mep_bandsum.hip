@@ -468,7 +468,8 @@ __global__ __launch_bounds__(BS_THREADS, 2) void bandsum_kernel(BandArgs b, doub
           const zd denv = zd{dE * dE - w2.re, -w2.im};
           const zd deno = zmul(zd{dE, 0.0}, zd{dE - wq.re, -wq.im});
           const double iv = 1.0 / zabs2(denv), io = 1.0 / zabs2(deno);
-          const bool off = nn != p0;
+          // (the padding's energy, 0, may be a band's)
+          const bool off = nn != p0 && p0 < n;
           const zd rv = off ? zd{denv.re * iv * dfv, -denv.im * iv * dfv} : zd{0.0, 0.0};
           const zd ro = off ? zd{deno.re * io * dfv, -deno.im * io * dfv} : zd{0.0, 0.0};
 #pragma unroll

@@ -114,3 +114,22 @@ def test_given_bands_out_of_order(n):
                   for i in range(nk))
         # 1e-9, the sums' tolerance
         assert np.max(np.abs(g[q] - ref)) <= 1e-9 * np.max(np.abs(ref)), q
+
+
+@pytest.mark.parametrize("n", [3, 16, 24])
+def test_a_band_at_zero_energy(n):
+    """The padding of the band tables holds zeros too."""
+    import oracle as O
+    from mepinterp_amd import capi, models
+    rng = np.random.default_rng(n)
+    e = 0.1 * np.arange(n)
+    V = np.asfortranarray(rng.standard_normal((3, n, n)) + 1j * rng.standard_normal((3, n, n)))
+    fd = np.asfortranarray(np.linspace(0.9, 0.2, n)[None])
+    m = models.make_random(seed=n, n=n, L=1)
+    with capi.Engine(m["R_frac"], m["H"], a_latt=m["a_latt"]) as eng:
+        g = eng.bandsum(e, V[..., None], capi.Engine.params(
+            jobs=capi.MEP_JOB_AHC | capi.MEP_JOB_KUBO, n_hw=1, hw_min=0.03, hw_max=0.03, eta=0.01), fd=fd)
+    for q, f in (("ahc_velo", O.velo_ahc_tens), ("ohc", O.kubo_ohc_tens)):
+        ref = f(e, V, np.array([0.03]), fd, 0.01).reshape(g[q].shape, order="F")
+        # 1e-9, the sums' tolerance
+        assert np.max(np.abs(g[q] - ref)) <= 1e-9 * np.max(np.abs(ref)), q
