@@ -1590,25 +1590,38 @@ size_t bandsum_wide_lds_bytes(const BandArgs& b) {
 //   velo  g Im(P_ji - P_ij),  g = f / (dE^2 - w^2)
 //   ohc   f / (dE (dE - w)) P_ij - f / (dE (dE + w)) P_ji
 //         = g (P_ij - P_ji) + w g (P_ij + P_ji) / dE
-// so one complex g serves all of them: the sums of g A, A_c = P_ij - P_ji, and
-// of g S, S_ij = (P_ij + P_ji) / dE, are what the items keep, and w enters once
-// at the end.  With D = (dE - hw)(dE + hw) + eta^2 (no cancellation at
-// resonance) and B = 2 hw eta, g = (D + i B) r, r = f / (D^2 + B^2): the items
-// sum D r v and r v over the real values v of A and S, and B waits as well.
-// Hermitian V: Im A (3), Re S (3) and S_ii (3), the others being zero; general
-// V: those of all 18.
+// so with Hermitian V one complex g serves all of them: the sums of g A, A_c =
+// P_ij - P_ji, and of g S, S_ij = (P_ij + P_ji) / dE, are what the items keep,
+// and w enters once at the end.  With D = (dE - hw)(dE + hw) + eta^2 (no
+// cancellation at resonance) and B = 2 hw eta, g = (D + i B) r, r = f / (D^2 +
+// B^2): the items sum D r v and r v over the real values v of A and S, and B
+// waits as well: Im A (3), Re S (3) and S_ii (3), the others being zero.
+//
+// General V: P_ij and P_ji are of different sizes.  The weight of the order
+// that is not in resonance would be the difference of two terms larger by dE /
+// eta, so the off-diagonal ohc sums (6, complex) take each order's own weight,
+//   f / (dE - w) = (dE - hw + i eta) f m2 / (m1 m2),  m1 = |dE - w|^2
+//   f / (dE + w) = (dE + hw - i eta) f m1 / (m1 m2),  m2 = |dE + w|^2
+// (1 / dE is in the record), which share g's one reciprocal, m1 m2 = D^2 + B^2;
+// S_ii (3, complex), where both orders weigh the same value, and Im A (3) as
+// above.
 //
 // Bound by FP64 VALU issue: 2 x 9 fma and about 13 more a record and item
 // (Hermitian V); four items a thread take the reads of a record from LDS off
 // the LDS return path.
 // n = 96, 256 frequencies, 2,744 k-points: 2.8 ms (three denominators for the
 // two orders, 24 sums an item: 4.2); n = 20, 80 items, 24,273: 0.50 ms (0.88);
-// general V, n = 14, 16 items, 2,730: 40 us (59).
+// general V, n = 14, 16 items, 2,730: 50 us (59 with a reciprocal for each
+// weight and ordered pair; 40 with g alone, at the loss above: 7e-9 of an element
+// at eta = 1e-8, now 3e-16).
 // ===========================================================================
 constexpr int HW_CH = 256;  // pair candidates per chunk (one per thread)
 
+// values of a record; real sums of an item, in three parts of at most hw_part
 template <bool HERM>
-__host__ __device__ constexpr int hw_vals() { return HERM ? 9 : 18; }
+__host__ __device__ constexpr int hw_vals() { return HERM ? 9 : 21; }
+template <bool HERM>
+__host__ __device__ constexpr int hw_part() { return HERM ? 6 : 12; }
 
 template <bool HERM, int IPT>
 __global__ __launch_bounds__(256, 2) void hwsum_kernel(BandArgs b, double Tsmear, AccLayout L,
@@ -1616,7 +1629,7 @@ __global__ __launch_bounds__(256, 2) void hwsum_kernel(BandArgs b, double Tsmear
                                                        const zd* __restrict__ V,
                                                        const double* __restrict__ w,
                                                        double* __restrict__ part) {
-  constexpr int NV = hw_vals<HERM>(), NP = NV / 3;  // values; values of A, S and S_ii each
+  constexpr int NV = hw_vals<HERM>(), NP = hw_part<HERM>();
   extern __shared__ double smem[];
   const int n = b.n, nef = b.n_ef, nhw = b.n_hw;
   const int PS = 1 + nef + NV;  // doubles per record: dE, f[nef], v[NV]
@@ -1649,11 +1662,13 @@ __global__ __launch_bounds__(256, 2) void hwsum_kernel(BandArgs b, double Tsmear
       wr[u] = b.hw[it % nhw];
       B2[u] = 4.0 * wr[u] * wr[u] * eta2;
     }
-    double aD[IPT][NV], aR[IPT][NV];  // sums of D r v and of r v
+    // HERM: sums of D r v and of r v of A, S, S_ii; general V: the ohc sums, then
+    // those of S_ii and of Im A
+    double acc[IPT][3][NP];
 #pragma unroll
     for (int u = 0; u < IPT; ++u)
 #pragma unroll
-      for (int q = 0; q < NV; ++q) aD[u][q] = aR[u][q] = 0.0;
+      for (int q = 0; q < 3 * NP; ++q) acc[u][q / NP][q % NP] = 0.0;
     for (int64_t k = blockIdx.x; k < nk; k += gridDim.x) {
       const double wk = w ? w[k] : 1.0;
       const zd* Vk = V + k * 3 * (int64_t)n2;
@@ -1699,7 +1714,8 @@ __global__ __launch_bounds__(256, 2) void hwsum_kernel(BandArgs b, double Tsmear
           zd vxy[3];
 #pragma unroll
           for (int a = 0; a < 3; ++a) vxy[a] = Vk[a * (int64_t)n2 + x + (int64_t)n * y];
-          // v: A_c, S_c (c = (0,1), (0,2), (1,2)), S_ii
+          // v: A_c, S_c (c = (0,1), (0,2), (1,2)), S_ii; general V: P_ij / dE and
+          // P_ji / dE of each c, S_ii, Im A_c
           if constexpr (HERM) {  // V(y, x) = conj V(x, y): Im A, Re S, S_ii
 #pragma unroll
             for (int c = 0; c < 3; ++c) {
@@ -1716,14 +1732,14 @@ __global__ __launch_bounds__(256, 2) void hwsum_kernel(BandArgs b, double Tsmear
             for (int c = 0; c < 3; ++c) {
               const int i = c == 2 ? 1 : 0, j = c == 0 ? 1 : 2;
               const zd pij = zmul(vyx[i], vxy[j]), pji = zmul(vyx[j], vxy[i]);
-              const zd A = zsub(pij, pji), Sc = zscale(zadd(pij, pji), iE);
               const zd Sd = zscale(zmul(vyx[c], vxy[c]), 2.0 * iE);
-              v[2 * c] = A.re;
-              v[2 * c + 1] = A.im;
-              v[6 + 2 * c] = Sc.re;
-              v[7 + 2 * c] = Sc.im;
+              v[4 * c] = pij.re * iE;
+              v[4 * c + 1] = pij.im * iE;
+              v[4 * c + 2] = pji.re * iE;
+              v[4 * c + 3] = pji.im * iE;
               v[12 + 2 * c] = Sd.re;
               v[13 + 2 * c] = Sd.im;
+              v[18 + c] = pij.im - pji.im;
             }
           }
         }
@@ -1738,22 +1754,46 @@ __global__ __launch_bounds__(256, 2) void hwsum_kernel(BandArgs b, double Tsmear
 #pragma unroll
             for (int u = 0; u < IPT; ++u) {
               // f = 0 records (another E_F differs) contribute exactly zero
-              const double D = (dE - wr[u]) * (dE + wr[u]) + eta2;
-              const double r = sp[1 + ef[u]] * rcp_nr(D * D + B2[u]), Dr = D * r;
+              const double D1 = dE - wr[u], D2 = dE + wr[u];
+              const double D = D1 * D2 + eta2;
+              if constexpr (HERM) {
+                const double r = sp[1 + ef[u]] * rcp_nr(D * D + B2[u]), Dr = D * r;
 #pragma unroll
-              for (int q = 0; q < NV; ++q) {
-                aD[u][q] += Dr * v[q];
-                aR[u][q] += r * v[q];
+                for (int q = 0; q < NV; ++q) {
+                  acc[u][q / 3][q % 3] += Dr * v[q];
+                  acc[u][q / 3][3 + q % 3] += r * v[q];
+                }
+              } else {
+                const double m1 = D1 * D1 + eta2, m2 = D2 * D2 + eta2;
+                const double r = sp[1 + ef[u]] * rcp_nr(m1 * m2), Dr = D * r;
+                const double t1 = r * m2, t2 = r * m1;
+                const zd w1 = zd{D1 * t1, b.eta * t1}, w2 = zd{D2 * t2, -b.eta * t2};
+#pragma unroll
+                for (int c = 0; c < 3; ++c) {
+                  const zd pij = zd{v[4 * c], v[4 * c + 1]}, pji = zd{v[4 * c + 2], v[4 * c + 3]};
+                  const zd xij = zsub(zmul(w1, pij), zmul(w2, pji));
+                  const zd xji = zsub(zmul(w1, pji), zmul(w2, pij));
+                  acc[u][0][4 * c] += xij.re;
+                  acc[u][0][4 * c + 1] += xij.im;
+                  acc[u][0][4 * c + 2] += xji.re;
+                  acc[u][0][4 * c + 3] += xji.im;
+                  acc[u][2][c] += Dr * v[18 + c];
+                  acc[u][2][3 + c] += r * v[18 + c];
+                }
+#pragma unroll
+                for (int q = 0; q < 6; ++q) {
+                  acc[u][1][q] += Dr * v[12 + q];
+                  acc[u][1][6 + q] += r * v[12 + q];
+                }
               }
             }
           }
       }
     }
-    // combine the splits of each item, A, S and S_ii in turn, in
-    // red[split][item][2 NP] over the staging area, and add what each gives:
-    // with G = sum g v (g = (D + i B) r), velo_ij = -Im part of A's sums (as a
-    // complex g), ohc_ij = i (G_A + w G_S), ohc_ji = i (w G_S - G_A), ohc_ii =
-    // i w G_Sii
+    // combine the splits of each item, part by part, in red[split][item][NP] over
+    // the staging area, and add what each gives.  With G = sum g v (g = (D + i B)
+    // r): velo_ij = -G(Im A) (+ for ji), ohc_ij = i (G(A) + w G(S)), ohc_ji = i (w
+    // G(S) - G(A)), ohc_ii = i w G(S_ii); general V: ohc_ij is i times its own sum
 #pragma unroll
     for (int third = 0; third < 3; ++third) {
       __syncthreads();
@@ -1762,35 +1802,18 @@ __global__ __launch_bounds__(256, 2) void hwsum_kernel(BandArgs b, double Tsmear
         for (int u = 0; u < IPT; ++u)
           if (iok[u])
 #pragma unroll
-            for (int q = 0; q < NP; ++q) {
-              double* o = st + (split * IW + slot + IWT * u) * 2 * NP;
-              o[q] = aD[u][third * NP + q];
-              o[NP + q] = aR[u][third * NP + q];
-            }
+            for (int q = 0; q < NP; ++q) st[(split * IW + slot + IWT * u) * NP + q] = acc[u][third][q];
       __syncthreads();
       for (int o = t; o < IW * 3; o += 256) {
         const int i2 = o / 3, c = o % 3;
         const int item = g0 + i2, hh = item % nhw, e2 = item / nhw;
         const zd wq = zd{b.hw[hh], b.eta};
         const double B = 2.0 * wq.re * wq.im;
-        auto G = [&](int q) {  // sum of g v_q over the splits
-          double sD = 0.0, sR = 0.0;
-          for (int u = 0; u < S; ++u) {
-            sD += st[(u * IW + i2) * 2 * NP + q];
-            sR += st[(u * IW + i2) * 2 * NP + NP + q];
-          }
-          return zd{sD, B * sR};
+        auto sum = [&](int q) {  // over the splits
+          double s_ = 0.0;
+          for (int u = 0; u < S; ++u) s_ += st[(u * IW + i2) * NP + q];
+          return s_;
         };
-        zd Gi = zd{0.0, 0.0}, Z;  // sum of g Im v; sum of g v
-        if constexpr (HERM) {
-          const zd x = G(c);
-          Gi = x;
-          Z = third == 0 ? zmuli(x) : x;
-        } else {
-          const zd x = G(2 * c);
-          Gi = G(2 * c + 1);
-          Z = zadd(x, zmuli(Gi));
-        }
         double* av = accp + L.velo + 2 * 9 * (hh + (int64_t)nhw * e2);
         double* ao = accp + L.ohc + 2 * 9 * (hh + (int64_t)nhw * e2);
         const int i = c == 2 ? 1 : 0, j = c == 0 ? 1 : 2;
@@ -1798,19 +1821,32 @@ __global__ __launch_bounds__(256, 2) void hwsum_kernel(BandArgs b, double Tsmear
           p[0] += sgn * z.re;
           p[1] += sgn * z.im;
         };
-        if (third == 0) {
-          add(av + 2 * (i + 3 * j), Gi, -1.0);
-          add(av + 2 * (j + 3 * i), Gi, 1.0);
-          add(ao + 2 * (i + 3 * j), zmuli(Z), 1.0);
-          add(ao + 2 * (j + 3 * i), zmuli(Z), -1.0);
-        } else {
-          const zd iwZ = zmuli(zmul(wq, Z));
-          if (third == 1) {
-            add(ao + 2 * (i + 3 * j), iwZ, 1.0);
-            add(ao + 2 * (j + 3 * i), iwZ, 1.0);
+        if constexpr (HERM) {
+          const zd x = zd{sum(c), B * sum(3 + c)};  // sum of g v
+          if (third == 0) {                         // v = Im A
+            add(av + 2 * (i + 3 * j), x, -1.0);
+            add(av + 2 * (j + 3 * i), x, 1.0);
+            add(ao + 2 * (i + 3 * j), x, -1.0);
+            add(ao + 2 * (j + 3 * i), x, 1.0);
           } else {
-            add(ao + 2 * 4 * c, iwZ, 1.0);
+            const zd iwZ = zmuli(zmul(wq, x));
+            if (third == 1) {
+              add(ao + 2 * (i + 3 * j), iwZ, 1.0);
+              add(ao + 2 * (j + 3 * i), iwZ, 1.0);
+            } else {
+              add(ao + 2 * 4 * c, iwZ, 1.0);
+            }
           }
+        } else if (third == 0) {
+          add(ao + 2 * (i + 3 * j), zmuli(zd{sum(4 * c), sum(4 * c + 1)}), 1.0);
+          add(ao + 2 * (j + 3 * i), zmuli(zd{sum(4 * c + 2), sum(4 * c + 3)}), 1.0);
+        } else if (third == 1) {
+          const zd gr = zd{sum(2 * c), B * sum(6 + 2 * c)}, gi = zd{sum(2 * c + 1), B * sum(7 + 2 * c)};
+          add(ao + 2 * 4 * c, zmuli(zmul(wq, zadd(gr, zmuli(gi)))), 1.0);
+        } else {
+          const zd x = zd{sum(c), B * sum(3 + c)};
+          add(av + 2 * (i + 3 * j), x, -1.0);
+          add(av + 2 * (j + 3 * i), x, 1.0);
         }
       }
     }
@@ -1818,8 +1854,9 @@ __global__ __launch_bounds__(256, 2) void hwsum_kernel(BandArgs b, double Tsmear
 }
 
 // items per thread: four from eight items on (n = 96, 256 items: 2.8 ms, one
-// 3.1; n = 20, 80 items: 0.50, 0.51); general V's 36 sums an item leave
-// registers for two, which was slower (n = 14, 16 items: 52 us, one 40)
+// 3.1; n = 20, 80 items: 0.50, 0.51); general V's 30 sums an item leave no
+// registers for four, and two were slower (with 36 sums, n = 14, 16 items: 52
+// us, one 40)
 static int hwsum_ipt(const BandArgs& b) {
   return b.v_herm && (int64_t)b.n_hw * b.n_ef >= 8 ? 4 : 1;
 }
@@ -1964,7 +2001,7 @@ __global__ __launch_bounds__(256, 2) void hall_kernel(BandArgs b, double Tsmear,
                                                       const double* __restrict__ w,
                                                       double* __restrict__ part) {
   static_assert(!PMODE || NEF == 1, "");
-  constexpr int NA = 9 * NEF, NQ = PMODE ? 36 : 0;
+  constexpr int NA = 9 * NEF, NQ = PMODE ? 30 : 0;
   __shared__ double Es[128], fd[NEF * 128], wks[HALL_KB], red[4 * (NA + NQ + NEF)];
   const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
   const int n = b.n, n2 = n * n, npair = n * (n - 1) / 2;
@@ -1972,8 +2009,10 @@ __global__ __launch_bounds__(256, 2) void hall_kernel(BandArgs b, double Tsmear,
   // k-points at a time: KB n <= 128
   int KB = npair ? 256 / npair : HALL_KB;
   KB = KB < 1 ? 1 : KB > HALL_KB ? HALL_KB : KB;
-  const double wr = b.hw[0], eta2 = b.eta * b.eta, B2 = 4.0 * wr * wr * eta2;
-  double ah[NA], pv[NQ + 1], ne[NEF];  // per level: S (3), A (3), S_ii (3); D q v, q v
+  const double wr = b.hw[0], eta2 = b.eta * b.eta;
+  // per level: S (3), A (3), S_ii (3); the ohc sums (6, complex), then D q v and
+  // q v of S_ii and of Im A
+  double ah[NA], pv[NQ + 1], ne[NEF];
 #pragma unroll
   for (int q = 0; q < NA; ++q) ah[q] = 0.0;
 #pragma unroll
@@ -2039,23 +2078,28 @@ __global__ __launch_bounds__(256, 2) void hall_kernel(BandArgs b, double Tsmear,
         // selects drop pairs of equal occupation
         const double f = fx[0] - fy[0];
         const bool on = f != 0.0;
-        const double D = (dE - wr) * (dE + wr) + eta2;
-        const double g = on ? wk * f * rcp_nr(D * D + B2) : 0.0, Dg = D * g;
+        const double D1 = dE - wr, D2 = dE + wr, D = D1 * D2 + eta2;
+        const double m1 = D1 * D1 + eta2, m2 = D2 * D2 + eta2;
+        const double g = on ? wk * f * rcp_nr(m1 * m2) : 0.0, Dg = D * g;
         const double rs = on ? r : 0.0, gr = g * rs, Dgr = Dg * rs;
+        const double t1 = gr * m2, t2 = gr * m1;
+        const zd w1 = zd{D1 * t1, b.eta * t1}, w2 = zd{D2 * t2, -b.eta * t2};
 #pragma unroll
         for (int q = 0; q < 3; ++q) {
-          pv[2 * q] += Dg * A[q].re;
-          pv[2 * q + 1] += Dg * A[q].im;
-          pv[6 + 2 * q] += Dgr * S[q].re;
-          pv[7 + 2 * q] += Dgr * S[q].im;
+          const int i = q == 2 ? 1 : 0, j = q == 0 ? 1 : 2;
+          const zd pij = zmul(vyx[i], vxy[j]), pji = zmul(vyx[j], vxy[i]);
+          const zd xij = zsub(zmul(w1, pij), zmul(w2, pji));
+          const zd xji = zsub(zmul(w1, pji), zmul(w2, pij));
+          pv[4 * q] += xij.re;
+          pv[4 * q + 1] += xij.im;
+          pv[4 * q + 2] += xji.re;
+          pv[4 * q + 3] += xji.im;
           pv[12 + 2 * q] += Dgr * Sd[q].re;
           pv[13 + 2 * q] += Dgr * Sd[q].im;
-          pv[18 + 2 * q] += g * A[q].re;
-          pv[19 + 2 * q] += g * A[q].im;
-          pv[24 + 2 * q] += gr * S[q].re;
-          pv[25 + 2 * q] += gr * S[q].im;
-          pv[30 + 2 * q] += gr * Sd[q].re;
-          pv[31 + 2 * q] += gr * Sd[q].im;
+          pv[18 + 2 * q] += gr * Sd[q].re;
+          pv[19 + 2 * q] += gr * Sd[q].im;
+          pv[24 + q] += Dg * A[q].im;
+          pv[27 + q] += g * A[q].im;
         }
       }
     }
@@ -2087,19 +2131,16 @@ __global__ __launch_bounds__(256, 2) void hall_kernel(BandArgs b, double Tsmear,
     const int o = t - 64, i = o % 3, j = o / 3, c = i + j - 1;
     const zd wq = zd{wr, b.eta};
     const double B = 2.0 * wr * b.eta;
-    auto G = [&](int q) {  // sum of g v over the complex value q of A, S or S_ii
-      const double dr = R(NA + 2 * q), di = R(NA + 2 * q + 1);
-      const double br = B * R(NA + 18 + 2 * q), bi = B * R(NA + 19 + 2 * q);
-      return zd{dr - bi, di + br};
-    };
-    auto Gi = [&](int q) { return zd{R(NA + 2 * q + 1), B * R(NA + 19 + 2 * q)}; };  // g Im v
     zd av = zd{0.0, 0.0}, ao;
-    if (i == j) {
-      ao = zmuli(zmul(wq, G(6 + i)));
+    if (i == j) {  // i w sum g S_ii / dE
+      const zd gr = zd{R(NA + 12 + 2 * i), B * R(NA + 18 + 2 * i)};
+      const zd gi = zd{R(NA + 13 + 2 * i), B * R(NA + 19 + 2 * i)};
+      ao = zmuli(zmul(wq, zadd(gr, zmuli(gi))));
     } else {
-      const zd gi = Gi(c), iA = zmuli(G(c)), iwS = zmuli(zmul(wq, G(3 + c)));
+      const zd gi = zd{R(NA + 24 + c), B * R(NA + 27 + c)};  // sum g Im A
+      const int q = NA + 4 * c + (i < j ? 0 : 2);
       av = i < j ? zd{-gi.re, -gi.im} : gi;
-      ao = i < j ? zadd(iwS, iA) : zsub(iwS, iA);
+      ao = zmuli(zd{R(q), R(q + 1)});
     }
     out[L.velo + 2 * o] += av.re;
     out[L.velo + 2 * o + 1] += av.im;

@@ -37,3 +37,28 @@ def test_item_sums_match_oracle(n, n_hw, n_eF, pos, eta):
         # eigenvalues' 1e-15 by at most 1e9 where a gap meets a frequency
         # to that width, which these few points do to 1e-4 at the nearest
         assert np.max(np.abs(g[q] - ref[q])) < 1e-9 * np.max(np.abs(ref[q])), q
+
+
+@pytest.mark.parametrize("n,n_hw,jobs", [(4, 1, "hall"), (4, 3, "hall"), (24, 1, "hall"), (24, 1, "kubo"),
+                                         (20, 300, "hall"), (40, 1, "hall"), (40, 5, "hall")])
+def test_the_order_that_is_not_in_resonance(n, n_hw, jobs):
+    """General V with P_ij and P_ji of different sizes, at a resonance 1e-8 wide:
+    every element by itself.  One pair has a velocity, so an element holds the two
+    orders of that pair and nothing else."""
+    import oracle as O
+    from mepinterp_amd import capi, models
+    m = models.make_random(seed=n, n=n, L=1)
+    e, x, y, eta = 0.25 * np.arange(n), 1, 3, 1e-8
+    hw = np.linspace(0.5, 2.0, n_hw)  # the first one is the pair's gap
+    V = np.zeros((3, n, n), np.complex128, order="F")
+    V[:, y, x] = 1.0 + 0.3j, 1e-9 * (0.5 - 0.7j), 1e-4 * (0.2 + 1.1j)
+    V[:, x, y] = 1e-9 * (0.9 + 0.2j), 0.8 - 0.5j, 1e-5 * (1.0 + 0.6j)
+    fd = np.asfortranarray(np.linspace(0.9, 0.2, n)[None])
+    p = capi.Engine.params(jobs=capi.MEP_JOB_AHC | (capi.MEP_JOB_KUBO if jobs == "kubo" else 0),
+                           hw_lst=hw, eta=eta)
+    with capi.Engine(m["R_frac"], m["H"], a_latt=m["a_latt"]) as eng:
+        g = eng.bandsum(e, V[..., None], p, fd=fd)
+    ref = O.kubo_ohc_tens(e, V, hw, fd, eta).reshape(g["ohc"].shape, order="F")
+    assert np.all(ref != 0)
+    # about 30 roundings of 1.1e-16 on the way to an element
+    assert np.all(np.abs(g["ohc"] - ref) <= 4e-15 * np.abs(ref))
