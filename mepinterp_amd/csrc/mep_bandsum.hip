@@ -1346,8 +1346,11 @@ __global__ __launch_bounds__(256, 2) void bandsum_wide_kernel(BandArgs b, double
     }
     }
     // ---- itinerant (IC) terms on MFMA ----------------------------------------
-    // B_a(m, n0) = V_a(m, n0) r(m, n0), r(m, n0) = 1 / (E_n0 - E_m) (0 on the
-    // diagonal).  Hermitian V: formed in the step from conj V_a(n0, m), which
+    // B_a(m, n0) = V_a(m, n0) r(m, n0), r(m, n0) = 1 / (E_n0 - E_m), 0 for m = n0
+    // and for an m of exactly n0's energy, in the product and in the windows'
+    // terms alike: the Niu guards exclude such an m whatever n is, and the Kubo
+    // sum is not finite all the same, through its row m of the contraction.
+    // Hermitian V: formed in the step from conj V_a(n0, m), which
     // loads as one run of the 16 columns n0, so V is all that is read (a scaled
     // copy per workgroup doubled a working set that the caches miss as it is);
     // general V: scaled planes in the workgroup's slot of Bscr, transposed.
@@ -1370,7 +1373,7 @@ __global__ __launch_bounds__(256, 2) void bandsum_wide_kernel(BandArgs b, double
       if constexpr (!HERM) {
         for (int idx = t; idx < n2; idx += 256) {
           const int n0 = idx % n, m = idx / n;
-          const double rr = m == n0 ? 0.0 : rcp_nr(Es[n0] - Es[m]);
+          const double dE = Es[n0] - Es[m], rr = dE != 0.0 ? rcp_nr(dE) : 0.0;
 #pragma unroll
           for (int a = 0; a < 3; ++a)
             Bw[a * (int64_t)n2 + idx] = zscale(Vk[a * (int64_t)n2 + m + (int64_t)n * n0], rr);
@@ -1485,12 +1488,13 @@ __global__ __launch_bounds__(256, 2) void bandsum_wide_kernel(BandArgs b, double
           auto terms = [&](int from, int to) {
             for (int mm = from; mm < to; ++mm) {
               zd vm[3], bm[3];
-              const double rm = HERM ? (mm == n0 ? 0.0 : rcp_nr(Es[n0] - Es[mm])) : 1.0;
+              const double dm = Es[n0] - Es[mm];
+              const double rm = HERM ? (dm != 0.0 ? rcp_nr(dm) : 0.0) : 1.0;
 #pragma unroll
               for (int c = 0; c < 3; ++c) {
                 vm[c] = Vk[c * (int64_t)n2 + row + (int64_t)n * mm];
                 bm[c] = HERM ? zscale(zconj(Vk[c * (int64_t)n2 + n0 + (int64_t)n * mm]), rm)
-                             : Bw[c * (int64_t)n2 + n0 + (int64_t)n * mm];  // 0 for mm = n0
+                             : Bw[c * (int64_t)n2 + n0 + (int64_t)n * mm];
               }
 #pragma unroll
               for (int j = 0; j < 3; ++j) {

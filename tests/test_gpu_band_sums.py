@@ -133,3 +133,26 @@ def test_a_band_at_zero_energy(n):
         ref = f(e, V, np.array([0.03]), fd, 0.01).reshape(g[q].shape, order="F")
         # 1e-9, the sums' tolerance
         assert np.max(np.abs(g[q] - ref)) <= 1e-9 * np.max(np.abs(ref)), q
+
+
+@pytest.mark.parametrize("n", [33, 48, 70])
+def test_two_bands_of_the_same_energy(n):
+    """Above 32 bands: the Niu guards exclude the pair, the Kubo sums are not
+    finite (1 / 0 in the reference), and nothing else notices."""
+    import oracle as O
+    from mepinterp_amd import capi, models
+    tol, nv = 1e-5, n // 2
+    rng = np.random.default_rng(n)
+    e = 0.05 * np.arange(n)
+    e[4] = e[3]    # valence and valence
+    e[nv] = e[nv - 1]
+    V = np.asfortranarray(rng.standard_normal((3, n, n)) + 1j * rng.standard_normal((3, n, n)))
+    m = models.make_random(seed=n, n=n, L=1)
+    with capi.Engine(m["R_frac"], m["H"], a_latt=m["a_latt"], kubo_tol=tol) as eng:
+        g = eng.bandsum(e, V[..., None], capi.Engine.params(
+            jobs=capi.MEP_JOB_MEP | capi.MEP_JOB_KUBO, valence_bands=nv, eF_min=0.5, eF_max=0.5))
+    for q, f in (("niu_ic", O.mep_niu_ic), ("niu_lc", O.mep_niu_lc)):
+        ref = f(V, e, nv, tol)
+        # 1e-9, the sums' tolerance
+        assert np.max(np.abs(g[q] - ref)) <= 1e-9 * np.max(np.abs(ref)), q
+    assert not np.any(np.isfinite(g["kubo_ic"]))
