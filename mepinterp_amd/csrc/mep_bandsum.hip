@@ -75,10 +75,11 @@ struct BsLds {
                              (OM + 9) * NMAX + (size_t)total);
   }
 };
-// what the number of Fermi levels is limited by (above a few levels more than
-// the kernel takes): V and r, E and the occupations, per-band tables of 27 (45
-// with two row tiles) rows and one more, sums of 9 per level and tile, 96, the
-// record and two bytes per pair of bands
+// what the number of Fermi levels is limited by, where it is more than the kernel
+// takes (from a few levels on): V and r, E and the occupations, per-band tables
+// of 27 (45 with two row tiles) rows and one more, sums of 9 per level and tile,
+// 96, the record and two bytes per pair of bands.  A limit that callers know; the
+// kernel's own tables would admit more levels.
 static size_t bs_limit_bytes(int nmax, int nef, int64_t total) {
   const size_t pl = (size_t)nmax * (nmax + 1), nt = nmax / 16, m = nmax;
   return sizeof(zd) * 3 * pl + 2 * m * m +
@@ -949,13 +950,19 @@ static __device__ inline double rinv(const double* Es, int m, int c) {
   return (m == c) ? 0.0 : 1.0 / (Es[c] - Es[m]);  // 1 / (E_c - E_m)
 }
 
-// complex elements of a workgroup's slot: three scaled planes (general V) and 18
-// sums of 16 columns for each 16 x 16 tile (at most the eigensolver record of a k-point)
-__host__ __device__ inline int64_t wide_slot(int n) {
-  const int64_t nt = (n + 15) / 16;
-  return 3 * (int64_t)n * n + nt * nt * (18 * 16 / 2);
+// complex elements of a workgroup's slot: three scaled planes (general V only) and
+// 18 sums of 16 columns for each 16 x 16 tile (at most the eigensolver record of a
+// k-point)
+__host__ __device__ inline int64_t wide_planes(int n, bool herm) {
+  return herm ? 0 : 3 * (int64_t)n * n;
 }
-size_t bandsum_wide_scratch(int n, int nblocks) { return sizeof(zd) * (size_t)wide_slot(n) * nblocks; }
+__host__ __device__ inline int64_t wide_slot(int n, bool herm) {
+  const int64_t nt = (n + 15) / 16;
+  return wide_planes(n, herm) + nt * nt * (18 * 16 / 2);
+}
+size_t bandsum_wide_scratch(const BandArgs& b, int nblocks) {
+  return b.n > 32 ? sizeof(zd) * (size_t)wide_slot(b.n, b.v_herm) * nblocks : 0;
+}
 
 constexpr int BW_SLOTS = 21;  // per-band partial sums a thread leaves in LDS
 // lane group of 8 sums f over the bands and adds it to *dst (uniform call)
@@ -1368,8 +1375,8 @@ __global__ __launch_bounds__(256, 2) void bandsum_wide_kernel(BandArgs b, double
     if (doK || doNjob) {
       const int nt = (n + 15) / 16;
       const int lr = lane & 15, kq = lane >> 4;
-      zd* Bw = Bscr + (int64_t)blockIdx.x * wide_slot(n);
-      double* Pw = reinterpret_cast<double*>(Bw + 3 * (int64_t)n2);  // [item][18][16]
+      zd* Bw = Bscr + (int64_t)blockIdx.x * wide_slot(n, HERM);
+      double* Pw = reinterpret_cast<double*>(Bw + wide_planes(n, HERM));  // [item][18][16]
       if constexpr (!HERM) {
         for (int idx = t; idx < n2; idx += 256) {
           const int n0 = idx % n, m = idx / n;
@@ -2181,12 +2188,15 @@ static AccLayout lds_layout(const AccLayout& L, bool drop, int64_t* gap) {
   return S;
 }
 
+// the velo / ohc block is not the band-sum kernel's to fill
+static bool bs_drop(const BandArgs& b) { return hw_many(b) || !(b.jobs & MEP_JOB_AHC); }
+
 template <int NMAX, bool FUSED, bool HERM>
 static void launch_bs(hipStream_t s, const BandArgs& b, double Tsmear, const AccLayout& L,
                       int64_t nk, const double* E, const zd* V, const zd* A, const zd* Om,
                       const double* w, int nblocks, double* part, const VeloFuse* f) {
   int64_t gap;
-  const AccLayout S = lds_layout(L, hw_many(b) || !(b.jobs & MEP_JOB_AHC), &gap);
+  const AccLayout S = lds_layout(L, bs_drop(b), &gap);
   size_t lds = BsLds<NMAX, HERM>::bytes(b.n_ef, S.total);
   (void)hipFuncSetAttribute((const void*)bandsum_kernel<NMAX, FUSED, HERM>,
                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
@@ -2203,7 +2213,14 @@ size_t bandsum_lds_bytes(const BandArgs& b) {
   }
   int64_t gap;
   const AccLayout S = lds_layout(L, hw_many(b), &gap);
-  const size_t a = bs_limit_bytes(b.n <= 16 ? 16 : 32, b.n_ef, S.total);
+  size_t a = bs_limit_bytes(b.n <= 16 ? 16 : 32, b.n_ef, S.total);
+  // never less than launch_bs asks for
+  const AccLayout K = lds_layout(L, bs_drop(b), &gap);
+  const size_t k = b.n <= 16 ? (b.v_herm ? BsLds<16, true>::bytes(b.n_ef, K.total)
+                                         : BsLds<16, false>::bytes(b.n_ef, K.total))
+                             : (b.v_herm ? BsLds<32, true>::bytes(b.n_ef, K.total)
+                                         : BsLds<32, false>::bytes(b.n_ef, K.total));
+  if (k > a) a = k;
   const size_t h = hw_many(b) ? hwsum_lds_bytes(b) : 0;
   return a > h ? a : h;
 }

@@ -844,21 +844,21 @@ static int band_setup(mep_ctx* c, const mep_run_params* p, int64_t kblock, BandS
 // velocity kernel is not launched and V never reaches HBM)
 static int band_block(mep_ctx* c, BandSetup& bs, int64_t nb, const double* w, bool fuse = false) {
   int nblk = (int)(nb < bs.nblocks ? nb : bs.nblocks);
-  if (c->n > 32 && bandsum_wide_scratch((int)c->n, nblk) > eigh_scratch_bytes((int)c->n, c->kcap))
+  const size_t have = eigh_scratch_bytes((int)c->n, c->kcap);
+  if (bandsum_wide_scratch(bs.b, nblk) > have || (bs.ext && extsum_scratch(bs.b, nblk) > have))
     return fail(MEP_ERR_ARG, "band sums: the k-block is too small for the workgroups' slots");
   VeloFuse vf;
   vf.Hk = c->dHk;
   vf.strideHk = c->ncols;
   vf.U = c->dU;
   timed(c, K_BANDSUM, [&] {
-    // n > 32: the eigensolver records (consumed by now) hold the wide
-    // kernel's slots; nblk <= nb workgroups
+    // the eigensolver records (consumed by now) hold the kernels' slots, a slot
+    // at most as large as a k-point's record; nblk <= nb workgroups
     launch_bandsum(c->st, bs.b, nb, c->dE, c->dV, c->dA, c->dOm, w, nblk, c->dpart,
                    fuse ? &vf : nullptr, reinterpret_cast<zd*>(c->dscr));
     if (bs.ext)
       launch_extsum(c->st, bs.b, nb, c->dE, c->dV, c->dA, c->dOm, w, nblk,
-                    c->dpart + (int64_t)bs.nblocks * bs.L.total,
-                    c->n > 32 ? reinterpret_cast<zd*>(c->dscr) : nullptr);
+                    c->dpart + (int64_t)bs.nblocks * bs.L.total, reinterpret_cast<zd*>(c->dscr));
   });
   HIPCHK(hipGetLastError());
   return MEP_OK;

@@ -212,8 +212,8 @@ static bool photo_fast(const BandArgs& b) {
 // (3 x 128 complex) | fd (n_ef x n) | fd_stat_deriv (n_ef x n) | work area:
 // photo_2nd_cond here (n > 32): P (n^2 complex) where it fits, split sums
 // (XS_THREADS complex); kubo_opt_tens: pair records and split sums; get_gyro_Dw:
-// frequency-resolved curvatures.  The last two take what is left, up to
-// XS_WORK doubles.
+// frequency-resolved curvatures, one frequency at the least.  The last two take
+// what is left, up to XS_WORK doubles.
 constexpr size_t XS_WORK = 18 * XS_THREADS;
 __host__ __device__ inline size_t ext_base_doubles(int n, int nef, bool ldsv) {
   return (ldsv ? 2 * 3 * (size_t)XS_PL : 0) + 128 + 2 * 3 * 128 + 2 * (size_t)nef * n;
@@ -231,6 +231,7 @@ static size_t ext_work(const BandArgs& b, bool ldsv) {
   const size_t base = ext_base_doubles(b.n, b.n_ef, ldsv);
   size_t least = opt ? 2 * XS_THREADS : 0;
   if (opt && !photo_fast(b) && ext_photo_p(b.n, b.n_ef)) least += 2 * (size_t)b.n * b.n;
+  if ((b.jobs & MEP_JOB_GYRO) && b.pos_op && least < 3 * (size_t)b.n) least = 3 * (size_t)b.n;
   const size_t left = XS_LDS / sizeof(double) > base ? XS_LDS / sizeof(double) - base : 0;
   const size_t most = left < XS_WORK ? left : XS_WORK;
   return least > most ? least : most;
@@ -485,8 +486,8 @@ __global__ __launch_bounds__(XS_THREADS) void extsum_kernel(BandArgs b, double T
       }
       // get_curvTilde_hw (gyro.f90:271-300) of (band, hw), three components,
       // for as many frequencies as the work area holds, then the items
-      const int hc = nwork / (3 * n);
-      if (pos && hc > 0)
+      const int hc = nwork / (3 * n);  // at least 1 (ext_work)
+      if (pos)
         for (int h0 = 0; h0 < nhw; h0 += hc) {
           const int nh = nhw - h0 < hc ? nhw - h0 : hc;
           __syncthreads();
@@ -523,30 +524,6 @@ __global__ __launch_bounds__(XS_THREADS) void extsum_kernel(BandArgs b, double T
             rec[X.gyro_Dw + o + 1] += wk * dw.im;
           }
         }
-      if (pos && hc <= 0)  // occupation tables that leave no room
-        for (int it = t; it < 9 * nhw * nef; it += XS_THREADS) {
-          const int q = it % 9, h = (it / 9) % nhw, ef = it / (9 * nhw);
-          const int a = q % 3, bb = q / 3;
-          const double hwv = b.hw[h];
-          zd dw = zd{0.0, 0.0};
-          for (int nn = 0; nn < n; ++nn) {
-            // get_curvTilde_hw (gyro.f90:271-300), component bb
-            double omt = 0.0;
-            for (int m = 0; m < n; ++m) {
-              if (m == nn) continue;
-              const double ww = (Es[m] - Es[nn]) * (Es[m] - Es[nn]);
-              const int b1 = (bb + 1) % 3, b2 = (bb + 2) % 3;
-              const zd cr = zsub(zmul(Aat(k, b1, nn, m), Aat(k, b2, m, nn)),
-                                 zmul(Aat(k, b2, nn, m), Aat(k, b1, m, nn)));
-              omt -= cr.im * ww / (ww - hwv);
-            }
-            const zd va = Vat(a, nn, nn);
-            dw = zsub(dw, zscale(va, omt * fdd[ef + nef * nn]));
-          }
-          const int64_t o = 2 * (q + 9 * (h + (int64_t)nhw * ef));
-          rec[X.gyro_Dw + o] += wk * dw.re;
-          rec[X.gyro_Dw + o + 1] += wk * dw.im;
-        }
     }
   }
   if (doOpt && pos && npass == 1) opt_flush(0);
@@ -562,6 +539,11 @@ static bool ext_ldsv(const BandArgs& b) {
 size_t ext_lds_bytes(const BandArgs& b) {
   const bool ldsv = ext_ldsv(b);
   return sizeof(double) * (ext_base_doubles(b.n, b.n_ef, ldsv) + ext_work(b, ldsv));
+}
+
+size_t extsum_scratch(const BandArgs& b, int nblocks) {
+  const bool slots = (b.jobs & MEP_JOB_OPT) && !photo_fast(b) && !ext_photo_p(b.n, b.n_ef);
+  return slots ? sizeof(zd) * (size_t)b.n * b.n * nblocks : 0;
 }
 
 void launch_extsum(hipStream_t s, const BandArgs& b, int64_t nk, const double* E, const zd* V,

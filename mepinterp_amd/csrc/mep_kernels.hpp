@@ -135,9 +135,10 @@ struct VeloFuse {
   const zd* U;
 };
 bool bandsum_can_fuse(const BandArgs& b);
-// wide_scr (n > 32): bandsum_wide_scratch bytes, a slot per workgroup for the
-// columns of V scaled by 1 / (E_n0 - E_m) of the itinerant products and their sums
-size_t bandsum_wide_scratch(int n, int nblocks);
+// wide_scr: bandsum_wide_scratch bytes (none up to 32 bands), a slot per workgroup
+// for the sums of the itinerant products and, general V, the columns of V scaled
+// by 1 / (E_n0 - E_m)
+size_t bandsum_wide_scratch(const BandArgs& b, int nblocks);
 void launch_bandsum(hipStream_t s, const BandArgs& b, int64_t nk, const double* E, const zd* V,
                     const zd* A, const zd* Om, const double* w, int nblocks, double* part,
                     const VeloFuse* fuse = nullptr, zd* wide_scr = nullptr);
@@ -153,8 +154,9 @@ struct ExtLayout {
 ExtLayout ext_layout(const BandArgs& b);
 // dynamic LDS of the optical / gyrotropic kernel (must stay within 160 KiB)
 size_t ext_lds_bytes(const BandArgs& b);
-// scr: nblocks slots of n^2 complex (photo_2nd_cond's per-(b, c) product
-// where it does not fit in LDS), or null to keep the per-item loop there
+// scr: extsum_scratch bytes, nblocks slots of n^2 complex for photo_2nd_cond's
+// per-(b, c) product where that does not fit in LDS
+size_t extsum_scratch(const BandArgs& b, int nblocks);
 void launch_extsum(hipStream_t s, const BandArgs& b, int64_t nk, const double* E, const zd* V,
                    const zd* A, const zd* Om, const double* w, int nblocks, double* part,
                    zd* scr);

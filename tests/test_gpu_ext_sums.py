@@ -57,3 +57,23 @@ def test_ext_sums_at_the_edges_of_the_register_ql(n):
     for key in ("opt_s", "opt_a", "photo"):
         # 1e-9, the sums' tolerance
         assert np.max(np.abs(g[key] - o[key])) <= 1e-9 * np.max(np.abs(o[key])), key
+
+
+@pytest.mark.parametrize("n,most", [(16, 182), (32, 81), (33, 45)])
+def test_as_many_fermi_levels_as_the_tables_take(n, most):
+    import oracle as O
+    from mepinterp_amd import capi, models
+    m = models.make_random(seed=90 + n, n=n, L=1, with_r=True)
+    k = rand_kpts(2, seed=n)
+    width = 2.0 * np.max(np.sum(np.abs(m["H"]), axis=(1, 2)))  # above every gap: no pole near
+    kw = dict(eF_min=-0.05, eF_max=0.05, n_hw=1, hw_min=width, hw_max=width, T_kelvin=300.0,
+              eta=0.004, valence_bands=1)
+    jobs = capi.MEP_JOB_OPT | capi.MEP_JOB_GYRO
+    with capi.Engine(m["R_frac"], m["H"], r=m["r"], a_latt=m["a_latt"]) as eng:
+        g = eng.run_kpts(k, capi.Engine.params(jobs=jobs, n_eF=most, **kw))
+        with pytest.raises(capi.MepError):
+            eng.run_kpts(k, capi.Engine.params(jobs=jobs, n_eF=most + 1, **kw))
+    o = O.accumulate(oracle_model(m), O.RunParams(do_opt=True, do_gyro=True, n_eF=most, **kw), k)
+    for key in ("opt_s", "opt_a", "photo", "gyro_C", "gyro_D"):
+        # 1e-9, the sums' tolerance
+        assert np.max(np.abs(g[key] - o[key])) <= 1e-9 * np.max(np.abs(o[key])), key
