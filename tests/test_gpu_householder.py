@@ -28,3 +28,11 @@ def test_householder_variants_match_oracle(n, tb, variant):
         # FP64 on both sides; eigenvectors divide by gaps down to 1e-4 of the spectrum
         assert np.max(np.abs(e[:, ik] - eo)) < 1e-12 * np.max(np.abs(eo))
         assert np.max(np.abs(V[..., ik] - Vo)) < 1e-10 * np.max(np.abs(Vo))
+
+
+@pytest.mark.parametrize("n,tb", [(33, True), (35, False), (48, True), (49, False), (64, True), (65, False), (128, False)])
+@pytest.mark.parametrize("variant", [1, 2])
+def test_householder_in_lds_matches_oracle(n, tb, variant):
+    """The matrix in a workgroup's LDS (1) and in one wavefront's (2, which above
+    64 bands is 1)."""
+    test_householder_variants_match_oracle(n, tb, variant)

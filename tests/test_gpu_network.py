@@ -90,3 +90,31 @@ def test_training_chunks_of_a_data_set_after_a_larger_one():
     np.testing.assert_array_equal(out[0][0][0], out[1][0][0])
     # the Adam moments of the first calls differ, the fits do not by much
     assert np.linalg.norm(out[0][1] - out[1][1]) < 0.5 * np.linalg.norm(out[1][1])
+
+
+@pytest.mark.parametrize("n,epochs", [(700, 200), (1000, 131), (140000, 3)])
+def test_chunks_of_epochs_equal_single_epochs(n, epochs):
+    """Epoch e of a run with seed s is shuffled from s + (e + 1) times a constant,
+    so single-epoch calls whose seeds step by it see the same rows in the same
+    batches: the same bits, whichever part of the index buffers a chunk of epochs
+    went through (1, 2, 4, ... epochs, up to 131,072 points), and whether the
+    buffers were made for this data set or for a larger one."""
+    from mepinterp_amd import capi
+    rng = np.random.default_rng(n)
+    k = rng.uniform(-0.5, 0.5, size=(3, n))
+    t = rng.normal(size=n).astype(np.float32)
+    big = rng.uniform(-0.5, 0.5, size=(3, 200000))
+    kw = dict(batch=8192 if n > 8192 else 128, lr=1e-3)
+    out = []
+    for first in (False, True):
+        with capi.MLP(n_freq=2, hidden=32, seed=2) as net:
+            if first:
+                net.predict(big)
+            out.append((net.train(k, t, epochs=epochs, seed=1, **kw), net.params))
+    with capi.MLP(n_freq=2, hidden=32, seed=2) as net:
+        for e in range(epochs):
+            loss = net.train(k, t, epochs=1, seed=(1 + 0x9e3779b97f4a7c15 * e) % 2 ** 64, **kw)
+        out.append((loss, net.params))
+    for loss, p in out[1:]:
+        assert loss == out[0][0]
+        np.testing.assert_array_equal(p, out[0][1])
