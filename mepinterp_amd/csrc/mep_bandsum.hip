@@ -1635,7 +1635,7 @@ template <bool HERM>
 __host__ __device__ constexpr int hw_part() { return HERM ? 6 : 12; }
 
 template <bool HERM, int IPT>
-__global__ __launch_bounds__(256, 2) void hwsum_kernel(BandArgs b, double Tsmear, AccLayout L,
+__global__ __launch_bounds__(256, HERM ? 2 : 3) void hwsum_kernel(BandArgs b, double Tsmear, AccLayout L,
                                                        int64_t nk, const double* __restrict__ E,
                                                        const zd* __restrict__ V,
                                                        const double* __restrict__ w,
@@ -1872,14 +1872,15 @@ static int hwsum_ipt(const BandArgs& b) {
   return b.v_herm && (int64_t)b.n_hw * b.n_ef >= 8 ? 4 : 1;
 }
 
-// (the records' room is what the number of Fermi levels is limited by: 13 and
-// 28 doubles beside a record's levels)
-size_t hwsum_lds_bytes(const BandArgs& b) {
-  const size_t ps = (size_t)b.n_ef + (b.v_herm ? 13 : 28);
+// LDS of a record of `beside` doubles beside its Fermi levels
+static size_t hwsum_lds(const BandArgs& b, int beside) {
   const size_t red = 256 * 24;  // the split reduction: 24 doubles a thread at most
-  const size_t stage = (size_t)HW_CH * ps > red ? (size_t)HW_CH * ps : red;
-  return sizeof(double) * ((size_t)b.n + (size_t)b.n_ef * b.n + 4 + stage);
+  const size_t st = (size_t)HW_CH * (b.n_ef + beside);
+  return sizeof(double) * ((size_t)b.n + (size_t)b.n_ef * b.n + 4 + (st > red ? st : red));
 }
+// (13 and 28 doubles are what the number of Fermi levels is limited by.  General V
+// is launched with its own 22: 51 KB at three levels, three workgroups a CU.)
+size_t hwsum_lds_bytes(const BandArgs& b) { return hwsum_lds(b, b.v_herm ? 13 : 28); }
 
 // ===========================================================================
 // Per-k Berry curvature at one Fermi level: out[k][i + 3j] = the k-point's
@@ -2234,7 +2235,7 @@ bool bandsum_can_fuse(const BandArgs& b) {
 static void launch_hwsum(hipStream_t s, const BandArgs& b, double Tsmear, const AccLayout& L,
                          int64_t nk, const double* E, const zd* V, const double* w, int nblocks,
                          double* part) {
-  const size_t lh = hwsum_lds_bytes(b);
+  const size_t lh = b.v_herm ? hwsum_lds_bytes(b) : hwsum_lds(b, 1 + hw_vals<false>());
   auto go = [&](auto kernel) {
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lh);
