@@ -214,7 +214,12 @@ int mep_curv_batch(mep_ctx *ctx, int64_t nk, const double *kpts, double eF, doub
    log|Omega(k)| from a coarse mesh and ranks the cells to refine.  Training
    (mean squared error, Adam) and inference run in HIP kernels.
    Parameters: W1[6 n_freq padded to 16][hidden] b1 W2[hidden][hidden] b2
-   W3[hidden][hidden] b3 W4[hidden][16] b4[16] (column 0 is the output).    */
+   W3[hidden][hidden] b3 W4[hidden][16] b4[16] (column 0 is the output).
+   Device memory of a network: four times its parameters, the largest batch's
+   activations ((6 n_freq padded + 6 hidden) floats a row), up to 64 copies of
+   the parameters for the partial gradients of a batch (one per 64 rows: 10 MB at
+   128 units and 4,096 rows, 550 MB at 1,024), and the largest data set (48
+   bytes a point, at least 2 MB).                                           */
 typedef struct mep_mlp mep_mlp;
 int mep_mlp_create(int32_t n_freq, int32_t hidden, uint64_t seed, mep_mlp **mlp);
 int mep_mlp_destroy(mep_mlp *mlp);

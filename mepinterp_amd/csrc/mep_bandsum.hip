@@ -95,9 +95,9 @@ static size_t bs_limit_bytes(int nmax, int nef, int64_t total) {
 // to the two-kernel path).  n in 17..32, no position operator, Wannier
 // convention.
 //
-// Bound by issue: the FP64 MFMA products take 0.45 of the time at n = 32 and do
-// not overlap with the VALU work of the other phases, so what counts is the
-// instructions: one sum instead of two where the Niu guards exclude nothing
+// Bound by issue: at n = 32 the FP64 MFMA products take 0.52 of the SIMD-cycles and
+// do not overlap with the VALU work of the other phases (0.27; LDS 0.2 of the
+// CU-cycles), so what counts is the instructions: one sum instead of two where the Niu guards exclude nothing
 // (decided per k-point), per-k reductions scattered over the lanes or kept in
 // registers over all k-points, one weight per pair.
 // n = 32, 262,144 k-points, all tensors: 15.2 ms (17.6 before these); n = 20,
@@ -811,8 +811,8 @@ __global__ __launch_bounds__(BS_THREADS, 2) void bandsum_kernel(BandArgs b, doub
     __syncthreads();
     if constexpr (FUSED) fetch(k + gridDim.x);  // in flight during the sums below
     // ---- sums over the bands n0 and over the waves' partial records --------
-    // Ne, kubo_ahc_tens (-sum f Omega), kubo_mep_LC and kubo_mep_IC for every E_F
-    // for every E_F; item (c, ef) is summed by 8 lanes, lane g taking the
+    // Ne, kubo_ahc_tens (-sum f Omega), kubo_mep_LC and kubo_mep_IC for every E_F;
+    // item (c, ef) is summed by 8 lanes, lane g taking the
     // bands m0 = g, g + 8, ...
     // (Hermitian V: the three Berry sums are each two entries)
     constexpr int NO = S_::OM, NI = 1 + NO + 18;
@@ -965,7 +965,7 @@ size_t bandsum_wide_scratch(const BandArgs& b, int nblocks) {
 }
 
 constexpr int BW_SLOTS = 21;  // per-band partial sums a thread leaves in LDS
-// lane group of 8 sums f over the bands and adds it to *dst (uniform call)
+// lane group of 8 sums f over the bands and adds it to *dst (all 8 lanes call)
 static __device__ inline void band_item(int n, int nef, int ef, int g, bool valid, const double* fd,
                                         const double* src, double w, double* dst) {
   double s = 0.0;
@@ -1367,8 +1367,9 @@ __global__ __launch_bounds__(256, 2) void bandsum_wide_kernel(BandArgs b, double
     // operands they share in L1.  Two row tiles an item (9 operands for 36
     // products) spill, three wavefronts a SIMD too.  The contraction with
     // A_i(n0, n) = V_i(n0, n) r(n, n0)^2 comes straight from the accumulators;
-    // the items' sums go through the slot.  Bound by the operands' way from
-    // beyond L2 and by MFMA issue (0.5 of it).
+    // the items' sums go through the slot.  Bound by the operands' way from beyond
+    // L2 (n = 96: 9.9 GB at 4.0 TB/s; n = 44: 1.5 TB/s) and by issue (MFMA 0.45 and
+    // VALU 0.20 of the SIMD-cycles; 0.33 and 0.24), at two wavefronts a SIMD.
     // n = 96, 2,744 k-points: 2.5 ms (one C_j an item, V read three times: 5.6;
     // with scaled planes and tiles in row order 3.0); n = 44, 9,261: 1.48 ms
     // (3.0 with its velo / ohc kernel; 1.72).
@@ -1617,12 +1618,13 @@ size_t bandsum_wide_lds_bytes(const BandArgs& b) {
 // S_ii (3, complex), where both orders weigh the same value, and Im A (3) as
 // above.
 //
-// Bound by FP64 VALU issue: 2 x 9 fma and about 13 more a record and item
+// Bound by FP64 VALU issue (n = 96: 0.69 of the SIMD-cycles, n = 20: 0.61; general
+// V, with its few items, by latency): 2 x 9 fma and about 13 more a record and item
 // (Hermitian V); four items a thread take the reads of a record from LDS off
 // the LDS return path.
-// n = 96, 256 frequencies, 2,744 k-points: 2.8 ms (three denominators for the
+// n = 96, 256 frequencies, 2,744 k-points: 2.6 ms (three denominators for the
 // two orders, 24 sums an item: 4.2); n = 20, 80 items, 24,273: 0.50 ms (0.88);
-// general V, n = 14, 16 items, 2,730: 50 us (59 with a reciprocal for each
+// general V, n = 14, 16 items, 2,730: 45 us (59 with a reciprocal for each
 // weight and ordered pair; 40 with g alone, at the loss above: 7e-9 of an element
 // at eta = 1e-8, now 3e-16).
 // ===========================================================================
@@ -1867,7 +1869,7 @@ __global__ __launch_bounds__(256, HERM ? 2 : 3) void hwsum_kernel(BandArgs b, do
 // items per thread: four from eight items on (n = 96, 256 items: 2.8 ms, one
 // 3.1; n = 20, 80 items: 0.50, 0.51); general V's 30 sums an item leave no
 // registers for four, and two were slower (with 36 sums, n = 14, 16 items: 52
-// us, one 40)
+// us, one 40); one leaves room for three workgroups a CU
 static int hwsum_ipt(const BandArgs& b) {
   return b.v_herm && (int64_t)b.n_hw * b.n_ef >= 8 ? 4 : 1;
 }
@@ -2000,8 +2002,9 @@ __global__ __launch_bounds__(RP_COLS * RP_ROWS) void reduce_parts_kernel(
 //   ahc_ij = sum ((f_x + f_y) Im S_ij - (f_x - f_y) Im A_c) / dE^2   (ji: + A)
 // and the velo / ohc sums are hwsum_kernel's.  General V: nothing is assumed of
 // V(y, x).
-// Bound by the reads of V (at 8 bands, 32,768 k-points: 34 us; the band-sum
-// kernel, with three of its wavefronts waiting on the fourth's shuffles, 411).
+// Bound by the reads of V and by VALU issue (at 8 bands, 32,768 k-points: 31 us for
+// 100 MB, VALU 0.59 of the SIMD-cycles; the band-sum kernel, with three of its
+// wavefronts waiting on the fourth's shuffles, 411).
 // Several Fermi levels cost 9 sums each: from HALL_EF on, the band-sum kernel.
 // ===========================================================================
 constexpr int HALL_EF = 4, HALL_KB = 32;

@@ -1151,7 +1151,7 @@ __global__ __launch_bounds__(64) void eigh_sturm_kernel(
 }
 
 // The same for 32 < n <= 128: one workgroup of ceil(n / 64) wavefronts per
-// k-point.  n = 96, 2,744 k-points: 107 us (QL in LDS columns 5.8 ms); n = 44,
+// k-point.  n = 96, 2,744 k-points: 107 us (QL in LDS columns 6.4 ms); n = 44,
 // 9,261 k-points: 93 us (QL in registers 820 us).
 template <int WAVES>
 __global__ __launch_bounds__(64 * WAVES) void eigh_sturm_wide_kernel(
@@ -1992,9 +1992,10 @@ __device__ inline zd zsel(bool c, zd a, zd b) { return zd{c ? a.re : b.re, c ? a
 // buffers alternate between columns).  Same outputs as the other kernels.
 // The loops take CH or CU entries at a time, their LDS reads first, with zeros
 // past the end instead of a test per entry, and v's one corrected element (at
-// kc + 1) is selected in the two entries that can hold it: bound by the LDS
-// return path and the chain of sums at three wavefronts a SIMD.  n = 96, 2,744
-// k-points: 2.51 ms (one entry at a time, selects on each: 3.73); n = 52,
+// kc + 1) is selected in the two entries that can hold it.  Bound by FP64 VALU issue
+// up to 48 bands (0.75 of the SIMD-cycles at n = 44; LDS 0.3 of the CU-cycles), by
+// the chain of sums and barriers of each column above (n = 96: VALU 0.38, LDS 0.18,
+// 1.4 wavefronts a SIMD).  n = 96, 2,744 k-points: 2.47 ms (one entry at a time, selects on each: 3.73); n = 52,
 // 3,570: 0.62 ms (0.84).
 template <int NMAX>
 __global__ __launch_bounds__(4 * NMAX, NMAX <= 48 ? 4 : NMAX <= 96 ? 3 : 2) void eigh_house_rows_kernel(int n, int64_t nk,

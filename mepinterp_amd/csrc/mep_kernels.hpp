@@ -85,8 +85,7 @@ struct VeloArgs {
   int pos_op;
   int textbook;
   double kubo_tol;
-  zd* scratch;  // n > 32: 3 n x n per workgroup (up to 2048 workgroups); with a
-                // position operator 18 n x n per workgroup
+  zd* scratch;  // position operator and n > 32: 18 n x n per workgroup (up to 2048)
   size_t scratch_bytes = 0;
 };
 // the scratch holds at least one position-operator slot (or none is needed)

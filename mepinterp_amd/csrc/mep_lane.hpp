@@ -1,7 +1,8 @@
 // mep_lane.hpp -- cross-lane sums and broadcasts on the VALU: DPP row
 // patterns, the gfx950 permlane swaps and readlane (no LDS round trip).
 // Every function here reads other lanes, so the lanes it names must all be
-// active: call them from wave-uniform control flow only.
+// active: call them from wave-uniform control flow (group8_sum: where all lanes
+// of an aligned group of 8 go the same way).
 #pragma once
 #include "mep_common.hpp"
 

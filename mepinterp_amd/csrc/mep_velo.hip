@@ -311,8 +311,8 @@ __global__ __launch_bounds__(256) void velo_tb_kernel(int n, int64_t nk, zd* __r
 // 2.4 ms so against 1.9).
 // The wavefronts of one k-point follow each other on one XCD (workgroup index
 // mod 8), so that dH_a and U come from its L2 after the first.  Bound by the
-// operand loads: 0.55 (n = 44) and 0.46 (n = 96) of the MFMA issue at two
-// wavefronts a SIMD; three with spills took 1.2 and 2.6 ms, two columns a
+// operand loads: MFMA 0.57 (n = 44) and 0.46 (n = 96, where 12 GB come from beyond
+// L2 at 6.3 TB/s) of the SIMD-cycles at two wavefronts a SIMD; three with spills took 1.2 and 2.6 ms, two columns a
 // wavefront at one wavefront a SIMD 1.1 and 2.0.
 // n = 44, 9,261 k-points: 0.70 ms (U and one component at a time in LDS, T_a
 // through memory: 1.42); n = 96, 2,744: 1.92 ms (T_a through memory: 4.07).
