@@ -238,7 +238,7 @@ def main():
                                   "at most 3/4 of frac",
                     "mfma_issued_frac_bound": 0.75 * d["frac"],
                     "kernel": {"velo": "velo_mfma_kernel<zd>",
-                               "bandsum": "bandsum_kernel<32, %s>" % ("true" if fused else "false")}[dom],
+                               "bandsum": "bandsum_kernel<32, %s, true>" % ("true" if fused else "false")}[dom],
                     "launch_ms": d["launch_ms"], "stages": stages}
     out = host.finalize(sums, p, mp, m["a_latt"])
     # the mixed-precision path on the same mesh: throughput and error per
